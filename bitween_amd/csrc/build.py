@@ -1,6 +1,6 @@
 """Builds libbitween_hip.so (gfx950) next to its sources.
 
-    python -m bitween_amd.csrc.build            the library
+    python -m bitween_amd.csrc.build            the library and _bw_host.so, the package's native host path
     python -m bitween_amd.csrc.build --tune     also libbitween_hip_tune.so, the measurement build (see build)
 
 hipcc cross-compiles without a GPU.  The library is loaded by
@@ -14,6 +14,7 @@ HERE = os.path.dirname(os.path.abspath(__file__))
 SOURCES = ["bw_quantize.hip", "bw_qgemv.hip", "bw_qgemm.hip", "bw_qgemm_rows.hip", "bw_qdgrad.hip"]
 TUNE_SOURCES = ["bw_qgemm.hip", "bw_qgemm_rows.hip"]      # compiled a second time with -DBW_TUNE for the measurement build
 LIB = os.path.join(HERE, "libbitween_hip.so")
+HOST_SOURCE, HOST_LIB = os.path.join(HERE, "bw_host.cpp"), os.path.join(HERE, "_bw_host.so")
 FLAGS = [
     "--offload-arch=gfx950", "-O3", "-std=c++17", "-fPIC", "-shared",
     "-ffp-contract=off",                      # the quantiser's roundings must stay separate operations
@@ -32,6 +33,18 @@ def _run(cmd, verbose):
         raise RuntimeError(f"hipcc failed ({proc.returncode}):\n{err}")
     if verbose and err.strip():
         print(err, file=sys.stderr)
+
+
+def _host_command():
+    """The compiler's command line for _bw_host.so: a CPython extension over torch's C++ API (host code only; the kernel
+    library is reached through addresses handed over at run time, so nothing of it is linked)."""
+    import sysconfig
+    from torch.utils import cpp_extension
+    torch_lib = os.path.join(os.path.dirname(os.path.dirname(cpp_extension.__file__)), "lib")
+    includes = cpp_extension.include_paths("cuda") + [sysconfig.get_paths()["include"]]
+    return ([os.environ.get("CXX", "g++"), "-O2", "-std=c++17", "-fPIC", "-shared"] + cpp_extension.COMMON_HIP_FLAGS +
+            ["-isystem" + d for d in includes] + ["-o", HOST_LIB, HOST_SOURCE, "-L" + torch_lib] +
+            ["-l" + n for n in ("c10", "c10_hip", "torch_cpu", "torch_hip", "torch", "torch_python")])
 
 
 TUNE_LIB = os.path.join(HERE, "libbitween_hip_tune.so")
@@ -55,6 +68,7 @@ def build(verbose=False, tune=False):
     tune_objs = [os.path.join(objdir, s.replace(".hip", "_tune.o")) for s in TUNE_SOURCES]
     if tune:
         jobs += [[hipcc] + compile_flags + ["-DBW_TUNE", "-o", o, os.path.join(HERE, s)] for s, o in zip(TUNE_SOURCES, tune_objs)]
+    jobs.append(_host_command())
     with ThreadPoolExecutor(max_workers=min(len(jobs), os.cpu_count() or 1)) as pool:
         list(pool.map(lambda cmd: _run(cmd, verbose), jobs))
     _run([hipcc, "--offload-arch=gfx950", "-shared", "-fPIC", "-o", LIB] + objs, verbose)

@@ -1,0 +1,500 @@
+// Host path of the Python package in native code: from a module call to the launch without the interpreter in between.
+//
+// A decode kernel runs for 3 ... 12 us, so what a call costs on the host decides how fast eager code decodes.  The same
+// steps written in Python (views, checks, the output tensor, a ctypes call with sixteen arguments) took 8 ... 9 us a
+// call, and an autograd node written in Python about 50 us per forward + backward.  Here: a layer's buffers are validated
+// once into a Plan (kept in the module's __dict__, compared with the module's current buffers by identity and address on
+// every call), the output comes straight from the caching allocator, and the node that backward runs is a C++ node.
+//
+// The kernels are reached through function pointers of the C ABI (bind(), called once by hip_loader), so this file
+// neither links the kernel library nor knows where it lies.  Anything a function here does not take - CPU tensors,
+// tensor subclasses, buffers of another dtype or layout - it answers with None, and the Python code that it stands in
+// front of deals with the call and raises what has to be raised.
+#include <ATen/ATen.h>
+#include <ATen/hip/EmptyTensor.h>
+#include <c10/core/DeviceGuard.h>
+#include <c10/core/GradMode.h>
+#include <c10/hip/HIPFunctions.h>
+#include <c10/hip/HIPStream.h>
+#include <torch/csrc/autograd/function.h>
+#include <torch/csrc/autograd/functions/utils.h>
+#include <torch/csrc/autograd/python_variable.h>
+#include <torch/csrc/autograd/saved_variable.h>
+#include <torch/csrc/autograd/variable.h>
+
+#include "../../include/bitween_hip.h"
+
+namespace {
+
+using at::Tensor;
+
+struct Library {
+    decltype(&bw_qlinear) qlinear = nullptr;
+    decltype(&bw_qlinear_decode_rows) decode_rows = nullptr;
+    decltype(&bw_qgemm_ws) qgemm_ws = nullptr;
+    decltype(&bw_qgemm_workspace_bytes) qgemm_ws_bytes = nullptr;
+    decltype(&bw_cast_bf16_f16) cast = nullptr;
+    decltype(&bw_qdgrad) qdgrad = nullptr;
+    decltype(&bw_qdgrad_workspace_bytes) qdgrad_ws_bytes = nullptr;
+    decltype(&bw_qdgrad_tile_rows) qdgrad_tile_rows = nullptr;
+    decltype(&bw_quantize_pack_add) quantize = nullptr;
+    decltype(&bw_dequantize) dequantize = nullptr;
+} lib;
+
+PyObject* g_check = nullptr;          // Python: check(status, entry point's name) raises for a status other than 0
+int64_t g_fused_rows = 0, g_fused_large_rows = 0;
+
+PyObject *s_buffers, *s_qweight, *s_scale, *s_zero, *s_bias, *s_bits, *s_group, *s_plan;
+
+int dtype_code(at::ScalarType t) {
+    switch (t) {
+        case at::kHalf: return BW_F16;
+        case at::kBFloat16: return BW_BF16;
+        case at::kFloat: return BW_F32;
+        case at::kInt: return BW_I32;
+        case at::kDouble: return BW_F64;
+        default: return -1;
+    }
+}
+
+at::ScalarType dtype_of(int code) {
+    switch (code) {
+        case BW_F16: return at::kHalf;
+        case BW_BF16: return at::kBFloat16;
+        case BW_F32: return at::kFloat;
+        case BW_F64: return at::kDouble;
+        default: return at::kInt;
+    }
+}
+
+inline bool aligned16(const void* p) { return ((uintptr_t)p & 15) == 0; }
+
+inline Tensor empty(at::IntArrayRef sizes, at::ScalarType t, const at::Device& dev) {
+    return Tensor(at::detail::empty_cuda(sizes, t, dev, std::nullopt));
+}
+
+inline void* stream_of(at::DeviceIndex index) { return (void*)c10::hip::getCurrentHIPStream(index).stream(); }
+
+// The device of a call made current, only where it is not already.
+struct OnDevice {
+    std::optional<c10::DeviceGuard> guard;
+    explicit OnDevice(const at::Device& d) {
+        if (c10::hip::current_device() != d.index()) guard.emplace(d);
+    }
+};
+
+struct Layer {
+    const void *qweight, *scale, *zero, *bias;
+    int64_t n, k, decode_rows;
+    int bits, group;
+    at::DeviceIndex device;
+};
+
+// What the kernels ask of a layer's buffers; false = the general Python path has to look at them.
+bool layer_of(const Tensor& qweight, const Tensor& scale, const Tensor& zero, const Tensor* bias, int64_t bits, int64_t group, Layer& l) {
+    if (!lib.qlinear || (bits != 2 && bits != 4 && bits != 8) || group < 1) return false;
+    if (!qweight.is_cuda() || qweight.scalar_type() != at::kInt || qweight.dim() != 2 || !qweight.is_contiguous()) return false;
+    const int64_t n = qweight.size(0), k = qweight.size(1) * (32 / bits);
+    if (n < 1 || k < 1 || k % group) return false;
+    for (const Tensor* t : {&scale, &zero})
+        if (t->device() != qweight.device() || t->scalar_type() != at::kHalf || t->dim() != 2 || !t->is_contiguous() || t->size(0) != n ||
+            t->size(1) != k / group)
+            return false;
+    if (bias && (bias->device() != qweight.device() || bias->scalar_type() != at::kHalf || bias->dim() != 1 || bias->size(0) != n ||
+                 !bias->is_contiguous()))
+        return false;
+    l = {qweight.const_data_ptr(), scale.const_data_ptr(), zero.const_data_ptr(), bias ? bias->const_data_ptr() : nullptr,
+         n, k, lib.decode_rows(n, k, (int)bits), (int)bits, (int)group, qweight.device().index()};
+    return true;
+}
+
+// x.to(float16) of a bfloat16 matrix [m, k] with row pitch ldx: the library's streaming kernel where the layout qualifies.
+Tensor cast_to_f16(const Tensor& x, int64_t m, int64_t k, int64_t ldx, void* stream) {
+    if (k % 8 == 0 && ldx % 8 == 0 && aligned16(x.const_data_ptr())) {
+        Tensor y = empty({m, k}, at::kHalf, x.device());
+        if (lib.cast(x.const_data_ptr(), m, k, ldx, y.mutable_data_ptr(), k, stream) == BW_OK) return y;
+    }
+    return x.to(at::kHalf).contiguous();
+}
+
+// y = x W16^T (+ bias); the result keeps x's leading dimensions.  An undefined tensor with status 0 = not taken here.
+Tensor linear(const Layer& l, Tensor x, int& status, const char*& what) {
+    status = 0;
+    if (!x.is_cuda() || x.device().index() != l.device || x.dim() < 1 || x.size(-1) != l.k || x.numel() == 0) return {};
+    c10::SmallVector<int64_t, 5> shape(x.sizes().begin(), x.sizes().end());
+    shape.back() = l.n;
+    OnDevice on(x.device());
+    at::ScalarType t = x.scalar_type();
+    if (t != at::kHalf && t != at::kBFloat16) {
+        x = x.to(at::kHalf);
+        t = at::kHalf;
+    }
+    const int64_t m = x.numel() / l.k;
+    int64_t ldx = l.k;
+    if (!x.is_contiguous()) {
+        if (x.dim() != 2) x = x.reshape({m, l.k});
+        if (x.stride(1) == 1 && x.stride(0) >= l.k) ldx = x.stride(0);
+        else x = x.contiguous();
+    }
+    if ((ldx * 2) % 16 || !aligned16(x.const_data_ptr())) {
+        x = x.clone(at::MemoryFormat::Contiguous);
+        ldx = l.k;
+    }
+    void* stream = stream_of(l.device);
+    Tensor y = empty(shape, at::kHalf, x.device());
+    if (m <= l.decode_rows) {
+        what = "bw_qlinear";
+        const int act = t == at::kHalf ? BW_F16 : BW_BF16;
+        status = lib.qlinear(x.const_data_ptr(), act, m, l.k, ldx, (const int32_t*)l.qweight, l.scale, l.zero, l.bias, l.n, l.bits, l.group,
+                             y.mutable_data_ptr(), l.n, stream);
+        if (status == BW_EUNSUPPORTED && act == BW_BF16) {     // a shape only the generic kernel takes: float16 in memory
+            x = cast_to_f16(x, m, l.k, ldx, stream);
+            status = lib.qlinear(x.const_data_ptr(), BW_F16, m, l.k, l.k, (const int32_t*)l.qweight, l.scale, l.zero, l.bias, l.n, l.bits,
+                                 l.group, y.mutable_data_ptr(), l.n, stream);
+        }
+        return y;
+    }
+    what = "bw_qgemm_ws";
+    if (t == at::kBFloat16) {                                  // the prefill kernel wants float16 in memory
+        x = cast_to_f16(x, m, l.k, ldx, stream);
+        ldx = l.k;
+    }
+    const size_t bytes = lib.qgemm_ws_bytes(m, l.n, l.k, l.bits, l.group);
+    Tensor ws;
+    if (bytes) ws = empty({(int64_t)bytes}, at::kByte, x.device());
+    status = lib.qgemm_ws(x.const_data_ptr(), BW_F16, m, l.k, ldx, (const int32_t*)l.qweight, l.scale, l.zero, l.bias, l.n, l.bits, l.group,
+                          y.mutable_data_ptr(), l.n, bytes ? ws.mutable_data_ptr() : nullptr, bytes, stream);
+    return y;
+}
+
+// grad_x = grad_y @ W, W the dequantised weight in grad_y's dtype (bitween/modules.py:108-141).  float16 / bfloat16
+// gradients run the fused kernel - up to g_fused_rows rows always, up to g_fused_large_rows where the library plans its
+// 256 x 256 kernel - and dequantise + library GEMM beyond, which is faster there; so does a backward that is itself
+// recorded (create_graph).
+Tensor input_grad(const Tensor& go, const Tensor& qweight, const Tensor& scale, const Tensor& zero, int bits, int group) {
+    const int64_t n = qweight.size(0), k = qweight.size(1) * (32 / bits);
+    OnDevice on(go.device());
+    void* stream = stream_of(go.device().index());
+    const at::ScalarType t = go.scalar_type();
+    const int64_t m = go.numel() / n;
+    const bool recorded = c10::GradMode::is_enabled() && go.requires_grad();
+    if ((t == at::kHalf || t == at::kBFloat16) && !recorded && m > 0 &&
+        (m <= g_fused_rows || (m <= g_fused_large_rows && lib.qdgrad_tile_rows(m, n, k, bits, group) == 257))) {
+        Tensor g = go;
+        int64_t ldg = n;
+        if (!g.is_contiguous()) {
+            if (g.dim() != 2) g = g.reshape({m, n});
+            if (g.stride(1) == 1 && g.stride(0) >= n && g.stride(0) % 8 == 0) ldg = g.stride(0);
+            else g = g.contiguous();
+        }
+        if (!aligned16(g.const_data_ptr())) {
+            g = g.clone(at::MemoryFormat::Contiguous);
+            ldg = n;
+        }
+        if (ldg % 8 == 0) {
+            c10::SmallVector<int64_t, 5> shape(go.sizes().begin(), go.sizes().end());
+            shape.back() = k;
+            Tensor gx = empty(shape, t, go.device());
+            const size_t bytes = lib.qdgrad_ws_bytes(m, n, k, bits, group);
+            Tensor ws;
+            if (bytes) ws = empty({(int64_t)bytes}, at::kByte, go.device());
+            const int st = lib.qdgrad(g.const_data_ptr(), dtype_code(t), m, n, ldg, (const int32_t*)qweight.const_data_ptr(),
+                                      scale.const_data_ptr(), zero.const_data_ptr(), k, bits, group, gx.mutable_data_ptr(), k,
+                                      bytes ? ws.mutable_data_ptr() : nullptr, bytes, stream);
+            if (st == BW_OK) return gx;
+            TORCH_CHECK(st == BW_EUNSUPPORTED || st == BW_EALIGN, "bw_qdgrad failed (status ", st, ")");
+        }
+    }
+    // W = scale * (q - zp) in float32, cast to grad_output's dtype: the float32 product is exact, so dequantising straight
+    // to that dtype gives the same bits
+    const at::ScalarType wt = (t == at::kHalf || t == at::kBFloat16 || t == at::kFloat) ? t : at::kFloat;
+    Tensor w = empty({n, k}, wt, go.device());
+    const int st = lib.dequantize((const int32_t*)qweight.const_data_ptr(), scale.const_data_ptr(), BW_F16, zero.const_data_ptr(), BW_F16, n, k,
+                                  bits, group, w.mutable_data_ptr(), dtype_code(wt), k, stream);
+    TORCH_CHECK(st == BW_OK, "bw_dequantize failed (status ", st, ")");
+    return at::matmul(go, wt == t ? w : w.to(t));
+}
+
+struct QuantizedLinearBackward : public torch::autograd::Node {
+    torch::autograd::SavedVariable qweight, scale, zero;
+    int bits = 0, group = 0;
+    std::string name() const override { return "QuantizedLinearBackward"; }
+    void release_variables() override {
+        std::lock_guard<std::mutex> lock(mutex_);
+        qweight.reset_data();
+        scale.reset_data();
+        zero.reset_data();
+    }
+    torch::autograd::variable_list apply(torch::autograd::variable_list&& grads) override {
+        std::lock_guard<std::mutex> lock(mutex_);
+        if (!grads[0].defined() || !task_should_compute_output(0)) return {Tensor()};
+        const Tensor q = qweight.unpack(), s = scale.unpack(), z = zero.unpack();
+        return {input_grad(grads[0], q.contiguous(), s.contiguous(), z.contiguous(), bits, group)};
+    }
+};
+
+// ---- Python side ----
+
+struct Plan {
+    PyObject_HEAD
+    PyObject* tensor[4];              // qweight, scale, zero_point, bias (or None): the objects that were validated
+    const void* address[4];
+    Layer layer;
+    bool usable;                      // false: these buffers go through the general path
+};
+
+void plan_dealloc(PyObject* self) {
+    for (PyObject* t : ((Plan*)self)->tensor) Py_XDECREF(t);
+    Py_TYPE(self)->tp_free(self);
+}
+
+PyTypeObject PlanType = {PyVarObject_HEAD_INIT(nullptr, 0)};
+
+// A plain tensor or parameter; subclasses have their own ideas of every operation and go through Python.
+inline bool plain(PyObject* o) { return THPVariable_CheckExact(o); }
+inline const Tensor& unpack(PyObject* o) { return THPVariable_Unpack(o); }
+inline const void* address(PyObject* o) { return o == Py_None ? nullptr : unpack(o).unsafeGetTensorImpl()->data(); }
+
+PyObject* none() { Py_RETURN_NONE; }
+
+PyObject* checked(Tensor y, int status, const char* what) {
+    if (status == 0) return y.defined() ? THPVariable_Wrap(std::move(y)) : none();
+    PyObject* r = PyObject_CallFunction(g_check, "is", status, what);   // raises
+    Py_XDECREF(r);
+    if (!PyErr_Occurred()) PyErr_SetString(PyExc_RuntimeError, what);
+    return nullptr;
+}
+
+// The C++ exceptions of torch as Python ones.
+template <class F>
+PyObject* guarded(F&& f) {
+    HANDLE_TH_ERRORS
+    return f();
+    END_HANDLE_TH_ERRORS
+}
+
+// The layer's plan: the one the module keeps while its four buffers are the same objects at the same addresses (a buffer
+// replaced through .data, .set_(), a load or a move is seen whichever one it is), a new one otherwise.
+Plan* plan_of(PyObject* dict) {
+    PyObject* buffers = PyDict_GetItemWithError(dict, s_buffers);
+    if (!buffers || !PyDict_Check(buffers)) return nullptr;
+    PyObject* now[4] = {PyDict_GetItem(buffers, s_qweight), PyDict_GetItem(buffers, s_scale), PyDict_GetItem(buffers, s_zero),
+                        PyDict_GetItem(buffers, s_bias)};
+    if (!now[3]) now[3] = Py_None;
+    PyObject* kept = PyDict_GetItem(dict, s_plan);
+    if (kept && Py_TYPE(kept) == &PlanType) {
+        Plan* p = (Plan*)kept;
+        bool same = true;
+        for (int i = 0; i < 4; i++) same = same && p->tensor[i] == now[i];
+        for (int i = 0; same && i < 4; i++) same = p->address[i] == address(now[i]);
+        if (same) return p;
+    }
+    for (int i = 0; i < 4; i++)
+        if (!now[i] || !(plain(now[i]) || (i == 3 && now[i] == Py_None))) return nullptr;
+    PyObject *bits = PyDict_GetItem(dict, s_bits), *group = PyDict_GetItem(dict, s_group);
+    if (!bits || !group || !PyLong_Check(bits) || !PyLong_Check(group)) return nullptr;
+    Plan* p = PyObject_New(Plan, &PlanType);
+    if (!p) return nullptr;
+    for (int i = 0; i < 4; i++) {
+        Py_INCREF(now[i]);
+        p->tensor[i] = now[i];
+        p->address[i] = address(now[i]);
+    }
+    p->usable = layer_of(unpack(now[0]), unpack(now[1]), unpack(now[2]), now[3] == Py_None ? nullptr : &unpack(now[3]),
+                         PyLong_AsLong(bits), PyLong_AsLong(group), p->layer);
+    PyDict_SetItem(dict, s_plan, (PyObject*)p);
+    Py_DECREF(p);                                             // the module's dict holds it
+    return p;
+}
+
+// forward(module.__dict__, x) -> y or None
+PyObject* py_forward(PyObject*, PyObject* const* args, Py_ssize_t nargs) {
+    return guarded([&]() -> PyObject* {
+        if (nargs != 2 || !PyDict_Check(args[0]) || !plain(args[1])) return none();
+        const Tensor& x = unpack(args[1]);
+        if (!x.is_cuda()) return none();
+        Plan* p = plan_of(args[0]);
+        if (!p) {
+            if (PyErr_Occurred()) return nullptr;
+            return none();
+        }
+        if (!p->usable) return none();
+        int status = 0;
+        const char* what = "";
+        if (!(c10::GradMode::is_enabled() && x.requires_grad())) return checked(linear(p->layer, x, status, what), status, what);
+        Tensor y;
+        {
+            c10::AutoGradMode off(false);
+            y = linear(p->layer, x, status, what);
+        }
+        if (status == 0 && y.defined()) {
+            std::shared_ptr<QuantizedLinearBackward> node(new QuantizedLinearBackward(), torch::autograd::deleteNode);
+            node->set_next_edges(torch::autograd::collect_next_edges(x));
+            node->qweight = torch::autograd::SavedVariable(unpack(p->tensor[0]), false);
+            node->scale = torch::autograd::SavedVariable(unpack(p->tensor[1]), false);
+            node->zero = torch::autograd::SavedVariable(unpack(p->tensor[2]), false);
+            node->bits = p->layer.bits;
+            node->group = p->layer.group;
+            torch::autograd::set_history(y, node);
+        }
+        return checked(std::move(y), status, what);
+    });
+}
+
+// matmul(x, qweight, scale, zero_point, bias, bits, group_size) -> y or None
+PyObject* py_matmul(PyObject*, PyObject* const* args, Py_ssize_t nargs) {
+    return guarded([&]() -> PyObject* {
+        if (nargs != 7 || !PyLong_Check(args[5]) || !PyLong_Check(args[6])) return none();
+        for (int i = 0; i < 5; i++)
+            if (!plain(args[i]) && !(i == 4 && args[i] == Py_None)) return none();
+        const Tensor& x = unpack(args[0]);
+        if (x.scalar_type() != at::kHalf && x.scalar_type() != at::kBFloat16) return none();
+        Layer l;
+        if (!layer_of(unpack(args[1]), unpack(args[2]), unpack(args[3]), args[4] == Py_None ? nullptr : &unpack(args[4]),
+                      PyLong_AsLong(args[5]), PyLong_AsLong(args[6]), l))
+            return none();
+        int status = 0;
+        const char* what = "";
+        c10::AutoGradMode off(false);
+        Tensor y = linear(l, x, status, what);
+        return checked(std::move(y), status, what);
+    });
+}
+
+// input_grad(grad_output, qweight, scale, zero_point, bits, group_size) -> grad_input or None
+PyObject* py_input_grad(PyObject*, PyObject* const* args, Py_ssize_t nargs) {
+    return guarded([&]() -> PyObject* {
+        if (nargs != 6 || !PyLong_Check(args[4]) || !PyLong_Check(args[5])) return none();
+        for (int i = 0; i < 4; i++)
+            if (!plain(args[i])) return none();
+        const Tensor& go = unpack(args[0]);
+        Layer l;
+        if (!go.is_cuda() || !layer_of(unpack(args[1]), unpack(args[2]), unpack(args[3]), nullptr, PyLong_AsLong(args[4]), PyLong_AsLong(args[5]), l))
+            return none();
+        if (go.dim() < 1 || go.size(-1) != l.n || !go.is_floating_point() || go.device().index() != l.device) return none();
+        return THPVariable_Wrap(input_grad(go, unpack(args[1]), unpack(args[2]), unpack(args[3]), l.bits, l.group));
+    });
+}
+
+// quantize(weight, delta or None, bits, group_size, math code with flags, scale code, zero-point code) -> (qweight, scale, zero_point) or None
+PyObject* py_quantize(PyObject*, PyObject* const* args, Py_ssize_t nargs) {
+    return guarded([&]() -> PyObject* {
+        if (nargs != 7 || !plain(args[0]) || !(args[1] == Py_None || plain(args[1]))) return none();
+        c10::AutoGradMode off(false);
+        Tensor w = unpack(args[0]), delta;
+        const int64_t bits = PyLong_AsLong(args[2]), group = PyLong_AsLong(args[3]);
+        const int math = (int)PyLong_AsLong(args[4]), sc = (int)PyLong_AsLong(args[5]), zc = (int)PyLong_AsLong(args[6]);
+        if (PyErr_Occurred()) return nullptr;
+        const int code = dtype_code(w.scalar_type());
+        if (!lib.quantize || !w.is_cuda() || w.dim() != 2 || code < 0 || (bits != 2 && bits != 4 && bits != 8) || group < 1) return none();
+        if (w.stride(1) != 1) w = w.contiguous();
+        if (args[1] != Py_None) {
+            delta = unpack(args[1]);
+            if (delta.device() != w.device() || delta.sizes() != w.sizes() || delta.scalar_type() != w.scalar_type()) return none();
+            if (delta.stride(1) != 1) delta = delta.contiguous();
+        }
+        const int64_t n = w.size(0), k = w.size(1);
+        OnDevice on(w.device());
+        Tensor q = empty({n, k / (32 / bits)}, at::kInt, w.device());
+        Tensor s = empty({n, k / group}, dtype_of(sc), w.device()), z = empty({n, k / group}, dtype_of(zc), w.device());
+        const int st = lib.quantize(w.const_data_ptr(), delta.defined() ? delta.const_data_ptr() : nullptr, code, math, n, k, w.stride(0),
+                                    delta.defined() ? delta.stride(0) : 0, (int)bits, (int)group, (int32_t*)q.mutable_data_ptr(),
+                                    s.mutable_data_ptr(), sc, z.mutable_data_ptr(), zc, stream_of(w.device().index()));
+        if (st) return checked({}, st, "bw_quantize_pack");
+        PyObject* r = PyTuple_New(3);
+        if (!r) return nullptr;
+        PyTuple_SET_ITEM(r, 0, THPVariable_Wrap(std::move(q)));
+        PyTuple_SET_ITEM(r, 1, THPVariable_Wrap(std::move(s)));
+        PyTuple_SET_ITEM(r, 2, THPVariable_Wrap(std::move(z)));
+        return r;
+    });
+}
+
+// dequantize(qweight, scale, zero_point, group_size, bits, output code) -> weight or None
+PyObject* py_dequantize(PyObject*, PyObject* const* args, Py_ssize_t nargs) {
+    return guarded([&]() -> PyObject* {
+        if (nargs != 6 || !plain(args[0]) || !plain(args[1]) || !plain(args[2])) return none();
+        c10::AutoGradMode off(false);
+        const int64_t group = PyLong_AsLong(args[3]), bits = PyLong_AsLong(args[4]);
+        const int oc = (int)PyLong_AsLong(args[5]);
+        if (PyErr_Occurred()) return nullptr;
+        const Tensor q = unpack(args[0]).contiguous(), s = unpack(args[1]).contiguous(), z = unpack(args[2]).contiguous();
+        const int sc = dtype_code(s.scalar_type()), zc = dtype_code(z.scalar_type());
+        if (!lib.dequantize || !q.is_cuda() || s.device() != q.device() || z.device() != q.device() || q.scalar_type() != at::kInt || q.dim() != 2 ||
+            sc < 0 || zc < 0 || (bits != 2 && bits != 4 && bits != 8) || group < 1)
+            return none();
+        const int64_t n = q.size(0), k = q.size(1) * (32 / bits);
+        if (s.numel() < n * (k / group) || z.numel() < n * (k / group)) return none();
+        OnDevice on(q.device());
+        Tensor w = empty({n, k}, dtype_of(oc), q.device());
+        const int st = lib.dequantize((const int32_t*)q.const_data_ptr(), s.const_data_ptr(), sc, z.const_data_ptr(), zc, n, k, (int)bits, (int)group,
+                                      w.mutable_data_ptr(), oc, k, stream_of(q.device().index()));
+        return checked(std::move(w), st, "bw_dequantize");
+    });
+}
+
+// bind({entry point name: address}, check, fused rows, fused rows of the large kernel): once, after the kernel library is loaded
+PyObject* py_bind(PyObject*, PyObject* args) {
+    PyObject *table, *check;
+    long long rows, large;
+    if (!PyArg_ParseTuple(args, "O!OLL", &PyDict_Type, &table, &check, &rows, &large)) return nullptr;
+    bool ok = true;
+    auto get = [&](auto& fn, const char* name) {
+        PyObject* v = PyDict_GetItemString(table, name);
+        void* p = v ? PyLong_AsVoidPtr(v) : nullptr;
+        if (!p) ok = false;
+        fn = reinterpret_cast<std::decay_t<decltype(fn)>>(p);
+    };
+    Library l;
+    get(l.qlinear, "bw_qlinear");
+    get(l.decode_rows, "bw_qlinear_decode_rows");
+    get(l.qgemm_ws, "bw_qgemm_ws");
+    get(l.qgemm_ws_bytes, "bw_qgemm_workspace_bytes");
+    get(l.cast, "bw_cast_bf16_f16");
+    get(l.qdgrad, "bw_qdgrad");
+    get(l.qdgrad_ws_bytes, "bw_qdgrad_workspace_bytes");
+    get(l.qdgrad_tile_rows, "bw_qdgrad_tile_rows");
+    get(l.quantize, "bw_quantize_pack_add");
+    get(l.dequantize, "bw_dequantize");
+    if (PyErr_Occurred()) return nullptr;
+    if (!ok) {
+        PyErr_SetString(PyExc_RuntimeError, "bind: an entry point is missing");
+        return nullptr;
+    }
+    lib = l;
+    Py_INCREF(check);
+    Py_XSETREF(g_check, check);
+    g_fused_rows = rows;
+    g_fused_large_rows = large;
+    Py_RETURN_NONE;
+}
+
+PyMethodDef methods[] = {
+    {"bind", py_bind, METH_VARARGS, nullptr},
+    {"forward", (PyCFunction)(void*)py_forward, METH_FASTCALL, nullptr},
+    {"matmul", (PyCFunction)(void*)py_matmul, METH_FASTCALL, nullptr},
+    {"input_grad", (PyCFunction)(void*)py_input_grad, METH_FASTCALL, nullptr},
+    {"quantize", (PyCFunction)(void*)py_quantize, METH_FASTCALL, nullptr},
+    {"dequantize", (PyCFunction)(void*)py_dequantize, METH_FASTCALL, nullptr},
+    {nullptr, nullptr, 0, nullptr}};
+
+PyModuleDef module_def = {PyModuleDef_HEAD_INIT, "_bw_host", "Native host path of bitween_amd", -1, methods};
+
+}  // namespace
+
+PyMODINIT_FUNC PyInit__bw_host() {
+    PlanType.tp_name = "bitween_amd.Plan";
+    PlanType.tp_basicsize = sizeof(Plan);
+    PlanType.tp_flags = Py_TPFLAGS_DEFAULT;
+    PlanType.tp_dealloc = plan_dealloc;
+    if (PyType_Ready(&PlanType) < 0) return nullptr;
+    s_buffers = PyUnicode_InternFromString("_buffers");
+    s_qweight = PyUnicode_InternFromString("qweight");
+    s_scale = PyUnicode_InternFromString("scale");
+    s_zero = PyUnicode_InternFromString("zero_point");
+    s_bias = PyUnicode_InternFromString("bias");
+    s_bits = PyUnicode_InternFromString("bits");
+    s_group = PyUnicode_InternFromString("group_size");
+    s_plan = PyUnicode_InternFromString("_decode_plan");
+    return PyModule_Create(&module_def);
+}

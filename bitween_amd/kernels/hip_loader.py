@@ -8,6 +8,7 @@ bias, bits, group_size)` (main.py:433).
 There is no CPU path: a missing library or a missing GPU raises.
 """
 import ctypes
+import importlib.util
 import os
 
 import torch
@@ -83,6 +84,28 @@ def load():
 
 _ENTRY = {}
 
+_HOST_PATH = os.path.join(os.path.dirname(os.path.dirname(os.path.abspath(__file__))), "csrc", "_bw_host.so")
+_host = None
+
+FUSED_DGRAD_MAX_ROWS = 512       # measured on MI355X, Llama-shaped layers: the 128-row fused kernel wins up to here (3x at 128 rows)
+FUSED_DGRAD_LARGE_MAX_ROWS = 2048  # ... and the 256 x 256 kernel, where the library plans it (large layers), up to here
+
+
+def host():
+    """The native host path (csrc/bw_host.cpp) bound to the kernel library; both are loaded once."""
+    global _host
+    if _host is None:
+        lib = load()
+        if not os.path.exists(_HOST_PATH):
+            raise BitweenHipError(f"{_HOST_PATH} is missing: build it with `python -m bitween_amd.csrc.build`")
+        spec = importlib.util.spec_from_file_location("bitween_amd.csrc._bw_host", _HOST_PATH)
+        module = importlib.util.module_from_spec(spec)
+        spec.loader.exec_module(module)
+        table = {name: ctypes.cast(getattr(lib, name), ctypes.c_void_p).value for name in ENTRY_POINTS}
+        module.bind(table, _check, FUSED_DGRAD_MAX_ROWS, FUSED_DGRAD_LARGE_MAX_ROWS)
+        _host = module
+    return _host
+
 
 def _check(status, what):
     if status == 0:
@@ -99,53 +122,39 @@ def require_gpu(t, what):
                               "(bitween_amd has no CPU path)")
 
 
-def _stream(device):
-    return torch._C._cuda_getCurrentRawStream(device.index if device.index is not None else torch.cuda.current_device())
-
-
 def quantize_pack(weight, bits, group_size, math_dtype, scale_dtype, zp_dtype, delta=None, scale_reciprocal=False):
     """weight [N,K] on GPU (f16/bf16/f32, or f64 with f64 math and scale) -> (qweight int32, scale, zero_point) per bw_quantize_pack; with
     `delta` (same shape and dtype) the kernel quantises weight + delta (bw_quantize_pack_add).
     `scale_reciprocal`: the scale as eager torch forms it on a GPU (BW_SCALE_RECIPROCAL)."""
     require_gpu(weight, "quantize_pack")
-    if weight.stride(-1) != 1:
-        weight = weight.contiguous()
-    n, k = weight.shape
-    vpi = 32 // bits
-    dev = weight.device
     if delta is not None:
         require_gpu(delta, "quantize_pack")
         if delta.shape != weight.shape or delta.dtype != weight.dtype:
             raise ValueError("delta must have the shape and dtype of weight")
-        if delta.stride(-1) != 1:
-            delta = delta.contiguous()
-    qweight = torch.empty((n, k // vpi), dtype=torch.int32, device=dev)
-    scale = torch.empty((n, k // group_size), dtype=scale_dtype, device=dev)
-    zp = torch.empty((n, k // group_size), dtype=zp_dtype, device=dev)
-    with torch.cuda.device(dev):
-        st = load().bw_quantize_pack_add(weight.data_ptr(), None if delta is None else delta.data_ptr(),
-                                         _DTYPE_CODE[weight.dtype], _DTYPE_CODE[math_dtype] | (BW_SCALE_RECIPROCAL if scale_reciprocal else 0), n, k, weight.stride(0),
-                                         0 if delta is None else delta.stride(0), bits, group_size, qweight.data_ptr(),
-                                         scale.data_ptr(), _DTYPE_CODE[scale_dtype], zp.data_ptr(),
-                                         _DTYPE_CODE[zp_dtype], _stream(dev))
-    _check(st, "bw_quantize_pack")
-    return qweight, scale, zp
+    args = (bits, group_size, _DTYPE_CODE[math_dtype] | (BW_SCALE_RECIPROCAL if scale_reciprocal else 0), _DTYPE_CODE[scale_dtype],
+            _DTYPE_CODE[zp_dtype])
+    out = host().quantize(weight, delta, *args)
+    if out is None:                                        # a tensor subclass: the same call on the plain tensor underneath
+        out = host().quantize(_plain(weight), None if delta is None else _plain(delta), *args)
+    if out is None:
+        raise TypeError(f"quantize_pack does not take a {weight.dim()}-D {weight.dtype} weight")
+    return out
 
 
 def dequantize(qweight, scale, zero_point, group_size, bits, out_dtype):
     """(qweight, scale f32|f16, zero_point i32|f16) on GPU -> weight [N,K] of out_dtype per bw_dequantize; a float64
     scale goes with out_dtype float64."""
     require_gpu(qweight, "dequantize")
-    qweight, scale, zero_point = qweight.contiguous(), scale.contiguous(), zero_point.contiguous()
-    n, words = qweight.shape
-    k = words * (32 // bits)
-    out = torch.empty((n, k), dtype=out_dtype, device=qweight.device)
-    with torch.cuda.device(qweight.device):
-        st = load().bw_dequantize(qweight.data_ptr(), scale.data_ptr(), _DTYPE_CODE[scale.dtype], zero_point.data_ptr(),
-                                  _DTYPE_CODE[zero_point.dtype], n, k, bits, group_size, out.data_ptr(),
-                                  _DTYPE_CODE[out_dtype], k, _stream(qweight.device))
-    _check(st, "bw_dequantize")
+    out = host().dequantize(qweight, scale, zero_point, group_size, bits, _DTYPE_CODE[out_dtype])
+    if out is None:
+        out = host().dequantize(_plain(qweight), _plain(scale), _plain(zero_point), group_size, bits, _DTYPE_CODE[out_dtype])
+    if out is None:
+        raise TypeError("dequantize needs int32 packed weights [N, words] with scale / zero_point of N * (K // group_size) values on the same GPU")
     return out
+
+
+def _plain(t):
+    return t.detach().as_subclass(torch.Tensor)
 
 
 def _raw_stream(index):
@@ -260,64 +269,11 @@ def _matmul(entry, x, qweight, scale, zero_point, bias, bits, group_size):
     return y
 
 
-def make_decode_plan(qweight, scale, zero_point, bias, bits, group_size):
-    """Validate a layer's buffers once for decode_with_plan: returns a tuple holding the tensors (so that the
-    caller can tell by identity whether they are still the ones validated), their device addresses and the
-    layer's sizes - or None when the buffers do not qualify and the general path has to look at them."""
-    if not qweight.is_cuda or qweight.dtype is not torch.int32 or scale.dtype is not torch.float16 or \
-            zero_point.dtype is not torch.float16 or (bias is not None and bias.dtype is not torch.float16):
-        return None
-    if not (qweight.is_contiguous() and scale.is_contiguous() and zero_point.is_contiguous()) or \
-            (bias is not None and not bias.is_contiguous()):
-        return None
-    n, words = qweight.shape
-    k = words * (32 // bits)
-    if k % group_size or scale.shape != (n, k // group_size) or zero_point.shape != scale.shape or \
-            (bias is not None and bias.shape != (n,)):
-        return None
-    load()
-    index = qweight.device.index if qweight.device.index is not None else torch.cuda.current_device()
-    return (qweight, scale, zero_point, bias, qweight.data_ptr(), scale.data_ptr(), zero_point.data_ptr(),
-            None if bias is None else bias.data_ptr(), n, k, bits, group_size, index,
-            load().bw_qlinear_decode_rows(n, k, bits))
-
-
-def decode_with_plan(plan, x, m):
-    """bw_qlinear on its decode path with buffers validated by make_decode_plan: only x is looked at.  Returns None
-    when x does not qualify (layout, device, dtype, more rows than the decode path takes for this layer) - the
-    caller then takes quantized_matmul_hip."""
-    if m > plan[13]:
-        return None
-    dt = x.dtype
-    if dt is torch.float16:
-        act = BW_F16
-    elif dt is torch.bfloat16:
-        act = BW_BF16
-    else:
-        return None
-    ldx = x.stride(0)
-    xp = x.data_ptr()
-    index = plan[12]
-    if not x.is_cuda or x.stride(1) != 1 or (ldx * 2) % 16 or xp % 16 or x.shape[1] != plan[9] or \
-            torch.cuda.current_device() != index:
-        return None
-    n = plan[8]
-    y = torch.empty((m, n), dtype=torch.float16, device=x.device)
-    st = _ENTRY["bw_qlinear"](xp, act, m, plan[9], ldx, plan[4], plan[5], plan[6], plan[7], n, plan[10], plan[11],
-                              y.data_ptr(), n, _raw_stream(index))
-    if st:
-        if st == -2:
-            return None
-        _check(st, "bw_qlinear")
-    return y
-
-
-def input_grad_prefers_fused(m, n, k, bits, group_size, max_rows, large_max_rows):
-    """Whether the backward should take the fused kernel for an m-row gradient: up to `max_rows` rows always (the
-    kernel that walks N in steps of 32 rows); up to `large_max_rows` where the library's plan is its 256 x 256 kernel,
-    which beats dequantise + library GEMM there (measured on Llama-shaped layers: 0.45-1.0 of its time up to 2048
-    rows, 1.0-1.13 at 4096)."""
-    return m <= max_rows or (m <= large_max_rows and load().bw_qdgrad_tile_rows(m, n, k, bits, group_size) == 257)
+def input_grad(grad_output, qweight, scale, zero_point, bits, group_size):
+    """grad_output [..., N] @ W -> [..., K] in grad_output's dtype: the fused kernel (bw_qdgrad) for float16 / bfloat16 gradients of
+    up to FUSED_DGRAD_MAX_ROWS rows, and of up to FUSED_DGRAD_LARGE_MAX_ROWS where the library plans its 256 x 256 kernel;
+    dequantise + library GEMM otherwise.  None for buffers that are not the contiguous ones a QuantizedLinear keeps."""
+    return host().input_grad(grad_output, qweight, scale, zero_point, bits, group_size)
 
 
 def quantized_input_grad(grad_y, qweight, scale, zero_point, bits, group_size):
@@ -360,6 +316,10 @@ def last_decode_kernel():
 
 def quantized_matmul_hip(x, qweight, scale, zero_point, bias, bits, group_size):
     """y[M,N] = x[M,K] @ dequant(qweight, scale, zero_point)^T + bias, float16 (main.py:433's operator)."""
+    if x.dim() == 2:
+        y = host().matmul(x, qweight, scale, zero_point, bias, bits, group_size)
+        if y is not None:
+            return y
     return _matmul("bw_qlinear", x, qweight, scale, zero_point, bias, bits, group_size)
 
 

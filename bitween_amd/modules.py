@@ -13,8 +13,11 @@ from . import functional as _functional
 from .kernels import hip_loader as _hip
 
 
-FUSED_DGRAD_MAX_ROWS = 512       # measured on MI355X, Llama-shaped layers: the 128-row fused kernel wins up to here (3x at 128 rows)
-FUSED_DGRAD_LARGE_MAX_ROWS = 2048  # ... and the 256 x 256 kernel, where the library plans it (large layers), up to here
+def _host_forward(fields, x):
+    """First call: loads the native host path and puts its forward(module.__dict__, x) in this function's place."""
+    global _host_forward
+    _host_forward = _hip.host().forward
+    return _host_forward(fields, x)
 
 
 class QuantizedLinearFunction(torch.autograd.Function):
@@ -38,15 +41,9 @@ class QuantizedLinearFunction(torch.autograd.Function):
         x, qweight, scale, zero_point, bias = ctx.saved_tensors
         grad_input = None
         if ctx.needs_input_grad[0]:
-            # float16 / bfloat16 gradients: one fused kernel, the weights are never materialised - up to
-            # FUSED_DGRAD_MAX_ROWS rows always, up to FUSED_DGRAD_LARGE_MAX_ROWS where the library runs its 256 x 256
-            # kernel (large layers); otherwise the library GEMM on dequantised weights is faster.
-            go2 = grad_output.reshape(-1, grad_output.shape[-1])
-            if grad_output.dtype in (torch.float16, torch.bfloat16) and grad_output.is_cuda and _hip.input_grad_prefers_fused(
-                    go2.shape[0], qweight.shape[0], x.shape[-1], ctx.bits, ctx.group_size, FUSED_DGRAD_MAX_ROWS, FUSED_DGRAD_LARGE_MAX_ROWS):
-                gx = _hip.quantized_input_grad(go2, qweight, scale, zero_point, ctx.bits, ctx.group_size)
-                if gx is not None:
-                    return gx.view(*grad_output.shape[:-1], gx.shape[-1]), None, None, None, None, None, None
+            grad_input = _hip.input_grad(grad_output, qweight, scale, zero_point, ctx.bits, ctx.group_size)
+            if grad_input is not None:
+                return grad_input, None, None, None, None, None, None
             # W = scale * (q - zp) in float32, cast to grad_output.dtype: the float32 product is exact,
             # so dequantising straight to that dtype gives the same bits.
             gdt = grad_output.dtype if grad_output.dtype in (torch.float16, torch.bfloat16, torch.float32) else torch.float32
@@ -85,34 +82,22 @@ class QuantizedLinear(nn.Module):
             self.bias = None
 
     def forward(self, x):
-        if x.requires_grad and torch.is_grad_enabled():
-            return QuantizedLinearFunction.apply(x, self.qweight, self.scale, self.zero_point, self.bias, self.bits,
-                                                 self.group_size)
-        group = self.__dict__.get("_sibling_group")
-        if group is not None:
+        fields = self.__dict__
+        group = fields.get("_sibling_group")
+        if group is not None and not (x.requires_grad and torch.is_grad_enabled()):
             y = group.forward(self, x)
             if y is not None:
                 return y
-        # nothing to differentiate (the buffers never require grad): same arithmetic without the autograd node
+        # The native path: the buffers were validated once and are looked at again only when one of them has been replaced
+        # (module.to(), load with assign, sibling fusion) or moved; records its own autograd node where x asks for one.
+        y = _host_forward(fields, x)
+        if y is not None:
+            return y
+        if x.requires_grad and torch.is_grad_enabled():
+            return QuantizedLinearFunction.apply(x, self.qweight, self.scale, self.zero_point, self.bias, self.bits,
+                                                 self.group_size)
         shape = x.shape
         x2 = x.reshape(-1, shape[-1])
-        m = x2.shape[0]
-        if 0 < m <= 48:
-            # decode: the buffers were validated once; they are looked at again only when one of them has been
-            # replaced (module.to(), load with assign, sibling fusion) or moved
-            plan = self.__dict__.get("_decode_plan")
-            b = self._buffers
-            if plan is None or plan[0] is not b["qweight"] or plan[1] is not b["scale"] or \
-                    plan[2] is not b["zero_point"] or plan[3] is not b.get("bias") or plan[4] != plan[0].data_ptr() or \
-                    plan[5] != plan[1].data_ptr() or plan[6] != plan[2].data_ptr() or \
-                    (plan[3] is not None and plan[7] != plan[3].data_ptr()):
-                plan = _hip.make_decode_plan(b["qweight"], b["scale"], b["zero_point"], b.get("bias"), self.bits,
-                                             self.group_size) if b["qweight"].is_cuda else None
-                self.__dict__["_decode_plan"] = plan
-            if plan is not None:
-                y = _hip.decode_with_plan(plan, x2, m)
-                if y is not None:
-                    return y.view(*shape[:-1], self.out_features)
         if x2.dtype is not torch.float16 and x2.dtype is not torch.bfloat16:    # bfloat16 is converted by the kernel
             x2 = x2.to(torch.float16)
         y = _hip.quantized_matmul_hip(x2, self.qweight, self.scale, self.zero_point, self.bias, self.bits, self.group_size)
@@ -144,19 +129,27 @@ class QuantizedLinear(nn.Module):
         qweight, scale, zero_point = _hip.quantize_pack(weight, bits, group_size, math_dtype=torch.float32,
                                                         scale_dtype=torch.float16, zp_dtype=torch.float16,
                                                         scale_reciprocal=_functional.scale_reciprocal_for(float_layer.weight))
-        # the constructor's zero buffers are built on the meta device (no memory, no host-to-device copy) and
-        # replaced by the kernel's outputs, which already have the buffers' shapes and dtypes
-        with torch.device("meta"):
-            q_layer = cls(float_layer.in_features, float_layer.out_features, bits, group_size,
-                          bias=float_layer.bias is not None, dtype=torch.float16)
-        new = {"qweight": qweight, "scale": scale, "zero_point": zero_point}
+        if qweight.shape[0] != float_layer.out_features or weight.shape[1] != float_layer.in_features:
+            raise BitweenShapeError(f"the layer declares {float_layer.out_features} x {float_layer.in_features}, its weight is {tuple(weight.shape)}")
+        buffers = {"qweight": qweight, "scale": scale, "zero_point": zero_point}
         if float_layer.bias is not None:
-            new["bias"] = float_layer.bias.data.to(device="cuda", dtype=torch.float16, copy=True)
-        for name, value in new.items():
-            if value.shape != q_layer._buffers[name].shape or value.dtype != q_layer._buffers[name].dtype:
-                raise BitweenShapeError(f"{name}: kernel produced {tuple(value.shape)} {value.dtype}, the module "
-                                        f"declares {tuple(q_layer._buffers[name].shape)} {q_layer._buffers[name].dtype}")
-            q_layer._buffers[name] = value if device.type == "cuda" else value.to(device)
+            buffers["bias"] = float_layer.bias.data.to(device="cuda", dtype=torch.float16, copy=True)
+        if device.type != "cuda":
+            buffers = {name: value.to(device) for name, value in buffers.items()}
+        if cls.__init__ is not QuantizedLinear.__init__:   # a subclass with a constructor of its own
+            with torch.device("meta"):                     # its zero buffers without memory; the kernel's outputs take their place
+                q_layer = cls(float_layer.in_features, float_layer.out_features, bits, group_size,
+                              bias=float_layer.bias is not None, dtype=torch.float16)
+        else:
+            # what the constructor does, without zero buffers to throw away and without nn.Module's attribute hooks
+            # (30 us of a call whose kernel runs for 10 ... 25)
+            q_layer = cls.__new__(cls)
+            nn.Module.__init__(q_layer)
+            q_layer.__dict__.update(in_features=float_layer.in_features, out_features=float_layer.out_features, bits=bits,
+                                    group_size=group_size, requires_grad=False, dtype=torch.float16)
+            if float_layer.bias is None:
+                q_layer.__dict__["bias"] = None
+        q_layer._buffers.update(buffers)
         return q_layer
 
     def __repr__(self):

@@ -1,0 +1,109 @@
+"""The native host path (csrc/bw_host.cpp) against the C ABI call it stands for: every layout, dtype and leading shape of x that
+the module forward accepts, the autograd node, and the calls it leaves to the general path."""
+import pytest
+import torch
+
+pytestmark = pytest.mark.gpu
+
+
+def _layer(k, n, bits, g, bias=True, seed=0):
+    from bitween_amd import QuantizedLinear
+    torch.manual_seed(seed)
+    return QuantizedLinear.from_float(torch.nn.Linear(k, n, bias=bias, device="cuda", dtype=torch.float16), bits, g)
+
+
+def _w16(q):
+    from bitween_amd.kernels import hip_loader as hip
+    return hip.dequantize(q.qweight, q.scale, q.zero_point, q.group_size, q.bits, torch.float16)
+
+
+def _close(y, x16, q):
+    """2^-10 of the value (two float16 roundings) and float32 accumulation on sum |x| |w|, as the sweep's bound."""
+    w = _w16(q).double()
+    x64 = x16.double()
+    ref = x64 @ w.T + (0 if q.bias is None else q.bias.double())
+    return ((y.double() - ref).abs() <= 2.0 ** -10 * ref.abs() + 2.0 ** -12 * (x64.abs() @ w.abs().T) + 1e-6).all()
+
+
+@pytest.mark.parametrize("dtype", [torch.float16, torch.bfloat16, torch.float32])
+@pytest.mark.parametrize("rows", [1, 16, 17, 49, 130])         # one decode launch, two, and the prefill kernel
+def test_layouts_of_x(dtype, rows):
+    q = _layer(256, 97, 4, 64)
+    base = torch.randn(rows, 3, 2 * 256 + 8, device="cuda").to(dtype)
+    views = [base[:, 0, :256],                                  # padded rows
+             base[:, :, 8:264],                                 # 3-D, padded
+             base[:, 1, 4:260],                                 # rows that start off a 16-byte boundary
+             base[:, 2, :512:2],                                # strided columns
+             base[:1, 0, :256].expand(rows, 256),               # one row repeated
+             base[:, 0, :256].contiguous().view(1, rows, 1, 256)]
+    for x in views:
+        y = q(x)
+        assert y.shape == x.shape[:-1] + (97,) and y.dtype is torch.float16
+        assert _close(y.reshape(-1, 97), x.reshape(-1, 256).to(torch.float16), q)
+    assert q(base[:0, 0, :256]).shape == (0, 97)                # no rows: the general path
+
+
+@pytest.mark.parametrize("bits,g,k,n", [(4, 128, 256, 96), (4, 64, 192, 61), (8, 32, 128, 33)])
+@pytest.mark.parametrize("dtype", [torch.float16, torch.bfloat16, torch.float32])
+def test_gradient_matches_the_autograd_function(bits, g, k, n, dtype):
+    """module(x).backward against QuantizedLinearFunction (the Python node with the reference's interface): same kernels, same bits."""
+    from bitween_amd import QuantizedLinearFunction
+    q = _layer(k, n, bits, g, seed=n)
+    x = torch.randn(2, 5, k, device="cuda").to(dtype).requires_grad_(True)
+    x2 = x.detach().clone().requires_grad_(True)
+    y, y2 = q(x), QuantizedLinearFunction.apply(x2, q.qweight, q.scale, q.zero_point, q.bias, q.bits, q.group_size)
+    assert torch.equal(y, y2) and y.requires_grad
+    go = torch.randn_like(y)
+    y.backward(go)
+    y2.backward(go)
+    assert x.grad.dtype is dtype and torch.equal(x.grad, x2.grad)
+    with pytest.raises(RuntimeError):                           # the node's buffers are released
+        y.backward(go)
+    with torch.no_grad():
+        assert not q(x).requires_grad
+
+
+def test_gradient_of_a_recorded_backward_and_of_a_changed_layer():
+    q = _layer(128, 64, 4, 64)
+    x = torch.randn(3, 128, device="cuda", dtype=torch.float16, requires_grad=True)
+    go = torch.randn(3, 64, device="cuda", dtype=torch.float16, requires_grad=True)
+    gx, = torch.autograd.grad(q(x), x, go, create_graph=True)
+    v = torch.randn_like(gx)
+    gg, = torch.autograd.grad(gx, go, v)                        # d(go W)/d(go) applied to v = v W^T
+    ref = v.float() @ _w16(q).float().T
+    assert (gg.float() - ref).abs().max() <= 2.0 ** -9 * ref.abs().max()
+    y = q(x)
+    q.scale.mul_(2.0)                                           # the weights of a recorded forward changed in place
+    with pytest.raises(RuntimeError, match="modified by an inplace"):
+        y.sum().backward()
+
+
+def test_subclasses_and_parameters_as_inputs():
+    class Sub(torch.Tensor):
+        pass
+
+    q = _layer(128, 64, 4, 64)
+    x = torch.randn(3, 128, device="cuda", dtype=torch.float16)
+    want = q(x)
+    assert torch.equal(q(x.as_subclass(Sub)).as_subclass(torch.Tensor), want)
+    assert torch.equal(q(torch.nn.Parameter(x)), want)
+    with torch.inference_mode():
+        y = q(x)
+    assert y.is_inference() and torch.equal(y, want)
+
+
+def test_quantize_copies_what_it_does_not_replace():
+    """The copy that Bitween.quantize returns shares nothing with the model: containers, hooks, plain attributes."""
+    import bitween_amd
+    model = torch.nn.Sequential(torch.nn.Linear(128, 64, device="cuda", dtype=torch.float16), torch.nn.LayerNorm(64, device="cuda"))
+    model.notes, model.empty = {"a": [1]}, {}
+    calls = []
+    model[1].register_forward_hook(lambda *a: calls.append(1))
+    out = bitween_amd.Bitween(model, bits=4, group_size=64).quantize(rtn=True, verbose=False)
+    assert isinstance(out[0], bitween_amd.QuantizedLinear) and isinstance(model[0], torch.nn.Linear)
+    assert out.notes == {"a": [1]} and out.notes["a"] is not model.notes["a"] and out.empty == {} and out.empty is not model.empty
+    assert out[1].weight is not model[1].weight and torch.equal(out[1].weight, model[1].weight)
+    for name, value in model[1].__dict__.items():
+        if isinstance(value, (dict, set)):
+            assert out[1].__dict__[name] is not value and type(out[1].__dict__[name]) is type(value) and len(out[1].__dict__[name]) == len(value)
+    assert len(out[1]._forward_hooks) == 1
