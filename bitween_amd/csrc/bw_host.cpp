@@ -29,10 +29,8 @@ namespace {
 using at::Tensor;
 
 struct Library {
-    decltype(&bw_qlinear) qlinear = nullptr;
-    decltype(&bw_qlinear_decode_rows) decode_rows = nullptr;
-    decltype(&bw_qgemm_ws) qgemm_ws = nullptr;
-    decltype(&bw_qgemm_workspace_bytes) qgemm_ws_bytes = nullptr;
+    decltype(&bw_qlinear_ws) qlinear = nullptr;
+    decltype(&bw_qlinear_workspace_bytes) qlinear_ws_bytes = nullptr;
     decltype(&bw_cast_bf16_f16) cast = nullptr;
     decltype(&bw_qdgrad) qdgrad = nullptr;
     decltype(&bw_qdgrad_workspace_bytes) qdgrad_ws_bytes = nullptr;
@@ -85,7 +83,7 @@ struct OnDevice {
 
 struct Layer {
     const void *qweight, *scale, *zero, *bias;
-    int64_t n, k, decode_rows;
+    int64_t n, k;
     int bits, group;
     at::DeviceIndex device;
 };
@@ -104,7 +102,7 @@ bool layer_of(const Tensor& qweight, const Tensor& scale, const Tensor& zero, co
                  !bias->is_contiguous()))
         return false;
     l = {qweight.const_data_ptr(), scale.const_data_ptr(), zero.const_data_ptr(), bias ? bias->const_data_ptr() : nullptr,
-         n, k, lib.decode_rows(n, k, (int)bits), (int)bits, (int)group, qweight.device().index()};
+         n, k, (int)bits, (int)group, qweight.device().index()};
     return true;
 }
 
@@ -142,28 +140,20 @@ Tensor linear(const Layer& l, Tensor x, int& status, const char*& what) {
     }
     void* stream = stream_of(l.device);
     Tensor y = empty(shape, at::kHalf, x.device());
-    if (m <= l.decode_rows) {
-        what = "bw_qlinear";
-        const int act = t == at::kHalf ? BW_F16 : BW_BF16;
-        status = lib.qlinear(x.const_data_ptr(), act, m, l.k, ldx, (const int32_t*)l.qweight, l.scale, l.zero, l.bias, l.n, l.bits, l.group,
-                             y.mutable_data_ptr(), l.n, stream);
-        if (status == BW_EUNSUPPORTED && act == BW_BF16) {     // a shape only the generic kernel takes: float16 in memory
-            x = cast_to_f16(x, m, l.k, ldx, stream);
-            status = lib.qlinear(x.const_data_ptr(), BW_F16, m, l.k, l.k, (const int32_t*)l.qweight, l.scale, l.zero, l.bias, l.n, l.bits,
-                                 l.group, y.mutable_data_ptr(), l.n, stream);
-        }
-        return y;
-    }
-    what = "bw_qgemm_ws";
-    if (t == at::kBFloat16) {                                  // the prefill kernel wants float16 in memory
-        x = cast_to_f16(x, m, l.k, ldx, stream);
+    what = "bw_qlinear_ws";
+    auto launch = [&](int act) {
+        const size_t bytes = lib.qlinear_ws_bytes(m, l.n, l.k, l.bits, l.group, act);
+        Tensor ws;
+        if (bytes) ws = empty({(int64_t)bytes}, at::kByte, x.device());
+        return lib.qlinear(x.const_data_ptr(), act, m, l.k, ldx, (const int32_t*)l.qweight, l.scale, l.zero, l.bias, l.n, l.bits, l.group,
+                           y.mutable_data_ptr(), l.n, bytes ? ws.mutable_data_ptr() : nullptr, bytes, stream);
+    };
+    status = launch(t == at::kHalf ? BW_F16 : BW_BF16);
+    if (t == at::kBFloat16 && (status == BW_EUNSUPPORTED || status == BW_EALIGN || status == BW_EWORKSPACE)) {
+        x = cast_to_f16(x, m, l.k, ldx, stream);               // a shape or layout that wants float16 in memory
         ldx = l.k;
+        status = launch(BW_F16);
     }
-    const size_t bytes = lib.qgemm_ws_bytes(m, l.n, l.k, l.bits, l.group);
-    Tensor ws;
-    if (bytes) ws = empty({(int64_t)bytes}, at::kByte, x.device());
-    status = lib.qgemm_ws(x.const_data_ptr(), BW_F16, m, l.k, ldx, (const int32_t*)l.qweight, l.scale, l.zero, l.bias, l.n, l.bits, l.group,
-                          y.mutable_data_ptr(), l.n, bytes ? ws.mutable_data_ptr() : nullptr, bytes, stream);
     return y;
 }
 
@@ -446,10 +436,8 @@ PyObject* py_bind(PyObject*, PyObject* args) {
         fn = reinterpret_cast<std::decay_t<decltype(fn)>>(p);
     };
     Library l;
-    get(l.qlinear, "bw_qlinear");
-    get(l.decode_rows, "bw_qlinear_decode_rows");
-    get(l.qgemm_ws, "bw_qgemm_ws");
-    get(l.qgemm_ws_bytes, "bw_qgemm_workspace_bytes");
+    get(l.qlinear, "bw_qlinear_ws");
+    get(l.qlinear_ws_bytes, "bw_qlinear_workspace_bytes");
     get(l.cast, "bw_cast_bf16_f16");
     get(l.qdgrad, "bw_qdgrad");
     get(l.qdgrad_ws_bytes, "bw_qdgrad_workspace_bytes");

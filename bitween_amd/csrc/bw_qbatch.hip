@@ -1,0 +1,214 @@
+// The batch kernel's plan, its reduction, and bw_qlinear, which sends a call to the decode, the batch or the prefill kernel.
+#include "bw_qbatch_kernel.h"
+
+#include <stddef.h>
+
+bool bw_fast_shape(int64_t M, int64_t N, int64_t K, int64_t ldx, int bits, int group);
+
+namespace {
+
+// y = sum over the splits of the partial sums, plus bias, rounded once.  A thread owns four columns of one row.
+__global__ __launch_bounds__(256) void qbatch_reduce_kernel(const float* __restrict__ ws, const _Float16* __restrict__ bias, _Float16* __restrict__ y,
+                                                            int M, int N, int npad, int ldy, int splits) {
+    const int quads = npad >> 2, idx = (int)blockIdx.x * 256 + threadIdx.x;
+    if (idx >= M * quads) return;
+    const int m = idx / quads, n = (idx - m * quads) * 4;
+    const float* p = ws + (int64_t)m * npad + n;
+    const int64_t step = (int64_t)M * npad;
+    f4 v = {0.f, 0.f, 0.f, 0.f};
+    int s = 0;
+    for (; s + 4 <= splits; s += 4) {
+        f4 t[4];
+#pragma unroll
+        for (int i = 0; i < 4; i++) t[i] = *reinterpret_cast<const f4*>(p + (s + i) * step);
+#pragma unroll
+        for (int i = 0; i < 4; i++) v += t[i];
+    }
+    for (; s < splits; s++) v += *reinterpret_cast<const f4*>(p + s * step);
+    _Float16 h[4];
+#pragma unroll
+    for (int e = 0; e < 4; e++) h[e] = (_Float16)(v[e] + (bias && n + e < N ? (float)bias[n + e] : 0.f));
+    _Float16* dst = y + (int64_t)m * ldy + n;
+    if (n + 3 < N && ldy % 4 == 0 && ((uintptr_t)y & 7) == 0) {
+        *reinterpret_cast<u2*>(dst) = u2{as_u32(h2{h[0], h[1]}), as_u32(h2{h[2], h[3]})};
+    } else {
+#pragma unroll
+        for (int e = 0; e < 4; e++)
+            if (n + e < N) dst[e] = h[e];
+    }
+}
+
+// ---- plan ----
+struct BatchPlan { int ntw, splits; };
+
+inline int batch_mt(int64_t M) { const int t = (int)((M + 15) / 16); return t <= 4 ? t : t <= 6 ? 6 : 8; }
+
+// Column tiles per wave and cuts of K for a call, from a model of the launch fitted to 1500 timings (17 ... 96 rows, eleven
+// shapes, 2 / 4 / 8 bits; rms error 7 %, its choice within 0.7 % of the best on average): a round costs
+// -0.23 + 0.21 MT + (0.46 + 0.014 MT + 0.19 at 8 bits) NTW us (0.68 of it where rounds are 256 values), every wave of
+// workgroups 0.34 MT us more, a launch 2.1, a cut of K the reduction: 2.4 us and 2.9 us per million partial sums.
+BatchPlan batch_plan(int64_t M, int64_t N, int64_t K, int bits, bool may_split) {
+    struct Entry { int64_t m, n, k; int key; BatchPlan plan; };
+    static thread_local Entry cache[32] = {};              // the search takes 2 us of a call's host time
+    const int key = bits * 2 + may_split;
+    Entry& e = cache[(size_t)(M * 7 + N * 3 + K * 5 + key) % 32];
+    if (e.m == M && e.n == N && e.k == K && e.key == key) return e.plan;
+    const int mt = batch_mt(M), wk = mt <= 4 ? 4 : 2, nchunks = (int)((K + 127) / 128), cus = bw_device_cus();
+    BatchPlan best{1, 1};
+    float best_us = 1e30f;
+    for (int ntw = 1; ntw <= (mt <= 4 ? 3 : mt == 6 ? 2 : 1); ntw++) {
+        const int bn = 16 * (8 / wk) * ntw;
+        const int64_t tiles = (N + bn - 1) / bn;
+        const float round = (-0.23f + 0.21f * mt + (0.46f + 0.014f * mt + (bits == 8 ? 0.19f : 0.f)) * ntw) * (mt <= 4 ? 1.f : 0.68f);
+        for (int s = 1; s <= 16 && (s == 1 || (may_split && 2 * s <= nchunks)); s++) {
+            const int cps = (nchunks + s - 1) / s, used = (nchunks + cps - 1) / cps;
+            if (used != s) continue;
+            const float us = 2.1f + (float)((tiles * s + cus - 1) / cus) * (((cps + wk - 1) / wk) * round + 0.34f * mt) +
+                             (s > 1 ? 2.4f + 2.9e-6f * (float)M * (float)N * s : 0.f);
+            if (us < best_us) { best_us = us; best = {ntw, s}; }
+        }
+    }
+    e = {M, N, K, key, best};
+    return best;
+}
+
+inline size_t batch_ws_bytes(int64_t M, int64_t N, const BatchPlan& p) { return p.splits > 1 ? (size_t)p.splits * M * ((N + 3) & ~(int64_t)3) * 4 : 0; }
+
+// ---- which kernel ----
+enum Route { kDecode, kBatch, kPrefill };
+
+// Up to 16 rows the decode kernels keep the call except where they stage x several times over: rows longer than one round
+// of theirs (K > 4096), or more column tiles than their resident workgroups hold.  5 ... 16 rows, timed on 60 shapes x
+// nine formats (us, decode against this kernel): W4 g32 5120 -> 22016 36 ... 48 against 20 ... 22, W2 g64 5120 -> 14336 21 ...
+// 30 against 11 ... 13, W4 g128 4096 -> 22016 15.7 ... 18.3 against 13.5 ... 14.8, W8 g64 4096 -> 14336 16.0 ... 20.5 against
+// 15.4 ... 16.1; on the other side of the lines W4 g128 4096 -> 14336 9.5 ... 10.8 against 10.3 ... 11.4, W4 g128 11008 -> 4096
+// 8.8 ... 12.1 against 11.7 ... 12.9.
+inline bool batch_takes_decode_rows(int64_t M, int64_t N, int64_t K, int bits, int group) {
+    const int64_t tiles = (N + 15) / 16, cus = bw_device_cus();
+    if (M < 5) return false;
+    if (bits == 8) return tiles > 3 * cus || (M > 8 && K >= 8192);
+    if (K > 4096) {
+        if (tiles > cus) return !(bits == 4 && group == 128) || M > 8;
+        return M > 8 && (group == 32 || (bits == 4 && group == 64));
+    }
+    if (K >= 3072 && tiles > 4 * cus) return true;
+    return bits == 2 && M > 8 && tiles > 3 * cus && (group == 32 || K / group % 2);
+}
+
+// 17 ... 96 rows: this kernel (64 rows of the Llama shapes at 4 bits, us, prefill kernel against this one: 4096 x 4096 17.7
+// -> 11.7, 4096 -> 11008 20.4 -> 17.3, 11008 -> 4096 22.8 -> 19.1; 2048 x 2048 13.0 -> 8.1; 96 rows 1.03 ... 1.4 x faster).
+// Up to 128 rows on layers it unpacks fast enough: 32 M weights at 4 bits (4096 x 4096 20.8 -> 17.4; 4096 -> 11008 27.0
+// against 30.0), 64 M at 2 and 8 bits (4096 -> 14336 W8 38.2 -> 33.1).
+Route route(int64_t M, int64_t N, int64_t K, int bits, int group) {
+    if (M <= 16) return batch_takes_decode_rows(M, N, K, bits, group) ? kBatch : kDecode;
+    if (M <= 96) return kBatch;
+    return M <= 128 && N * K <= ((int64_t)(bits == 4 ? 32 : 64) << 20) ? kBatch : kPrefill;
+}
+
+// What the batch kernel asks of a call beyond bw_fast_shape: 4-byte words of scales, offsets of x in 31 bits.
+inline bool batch_takes(const void* x, int64_t M, int64_t N, int64_t K, int64_t ldx, const void* qweight, const void* scale16, const void* zp16, int bits, int group) {
+    return bw_fast_shape(M, N, K, ldx, bits, group) && bw_aligned(x, 16) && (ldx * 2) % 16 == 0 && bw_aligned(qweight, 16) && bw_aligned(scale16, 4) &&
+           bw_aligned(zp16, 4) && M * ldx * 2 < (int64_t)kBatchMaxBytes;
+}
+
+int launch_batch(const void* x, int act_dtype, int64_t M, int64_t K, int64_t ldx, const int32_t* qweight, const void* scale16, const void* zp16,
+                 const void* bias, int64_t N, int bits, int group, void* y, int64_t ldy, void* workspace, const BatchPlan& plan, hipStream_t st) {
+    BatchArgs a;
+    a.x = x; a.qweight = qweight; a.scale = scale16; a.zp = zp16; a.bias = (const _Float16*)bias; a.y = (_Float16*)y;
+    a.ws = (float*)workspace;
+    a.M = (int)M; a.N = (int)N; a.K = (int)K; a.ldx = (int)ldx; a.ldy = (int)ldy; a.npad = (int)((N + 3) & ~(int64_t)3);
+    a.groups = (int)(K / group);
+    a.row_bytes = (int)(K * bits / 8);
+    a.nchunks = (int)((K + 127) / 128);
+    a.x_bytes = (uint32_t)(((M - 1) * ldx + K) * 2);
+    a.w_bytes = (uint32_t)(N * a.row_bytes);
+    a.meta_bytes = (uint32_t)(N * a.groups * 2);
+    a.splits = plan.splits;
+    a.chunks_per_split = (a.nchunks + plan.splits - 1) / plan.splits;
+    a.x_bf16 = act_dtype == BW_BF16;
+    const int mt = batch_mt(M);
+    const int r = bits == 4 ? bw_launch_qbatch_w4(group, mt, plan.ntw, a, st) : bits == 8 ? bw_launch_qbatch_w8(group, mt, plan.ntw, a, st)
+                                                                                      : bw_launch_qbatch_w2(group, mt, plan.ntw, a, st);
+    if (r != BW_OK || a.splits == 1) return r;
+    const int64_t items = M * (a.npad / 4);
+    hipLaunchKernelGGL(qbatch_reduce_kernel, dim3((unsigned)((items + 255) / 256)), dim3(256), 0, st, a.ws, a.bias, a.y, a.M, a.N, a.npad, a.ldy, a.splits);
+    return hipGetLastError() == hipSuccess ? BW_OK : BW_ELAUNCH;
+}
+
+inline size_t cast_bytes(int64_t M, int64_t K) { return ((size_t)M * K * 2 + 255) & ~(size_t)255; }
+
+}  // namespace
+
+// Rows up to which bw_qlinear takes bfloat16 x and, without a workspace, stays off the prefill kernel.  (Set when more than
+// 16 rows ran as several decode launches; kept as part of the interface.)
+extern "C" int bw_qlinear_decode_rows(int64_t N, int64_t K, int bits) {
+    if (N < 1 || K < 1 || !bw_bits_ok(bits)) return 0;
+    const int64_t bytes = N * (K * bits / 8);
+    return bytes < ((int64_t)10 << 20) ? 48 : bytes < ((int64_t)40 << 20) ? 32 : 16;
+}
+
+extern "C" size_t bw_qlinear_workspace_bytes(int64_t M, int64_t N, int64_t K, int bits, int group, int act_dtype) {
+    if (!bw_shape_ok(N, K, bits, group) || M < 1 || M >= ((int64_t)1 << 31)) return 0;
+    const bool fast = bw_fast_shape(M, N, K, K, bits, group);
+    const Route r = fast ? route(M, N, K, bits, group) : M <= 16 ? kDecode : kPrefill;
+    // (a call that this kernel turns out not to take - unaligned scales - falls back to the prefill kernel)
+    const size_t prefill = M <= 16 ? 0 : bw_qgemm_workspace_bytes(M, N, K, bits, group);
+    size_t split = r == kPrefill ? prefill : 0;
+    if (r == kBatch) split = batch_ws_bytes(M, N, batch_plan(M, N, K, bits, true));
+    const bool cast = act_dtype == BW_BF16 && (r == kPrefill || !fast);
+    return split + (cast ? cast_bytes(M, K) : 0);
+}
+
+extern "C" int bw_qlinear_ws(const void* x, int act_dtype, int64_t M, int64_t K, int64_t ldx, const int32_t* qweight, const void* scale16,
+                             const void* zp16, const void* bias, int64_t N, int bits, int group, void* y, int64_t ldy, void* workspace,
+                             size_t workspace_bytes, void* stream) {
+    if (!x || !qweight || !scale16 || !zp16 || !y) return BW_EINVAL;
+    if (!bw_shape_ok(N, K, bits, group) || M < 1 || M >= ((int64_t)1 << 31) || ldx < K || ldy < N) return BW_EINVAL;
+    if (act_dtype != BW_F16 && act_dtype != BW_BF16) return BW_EUNSUPPORTED;
+    if (workspace && !bw_aligned(workspace, 16)) return BW_EALIGN;
+    if (!workspace) workspace_bytes = 0;
+    const bool fast = bw_fast_shape(M, N, K, ldx, bits, group);
+    Route r = fast ? route(M, N, K, bits, group) : M <= 16 ? kDecode : kPrefill;
+    if (r == kBatch && batch_takes(x, M, N, K, ldx, qweight, scale16, zp16, bits, group)) {
+        BatchPlan plan = batch_plan(M, N, K, bits, true);
+        if (batch_ws_bytes(M, N, plan) > workspace_bytes) plan = batch_plan(M, N, K, bits, false);
+        return launch_batch(x, act_dtype, M, K, ldx, qweight, scale16, zp16, bias, N, bits, group, y, ldy, workspace, plan, (hipStream_t)stream);
+    }
+    if (M <= 16) {
+        const int st = bw_qgemv(x, act_dtype, M, K, ldx, qweight, scale16, zp16, bias, N, bits, group, y, ldy, stream);
+        if (st != BW_EUNSUPPORTED || act_dtype != BW_BF16) return st;      // bfloat16 on a shape that only the generic kernel takes
+    }
+    if (act_dtype == BW_BF16) {                                            // the prefill kernel wants float16 in memory
+        const size_t need = cast_bytes(M, K);
+        if (workspace_bytes < need) return BW_EWORKSPACE;
+        const int st = bw_cast_bf16_f16(x, M, K, ldx, workspace, K, stream);
+        if (st != BW_OK) return st;
+        x = workspace;
+        ldx = K;
+        workspace_bytes -= need;
+        workspace = workspace_bytes ? (char*)workspace + need : nullptr;
+    }
+    const size_t need = bw_qgemm_workspace_bytes(M, N, K, bits, group);
+    const bool split = need && workspace_bytes >= need;
+    return bw_qgemm_ws(x, BW_F16, M, K, ldx, qweight, scale16, zp16, bias, N, bits, group, y, ldy, split ? workspace : nullptr, split ? workspace_bytes : 0, stream);
+}
+
+extern "C" int bw_qlinear(const void* x, int act_dtype, int64_t M, int64_t K, int64_t ldx, const int32_t* qweight,
+                          const void* scale16, const void* zp16, const void* bias, int64_t N, int bits, int group,
+                          void* y, int64_t ldy, void* stream) {
+    if (M >= 1 && M <= bw_qlinear_decode_rows(N, K, bits) && (act_dtype == BW_F16 || act_dtype == BW_BF16)) {
+        // the batch kernel where it is what bw_qlinear_ws runs too and K needs no cut for want of workgroups
+        if (x && qweight && scale16 && zp16 && y && bw_shape_ok(N, K, bits, group) && ldx >= K && ldy >= N &&
+            batch_takes(x, M, N, K, ldx, qweight, scale16, zp16, bits, group) && route(M, N, K, bits, group) == kBatch &&
+            batch_plan(M, N, K, bits, true).splits == 1)
+            return launch_batch(x, act_dtype, M, K, ldx, qweight, scale16, zp16, bias, N, bits, group, y, ldy, nullptr,
+                                batch_plan(M, N, K, bits, true), (hipStream_t)stream);
+        for (int64_t m0 = 0; m0 < M; m0 += 16) {
+            const int st = bw_qgemv((const _Float16*)x + m0 * ldx, act_dtype, M - m0 < 16 ? M - m0 : 16, K, ldx, qweight, scale16,
+                                    zp16, bias, N, bits, group, (_Float16*)y + m0 * ldy, ldy, stream);
+            if (st != BW_OK) return st;
+        }
+        return BW_OK;
+    }
+    return bw_qgemm(x, act_dtype, M, K, ldx, qweight, scale16, zp16, bias, N, bits, group, y, ldy, stream);
+}

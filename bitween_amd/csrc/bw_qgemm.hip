@@ -256,32 +256,3 @@ extern "C" int bw_qgemm(const void* x, int act_dtype, int64_t M, int64_t K, int6
                         void* y, int64_t ldy, void* stream) {
     return bw_qgemm_ws(x, act_dtype, M, K, ldx, qweight, scale16, zp16, bias, N, bits, group, y, ldy, nullptr, 0, stream);
 }
-
-// Rows up to which bw_qlinear stays on the decode kernel (16 rows per launch; the later launches find the weights
-// in L2 / Infinity Cache) before it hands the call to the prefill kernel, whose 64-row tiles take 17 ... 64 rows.  Measured
-// under graph replay over rotating layer copies (decode launches against one prefill launch, us):
-//   4096 x 4096 at 4 bits (8 MiB of packed weights): 8.9 / 10.6 / 15.2 against 13.9 / 14.9 / 16.9 at 17 / 32 / 48 rows, 18.2
-//   against 16.8 at 49 - three launches still win;
-//   4096 x 4096 at 8 bits (16 MiB), 4096 x 11008 at 2 and 4 bits (11 / 21.5 MiB), 4096 x 14336 at 4 bits (28 MiB): two
-//   launches win (12.7 / 15.2 / 16.6 / 19.0 against 15.8 / 18.9 / 19.0 / 19.4 at 32 rows), a third does not (16.0 ... 24.6
-//   against 16.0 ... 19.5 at 33);
-//   4096 x 11008 at 8 bits (43 MiB): even the second launch loses (22.3 against 19.7 at 17 rows).
-extern "C" int bw_qlinear_decode_rows(int64_t N, int64_t K, int bits) {
-    if (N < 1 || K < 1 || !bw_bits_ok(bits)) return 0;
-    const int64_t bytes = N * (K * bits / 8);
-    return bytes < ((int64_t)10 << 20) ? 48 : bytes < ((int64_t)40 << 20) ? 32 : 16;
-}
-
-extern "C" int bw_qlinear(const void* x, int act_dtype, int64_t M, int64_t K, int64_t ldx, const int32_t* qweight,
-                          const void* scale16, const void* zp16, const void* bias, int64_t N, int bits, int group,
-                          void* y, int64_t ldy, void* stream) {
-    if (M >= 1 && M <= bw_qlinear_decode_rows(N, K, bits) && (act_dtype == BW_F16 || act_dtype == BW_BF16)) {
-        for (int64_t m0 = 0; m0 < M; m0 += 16) {
-            const int st = bw_qgemv((const _Float16*)x + m0 * ldx, act_dtype, M - m0 < 16 ? M - m0 : 16, K, ldx, qweight, scale16,
-                                    zp16, bias, N, bits, group, (_Float16*)y + m0 * ldy, ldy, stream);
-            if (st != BW_OK) return st;
-        }
-        return BW_OK;
-    }
-    return bw_qgemm(x, act_dtype, M, K, ldx, qweight, scale16, zp16, bias, N, bits, group, y, ldy, stream);
-}

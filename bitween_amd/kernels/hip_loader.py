@@ -23,7 +23,7 @@ _DTYPE_CODE = {torch.float16: BW_F16, torch.bfloat16: BW_BF16, torch.float32: BW
 
 ABI_VERSION = 10           # what bw_abi_version() of a matching library returns
 ENTRY_POINTS = ("bw_abi_version", "bw_strerror", "bw_quantize_pack", "bw_quantize_pack_add", "bw_dequantize", "bw_qgemv", "bw_qgemm",
-                "bw_qgemm_ws", "bw_qgemm_static", "bw_qgemm_workspace_bytes", "bw_qgemm_tile_rows", "bw_qlinear", "bw_qdgrad", "bw_qdgrad_workspace_bytes", "bw_qdgrad_tile_rows", "bw_cast_bf16_f16", "bw_qlinear_decode_rows", "bw_qgemv_last_kernel")
+                "bw_qgemm_ws", "bw_qgemm_static", "bw_qgemm_workspace_bytes", "bw_qgemm_tile_rows", "bw_qlinear", "bw_qlinear_ws", "bw_qlinear_workspace_bytes", "bw_qdgrad", "bw_qdgrad_workspace_bytes", "bw_qdgrad_tile_rows", "bw_cast_bf16_f16", "bw_qlinear_decode_rows", "bw_qgemv_last_kernel")
 
 
 class BitweenHipError(RuntimeError):
@@ -60,6 +60,10 @@ def load():
     lib.bw_qgemm_ws.argtypes = mm[:-1] + [vp, ctypes.c_size_t, vp]
     lib.bw_qgemm_workspace_bytes.argtypes = [i64, i64, i64, i32, i32]
     lib.bw_qgemm_workspace_bytes.restype = ctypes.c_size_t
+    lib.bw_qlinear_ws.argtypes = lib.bw_qgemm_ws.argtypes
+    lib.bw_qlinear_ws.restype = i32
+    lib.bw_qlinear_workspace_bytes.argtypes = [i64, i64, i64, i32, i32, i32]
+    lib.bw_qlinear_workspace_bytes.restype = ctypes.c_size_t
     lib.bw_qgemm_tile_rows.argtypes = [i64, i64, i64, i32, i32]
     lib.bw_qgemm_tile_rows.restype = i32
     lib.bw_qdgrad_workspace_bytes.argtypes = [i64, i64, i64, i32, i32]
@@ -76,13 +80,9 @@ def load():
     lib.bw_qgemv_last_kernel.restype = ctypes.c_char_p
     for name in ("bw_quantize_pack", "bw_quantize_pack_add", "bw_dequantize", "bw_qgemv", "bw_qgemm", "bw_qgemm_ws", "bw_qgemm_static", "bw_qlinear"):
         getattr(lib, name).restype = i32
-    for name in ("bw_qgemv", "bw_qgemm", "bw_qlinear"):
-        _ENTRY[name] = getattr(lib, name)
     _lib = lib
     return lib
 
-
-_ENTRY = {}
 
 _HOST_PATH = os.path.join(os.path.dirname(os.path.dirname(os.path.abspath(__file__))), "csrc", "_bw_host.so")
 _host = None
@@ -201,69 +201,60 @@ def _bf16_to_f16(x):
     return x.to(torch.float16)
 
 
-def _matmul(entry, x, qweight, scale, zero_point, bias, bits, group_size):
+def _checked(entry, x, qweight, scale, zero_point, bias, bits, group_size):
+    """The operands of a matmul entry point, checked and in the layout the kernels read."""
     if not x.is_cuda:
         require_gpu(x, entry)
     if x.dim() != 2:
         raise ValueError("x must be [M, K]")
     if qweight.dtype is not torch.int32 or scale.dtype is not torch.float16 or zero_point.dtype is not torch.float16:
         raise TypeError("qweight must be int32 and scale / zero_point float16 (the QuantizedLinear buffers)")
-    m = x.shape[0]
-    # rows that bw_qlinear keeps on the decode kernel: always 16, and 32 or 48 for layers that are not too large
-    decode_rows = 16 if m <= 16 or entry != "bw_qlinear" else load().bw_qlinear_decode_rows(qweight.shape[0], x.shape[1], bits)
-    act = BW_F16
-    if x.dtype is torch.bfloat16:
-        # the decode kernels round bfloat16 to float16 as they stage x (the reference's x.to(float16),
-        # bitween/modules.py:74, without the extra kernel); the prefill kernel wants float16 in memory
-        if entry == "bw_qgemv" or (entry == "bw_qlinear" and m <= decode_rows):
-            act = BW_BF16
-        else:
-            x = _bf16_to_f16(x)
-    elif x.dtype is not torch.float16:
+    if x.dtype is not torch.float16 and x.dtype is not torch.bfloat16:
         raise TypeError("x must be float16 or bfloat16")
     if bias is not None and bias.dtype is not torch.float16:
         raise TypeError("bias must be float16")
-    ldx = x.stride(0)
-    if x.stride(1) != 1 or (ldx * 2) % 16 or x.data_ptr() % 16:
-        x = x.contiguous().clone()
-        ldx = x.stride(0)
-    if not qweight.is_contiguous():
-        qweight = qweight.contiguous()
-    if not scale.is_contiguous():
-        scale = scale.contiguous()
-    if not zero_point.is_contiguous():
-        zero_point = zero_point.contiguous()
-    m, k = x.shape
+    k = x.shape[1]
     n, words = qweight.shape
     if words * (32 // bits) != k:
         raise ValueError(f"x has K={k} but qweight packs K={words * (32 // bits)}")
     groups = k // group_size
     if scale.shape != (n, groups) or zero_point.shape != (n, groups):
         raise ValueError("scale / zero_point must be [N, K // group_size]")
+    if x.stride(1) != 1 or (x.stride(0) * 2) % 16 or x.data_ptr() % 16:
+        x = x.contiguous().clone()
+    return tuple(_plain(t) for t in (x, qweight.contiguous(), scale.contiguous(), zero_point.contiguous())) + (
+        None if bias is None else _plain(bias.contiguous()),)
+
+
+def _matmul(entry, x, qweight, scale, zero_point, bias, bits, group_size):
+    """One of the kernels by name: bw_qgemv (M <= 16) or bw_qgemm (with the split-K workspace the shape asks for)."""
+    x, qweight, scale, zero_point, bias = _checked(entry, x, qweight, scale, zero_point, bias, bits, group_size)
+    (m, k), n = x.shape, qweight.shape[0]
     y = torch.empty((m, n), dtype=torch.float16, device=x.device)
     if m == 0:
         return y
     lib = load()
-    bias_ptr = None
-    if bias is not None:
-        bias_ptr = (bias if bias.is_contiguous() else bias.contiguous()).data_ptr()
+    bias_ptr = None if bias is None else bias.data_ptr()
+    act = BW_F16
+    if x.dtype is torch.bfloat16:
+        if entry == "bw_qgemv":                            # the decode kernels round bfloat16 to float16 as they stage x
+            act = BW_BF16
+        else:                                              # the prefill kernel wants float16 in memory
+            x = _bf16_to_f16(x)
     with _on_device(x.device) as index:
-        if (entry == "bw_qgemm" and m > 16) or (entry == "bw_qlinear" and m > decode_rows):
-            # prefill (bw_qlinear itself keeps fewer rows on the decode kernel): give the library a split-K
-            # workspace when the shape wants one
+        if entry == "bw_qgemm":
             nbytes = lib.bw_qgemm_workspace_bytes(m, n, k, bits, group_size)
             ws = torch.empty(nbytes, dtype=torch.uint8, device=x.device) if nbytes else None
-            st = lib.bw_qgemm_ws(x.data_ptr(), BW_F16, m, k, ldx, qweight.data_ptr(), scale.data_ptr(),
+            st = lib.bw_qgemm_ws(x.data_ptr(), BW_F16, m, k, x.stride(0), qweight.data_ptr(), scale.data_ptr(),
                                  zero_point.data_ptr(), bias_ptr, n, bits, group_size, y.data_ptr(), n,
                                  None if ws is None else ws.data_ptr(), nbytes, _raw_stream(index))
-            entry = "bw_qgemm_ws"
         else:
-            st = _ENTRY[entry](x.data_ptr(), act, m, k, ldx, qweight.data_ptr(), scale.data_ptr(),
-                               zero_point.data_ptr(), bias_ptr, n, bits, group_size, y.data_ptr(), n, _raw_stream(index))
+            st = lib.bw_qgemv(x.data_ptr(), act, m, k, x.stride(0), qweight.data_ptr(), scale.data_ptr(),
+                              zero_point.data_ptr(), bias_ptr, n, bits, group_size, y.data_ptr(), n, _raw_stream(index))
             if st == -2 and act == BW_BF16:                # a shape only the generic kernel takes: float16 in memory
                 x = x.to(torch.float16)
-                st = _ENTRY[entry](x.data_ptr(), BW_F16, m, k, x.stride(0), qweight.data_ptr(), scale.data_ptr(),
-                                   zero_point.data_ptr(), bias_ptr, n, bits, group_size, y.data_ptr(), n, _raw_stream(index))
+                st = lib.bw_qgemv(x.data_ptr(), BW_F16, m, k, x.stride(0), qweight.data_ptr(), scale.data_ptr(),
+                                  zero_point.data_ptr(), bias_ptr, n, bits, group_size, y.data_ptr(), n, _raw_stream(index))
     if st:
         _check(st, entry)
     return y
@@ -316,11 +307,15 @@ def last_decode_kernel():
 
 def quantized_matmul_hip(x, qweight, scale, zero_point, bias, bits, group_size):
     """y[M,N] = x[M,K] @ dequant(qweight, scale, zero_point)^T + bias, float16 (main.py:433's operator)."""
-    if x.dim() == 2:
-        y = host().matmul(x, qweight, scale, zero_point, bias, bits, group_size)
-        if y is not None:
-            return y
-    return _matmul("bw_qlinear", x, qweight, scale, zero_point, bias, bits, group_size)
+    y = host().matmul(x, qweight, scale, zero_point, bias, bits, group_size) if x.dim() == 2 else None
+    if y is None:                                          # not the contiguous tensors a QuantizedLinear keeps: look closer, then again
+        args = _checked("bw_qlinear", x, qweight, scale, zero_point, bias, bits, group_size)
+        if x.shape[0] == 0:
+            return torch.empty((0, qweight.shape[0]), dtype=torch.float16, device=x.device)
+        y = host().matmul(*args, bits, group_size)
+        if y is None:
+            raise BitweenHipError("bw_qlinear: x and the layer's buffers must be on one GPU")
+    return y
 
 
 def quantized_gemv_hip(x, qweight, scale, zero_point, bias, bits, group_size):

@@ -102,7 +102,7 @@ int bw_dequantize(const int32_t* qweight, const void* scale, int scale_dtype, co
  * reference dequantizes; products accumulate in float32; y is rounded once
  * (the reference rounds before and after the bias add; within its 1e-2
  * tolerance, main.py:471-477).
- *   x      [M][ldx] of act_dtype: BW_F16, or BW_BF16 for bw_qgemv and for bw_qlinear while it stays on the decode kernel - the
+ *   x      [M][ldx] of act_dtype: BW_F16, or BW_BF16 for bw_qgemv, bw_qlinear_ws and (up to bw_qlinear_decode_rows rows) bw_qlinear - the
  *          kernel then rounds every value to float16 as it reads it, which is the reference's
  *          x.to(float16) (bitween/modules.py:74) without a separate pass; other entry points return
  *          BW_EUNSUPPORTED for BW_BF16.  y [M][ldy] is float16 in every case, as in the reference.
@@ -111,9 +111,10 @@ int bw_dequantize(const int32_t* qweight, const void* scale, int scale_dtype, co
  *   bias   [N] float16 or NULL
  * bw_qgemv: decode path, 1 <= M <= 16, HBM-bound, no workspace.
  * bw_qgemm: prefill path, any M >= 1, MFMA-bound.
- * bw_qlinear: picks between them by M (what the Python forward calls): the decode kernel, 16 rows per
- *             launch, up to M = bw_qlinear_decode_rows(N, K, bits) (48; 32 for layers of 10 MiB of packed
- *             weights and more; 16 from 40 MiB on); the prefill kernel (without a workspace) beyond. */
+ * bw_qlinear: picks between them and a third, the batch kernel (5 ... 128 rows, no entry point of its own), by shape; without
+ *             a workspace: up to M = bw_qlinear_decode_rows(N, K, bits) (48; 32 for layers of 10 MiB of packed
+ *             weights and more; 16 from 40 MiB on) the batch kernel where it needs none, else the decode kernel, 16
+ *             rows per launch; the prefill kernel beyond.  BW_BF16 x up to those rows. */
 int bw_qgemv(const void* x, int act_dtype, int64_t M, int64_t K, int64_t ldx,
              const int32_t* qweight, const void* scale16, const void* zp16, const void* bias,
              int64_t N, int bits, int group, void* y, int64_t ldy, void* stream);
@@ -155,6 +156,17 @@ int bw_qgemm_static(const void* x, int act_dtype, int64_t M, int64_t K, int64_t 
                     int64_t N, int bits, int group, void* y, int64_t ldy, void* stream);
 
 int bw_qlinear_decode_rows(int64_t N, int64_t K, int bits);
+
+/* bw_qlinear with a workspace: what the Python forward calls for any number of rows.  Adds to it the batch kernel with K cut
+ * across workgroups, the split-K plans of the prefill kernel, and BW_BF16 x for every M (cast into the workspace where the
+ * prefill kernel runs).  `workspace` (16-byte aligned) holds at least bw_qlinear_workspace_bytes(...) bytes (0 = none needed);
+ * with less, plans that need it are not used, and BW_BF16 x that has to be cast returns BW_EWORKSPACE. */
+size_t bw_qlinear_workspace_bytes(int64_t M, int64_t N, int64_t K, int bits, int group, int act_dtype);
+
+int bw_qlinear_ws(const void* x, int act_dtype, int64_t M, int64_t K, int64_t ldx,
+                  const int32_t* qweight, const void* scale16, const void* zp16, const void* bias,
+                  int64_t N, int bits, int group, void* y, int64_t ldy,
+                  void* workspace, size_t workspace_bytes, void* stream);
 
 /* Diagnostic, no counterpart in the reference: the name (with template arguments) of the decode kernel that the
  * calling thread's last bw_qgemv / bw_qlinear launch ran ("" before the first one, or when the generic kernel ran).

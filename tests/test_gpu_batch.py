@@ -1,0 +1,121 @@
+"""The batch kernel (bw_qlinear_ws from 5, 17 or so rows up to 128) against the oracle: every format, row counts at the edges of
+its row tiles, columns and K that end inside tiles and rounds, K cut across workgroups or not, float16 and bfloat16 x."""
+import ctypes
+
+import numpy as np
+import pytest
+import torch
+
+from gpu_util import check_matmul, quantized_layer, to_gpu
+from oracle import rtn_oracle as orc
+
+pytestmark = pytest.mark.gpu
+
+FORMATS = [(4, 128), (4, 64), (4, 32), (8, 128), (8, 64), (8, 32), (2, 128), (2, 64), (2, 32)]
+
+
+def _call(lib, x, d, n, bits, g, ldy, ws=True, bias=None):
+    m, k = x.shape
+    act = 0 if x.dtype is torch.float16 else 1
+    y = torch.full((m, ldy), 7.0, dtype=torch.float16, device="cuda")
+    need = lib.bw_qlinear_workspace_bytes(m, n, k, bits, g, act) if ws else 0
+    w = torch.full((max(need, 16) // 4,), float("nan"), dtype=torch.float32, device="cuda")
+    st = lib.bw_qlinear_ws(x.data_ptr(), act, m, k, x.stride(0), d[0].data_ptr(), d[1].data_ptr(), d[2].data_ptr(),
+                           None if bias is None else bias.data_ptr(), n, bits, g, y.data_ptr(), ldy, w.data_ptr() if need else None, need,
+                           ctypes.c_void_p(torch.cuda.current_stream().cuda_stream))
+    torch.cuda.synchronize()
+    return st, y, need
+
+
+@pytest.mark.parametrize("bits,g", FORMATS)
+@pytest.mark.parametrize("k,n", [(128, 33), (23 * 128, 97), (9 * 64 * 2 + 64, 1003), (4096, 130)])
+def test_rows_and_ragged_shapes_vs_oracle(bits, g, k, n):
+    """K of one chunk, of an odd number of groups, not a multiple of 128 (or of 256), of several rounds; x rows padded and y rows of an
+    odd pitch; with and without bias; with the workspace (K cut across workgroups on the narrow shapes) and without."""
+    from bitween_amd.kernels import hip_loader
+    lib = hip_loader.load()
+    if k % g:
+        k = k // g * g
+    _, qw, s16, z16, b16 = quantized_layer(n, k, bits, g, seed=n + k + bits + g, outliers=True)
+    w16 = orc.dequantize_f16(qw, s16, z16, g, bits)
+    d = [to_gpu(a) for a in (qw, s16, z16, b16)]
+    split = False
+    for m in (17, 32, 33, 48, 64, 65, 96, 97, 128):
+        gen = torch.Generator(device="cuda").manual_seed(m)
+        xbuf = torch.full((m, k + 8), float("nan"), dtype=torch.float16, device="cuda")
+        xbuf[:, :k] = torch.randn(m, k, device="cuda", generator=gen).half()
+        hot = {0: k - 1, m - 1: k // 2}
+        for r, c in hot.items():
+            xbuf[r, :k] = 0
+            xbuf[r, c] = 1.0
+        x = xbuf[:, :k]
+        st, y, need = _call(lib, x, d, n, bits, g, n + 1, bias=d[3])
+        split = split or need > 0
+        assert st == 0 and (y[:, n:] == 7.0).all()
+        check_matmul(y[:, :n].contiguous(), x.cpu().numpy(), qw, s16, z16, b16, bits, g)
+        st, y, _ = _call(lib, x, d, n, bits, g, n, ws=False)
+        assert st == 0
+        check_matmul(y, x.cpu().numpy(), qw, s16, z16, None, bits, g)
+        for r, c in hot.items():
+            assert np.array_equal(y[r].cpu().numpy().view(np.uint16), w16[:, c].view(np.uint16))
+    assert split or k < 2048
+
+
+@pytest.mark.parametrize("bits,g", FORMATS)
+def test_bfloat16_rows_equal_the_cast(bits, g):
+    """bfloat16 x is rounded to float16 as it is staged: the bits of a call on x.to(float16)."""
+    from bitween_amd.kernels import hip_loader
+    lib = hip_loader.load()
+    n, k = 500, 1536
+    _, qw, s16, z16, _ = quantized_layer(n, k, bits, g, seed=bits + g)
+    d = [to_gpu(a) for a in (qw, s16, z16)]
+    for m in (18, 40, 64, 80, 128):
+        x = (torch.randn(m, k, device="cuda") * 30).to(torch.bfloat16)
+        st, y, _ = _call(lib, x, d, n, bits, g, n)
+        st2, y2, _ = _call(lib, x.to(torch.float16), d, n, bits, g, n)
+        assert st == 0 and st2 == 0 and torch.equal(y, y2)
+
+
+@pytest.mark.parametrize("bits,g,k,n", [(4, 64, 3072, 16400), (8, 32, 256, 12300), (2, 32, 4352, 4100), (4, 32, 8192, 200), (4, 128, 4224, 4100)])
+@pytest.mark.parametrize("m", [5, 8, 9, 16])
+def test_decode_rows_on_large_layers(bits, g, k, n, m):
+    """Up to 16 rows the batch kernel takes layers with more column tiles, or longer rows, than the decode kernels stage once
+    (and hands the others to them): through the module, and without a workspace."""
+    from bitween_amd.kernels import hip_loader as hip
+    rows = np.unique(np.concatenate([np.arange(0, n, n // 25), [n - 1]]))
+    torch.manual_seed(m + k)
+    lin = torch.nn.Linear(k, n, bias=True, device="cuda", dtype=torch.float16)
+    import bitween_amd
+    q = bitween_amd.QuantizedLinear.from_float(lin, bits, g)
+    x = torch.randn(m, k, device="cuda", dtype=torch.float16)
+    part = [a[torch.from_numpy(rows).cuda()].cpu().numpy() for a in (q.qweight, q.scale, q.zero_point, q.bias)]
+    y = q(x)
+    check_matmul(y[:, rows], x.cpu().numpy(), *part, bits, g)
+    st, y2, _ = _call(hip.load(), x, (q.qweight, q.scale, q.zero_point), n, bits, g, n, ws=False, bias=q.bias)
+    assert st == 0
+    check_matmul(y2[:, rows], x.cpu().numpy(), *part, bits, g)
+    xb = x.to(torch.bfloat16)
+    assert torch.equal(q(xb), q(xb.to(torch.float16)))
+
+
+@pytest.mark.parametrize("m", [7, 17, 70])
+def test_layouts_the_batch_kernel_does_not_take(m):
+    """Scales off a 4-byte boundary go to the other kernels, with bfloat16 x too; a workspace that is too small is not used."""
+    from bitween_amd.kernels import hip_loader
+    lib = hip_loader.load()
+    bits, g, k, n = 4, 128, 1280, 260
+    _, qw, s16, z16, b16 = quantized_layer(n, k, bits, g, seed=m)
+    sbuf = torch.zeros(s16.size + 1, dtype=torch.float16, device="cuda")
+    sbuf[1:] = to_gpu(s16).reshape(-1)
+    s_odd = sbuf[1:].view(n, k // g)
+    x = torch.randn(m, k, device="cuda", dtype=torch.float16)
+    d = [to_gpu(qw), s_odd, to_gpu(z16)]
+    st, y, _ = _call(lib, x, d, n, bits, g, n)
+    assert st == 0
+    check_matmul(y, x.cpu().numpy(), qw, s16, z16, None, bits, g)
+    from bitween_amd.kernels import hip_loader as hip
+    xb = x.to(torch.bfloat16)
+    yb = hip.quantized_matmul_hip(xb, d[0], s_odd, d[2], to_gpu(b16), bits, g)
+    check_matmul(yb, xb.to(torch.float16).cpu().numpy(), qw, s16, z16, b16, bits, g)
+    assert lib.bw_qlinear_ws(None, 0, m, k, k, d[0].data_ptr(), d[1].data_ptr(), d[2].data_ptr(), None, n, bits, g, y.data_ptr(), n, None, 0, None) == -1
+    assert lib.bw_qlinear_ws(x.data_ptr(), 2, m, k, k, d[0].data_ptr(), d[1].data_ptr(), d[2].data_ptr(), None, n, bits, g, y.data_ptr(), n, None, 0, None) == -2
