@@ -162,6 +162,13 @@ __global__ __launch_bounds__(WAVES * 64) void qgemm_kernel(const GemmArgs a) {
     // WIDE_META (rows of scales on 4-byte boundaries): META4 = 8-byte requests over runs of K steps; PAIR = a lane whose
     // values span two groups fetches both scales (zero points) with one 4-byte request instead of two 2-byte ones
     constexpr bool META4 = WIDE_META && C::CAN_META4, PAIR = WIDE_META && !C::CAN_META4 && C::NG == 2;
+    // QMETA (natural order, one 2-byte scale and zero point per lane, tile and step): the lanes ask for them four to a row -
+    // 16 address-unit cycles a request; in operand order, neighbouring lanes on neighbouring rows, it is 60, and with groups of
+    // 32 at 8 bits the 8 requests of a step then set the pace of the loop - and the pair is handed to the lane that
+    // multiplies by ds_bpermute (4096 -> 11008, 509 rows, W8 g32: 75 -> 60 us; 4096 -> 14336, 512 rows, W4 g32 69.7 -> 62.0, W2 g32
+    // 60.5 -> 55.7).  Not at larger groups (an odd number of them), where several lanes share a scale anyway and it gained
+    // nothing, and not with 256-row tiles: their step has twice the MFMAs for the same requests, and no register to spare.
+    constexpr bool QMETA = NAT && !META4 && GROUP == 32 && MT <= 8;
     constexpr uint32_t kOob = 0x80000000u;
     extern __shared__ __attribute__((aligned(16))) char smem[];
 #ifdef BW_TUNE
@@ -191,7 +198,7 @@ __global__ __launch_bounds__(WAVES * 64) void qgemm_kernel(const GemmArgs a) {
         // (256-row tiles add a scalar chunk offset that is itself "out of range" past the last chunk: rows past N then
         // read the last row's bytes instead of relying on a sum that could wrap; their outputs are never stored)
         w_off[j] = row < a.N ? (uint32_t)row * a.row_bytes + kq * C::LB * C::WL : NAT ? (uint32_t)(a.N - 1) * a.row_bytes + kq * C::LB * C::WL : kOob;
-        m_off[j] = (uint32_t)min(row, a.N - 1) * groups * 2;
+        m_off[j] = (uint32_t)min(QMETA ? n0 + 16 * j + (lane >> 2) : row, a.N - 1) * groups * 2;
     }
     // 128-row tiles: byte offsets of the staging units of a thread
     uint32_t x_off[C::XL];
@@ -237,7 +244,7 @@ __global__ __launch_bounds__(WAVES * 64) void qgemm_kernel(const GemmArgs a) {
         ws.w[j][l] = __builtin_amdgcn_raw_buffer_load_b128(rw, in ? w_off[j] + b : kOob, 0, 0);
     };
     auto issue_meta = [&](int j, int which, int c, WSet& ws) {   // which: 0 = scales, 1 = zero points
-        const int g0 = min((c * C::CHUNK_K + kq * C::VPL) / GROUP, groups - C::NG);
+        const int g0 = min((c * C::CHUNK_K + (QMETA ? lane & 3 : kq) * C::VPL) / GROUP, groups - C::NG);
         if constexpr (PAIR) {                                       // g0 is even: both entries in one aligned word
             if (which == 0) ws.s[j][0] = __builtin_amdgcn_raw_buffer_load_b32(rs, m_off[j] + g0 * 2, 0, 0);
             else ws.z[j][0] = __builtin_amdgcn_raw_buffer_load_b32(rz, m_off[j] + g0 * 2, 0, 0);
@@ -290,6 +297,8 @@ __global__ __launch_bounds__(WAVES * 64) void qgemm_kernel(const GemmArgs a) {
     using GC = std::conditional_t<NAT, GroupConstNat<BITS>, GroupConst<BITS>>;
     h8 xf[C::XSETS][C::XRING];
     h2 wf[2][NT][4];                                      // weight fragments as 4 register pairs each
+    uint32_t pm[NT];                                      // QMETA: (scale | zero point << 16) of the lane's row and values
+    const uint32_t pm_from = (uint32_t)(((nl << 2) | kq) << 2);
     // group constants of tile j for the step that reads `from` (META4: half `half` of m_cur / m_next)
     auto set_consts = [&](GC* gj, int j, const WSet& from, const u2 (*m)[2], int half) {
 #pragma unroll
@@ -300,6 +309,8 @@ __global__ __launch_bounds__(WAVES * 64) void qgemm_kernel(const GemmArgs a) {
             else if constexpr (META4)                            // two groups per step: lanes kq >= 2 take the second
                 gj[g].set(__builtin_bit_cast(_Float16, (uint16_t)(m[j][0][half] >> (16 * (kq >> 1)))),
                           __builtin_bit_cast(_Float16, (uint16_t)(m[j][1][half] >> (16 * (kq >> 1)))));
+            else if constexpr (QMETA)
+                gj[g].set(__builtin_bit_cast(_Float16, (uint16_t)pm[j]), __builtin_bit_cast(_Float16, (uint16_t)(pm[j] >> 16)));
             else if constexpr (PAIR)
                 gj[g].set(__builtin_bit_cast(_Float16, (uint16_t)(from.s[j][0] >> (16 * g))), __builtin_bit_cast(_Float16, (uint16_t)(from.z[j][0] >> (16 * g))));
             else
@@ -550,6 +561,13 @@ __global__ __launch_bounds__(WAVES * 64) void qgemm_kernel(const GemmArgs a) {
                 static_for<0, count>([&](auto oc) { unpack_op(std::integral_constant<int, first + decltype(oc)::value>{}); });
                 // ---- the next chunk's activations: unit i of the wave in slot i of the first MFMA step ----
                 if constexpr (t == 0 && j == 1) x_dma16(i, c + 1, nxt);
+                // ---- QMETA: tile r's scale and zero point of the next chunk to the lanes that use them.  Assembly like the
+                // fragment reads: the constants are formed two MFMA steps later, behind the wait for a fragment that was asked
+                // for after this (LDS operations complete in order); one more operation in flight only makes the waits stricter.
+                if constexpr (QMETA && t == 0 && k == RG - 2) {
+                    const uint32_t pair = wsn.s[r][0] | (wsn.z[r][0] << 16);
+                    asm volatile("ds_bpermute_b32 %0, %1, %2" : "=v"(pm[r]) : "v"(pm_from), "v"(pair));
+                }
                 // ---- fragment ring ----
                 if constexpr (j == NT - 1) {
                     constexpr int i2 = (i + C::XRING) % MT, t2 = t + (i + C::XRING) / MT;
@@ -691,6 +709,7 @@ __global__ __launch_bounds__(WAVES * 64) void qgemm_kernel(const GemmArgs a) {
     GC gc0[NT][C::NG], gc1[NT][C::NG];
 #pragma unroll
     for (int j = 0; j < NT; j++) {
+        if constexpr (QMETA) pm[j] = __builtin_amdgcn_ds_bpermute((int)pm_from, (int)(set0.s[j][0] | (set0.z[j][0] << 16)));
         set_consts(gc0[j], j, set0, m_cur, 0);
         const h8 f = unpack(set0, j, 0, gc0[j]);
 #pragma unroll
