@@ -174,14 +174,10 @@ Tensor input_grad(const Tensor& go, const Tensor& qweight, const Tensor& scale, 
         int64_t ldg = n;
         if (!g.is_contiguous()) {
             if (g.dim() != 2) g = g.reshape({m, n});
-            if (g.stride(1) == 1 && g.stride(0) >= n && g.stride(0) % 8 == 0) ldg = g.stride(0);
+            if (g.stride(1) == 1 && g.stride(0) >= n) ldg = g.stride(0);
             else g = g.contiguous();
         }
-        if (!aligned16(g.const_data_ptr())) {
-            g = g.clone(at::MemoryFormat::Contiguous);
-            ldg = n;
-        }
-        if (ldg % 8 == 0) {
+        if (n >= 32) {
             c10::SmallVector<int64_t, 5> shape(go.sizes().begin(), go.sizes().end());
             shape.back() = k;
             Tensor gx = empty(shape, t, go.device());

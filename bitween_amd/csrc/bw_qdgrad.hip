@@ -9,7 +9,7 @@
 //
 // The reduction runs over N, the dimension the packed words do NOT run along, so a weight tile has to be
 // transposed on its way to the matrix core.  A workgroup owns a 128 or 256 (m) x 128 (k) tile of grad_x and walks
-// N in steps of 32 rows:
+// N in steps of 32 rows (any N from 32 on, any K of whole groups, any pitch of grad_y):
 //   * 256 threads each take 16 consecutive k of one row n (one group: groups are >= 32 wide), dequantise them to
 //     the reference's W16 in natural k order (magic-number unpack, exact q - z, one multiply by the scale) and write
 //     them as they are - 32 bytes - into an LDS tile stored n-major (row n holds the 128 k of the tile; the 32-byte
@@ -65,6 +65,9 @@ BW_DEV int w_swizzle(int n) { return (n & 3) | (((n >> 3) & 1) << 2); }
 
 typedef short s4 __attribute__((ext_vector_type(4)));
 
+// 16 bytes of a grad_y row at any element: rows of an odd pitch start off every wider boundary (one global load all the same)
+typedef u4 u4_any __attribute__((aligned(2)));
+
 template <int BITS> struct WLoad;
 template <> struct WLoad<4> { typedef u2 type; };
 template <> struct WLoad<8> { typedef u4 type; };
@@ -105,29 +108,30 @@ BW_DEV f4 mfma16(const h8& a, const h8& b, const f4& c) {
 template <int BITS, int GROUP, int MT, int DT>
 __global__ __launch_bounds__(DTHREADS, MT == 4 ? 3 : 2) void qdgrad_kernel(const DgradArgs a) {   // workgroups per CU: 3 (<= 168 registers) or 2
     constexpr int DM = DgradTile<MT>::DM, A_BYTES = DgradTile<MT>::A_BYTES, STAGE = DgradTile<MT>::STAGE;
-    constexpr int GR = DM / 128;                                      // grad_y rows a thread stages
+    constexpr int GR = DM / 64;                                       // grad_y rows a thread stages 16 bytes of
     constexpr int PD = 2;                                             // steps of global loads in flight (even)
     extern __shared__ __attribute__((aligned(16))) char smem[];
     typedef typename WLoad<BITS>::type wload_t;
     const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
     const int tile = blockIdx.x / a.splits, split = blockIdx.x % a.splits;
     const int m0 = (tile / a.tiles_k) * DM, k0 = (tile % a.tiles_k) * DK;
-    const int nsteps = a.N / DN;
+    const int nsteps = (a.N + DN - 1) / DN;
     const int s_begin = split * a.steps_per_split;
     const int s_end = min(s_begin + a.steps_per_split, nsteps);
 
-    // loader roles
+    // loader roles.  Of a last tile of k that is not whole, the segments past K repeat the last one and are not stored.
     const int wn = tid >> 3, wks = tid & 7;                           // weight: row of the step, 16-value segment
-    const int gm = tid >> 1, gpart = tid & 1;                         // grad_y: row of the tile, 32-byte half
-    const char* wp = a.qweight + (int64_t)wn * a.row_bytes + (int64_t)(k0 + wks * 16) * BITS / 8;
-    const int gcol = (k0 + wks * 16) / GROUP;
+    const int gm = tid >> 2, gpart = tid & 3;                         // grad_y: row of the tile, 16-byte piece - four lanes to a row's 64 bytes
+    const int wk0 = min(k0 + wks * 16, a.K - 16);
+    const char* wp = a.qweight + (int64_t)wn * a.row_bytes + (int64_t)wk0 * BITS / 8;
+    const int gcol = wk0 / GROUP;
     const _Float16* sp = a.scale + (int64_t)wn * a.groups + gcol;
     const _Float16* zp = a.zp + (int64_t)wn * a.groups + gcol;
     // rows past M repeat the last row: every output row depends on its own grad_y row only, and rows >= M are
     // never stored
     const _Float16* gp[GR];
 #pragma unroll
-    for (int r = 0; r < GR; r++) gp[r] = a.go + (int64_t)min(m0 + gm + 128 * r, a.M - 1) * a.ldg + gpart * 16;
+    for (int r = 0; r < GR; r++) gp[r] = a.go + (int64_t)min(m0 + gm + 64 * r, a.M - 1) * a.ldg + gpart * 8;
     // a thread's 16 values are one 32-byte piece of row wn of the weight tile
     const int b_dst = wn * (DK * 2) + ((wks ^ w_swizzle(wn)) * 32);
 
@@ -135,17 +139,15 @@ __global__ __launch_bounds__(DTHREADS, MT == 4 ? 3 : 2) void qdgrad_kernel(const
     // unconditional - past the slice's end they repeat its last step - so the wait counts stay exact.
     wload_t wreg[PD];
     _Float16 sreg[PD], zreg[PD];
-    u4 greg[PD][2 * GR];
+    u4 greg[PD][GR];
+    // a last step that is not whole covers the last 32 rows of W; those that an earlier step had are given a scale of zero
     auto issue = [&](int step, int slot) {
-        const int64_t n0 = (int64_t)min(step, s_end - 1) * DN;
+        const int64_t n0 = min(min(step, s_end - 1) * DN, a.N - DN);
         wreg[slot] = *reinterpret_cast<const wload_t*>(wp + n0 * a.row_bytes);
         sreg[slot] = sp[n0 * a.groups];
         zreg[slot] = zp[n0 * a.groups];
 #pragma unroll
-        for (int r = 0; r < GR; r++) {
-            greg[slot][2 * r] = *reinterpret_cast<const u4*>(gp[r] + n0);
-            greg[slot][2 * r + 1] = *reinterpret_cast<const u4*>(gp[r] + n0 + 8);
-        }
+        for (int r = 0; r < GR; r++) greg[slot][r] = *reinterpret_cast<const u4_any*>(gp[r] + n0);
     };
 
     f4 acc[4][MT];
@@ -161,11 +163,12 @@ __global__ __launch_bounds__(DTHREADS, MT == 4 ? 3 : 2) void qdgrad_kernel(const
     const int tr_swz = w_swizzle(8 * q + (l16 >> 2));
 
     // slot -> LDS stage: dequantise the 16 weights and scatter them transposed; copy the grad_y rows
-    auto fill = [&](int slot, int stage, bool live) {
+    auto fill = [&](int slot, int stage, int step) {
+        const bool live = step < s_end && min(step * DN, a.N - DN) + wn >= step * DN;
         char* As = smem + stage * STAGE;
         char* Bs = As + A_BYTES;
         GroupConstNat<BITS> gc;
-        gc.set(live ? sreg[slot] : (_Float16)0.f, zreg[slot]);        // past the slice's end: weights of zero
+        gc.set(live ? sreg[slot] : (_Float16)0.f, zreg[slot]);        // past the slice's end, or counted before: weights of zero
         h2 w16[8];
         uint32_t wd[8];                                               // the 8 pairs in the gradient's type
         if constexpr (DT == BW_F16) {
@@ -181,11 +184,7 @@ __global__ __launch_bounds__(DTHREADS, MT == 4 ? 3 : 2) void qdgrad_kernel(const
         *reinterpret_cast<u4*>(Bs + b_dst) = u4{wd[0], wd[1], wd[2], wd[3]};
         *reinterpret_cast<u4*>(Bs + b_dst + 16) = u4{wd[4], wd[5], wd[6], wd[7]};
 #pragma unroll
-        for (int r = 0; r < GR; r++) {
-            u4* dst = reinterpret_cast<u4*>(As + (gm + 128 * r) * DPITCH + gpart * 32);
-            dst[0] = greg[slot][2 * r];
-            dst[1] = greg[slot][2 * r + 1];
-        }
+        for (int r = 0; r < GR; r++) *reinterpret_cast<u4*>(As + (gm + 64 * r) * DPITCH + gpart * 16) = greg[slot][r];
     };
 
     // Step s: read the fragments of stage s & 1, then - in the shadow of the step's MFMAs - fill the other
@@ -194,7 +193,7 @@ __global__ __launch_bounds__(DTHREADS, MT == 4 ? 3 : 2) void qdgrad_kernel(const
     if (s_begin < s_end) {
 #pragma unroll
         for (int d = 0; d < PD; d++) issue(s_begin + d, d);
-        fill(0, 0, true);
+        fill(0, 0, s_begin);
         issue(s_begin + PD, 0);
         __syncthreads();
     }
@@ -220,7 +219,7 @@ __global__ __launch_bounds__(DTHREADS, MT == 4 ? 3 : 2) void qdgrad_kernel(const
             }
 #pragma unroll
             for (int j = 0; j < MT; j++) bf[j] = *reinterpret_cast<const h8*>(As + (wm + 16 * j + l16) * DPITCH + q * 16);
-            fill((d + 1) % PD, (d + 1) & 1, step + 1 < s_end);
+            fill((d + 1) % PD, (d + 1) & 1, step + 1);
             issue(step + 1 + PD, (d + 1) % PD);
 #pragma unroll
             for (int j = 0; j < MT; j++)
@@ -247,6 +246,7 @@ __global__ __launch_bounds__(DTHREADS, MT == 4 ? 3 : 2) void qdgrad_kernel(const
 #pragma unroll
             for (int i = 0; i < 4; i++) {
                 const f4 v = acc[i][j];
+                if (k0 + wk + 16 * i + 4 * q >= a.K) continue;
                 _Float16* dst = a.gx + (int64_t)m * a.ldx + k0 + wk + 16 * i + 4 * q;
                 *reinterpret_cast<u2*>(dst) = u2{pack2<DT>(v[0], v[1]), pack2<DT>(v[2], v[3])};
             }
@@ -261,7 +261,7 @@ __global__ __launch_bounds__(256) void qdgrad_reduce_kernel(const DgradArgs a) {
     const int quad = (int)(blockIdx.x * blockDim.x + threadIdx.x);    // < DM * DKT / 4
     const int ml = quad / (DKT / 4), kl = (quad % (DKT / 4)) * 4;
     const int m = (tile / a.tiles_k) * DM + ml, k = (tile % a.tiles_k) * DKT + kl;
-    if (m >= a.M) return;
+    if (m >= a.M || k >= a.K) return;
     const float* src = a.ws + (size_t)tile * a.splits * (DM * DKT) + ml * DKT + kl;
     f4 v = {0.f, 0.f, 0.f, 0.f};
     for (int z = 0; z < a.splits; z++) {
@@ -588,7 +588,7 @@ inline int dgrad_cus() {
 // Returns the rows of m per tile (256 or 128), 0 = the stepping kernel.
 inline int dgrad256_rows(int64_t M, int64_t N, int64_t K, int64_t ldg, int bits, int group) {
     const int64_t lim = (int64_t)1 << 31;
-    if (K % QK || N % QN || N * (K * bits / 8) >= lim || (M + QM) * ldg * 2 >= lim || N * (K / group) * 2 >= lim) return 0;
+    if (K % QK || N % QN || ldg % 8 || N * (K * bits / 8) >= lim || (M + QM) * ldg * 2 >= lim || N * (K / group) * 2 >= lim) return 0;
     const int64_t col_steps = (K / QK) * (N / QN);
     if (M > 384 && ((M + QM - 1) / QM) * col_steps >= 3072) return QM;
     if (M <= 512 && ((M + 127) / 128) * col_steps >= 2560) return 128;
@@ -624,9 +624,9 @@ inline DgradPlan dgrad_plan(int64_t M, int64_t N, int64_t K, bool have_workspace
     DgradPlan p;
     p.mt = M > 512 ? 8 : 4;
     const int DM = 32 * p.mt;
-    p.tiles_k = (int)(K / DK);
+    p.tiles_k = (int)((K + DK - 1) / DK);
     p.tiles = p.tiles_k * (int)((M + DM - 1) / DM);
-    const int nsteps = (int)(N / DN);
+    const int nsteps = (int)((N + DN - 1) / DN);
     p.splits = 1;
     p.steps_per_split = nsteps;
     p.ws_bytes = 0;
@@ -649,8 +649,7 @@ inline DgradPlan dgrad_plan(int64_t M, int64_t N, int64_t K, bool have_workspace
 }
 
 inline bool dgrad_fast_shape(int64_t M, int64_t N, int64_t K, int64_t ldg, int64_t ldx, int bits, int group) {
-    return (group == 32 || group == 64 || group == 128) && K % DK == 0 && N % DN == 0 && ldg % 8 == 0 && ldx % 4 == 0 &&
-           M >= 1 && M < ((int64_t)1 << 24) && N * (K * bits / 8) < ((int64_t)1 << 40);
+    return (group == 32 || group == 64 || group == 128) && N >= DN && ldx % 4 == 0 && M >= 1 && N < ((int64_t)1 << 30) && M < ((int64_t)1 << 24) && N * (K * bits / 8) < ((int64_t)1 << 40);
 }
 
 template <int BITS, int GROUP, int MT, int DT>
@@ -714,7 +713,7 @@ int launch_dgrad(DgradArgs a, void* workspace, size_t workspace_bytes, hipStream
     if (g_dgrad_force == 8) return launch_dgrad256<BITS, GROUP, DT, 8>(a, workspace, workspace_bytes, stream);
     if (g_dgrad_force != 1)
 #endif
-    if (const int rows = dgrad_use256(a.M, a.N, a.K, a.ldg, BITS, GROUP, workspace != nullptr))
+    if (const int rows = bw_aligned(a.go, 16) ? dgrad_use256(a.M, a.N, a.K, a.ldg, BITS, GROUP, workspace != nullptr) : 0)
         return rows == QM ? launch_dgrad256<BITS, GROUP, DT, 16>(a, workspace, workspace_bytes, stream)
                           : launch_dgrad256<BITS, GROUP, DT, 8>(a, workspace, workspace_bytes, stream);
     const DgradPlan p = dgrad_plan(a.M, a.N, a.K, workspace != nullptr);
@@ -753,7 +752,7 @@ extern "C" int bw_qdgrad(const void* grad_y, int act_dtype, int64_t M, int64_t N
     if (!bw_shape_ok(N, K, bits, group) || M < 1 || ldg < N || ldx < K) return BW_EINVAL;
     if (act_dtype != BW_F16 && act_dtype != BW_BF16) return BW_EUNSUPPORTED;
     if (!dgrad_fast_shape(M, N, K, ldg, ldx, bits, group)) return BW_EUNSUPPORTED;
-    if (!bw_aligned(grad_y, 16) || !bw_aligned(grad_x, 8) || !bw_aligned(qweight, 16)) return BW_EALIGN;
+    if (!bw_aligned(grad_y, 2) || !bw_aligned(grad_x, 8) || !bw_aligned(qweight, 16)) return BW_EALIGN;
     if (workspace && !bw_aligned(workspace, 16)) return BW_EALIGN;
     DgradArgs a;
     a.go = (const _Float16*)grad_y; a.qweight = (const char*)qweight; a.scale = (const _Float16*)scale16;

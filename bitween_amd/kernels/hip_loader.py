@@ -279,12 +279,8 @@ def quantized_input_grad(grad_y, qweight, scale, zero_point, bits, group_size):
     k = qweight.shape[1] * (32 // bits)
     if m == 0 or qweight.shape[0] != n:
         return None
-    if grad_y.stride(1) != 1 or grad_y.stride(0) % 8 or grad_y.data_ptr() % 16:
+    if grad_y.stride(1) != 1:
         grad_y = grad_y.contiguous()
-        if grad_y.data_ptr() % 16:                         # contiguous already, but at an odd offset of its storage
-            grad_y = grad_y.clone()
-        if grad_y.stride(0) % 8:
-            return None
     qweight, scale, zero_point = qweight.contiguous(), scale.contiguous(), zero_point.contiguous()
     lib = load()
     grad_x = torch.empty((m, k), dtype=grad_y.dtype, device=grad_y.device)

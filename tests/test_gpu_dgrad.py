@@ -285,3 +285,48 @@ def test_dgrad_256_tiles_vs_oracle(bits, g, dtype):
             assert (np.abs(got - ref) <= bound).all(), float((np.abs(got - ref) / bound).max())
             for r, c in hot.items():
                 assert np.array_equal(gx[r, :k].float().cpu().numpy(), wt[c].astype(np.float32))
+
+
+@pytest.mark.parametrize("dtype", ["f16", "bf16"])
+@pytest.mark.parametrize("bits,g", COMBOS)
+def test_dgrad_ragged_n_k_and_pitch(bits, g, dtype):
+    """N that ends inside a step of 32 rows (33: one row past the first step; 32: the smallest; odd), K that ends inside a tile
+    of 128, odd pitches of grad_y, a grad_y off every 16-byte boundary; sliced and unsliced, both tile heights; one-hot
+    rows return rows of the weight bit for bit, the padding of grad_y (NaN) is never read."""
+    from bitween_amd.kernels import hip_loader
+    lib = hip_loader.load()
+    stream = ctypes.c_void_p(torch.cuda.current_stream().cuda_stream)
+    tdt, code = (torch.float16, 0) if dtype == "f16" else (torch.bfloat16, 1)
+    for (n, k, m) in ((32, g, 3), (33, 128 + g, 17), (1001, 5 * g, 130), (95, 3 * 128 + 64 if g < 128 else 640, 600), (3001, 192 if g < 128 else 384, 40)):
+        _, qw, s16, z16, _ = quantized_layer(n, k, bits, g, seed=n + k + bits + g, outliers=True, bias=False)
+        d = [to_gpu(a) for a in (qw, s16, z16)]
+        wt = orc.dequantize_f16(qw, s16, z16, g, bits).astype(np.float32) if dtype == "f16" else orc.dequantize_bf16(qw, s16, z16, g, bits)
+        ldg = n + 3
+        buf = torch.full((m * ldg + 1,), float("nan"), dtype=tdt, device="cuda")
+        view = buf[1:].view(m, ldg)
+        gen = torch.Generator(device="cuda").manual_seed(n)
+        go = torch.randn(m, n, device="cuda", generator=gen).to(tdt)
+        hot = {0: n - 1, m // 2: 0, m - 1: n // 32 * 32 - 1}
+        for r, c in hot.items():
+            go[r] = 0
+            go[r, c] = 1.0
+        view[:, :n] = go
+        need = lib.bw_qdgrad_workspace_bytes(m, n, k, bits, g)
+        ws = torch.empty(max(need, 16), dtype=torch.uint8, device="cuda")
+        go_np = go.float().cpu().numpy()
+        ref = orc.qlinear_backward(go_np if dtype == "bf16" else go_np.astype(np.float16), qw, s16, z16, bits, g,
+                                   **({"dtype": "bf16"} if dtype == "bf16" else {}))
+        mag = np.abs(go_np.astype(np.float64)) @ np.abs(wt.astype(np.float64))
+        bound = (2.0 ** -10 if dtype == "f16" else 2.0 ** -8) * np.abs(ref) + 2e-6 * mag + 1e-7
+        for use_ws in (True, False):
+            gx = torch.full((m, k + 4), 7.0, dtype=tdt, device="cuda")
+            st = lib.bw_qdgrad(view.data_ptr(), code, m, n, ldg, d[0].data_ptr(), d[1].data_ptr(), d[2].data_ptr(), k, bits, g,
+                               gx.data_ptr(), k + 4, ws.data_ptr() if (use_ws and need) else None, need if use_ws else 0, stream)
+            torch.cuda.synchronize()
+            assert st == 0 and (gx[:, k:] == 7.0).all()
+            got = gx[:, :k].double().cpu().numpy()
+            assert (np.abs(got - ref) <= bound).all(), (n, k, m, float((np.abs(got - ref) / bound).max()))
+            for r, c in hot.items():
+                assert np.array_equal(gx[r, :k].float().cpu().numpy(), wt[c].astype(np.float32))
+    assert lib.bw_qdgrad(view.data_ptr(), code, 1, 31, 31, d[0].data_ptr(), d[1].data_ptr(), d[2].data_ptr(), 128, bits, g,
+                         gx.data_ptr(), 128, None, 0, stream) == -2     # fewer rows of W than a step
