@@ -33,30 +33,63 @@ BW_DEV void store_meta(void* p, int dtype, int64_t i, float v) {
     else ((int32_t*)p)[i] = (int32_t)v;
 }
 
-// Load the VPI consecutive weights of one output word as float32.
-template <int WDT, int VPI>
-BW_DEV void load_vals(const void* w, int64_t off, float* v) {
+// One 16-byte piece of weights as float32: 4 of them, or 8.
+template <int WDT>
+BW_DEV void widen(const u4& t, float* v) {
     if constexpr (WDT == BW_F32) {
-        const f4* p = reinterpret_cast<const f4*>((const float*)w + off);
 #pragma unroll
-        for (int i = 0; i < VPI / 4; i++) { f4 t = p[i]; v[4 * i] = t[0]; v[4 * i + 1] = t[1]; v[4 * i + 2] = t[2]; v[4 * i + 3] = t[3]; }
-    } else if constexpr (VPI == 4) {
-        const u2 t = *reinterpret_cast<const u2*>((const uint16_t*)w + off);
-        const uint16_t h[4] = {(uint16_t)t[0], (uint16_t)(t[0] >> 16), (uint16_t)t[1], (uint16_t)(t[1] >> 16)};
-#pragma unroll
-        for (int i = 0; i < 4; i++) v[i] = WDT == BW_F16 ? (float)__builtin_bit_cast(_Float16, h[i]) : bf16_to_f32(h[i]);
+        for (int i = 0; i < 4; i++) { const uint32_t e = t[i]; v[i] = __builtin_bit_cast(float, e); }   // (not of t[i] itself: that takes element 0)
     } else {
-        const u4* p = reinterpret_cast<const u4*>((const uint16_t*)w + off);
 #pragma unroll
-        for (int i = 0; i < VPI / 8; i++) {
-            const u4 t = p[i];
-#pragma unroll
-            for (int j = 0; j < 4; j++) {
-                const uint16_t lo = (uint16_t)t[j], hi = (uint16_t)(t[j] >> 16);
-                v[8 * i + 2 * j] = WDT == BW_F16 ? (float)__builtin_bit_cast(_Float16, lo) : bf16_to_f32(lo);
-                v[8 * i + 2 * j + 1] = WDT == BW_F16 ? (float)__builtin_bit_cast(_Float16, hi) : bf16_to_f32(hi);
-            }
+        for (int j = 0; j < 4; j++) {
+            const uint16_t lo = (uint16_t)t[j], hi = (uint16_t)(t[j] >> 16);
+            v[2 * j] = WDT == BW_F16 ? (float)__builtin_bit_cast(_Float16, lo) : bf16_to_f32(lo);
+            v[2 * j + 1] = WDT == BW_F16 ? (float)__builtin_bit_cast(_Float16, hi) : bf16_to_f32(hi);
         }
+    }
+}
+
+// The VPT consecutive weights of thread `tcol` of a row as float32.
+//
+// STAGED: loaded by the wave together (all lanes call this; the threads of a wave are neighbours in the row).  A thread's own
+// 64 bytes in one go make every request of the wave 64 pieces of 16 bytes that far apart; here neighbouring lanes ask for
+// neighbouring pieces - whole lines, which the non-temporal hint needs - and each thread picks up its own from the wave's
+// block of LDS (`lds`, 64 bytes per thread).  Piece p of thread t lies in slot 4 t + (p ^ (t >> 2 & 3)), so that both accesses
+// spread over all banks.
+template <int WDT, int VPT, bool STAGED>
+BW_DEV void load_vals(const void* w, int64_t row_off, int tcol, int tpr, char* lds, float* v) {
+    constexpr int ESZ = WDT == BW_F32 ? 4 : 2, BYTES = VPT * ESZ, P = BYTES / 16;
+    if constexpr (STAGED) {
+        static_assert(P == 4, "64 bytes per thread");
+        const u4* row = reinterpret_cast<const u4*>((const char*)w + row_off * ESZ);
+        const int lane = (int)threadIdx.x & 63;
+        const int64_t first = (int64_t)__builtin_amdgcn_readfirstlane((int)(blockIdx.x * blockDim.x + threadIdx.x)) * P, last = (int64_t)tpr * P - 1;
+        u4* block = reinterpret_cast<u4*>(lds);
+        u4 in[P];
+#pragma unroll
+        for (int j = 0; j < P; j++) {
+            const int slot = 64 * j + lane, thread = slot >> 2;
+            const int64_t piece = first + 4 * thread + ((slot & 3) ^ (thread >> 2 & 3));
+            in[j] = __builtin_nontemporal_load(row + (piece < last ? piece : last));   // (threads past the row's end: anything)
+        }
+#pragma unroll
+        for (int j = 0; j < P; j++) block[64 * j + lane] = in[j];
+        __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+        __builtin_amdgcn_wave_barrier();
+        __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+#pragma unroll
+        for (int p = 0; p < P; p++) widen<WDT>(block[4 * lane + (p ^ (lane >> 2 & 3))], v + p * (16 / ESZ));
+        __builtin_amdgcn_wave_barrier();
+    } else if constexpr (BYTES < 16) {                       // one 8-bit word of a 16-bit type
+        const u2 t = *reinterpret_cast<const u2*>((const uint16_t*)w + row_off + (int64_t)tcol * VPT);
+        float q[8];
+        widen<WDT>(u4{t[0], t[1], 0u, 0u}, q);
+#pragma unroll
+        for (int i = 0; i < VPT; i++) v[i] = q[i];
+    } else {
+        const u4* p = reinterpret_cast<const u4*>((const char*)w + (row_off + (int64_t)tcol * VPT) * ESZ);
+#pragma unroll
+        for (int i = 0; i < P; i++) widen<WDT>(p[i], v + i * (16 / ESZ));
     }
 }
 
@@ -93,7 +126,7 @@ BW_DEV float quant_exact(float w, float s, float zf) {
 // sized for the worst case - the exact path, which a wave enters when any of its lanes needs it, was what a third
 // of the kernel's arithmetic went into.  Values inside the window (and infinities, NaN, groups so lopsided that the
 // window exceeds 1/2) are redone with the true IEEE divide.
-template <int BITS, int WDT, int MATH, int WPT>
+template <int BITS, int WDT, int MATH, int WPT, bool STAGED>
 __global__ __launch_bounds__(256) void quantize_pack_kernel(const void* __restrict__ w, const void* __restrict__ delta,
                                                             int64_t N, int K, int64_t ldw, int64_t ldd,
                                                             int group, int lpg, int32_t* __restrict__ qweight,
@@ -101,6 +134,8 @@ __global__ __launch_bounds__(256) void quantize_pack_kernel(const void* __restri
                                                             void* __restrict__ zp, int zp_dtype, int recip) {
     constexpr int VPI = 32 / BITS, VPT = VPI * WPT;
     constexpr float QMAX = (float)((1 << BITS) - 1);
+    __shared__ __attribute__((aligned(16))) char stage[STAGED ? 256 * 64 : 16];
+    char* lds = stage + (STAGED ? (threadIdx.x >> 6) * (64 * 64) : 0);   // the wave's block
     const int tpr = K / VPT;                             // threads per row; grid.x covers them, grid.y the rows
     int tcol = (int)(blockIdx.x * blockDim.x + threadIdx.x);
     const bool live = tcol < tpr;
@@ -108,10 +143,10 @@ __global__ __launch_bounds__(256) void quantize_pack_kernel(const void* __restri
     const int groups = K / group;
     for (int64_t row = blockIdx.y; row < N; row += gridDim.y) {
         float v[VPT];
-        load_vals<WDT, VPT>(w, row * ldw + (int64_t)tcol * VPT, v);
+        load_vals<WDT, VPT, STAGED>(w, row * ldw, tcol, tpr, lds, v);
         if (delta) {                                     // w + delta, one rounding to the weights' own type
             float dv[VPT];
-            load_vals<WDT, VPT>(delta, row * ldd + (int64_t)tcol * VPT, dv);
+            load_vals<WDT, VPT, STAGED>(delta, row * ldd, tcol, tpr, lds, dv);
 #pragma unroll
             for (int i = 0; i < VPT; i++) v[i] = rnd<WDT>(__fadd_rn(v[i], dv[i]));
         }
@@ -345,69 +380,67 @@ __global__ __launch_bounds__(256) void dequantize_kernel(const uint32_t* __restr
     }
 }
 
-// The same for the usual layouts, four words per thread, 256 words apart so that every load and store instruction of
-// a wave stays contiguous.  All four words and their (scale, zero point) are requested before the first is used: with
-// one 4-byte load per thread the kernel waits a memory round trip per 16 bytes it writes.  The group is a power of
-// two and at least a word wide, so a shift finds it; scale / zero point float16 (the module buffers) or float32 /
-// int32 (what quantize_rtn returns) are told apart once per thread, not per value.
-template <int BITS, int ODT>
-__global__ __launch_bounds__(256) void dequantize_x4_kernel(const uint32_t* __restrict__ qweight, const void* __restrict__ scale,
-                                                            const void* __restrict__ zp, int module_buffers, int64_t N, int K,
-                                                            int group_shift, void* __restrict__ out, int64_t ldo) {
-    constexpr int VPI = 32 / BITS;
-    const int words = K / VPI, groups = K >> group_shift;
-    const int w0 = (int)(blockIdx.x * 1024 + threadIdx.x);
-    for (int64_t row = blockIdx.y; row < N; row += gridDim.y) {
-        uint32_t w[4];
-        float s[4], z[4];
+// The same for the usual layouts.  A thread owns two 16-byte pieces of the output, 256 pieces apart, so that every store of a
+// wave is whole lines; the word a piece comes from is read by the lanes that share it.  (A packed word per thread stored
+// 64 bytes of float32 per 2-bit word, 16 at a time and 64 apart from lane to lane: 4096 x 11008 70 us, now 48.6; 8 bits 51 ->
+// 45.7.)  Pieces are counted over the whole tensor, so a row of any length fills the blocks (16-bit output of 4 bits,
+// 35.4 -> 26.4), and with K a multiple of the group the scales too are one flat array; only an output with padded rows
+// (PITCH) needs its row.  Both loads are made before the first is used; one piece per thread costs a quarter more, three and
+// four lose a few percent.  The group is a power of two and at least a piece wide; scale / zero point float16 (the module
+// buffers) or float32 / int32 (what quantize_rtn returns).  Outputs of more than half the Infinity Cache carry the non-temporal hint.
+constexpr int PPT = 2;
+template <int BITS, int ODT, bool PITCH>
+__global__ __launch_bounds__(256) void dequantize_flat_kernel(const void* __restrict__ qweight, const void* __restrict__ scale,
+                                                              const void* __restrict__ zp, int module_buffers, int64_t pieces,
+                                                              int group_shift, void* __restrict__ out, int pieces_per_row,
+                                                              int64_t pitch, int streaming) {
+    constexpr int OV = ODT == BW_F32 ? 4 : 8, BYTES = OV * BITS / 8;   // values, and bytes of packed weights, of a piece
+    using Packed = std::conditional_t<BYTES == 1, uint8_t, std::conditional_t<BYTES == 2, uint16_t, std::conditional_t<BYTES == 4, uint32_t, uint64_t>>>;
+    const int64_t p0 = (int64_t)blockIdx.x * (256 * PPT) + threadIdx.x;
+    Packed w[PPT];
+    float s[PPT], z[PPT];
 #pragma unroll
-        for (int j = 0; j < 4; j++) {
-            const int wc = w0 + 256 * j;
-            if (wc < words) {
-                w[j] = qweight[row * words + wc];
-                const int64_t gi = row * groups + ((wc * VPI) >> group_shift);
-                if (module_buffers) {
-                    s[j] = (float)((const _Float16*)scale)[gi];
-                    z[j] = (float)((const _Float16*)zp)[gi];
-                } else {
-                    s[j] = ((const float*)scale)[gi];
-                    z[j] = (float)((const int32_t*)zp)[gi];
-                }
+    for (int j = 0; j < PPT; j++) {
+        const int64_t p = p0 + 256 * j < pieces ? p0 + 256 * j : pieces - 1;
+        w[j] = ((const Packed*)qweight)[p];
+        const int64_t gi = p >> group_shift;                  // log2 of the pieces in a group
+        if (module_buffers) {
+            s[j] = (float)((const _Float16*)scale)[gi];
+            z[j] = (float)((const _Float16*)zp)[gi];
+        } else {
+            s[j] = ((const float*)scale)[gi];
+            z[j] = (float)((const int32_t*)zp)[gi];
+        }
+    }
+#pragma unroll
+    for (int j = 0; j < PPT; j++) {
+        const int64_t p = p0 + 256 * j;
+        if (p >= pieces) break;
+        float r[OV];
+#pragma unroll
+        for (int i = 0; i < OV; i++) {
+            const float q = (float)(uint32_t)((w[j] >> (i * BITS)) & ((1u << BITS) - 1));
+            r[i] = __fmul_rn(s[j], __fsub_rn(q, z[j]));                        // functional.py:70, modules.py:55
+            asm volatile("" : "+v"(r[i]));                                     // see dequantize_kernel
+        }
+        u4 d;
+#pragma unroll
+        for (int i = 0; i < 4; i++) {
+            if constexpr (ODT == BW_F32) d[i] = __builtin_bit_cast(uint32_t, r[i]);
+            else {
+                const uint16_t lo = ODT == BW_F16 ? __builtin_bit_cast(uint16_t, (_Float16)r[2 * i]) : f32_to_bf16(r[2 * i]);
+                const uint16_t hi = ODT == BW_F16 ? __builtin_bit_cast(uint16_t, (_Float16)r[2 * i + 1]) : f32_to_bf16(r[2 * i + 1]);
+                d[i] = (uint32_t)lo | ((uint32_t)hi << 16);
             }
         }
-#pragma unroll
-        for (int j = 0; j < 4; j++) {
-            const int wc = w0 + 256 * j;
-            if (wc >= words) break;
-            float r[VPI];
-#pragma unroll
-            for (int i = 0; i < VPI; i++) {
-                const float q = (float)((w[j] >> (i * BITS)) & ((1u << BITS) - 1));
-                r[i] = __fmul_rn(s[j], __fsub_rn(q, z[j]));                        // functional.py:70, modules.py:55
-                asm volatile("" : "+v"(r[i]));                                     // see dequantize_kernel
-            }
-            const int64_t o = row * ldo + (int64_t)wc * VPI;
-            if constexpr (ODT == BW_F32) {
-                float* p = (float*)out + o;
-#pragma unroll
-                for (int i = 0; i < VPI; i += 4) *reinterpret_cast<f4*>(p + i) = f4{r[i], r[i + 1], r[i + 2], r[i + 3]};
-            } else {
-                uint32_t d[VPI / 2];
-#pragma unroll
-                for (int i = 0; i < VPI / 2; i++) {
-                    const uint16_t lo = ODT == BW_F16 ? __builtin_bit_cast(uint16_t, (_Float16)r[2 * i]) : f32_to_bf16(r[2 * i]);
-                    const uint16_t hi = ODT == BW_F16 ? __builtin_bit_cast(uint16_t, (_Float16)r[2 * i + 1]) : f32_to_bf16(r[2 * i + 1]);
-                    d[i] = (uint32_t)lo | ((uint32_t)hi << 16);
-                }
-                uint16_t* p = (uint16_t*)out + o;
-                if constexpr (VPI == 4) {
-                    *reinterpret_cast<u2*>(p) = u2{d[0], d[1]};
-                } else {
-#pragma unroll
-                    for (int i = 0; i < VPI / 2; i += 4) *reinterpret_cast<u4*>(p + 2 * i) = u4{d[i], d[i + 1], d[i + 2], d[i + 3]};
-                }
-            }
+        int64_t o = p;
+        if constexpr (PITCH) {
+            const int64_t row = pieces >> 32 ? p / pieces_per_row : (int64_t)((uint32_t)p / (uint32_t)pieces_per_row);
+            o = row * pitch + (p - row * pieces_per_row);
         }
+        u4* dst = (u4*)out + o;
+        if (streaming) __builtin_nontemporal_store(d, dst);
+        else *dst = d;
     }
 }
 
@@ -424,14 +457,14 @@ bool quantize_fits(const void* w, const void* delta, int64_t K, int64_t ldw, int
            (!delta || (bw_aligned(delta, need) && (ldd * esz) % need == 0));
 }
 
-template <int BITS, int WDT, int MATH, int WPT>
+template <int BITS, int WDT, int MATH, int WPT, bool STAGED = false>
 int launch_quantize(const void* w, const void* delta, int64_t N, int64_t K, int64_t ldw, int64_t ldd, int group,
                     int32_t* qweight, void* scale, int sdt, void* zp, int zdt, int recip, hipStream_t st) {
     constexpr int VPT = 32 / BITS * WPT;
     const int tpr = (int)(K / VPT);
     const int block = tpr >= 256 ? 256 : ((tpr + 63) / 64) * 64;
     dim3 grid((unsigned)((tpr + block - 1) / block), (unsigned)(N < 65535 ? N : 65535));
-    hipLaunchKernelGGL((quantize_pack_kernel<BITS, WDT, MATH, WPT>), grid, dim3(block), 0, st, w, delta, N, (int)K, ldw, ldd,
+    hipLaunchKernelGGL((quantize_pack_kernel<BITS, WDT, MATH, WPT, STAGED>), grid, dim3(block), 0, st, w, delta, N, (int)K, ldw, ldd,
                        group, group / VPT, qweight, scale, sdt, zp, zdt, recip);
     return hipGetLastError() == hipSuccess ? BW_OK : BW_ELAUNCH;
 }
@@ -439,14 +472,21 @@ int launch_quantize(const void* w, const void* delta, int64_t N, int64_t K, int6
 template <int BITS, int WDT, int MATH>
 int launch_quantize_bits(const void* w, const void* delta, int64_t N, int64_t K, int64_t ldw, int64_t ldd, int group,
                          int32_t* qweight, void* scale, int sdt, void* zp, int zdt, int recip, hipStream_t st) {
-    // 64 bytes of 16-bit input per thread (32 weights) where the shape allows - everything a thread does once per
-    // group share (extrema exchange, the two divisions of the group's parameters, addressing, the stores) then costs
-    // half as much per weight as with 32 bytes, and the kernel is bound by arithmetic, not memory: 28.6 -> see the
-    // benchmark - else 32 bytes, else one word per thread, else the generic kernel
-    constexpr int VPI = 32 / BITS;
-    constexpr int WIDE = (WDT == BW_F32 ? 8 : 16) / VPI;
+    // 64 bytes of 16-bit input per thread (32 weights) where the shape allows - everything a thread does once per group share
+    // (extrema exchange, the two divisions of the group's parameters, addressing, the stores) then costs half as much per
+    // weight as with 32 bytes, and at 2 and 4 bits the kernel is bound by arithmetic - else 32 bytes, else one word per
+    // thread, else the generic kernel.
+    // Loads through LDS where memory is the bound: float32 input, of which 64 bytes are 16 weights (11008 x 4096 at 4 bits
+    // 40.1 -> 36.8 us, 4096 x 11008 43.7 -> 37.4), and 8-bit weights (38.2 -> 33.5; at 2 and 4 bits of 16-bit input they
+    // cost 7 % instead).  Below 4 M weights the launch is one short wait for memory, and the detour only lengthens it (512 x
+    // 576 float32 3.3 -> 3.7).
+    constexpr int VPI = 32 / BITS, WIDE = (WDT == BW_F32 ? 8 : 16) / VPI, WIDER = 2 * WIDE > 1 ? 2 * WIDE : 1;
+    constexpr bool STAGES = WDT == BW_F32 || BITS == 8;
+    if constexpr (STAGES) {
+        if (N * K >= ((int64_t)4 << 20) && quantize_fits<BITS, WDT, WIDER>(w, delta, K, ldw, ldd, group, qweight))
+            return launch_quantize<BITS, WDT, MATH, WIDER, true>(w, delta, N, K, ldw, ldd, group, qweight, scale, sdt, zp, zdt, recip, st);
+    }
     if constexpr (WDT != BW_F32) {
-        constexpr int WIDER = 32 / VPI;
         if (quantize_fits<BITS, WDT, WIDER>(w, delta, K, ldw, ldd, group, qweight))
             return launch_quantize<BITS, WDT, MATH, WIDER>(w, delta, N, K, ldw, ldd, group, qweight, scale, sdt, zp, zdt, recip, st);
     }
@@ -536,20 +576,27 @@ extern "C" int bw_dequantize(const int32_t* qweight, const void* scale, int scal
     const bool vec = bw_aligned(w_out, 16) && (ldo * esz) % 16 == 0;
     hipStream_t st = (hipStream_t)stream;
     const bool module_buffers = scale_dtype == BW_F16 && zp_dtype == BW_F16, returned = scale_dtype == BW_F32 && zp_dtype == BW_I32;
-    if (vec && (module_buffers || returned) && words >= 512 && (group & (group - 1)) == 0 && group >= vpi) {
+    const int ov = (int)(16 / esz);                          // values of a 16-byte piece of the output
+    if (vec && (module_buffers || returned) && (group & (group - 1)) == 0 && group >= ov && bw_aligned(qweight, 8)) {
         int shift = 0;
-        while ((1 << shift) < group) shift++;
-        const int bsz = 256;
-        dim3 g4((unsigned)((words + 1023) / 1024), (unsigned)(N < 65535 ? N : 65535));
+        while ((ov << shift) < group) shift++;
+        const int64_t pieces = N * K / ov, blocks = (pieces + 256 * PPT - 1) / (256 * PPT);
+        const int streaming = (int64_t)(N * K * esz) > ((int64_t)128 << 20);
+        if (blocks < ((int64_t)1 << 31)) {
 #define BW_D4(B, OD)                                                                                                    \
     if (bits == B && out_dtype == OD) {                                                                                 \
-        hipLaunchKernelGGL((dequantize_x4_kernel<B, OD>), g4, dim3(bsz), 0, st, (const uint32_t*)qweight, scale, zp,    \
-                           (int)module_buffers, N, (int)K, shift, w_out, ldo);                                          \
+        if (ldo == K)                                                                                                   \
+            hipLaunchKernelGGL((dequantize_flat_kernel<B, OD, false>), dim3((unsigned)blocks), dim3(256), 0, st, qweight, scale, zp, \
+                               (int)module_buffers, pieces, shift, w_out, 1, (int64_t)0, streaming);                    \
+        else                                                                                                            \
+            hipLaunchKernelGGL((dequantize_flat_kernel<B, OD, true>), dim3((unsigned)blocks), dim3(256), 0, st, qweight, scale, zp,  \
+                               (int)module_buffers, pieces, shift, w_out, (int)(K / ov), ldo / ov, streaming);          \
         return hipGetLastError() == hipSuccess ? BW_OK : BW_ELAUNCH;                                                    \
     }
         BW_D4(2, BW_F32) BW_D4(4, BW_F32) BW_D4(8, BW_F32) BW_D4(2, BW_F16) BW_D4(4, BW_F16) BW_D4(8, BW_F16)
         BW_D4(2, BW_BF16) BW_D4(4, BW_BF16) BW_D4(8, BW_BF16)
 #undef BW_D4
+        }
     }
     dim3 grid((unsigned)((words + 255) / 256), (unsigned)(N < 65535 ? N : 65535)), block(256);
 #define BW_D(B, OD)                                                                                                     \
