@@ -2,9 +2,9 @@
 //
 // A decode kernel runs for 3 ... 12 us, so what a call costs on the host decides how fast eager code decodes.  The same
 // steps written in Python (views, checks, the output tensor, a ctypes call with sixteen arguments) took 8 ... 9 us a
-// call, and an autograd node written in Python about 50 us per forward + backward.  Here: a layer's buffers are validated
-// once into a Plan (kept in the module's __dict__, compared with the module's current buffers by identity and address on
-// every call), the output comes straight from the caching allocator, and the node that backward runs is a C++ node.
+// call, and an autograd node written in Python about 50 us per forward + backward.  Here: a layer's buffers are looked at
+// on every call (dtype, shape, strides, device, address: about 0.1 us, so nothing about them has to be remembered), the
+// output comes straight from the caching allocator, and the node that backward runs is a C++ node.
 //
 // The kernels are reached through function pointers of the C ABI (bind(), called once by hip_loader), so this file
 // neither links the kernel library nor knows where it lies.  Anything a function here does not take - CPU tensors,
@@ -91,7 +91,7 @@ struct Layer {
 // What the kernels ask of a layer's buffers; false = the general Python path has to look at them.
 bool layer_of(const Tensor& qweight, const Tensor& scale, const Tensor& zero, const Tensor* bias, int64_t bits, int64_t group, Layer& l) {
     if (!lib.qlinear || (bits != 2 && bits != 4 && bits != 8) || group < 1) return false;
-    if (!qweight.is_cuda() || qweight.scalar_type() != at::kInt || qweight.dim() != 2 || !qweight.is_contiguous()) return false;
+    if (!qweight.is_cuda() || !qweight.has_storage() || qweight.scalar_type() != at::kInt || qweight.dim() != 2 || !qweight.is_contiguous()) return false;
     const int64_t n = qweight.size(0), k = qweight.size(1) * (32 / bits);
     if (n < 1 || k < 1 || k % group) return false;
     for (const Tensor* t : {&scale, &zero})
@@ -221,25 +221,9 @@ struct QuantizedLinearBackward : public torch::autograd::Node {
 
 // ---- Python side ----
 
-struct Plan {
-    PyObject_HEAD
-    PyObject* tensor[4];              // qweight, scale, zero_point, bias (or None): the objects that were validated
-    const void* address[4];
-    Layer layer;
-    bool usable;                      // false: these buffers go through the general path
-};
-
-void plan_dealloc(PyObject* self) {
-    for (PyObject* t : ((Plan*)self)->tensor) Py_XDECREF(t);
-    Py_TYPE(self)->tp_free(self);
-}
-
-PyTypeObject PlanType = {PyVarObject_HEAD_INIT(nullptr, 0)};
-
 // A plain tensor or parameter; subclasses have their own ideas of every operation and go through Python.
 inline bool plain(PyObject* o) { return THPVariable_CheckExact(o); }
 inline const Tensor& unpack(PyObject* o) { return THPVariable_Unpack(o); }
-inline const void* address(PyObject* o) { return o == Py_None ? nullptr : unpack(o).unsafeGetTensorImpl()->data(); }
 
 PyObject* none() { Py_RETURN_NONE; }
 
@@ -259,38 +243,26 @@ PyObject* guarded(F&& f) {
     END_HANDLE_TH_ERRORS
 }
 
-// The layer's plan: the one the module keeps while its four buffers are the same objects at the same addresses (a buffer
-// replaced through .data, .set_(), a load or a move is seen whichever one it is), a new one otherwise.
-Plan* plan_of(PyObject* dict) {
+// The module's buffers as they are now; false = the general path (or, with a Python error set, none).
+struct Module {
+    Tensor qweight, scale, zero, bias;                         // held: the interpreter may run while a call is under way
+    Layer layer;
+};
+
+bool module_of(PyObject* dict, Module& m) {
     PyObject* buffers = PyDict_GetItemWithError(dict, s_buffers);
-    if (!buffers || !PyDict_Check(buffers)) return nullptr;
-    PyObject* now[4] = {PyDict_GetItem(buffers, s_qweight), PyDict_GetItem(buffers, s_scale), PyDict_GetItem(buffers, s_zero),
-                        PyDict_GetItem(buffers, s_bias)};
-    if (!now[3]) now[3] = Py_None;
-    PyObject* kept = PyDict_GetItem(dict, s_plan);
-    if (kept && Py_TYPE(kept) == &PlanType) {
-        Plan* p = (Plan*)kept;
-        bool same = true;
-        for (int i = 0; i < 4; i++) same = same && p->tensor[i] == now[i];
-        for (int i = 0; same && i < 4; i++) same = p->address[i] == address(now[i]);
-        if (same) return p;
-    }
-    for (int i = 0; i < 4; i++)
-        if (!now[i] || !(plain(now[i]) || (i == 3 && now[i] == Py_None))) return nullptr;
-    PyObject *bits = PyDict_GetItem(dict, s_bits), *group = PyDict_GetItem(dict, s_group);
-    if (!bits || !group || !PyLong_Check(bits) || !PyLong_Check(group)) return nullptr;
-    Plan* p = PyObject_New(Plan, &PlanType);
-    if (!p) return nullptr;
+    PyObject *bits = PyDict_GetItemWithError(dict, s_bits), *group = PyDict_GetItemWithError(dict, s_group);
+    if (!buffers || !PyDict_Check(buffers) || !bits || !group || !PyLong_Check(bits) || !PyLong_Check(group)) return false;
+    PyObject* names[4] = {s_qweight, s_scale, s_zero, s_bias};
+    Tensor* out[4] = {&m.qweight, &m.scale, &m.zero, &m.bias};
     for (int i = 0; i < 4; i++) {
-        Py_INCREF(now[i]);
-        p->tensor[i] = now[i];
-        p->address[i] = address(now[i]);
+        PyObject* t = PyDict_GetItemWithError(buffers, names[i]);
+        if (i == 3 && (!t || t == Py_None)) break;
+        if (!t || !plain(t)) return false;
+        *out[i] = unpack(t);
     }
-    p->usable = layer_of(unpack(now[0]), unpack(now[1]), unpack(now[2]), now[3] == Py_None ? nullptr : &unpack(now[3]),
-                         PyLong_AsLong(bits), PyLong_AsLong(group), p->layer);
-    PyDict_SetItem(dict, s_plan, (PyObject*)p);
-    Py_DECREF(p);                                             // the module's dict holds it
-    return p;
+    const long b = PyLong_AsLong(bits), g = PyLong_AsLong(group);
+    return !PyErr_Occurred() && layer_of(m.qweight, m.scale, m.zero, m.bias.defined() ? &m.bias : nullptr, b, g, m.layer);
 }
 
 // forward(module.__dict__, x) -> y or None
@@ -298,29 +270,31 @@ PyObject* py_forward(PyObject*, PyObject* const* args, Py_ssize_t nargs) {
     return guarded([&]() -> PyObject* {
         if (nargs != 2 || !PyDict_Check(args[0]) || !plain(args[1])) return none();
         const Tensor& x = unpack(args[1]);
-        if (!x.is_cuda()) return none();
-        Plan* p = plan_of(args[0]);
-        if (!p) {
+        if (!x.is_cuda() || !x.has_storage()) return none();    // (no storage: a wrapper of vmap or torch.func)
+        Module l;
+        if (!module_of(args[0], l)) {
             if (PyErr_Occurred()) return nullptr;
             return none();
         }
-        if (!p->usable) return none();
+        if (!PyDict_GetItemWithError(args[0], s_plan) && (PyErr_Occurred() || PyDict_SetItem(args[0], s_plan, Py_True)))
+            return nullptr;                                    // the mark says that the native path takes this layer
         int status = 0;
         const char* what = "";
-        if (!(c10::GradMode::is_enabled() && x.requires_grad())) return checked(linear(p->layer, x, status, what), status, what);
+        if (!(c10::GradMode::is_enabled() && x.requires_grad())) return checked(linear(l.layer, x, status, what), status, what);
+        if (x._fw_grad(0).defined()) return none();            // the Python function refuses forward-mode derivatives
         Tensor y;
         {
             c10::AutoGradMode off(false);
-            y = linear(p->layer, x, status, what);
+            y = linear(l.layer, x, status, what);
         }
         if (status == 0 && y.defined()) {
             std::shared_ptr<QuantizedLinearBackward> node(new QuantizedLinearBackward(), torch::autograd::deleteNode);
             node->set_next_edges(torch::autograd::collect_next_edges(x));
-            node->qweight = torch::autograd::SavedVariable(unpack(p->tensor[0]), false);
-            node->scale = torch::autograd::SavedVariable(unpack(p->tensor[1]), false);
-            node->zero = torch::autograd::SavedVariable(unpack(p->tensor[2]), false);
-            node->bits = p->layer.bits;
-            node->group = p->layer.group;
+            node->qweight = torch::autograd::SavedVariable(l.qweight, false);
+            node->scale = torch::autograd::SavedVariable(l.scale, false);
+            node->zero = torch::autograd::SavedVariable(l.zero, false);
+            node->bits = l.layer.bits;
+            node->group = l.layer.group;
             torch::autograd::set_history(y, node);
         }
         return checked(std::move(y), status, what);
@@ -334,7 +308,7 @@ PyObject* py_matmul(PyObject*, PyObject* const* args, Py_ssize_t nargs) {
         for (int i = 0; i < 5; i++)
             if (!plain(args[i]) && !(i == 4 && args[i] == Py_None)) return none();
         const Tensor& x = unpack(args[0]);
-        if (x.scalar_type() != at::kHalf && x.scalar_type() != at::kBFloat16) return none();
+        if (!x.has_storage() || (x.scalar_type() != at::kHalf && x.scalar_type() != at::kBFloat16)) return none();
         Layer l;
         if (!layer_of(unpack(args[1]), unpack(args[2]), unpack(args[3]), args[4] == Py_None ? nullptr : &unpack(args[4]),
                       PyLong_AsLong(args[5]), PyLong_AsLong(args[6]), l))
@@ -355,7 +329,8 @@ PyObject* py_input_grad(PyObject*, PyObject* const* args, Py_ssize_t nargs) {
             if (!plain(args[i])) return none();
         const Tensor& go = unpack(args[0]);
         Layer l;
-        if (!go.is_cuda() || !layer_of(unpack(args[1]), unpack(args[2]), unpack(args[3]), nullptr, PyLong_AsLong(args[4]), PyLong_AsLong(args[5]), l))
+        if (!go.is_cuda() || !go.has_storage() ||
+            !layer_of(unpack(args[1]), unpack(args[2]), unpack(args[3]), nullptr, PyLong_AsLong(args[4]), PyLong_AsLong(args[5]), l))
             return none();
         if (go.dim() < 1 || go.size(-1) != l.n || !go.is_floating_point() || go.device().index() != l.device) return none();
         return THPVariable_Wrap(input_grad(go, unpack(args[1]), unpack(args[2]), unpack(args[3]), l.bits, l.group));
@@ -467,11 +442,6 @@ PyModuleDef module_def = {PyModuleDef_HEAD_INIT, "_bw_host", "Native host path o
 }  // namespace
 
 PyMODINIT_FUNC PyInit__bw_host() {
-    PlanType.tp_name = "bitween_amd.Plan";
-    PlanType.tp_basicsize = sizeof(Plan);
-    PlanType.tp_flags = Py_TPFLAGS_DEFAULT;
-    PlanType.tp_dealloc = plan_dealloc;
-    if (PyType_Ready(&PlanType) < 0) return nullptr;
     s_buffers = PyUnicode_InternFromString("_buffers");
     s_qweight = PyUnicode_InternFromString("qweight");
     s_scale = PyUnicode_InternFromString("scale");

@@ -88,8 +88,7 @@ class QuantizedLinear(nn.Module):
             y = group.forward(self, x)
             if y is not None:
                 return y
-        # The native path: the buffers were validated once and are looked at again only when one of them has been replaced
-        # (module.to(), load with assign, sibling fusion) or moved; records its own autograd node where x asks for one.
+        # The native path: looks at the layer's buffers as they are now, records its own autograd node where x asks for one.
         y = _host_forward(fields, x)
         if y is not None:
             return y
@@ -103,7 +102,7 @@ class QuantizedLinear(nn.Module):
         y = _hip.quantized_matmul_hip(x2, self.qweight, self.scale, self.zero_point, self.bias, self.bits, self.group_size)
         return y.view(*shape[:-1], self.out_features)
 
-    def __getstate__(self):                                # the validated-buffers cache holds device addresses
+    def __getstate__(self):                                # the native path's mark belongs to this object's buffers
         state = self.__dict__.copy()
         state.pop("_decode_plan", None)
         return state

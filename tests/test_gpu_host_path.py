@@ -107,3 +107,34 @@ def test_quantize_copies_what_it_does_not_replace():
         if isinstance(value, (dict, set)):
             assert out[1].__dict__[name] is not value and type(out[1].__dict__[name]) is type(value) and len(out[1].__dict__[name]) == len(value)
     assert len(out[1]._forward_hooks) == 1
+
+
+def test_buffers_are_looked_at_on_every_call():
+    """A buffer whose tensor object and address stay but whose layout or type does not, and a changed group size, are seen by the next call."""
+    q = _layer(128, 64, 4, 64)
+    x = torch.randn(3, 128, device="cuda", dtype=torch.float16)
+    want = q(x)
+    scale, dt = q.scale.data, q.scale.data.clone().t().contiguous().t()
+    q.scale.data = dt                                           # same values, column-major
+    assert torch.equal(q(x), want)
+    q.scale.data = scale
+    q.scale.data = scale.view(torch.bfloat16)                   # same address, another type
+    with pytest.raises(TypeError):
+        q(x)
+    q.scale.data = scale
+    assert torch.equal(q(x), want)
+    q.group_size = 32                                           # the buffers do not belong to this one
+    with pytest.raises(ValueError):
+        q(x)
+
+
+def test_transforms_that_the_python_function_refuses_stay_refused():
+    q = _layer(128, 64, 4, 64)
+    x = torch.randn(3, 128, device="cuda", dtype=torch.float16)
+    with pytest.raises(RuntimeError):                           # no vmap rule
+        torch.func.vmap(q)(x)
+    with pytest.raises(RuntimeError):                           # no setup_context
+        torch.func.grad(lambda t: q(t).float().sum())(x)
+    import torch.autograd.forward_ad as fwd
+    with fwd.dual_level(), pytest.raises(RuntimeError):         # no jvp
+        q(fwd.make_dual(x.clone().requires_grad_(True), torch.ones_like(x)))
