@@ -176,14 +176,16 @@ __global__ __launch_bounds__(512, 2) void qbatch_kernel(const BatchArgs a) {
     constexpr int TASKS = PASSES + ML + NTW * WL, SLOTS = 4 * NTW;
     auto round = [&](auto more, const char* cur, char* nxt, XSet& xs, WSet& wq, const WSet& s, WSet& sn, int r) {
         constexpr bool MORE = decltype(more)::value;
-        // the lane's group of the round, kept inside the row: values past K meet zeros of x, but not another row's scale
+        // the lane's group of the round, kept inside the row
         const int g = min((kw * 128 + kq * 32) / GROUP, a.groups - 1 - (c_begin + WK * r) * 128 / GROUP);
         const uint32_t ko = x_offset(r + 3), so = w_scalar(r + 3);
         GC gc[NTW];
 #pragma unroll
         for (int j = 0; j < NTW; j++) {
             const _Float16* m = reinterpret_cast<const _Float16*>(cur + X_BYTES) + ((wn * NTW + j) * 16 + nl) * GR + g;
-            gc[j].set(m[0], m[BN * GR]);
+            // values past K (of the last round only) meet zeros of x; what is unpacked there must be finite
+            const bool past = !MORE && (c_begin + WK * r + kw) * 128 + kq * 32 >= a.K;
+            gc[j].set(past ? (_Float16)0.f : m[0], past ? (_Float16)0.f : m[BN * GR]);
         }
         const char* xp = cur + nl * PITCH + (kw * 128 + kq * 32) * 2;
         h8 xf[XF][MT];

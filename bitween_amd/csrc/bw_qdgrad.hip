@@ -183,6 +183,17 @@ __global__ __launch_bounds__(DTHREADS, MT == 4 ? 3 : 2) void qdgrad_kernel(const
         }
         *reinterpret_cast<u4*>(Bs + b_dst) = u4{wd[0], wd[1], wd[2], wd[3]};
         *reinterpret_cast<u4*>(Bs + b_dst + 16) = u4{wd[4], wd[5], wd[6], wd[7]};
+        // ... and their columns of grad_y of zero as well: an infinity there times a weight of zero would turn its sum into NaN
+        const int dup = step < s_end ? step * DN - min(step * DN, a.N - DN) : DN;
+        if (dup > 0) {                                                // (uniform)
+#pragma unroll
+            for (int e = 0; e < 4; e++) {
+                const int n = gpart * 8 + 2 * e;
+                const uint32_t keep = (n < dup ? 0u : 0xFFFFu) | (n + 1 < dup ? 0u : 0xFFFF0000u);
+#pragma unroll
+                for (int r = 0; r < GR; r++) greg[slot][r][e] &= keep;
+            }
+        }
 #pragma unroll
         for (int r = 0; r < GR; r++) *reinterpret_cast<u4*>(As + (gm + 64 * r) * DPITCH + gpart * 16) = greg[slot][r];
     };
@@ -198,7 +209,7 @@ __global__ __launch_bounds__(DTHREADS, MT == 4 ? 3 : 2) void qdgrad_kernel(const
         __syncthreads();
     }
     // whole passes of PD steps, no early exit (the steps past the end multiply by zero weights): the loop body
-    // is one straight block, which keeps the compiler's count of outstanding loads exact
+    // is one straight block but for the masking in fill(), which keeps the compiler's count of outstanding loads exact
     for (int base = s_begin; base < s_end; base += PD) {
 #pragma unroll
         for (int d = 0; d < PD; d++) {

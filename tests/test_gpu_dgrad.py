@@ -330,3 +330,21 @@ def test_dgrad_ragged_n_k_and_pitch(bits, g, dtype):
                 assert np.array_equal(gx[r, :k].float().cpu().numpy(), wt[c].astype(np.float32))
     assert lib.bw_qdgrad(view.data_ptr(), code, 1, 31, 31, d[0].data_ptr(), d[1].data_ptr(), d[2].data_ptr(), 128, bits, g,
                          gx.data_ptr(), 128, None, 0, stream) == -2     # fewer rows of W than a step
+
+
+@pytest.mark.parametrize("n,m", [(33, 5), (1001, 40), (3040, 600)])
+def test_dgrad_infinite_gradients_of_a_ragged_n(n, m):
+    """Columns of grad_y that a step of 32 rows sees twice (N that is no multiple of 32), or that the last pass of steps repeats (an
+    odd number of steps), count once: an infinite gradient gives infinities, not NaN - what a loss scaler, and anyone who looks for where
+    it came from, expects."""
+    from bitween_amd.kernels import hip_loader as hip
+    bits, g, k = 4, 64, 192
+    _, qw, s16, z16, _ = quantized_layer(n, k, bits, g, seed=n, bias=False)
+    w = torch.from_numpy(orc.dequantize_f16(qw, s16, z16, g, bits).astype(np.float64))
+    go = torch.randn(m, n, dtype=torch.float16)
+    for row, col in ((0, n - 1), (1, n // 32 * 32 - 1), (2, max(0, n - 32)), (3, 0)):
+        go[row, col] = float("inf")
+    want = go.double() @ w                                      # one infinity a row: +-inf, or NaN where its weight is 0
+    gx = hip.quantized_input_grad(go.cuda(), *(to_gpu(a) for a in (qw, s16, z16)), bits, g).double().cpu()
+    assert torch.equal(torch.isnan(gx), torch.isnan(want)) and torch.equal(torch.isinf(gx), torch.isinf(want))
+    assert torch.equal(gx[torch.isinf(want)], want[torch.isinf(want)])
