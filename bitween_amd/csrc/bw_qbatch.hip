@@ -43,28 +43,32 @@ struct BatchPlan { int ntw, splits; };
 
 inline int batch_mt(int64_t M) { const int t = (int)((M + 15) / 16); return t <= 4 ? t : t <= 6 ? 6 : 8; }
 
-// Column tiles per wave and cuts of K for a call, from a model of the launch fitted to 1500 timings (17 ... 96 rows, eleven
-// shapes, 2 / 4 / 8 bits; rms error 7 %, its choice within 0.7 % of the best on average): a round costs
-// -0.23 + 0.21 MT + (0.46 + 0.014 MT + 0.19 at 8 bits) NTW us (0.68 of it where rounds are 256 values), every wave of
-// workgroups 0.34 MT us more, a launch 2.1, a cut of K the reduction: 2.4 us and 2.9 us per million partial sums.
+// Column tiles per wave and cuts of K for a call, from a model of the launch fitted to timings (17 ... 64 rows: 1500, eleven
+// shapes, 2 / 4 / 8 bits; rms error 7 %, its choice within 0.7 % of the best on average; 65 ... 128 rows, rounds of 256 values: 800,
+// eight shapes, 6 %, 0.8 %): a round costs -0.23 + 0.21 MT + (0.46 + 0.014 MT + 0.19 at 8 bits) NTW us, beyond 64 rows 0.094 MT +
+// (0.258 + 0.004 MT + 0.136 at 8 bits) NTW; every wave of workgroups 0.34 (0.22) MT us more, a launch 2.1 (2.9), a cut of K
+// the reduction: 2.4 (2.7) us and 2.9 (2.5) us per million partial sums.
 BatchPlan batch_plan(int64_t M, int64_t N, int64_t K, int bits, bool may_split) {
     struct Entry { int64_t m, n, k; int key; BatchPlan plan; };
     static thread_local Entry cache[32] = {};              // the search takes 2 us of a call's host time
     const int key = bits * 2 + may_split;
     Entry& e = cache[(size_t)(M * 7 + N * 3 + K * 5 + key) % 32];
     if (e.m == M && e.n == N && e.k == K && e.key == key) return e.plan;
-    const int mt = batch_mt(M), wk = mt <= 4 ? 4 : 2, nchunks = (int)((K + 127) / 128), cus = bw_device_cus();
+    const int mt = batch_mt(M), nchunks = (int)((K + 127) / 128), cus = bw_device_cus();
+    const bool large = mt > 4;
     BatchPlan best{1, 1};
     float best_us = 1e30f;
-    for (int ntw = 1; ntw <= (mt <= 4 ? 3 : mt == 6 ? 2 : 1); ntw++) {
-        const int bn = 16 * (8 / wk) * ntw;
+    for (int ntw = 1; ntw <= (mt <= 6 ? 3 : 2); ntw++) {
+        const int bn = 32 * ntw;
         const int64_t tiles = (N + bn - 1) / bn;
-        const float round = (-0.23f + 0.21f * mt + (0.46f + 0.014f * mt + (bits == 8 ? 0.19f : 0.f)) * ntw) * (mt <= 4 ? 1.f : 0.68f);
+        const float round = large ? 0.094f * mt + (0.258f + 0.004f * mt + (bits == 8 ? 0.136f : 0.f)) * ntw
+                                  : -0.23f + 0.21f * mt + (0.46f + 0.014f * mt + (bits == 8 ? 0.19f : 0.f)) * ntw;
         for (int s = 1; s <= 16 && (s == 1 || (may_split && 2 * s <= nchunks)); s++) {
             const int cps = (nchunks + s - 1) / s, used = (nchunks + cps - 1) / cps;
             if (used != s) continue;
-            const float us = 2.1f + (float)((tiles * s + cus - 1) / cus) * (((cps + wk - 1) / wk) * round + 0.34f * mt) +
-                             (s > 1 ? 2.4f + 2.9e-6f * (float)M * (float)N * s : 0.f);
+            const float waves = (float)((tiles * s + cus - 1) / cus), sums = 1e-6f * (float)M * (float)N * s;
+            const float us = large ? 2.9f + waves * ((cps + 1) / 2 * round + 0.22f * mt) + (s > 1 ? 2.7f + 2.5f * sums : 0.f)
+                                   : 2.1f + waves * ((cps + 3) / 4 * round + 0.34f * mt) + (s > 1 ? 2.4f + 2.9f * sums : 0.f);
             if (us < best_us) { best_us = us; best = {ntw, s}; }
         }
     }
@@ -96,13 +100,17 @@ inline bool batch_takes_decode_rows(int64_t M, int64_t N, int64_t K, int bits, i
 }
 
 // 17 ... 96 rows: this kernel (64 rows of the Llama shapes at 4 bits, us, prefill kernel against this one: 4096 x 4096 17.7
-// -> 11.7, 4096 -> 11008 20.4 -> 17.3, 11008 -> 4096 22.8 -> 19.1; 2048 x 2048 13.0 -> 8.1; 96 rows 1.03 ... 1.4 x faster).
-// Up to 128 rows on layers it unpacks fast enough: 32 M weights at 4 bits (4096 x 4096 20.8 -> 17.4; 4096 -> 11008 27.0
-// against 30.0), 64 M at 2 and 8 bits (4096 -> 14336 W8 38.2 -> 33.1).
+// -> 11.7, 4096 -> 11008 20.4 -> 17.3, 11008 -> 4096 22.8 -> 19.1; 2048 x 2048 13.0 -> 8.1; 96 rows 1.1 ... 1.4 x faster).
+// Up to 128 rows while one wave of its 64-column tiles covers N and the layer has no more than 64 M weights (128 rows, us,
+// prefill kernel with its cast of bfloat16 against this one: 4096 -> 14336 W4 31.3 -> 27.4, bfloat16 34.0 -> 30.5, W8 g32 36.4 -> 31.3,
+// W2 31.5 -> 26.4; 4096 x 4096 20.9 -> 17.0; but 4096 -> 22016 W4 40.8 against 53.3) - 48 M where K has to be cut and
+// weights are few bytes (14336 -> 4096 W4 28.7 against 29.9, 11008 -> 4096 27.2 -> 26.5).
 Route route(int64_t M, int64_t N, int64_t K, int bits, int group) {
     if (M <= 16) return batch_takes_decode_rows(M, N, K, bits, group) ? kBatch : kDecode;
     if (M <= 96) return kBatch;
-    return M <= 128 && N * K <= ((int64_t)(bits == 4 ? 32 : 64) << 20) ? kBatch : kPrefill;
+    if (M > 128 || (N + 63) / 64 > bw_device_cus()) return kPrefill;
+    const int64_t most = bits == 8 || batch_plan(M, N, K, bits, true).splits == 1 ? 64 : 48;
+    return N * K <= (most << 20) ? kBatch : kPrefill;
 }
 
 // What the batch kernel asks of a call beyond bw_fast_shape: 4-byte words of scales, offsets of x in 31 bits.

@@ -5,8 +5,8 @@
 // bound by how many bytes a compute unit has to take in: every workgroup needs its slice of x, so x crosses from L2 to
 // the CUs N / BN times, next to the weights once from HBM.  A workgroup of 8 waves owns all M rows x BN = 32 NTW output
 // columns and a slice of K:
-//   * K is walked in rounds of 512 values; of a round's four chunks of 128 each wave takes one (kw) and NTW of the 2 NTW
-//     column tiles (wn), so that the grid has enough workgroups for narrow layers and a fragment of x read from LDS
+//   * K is walked in rounds of 512 values (256 beyond 64 rows); of a round's four chunks each wave takes one (kw) and NTW of the
+//     2 NTW column tiles (wn), so that the grid has enough workgroups for narrow layers and a fragment of x read from LDS
 //     feeds NTW MFMAs;
 //   * x goes global -> registers -> LDS (double buffered, one round ahead), converted from bfloat16 and permuted to the
 //     order the unpack emits on the way; scales and zero points of a round come in with it, whole rows at a time;
@@ -47,11 +47,13 @@ BW_DEV __amdgpu_buffer_rsrc_t batch_rsrc(const void* p, uint32_t bytes) {
     return __builtin_amdgcn_make_buffer_rsrc(const_cast<void*>(p), (short)0, (int)bytes, 0x00020000);
 }
 
-// Shape of a workgroup of 8 waves: KR values of K per round, cut over WK waves of 128 values; WN waves side by side over the
-// columns.  Up to 64 rows a round is 512 values; beyond, x of a round would not fit LDS twice.
+// Shape of a workgroup of 8 waves: KR values of K per round, cut over WK = 4 waves of CK values (VPL of them in a lane); WN = 2
+// waves side by side over the columns.  Up to 64 rows a round is 512 values; beyond, x of a round would not fit LDS twice.
+// (Beyond 64 rows as 2 waves of 128 values x 4 side by side, every fragment of x crossed LDS four times instead of twice, and
+// LDS was what the loop waited for.)
 template <int MT, int NTW>
 struct BatchCfg {
-    static constexpr int KR = MT <= 4 ? 512 : 256, WK = KR / 128, WN = 8 / WK, BN = 16 * WN * NTW;
+    static constexpr int KR = MT <= 4 ? 512 : 256, WK = 4, CK = KR / WK, VPL = CK / 4, WN = 2, BN = 16 * WN * NTW;
     static constexpr int PITCH = (KR + 8) * 2;                        // bytes of an LDS row of x
     static constexpr int X_BYTES = 16 * MT * PITCH;
     static constexpr int RPW = 512 / KR, PASSES = 2 * MT / RPW;       // rows a wave stages per pass, passes per round
@@ -65,9 +67,10 @@ template <int BITS, int GROUP, int MT, int NTW, bool BF16>
 __global__ __launch_bounds__(512, 2) void qbatch_kernel(const BatchArgs a) {
     constexpr uint32_t kOob = 0x80000000u, kOobRow = kBatchMaxBytes;   // beyond every buffer, also added to one another
     using C = BatchCfg<MT, NTW>;
-    constexpr int KR = C::KR, WK = C::WK, WN = C::WN, BN = C::BN, PITCH = C::PITCH, PASSES = C::PASSES, X_BYTES = C::X_BYTES;
-    constexpr int WL = BITS == 8 ? 2 : 1;                             // 16-byte pieces of a lane's 32 weights (8 bytes at 2 bits)
-    constexpr int CHUNK_BYTES = 16 * BITS, GR = KR / GROUP;           // groups per round
+    constexpr int KR = C::KR, WK = C::WK, CK = C::CK, VPL = C::VPL, BN = C::BN, PITCH = C::PITCH, PASSES = C::PASSES, X_BYTES = C::X_BYTES;
+    constexpr int LANE_BYTES = VPL * BITS / 8, STEPS = VPL / 8;       // packed bytes, and MFMA steps, of a lane's weights of a round
+    constexpr int WL = LANE_BYTES > 16 ? LANE_BYTES / 16 : 1, WW = LANE_BYTES > 16 ? 4 : LANE_BYTES / 4;   // requests, words of each
+    constexpr int CHUNK_BYTES = CK * BITS / 8, GR = KR / GROUP;       // groups per round
     constexpr int ML = (BN * GR / 2 + 255) / 256;                     // words of scales (zero points) a thread brings in
     constexpr int BUF = X_BYTES + 2 * BN * GR * 2;
     constexpr int XF = MT * NTW >= 12 ? 1 : 2;                        // sets of x fragments: the next step's are read early where registers allow
@@ -76,16 +79,17 @@ __global__ __launch_bounds__(512, 2) void qbatch_kernel(const BatchArgs a) {
     const int nl = lane & 15, kq = lane >> 4, kw = wave % WK, wn = wave / WK;
     const int tile = (int)blockIdx.x / a.splits, slice = (int)blockIdx.x - tile * a.splits;
     const int n_base = tile * BN;
-    const int c_begin = slice * a.chunks_per_split, c_end = min(a.nchunks, c_begin + a.chunks_per_split);
+    // chunks of CK values (the slices are counted in 128s)
+    const int c_begin = slice * a.chunks_per_split * (128 / CK), c_end = min(a.nchunks, (slice + 1) * a.chunks_per_split) * (128 / CK);
     const int rounds = (c_end - c_begin + WK - 1) / WK;
-    const int k_end = min(a.K, c_end * 128);
+    const int k_end = min(a.K, c_end * CK);
     const __amdgpu_buffer_rsrc_t rw = batch_rsrc(a.qweight, a.w_bytes), rx = batch_rsrc(a.x, a.x_bytes);
 
     uint32_t w_off[NTW];
 #pragma unroll
     for (int j = 0; j < NTW; j++) {
         const int row = min(n_base + (wn * NTW + j) * 16 + (lane >> 2), a.N - 1);   // columns past N repeat the last one and are not stored
-        w_off[j] = (uint32_t)row * a.row_bytes + (lane & 3) * (4 * BITS) + kw * CHUNK_BYTES;
+        w_off[j] = (uint32_t)row * a.row_bytes + (lane & 3) * LANE_BYTES + kw * CHUNK_BYTES;
     }
     struct WSet { u4 w[NTW][WL]; };
     WSet wset[2];
@@ -97,7 +101,9 @@ __global__ __launch_bounds__(512, 2) void qbatch_kernel(const BatchArgs a) {
     };
     auto issue_w = [&](WSet& s, int j, int l, uint32_t so) {
         const uint32_t off = w_off[j] + so;
-        if constexpr (BITS == 2) {
+        if constexpr (WW == 1) {
+            s.w[j][0][0] = __builtin_amdgcn_raw_buffer_load_b32(rw, off, 0, 0);
+        } else if constexpr (WW == 2) {
             const u2 v = __builtin_amdgcn_raw_buffer_load_b64(rw, off, 0, 0);
             s.w[j][0][0] = v[0];
             s.w[j][0][1] = v[1];
@@ -119,7 +125,7 @@ __global__ __launch_bounds__(512, 2) void qbatch_kernel(const BatchArgs a) {
         row_off[p] = __builtin_amdgcn_readfirstlane(row < a.M ? (uint32_t)row * a.ldx * 2 : kOobRow);
     }
     auto x_offset = [&](int r) {
-        const int k = (c_begin + WK * r) * 128 + col;
+        const int k = (c_begin + WK * r) * CK + col;
         return k < k_end ? (uint32_t)(k + sub * a.ldx) * 2 : kOob;
     };
     auto issue_x = [&](XSet& xs, int p, uint32_t ko) { xs.x[p] = __builtin_amdgcn_raw_buffer_load_b128(rx, ko + row_off[p], 0, 0); };
@@ -129,7 +135,7 @@ __global__ __launch_bounds__(512, 2) void qbatch_kernel(const BatchArgs a) {
 #pragma unroll
     for (int i = 0; i < ML; i++) {
         const int item = (tid & 255) + 256 * i, n = item / (GR / 2), w = item - n * (GR / 2);
-        const uint32_t off = (uint32_t)(min(n_base + n, a.N - 1) * a.groups + c_begin * (128 / GROUP)) * 2 + 4 * w;
+        const uint32_t off = (uint32_t)(min(n_base + n, a.N - 1) * a.groups + c_begin * CK / GROUP) * 2 + 4 * w;
         meta_off[i] = n < BN ? off & ~3u : kOob;
         meta_shift[i] = (off & 2) * 8;
     }
@@ -168,39 +174,39 @@ __global__ __launch_bounds__(512, 2) void qbatch_kernel(const BatchArgs a) {
     const int from = ((nl << 2) | kq) << 2;
     auto permute_w = [&](WSet& s, const WSet& q, int j, int l) {
 #pragma unroll
-        for (int e = 0; e < (BITS == 2 ? 2 : 4); e++) s.w[j][l][e] = __builtin_amdgcn_ds_bpermute(from, (int)q.w[j][l][e]);
+        for (int e = 0; e < WW; e++) s.w[j][l][e] = __builtin_amdgcn_ds_bpermute(from, (int)q.w[j][l][e]);
     };
     // One round: multiply what lies in `cur` and `s`; and, dealt out over the column tiles' MFMA groups so that neither the
     // address unit nor LDS sees a burst while the matrix pipe idles (12288 x 4096 at 40 rows 18.2 -> 15.9 us),
     // put round r + 1 into `nxt` and `sn` from the registers it was requested into, and request round r + 3 there.
-    constexpr int TASKS = PASSES + ML + NTW * WL, SLOTS = 4 * NTW;
+    constexpr int TASKS = PASSES + ML + NTW * WL, SLOTS = STEPS * NTW;
     auto round = [&](auto more, const char* cur, char* nxt, XSet& xs, WSet& wq, const WSet& s, WSet& sn, int r) {
         constexpr bool MORE = decltype(more)::value;
         // the lane's group of the round, kept inside the row
-        const int g = min((kw * 128 + kq * 32) / GROUP, a.groups - 1 - (c_begin + WK * r) * 128 / GROUP);
+        const int g = min((kw * CK + kq * VPL) / GROUP, a.groups - 1 - (c_begin + WK * r) * CK / GROUP);
         const uint32_t ko = x_offset(r + 3), so = w_scalar(r + 3);
         GC gc[NTW];
 #pragma unroll
         for (int j = 0; j < NTW; j++) {
             const _Float16* m = reinterpret_cast<const _Float16*>(cur + X_BYTES) + ((wn * NTW + j) * 16 + nl) * GR + g;
             // values past K (of the last round only) meet zeros of x; what is unpacked there must be finite
-            const bool past = !MORE && (c_begin + WK * r + kw) * 128 + kq * 32 >= a.K;
+            const bool past = !MORE && (c_begin + WK * r + kw) * CK + kq * VPL >= a.K;
             gc[j].set(past ? (_Float16)0.f : m[0], past ? (_Float16)0.f : m[BN * GR]);
         }
-        const char* xp = cur + nl * PITCH + (kw * 128 + kq * 32) * 2;
+        const char* xp = cur + nl * PITCH + (kw * CK + kq * VPL) * 2;
         h8 xf[XF][MT];
         auto read_x = [&](int t) {
 #pragma unroll
             for (int i = 0; i < MT; i++) xf[t % XF][i] = *reinterpret_cast<const h8*>(xp + i * (16 * PITCH) + t * 16);
         };
         if constexpr (XF == 2) read_x(0);
-        static_for<0, 4>([&](auto tc) {
+        static_for<0, STEPS>([&](auto tc) {
             constexpr int t = decltype(tc)::value;
             static_for<0, NTW>([&](auto jc) {
                 constexpr int j = decltype(jc)::value, slot = t * NTW + j;
                 __builtin_amdgcn_sched_barrier(0);
                 if constexpr (j == 0 && XF == 1) read_x(t);
-                if constexpr (j == 0 && XF == 2 && t < 3) read_x(t + 1);
+                if constexpr (j == 0 && XF == 2 && t + 1 < STEPS) read_x(t + 1);
                 h2 o[4];
                 if constexpr (BITS == 4) dequant_word4<true>(s.w[j][0][t], gc[j], o);
                 else if constexpr (BITS == 2) dequant_halfword2_nat(s.w[j][0][t / 2], t % 2, gc[j], o);
@@ -334,7 +340,7 @@ int launch_qbatch_bits(int group, int mt, int ntw, const BatchArgs& a, hipStream
 #define BW_CASE(G, T, W) \
     if (group == G && mt == T && ntw == W) return a.x_bf16 ? launch_qbatch<BITS, G, T, W, true>(a, stream) : launch_qbatch<BITS, G, T, W, false>(a, stream);
 #define BW_ROWS(G, T) BW_CASE(G, T, 1) BW_CASE(G, T, 2) BW_CASE(G, T, 3)
-#define BW_GROUP(G) BW_ROWS(G, 1) BW_ROWS(G, 2) BW_ROWS(G, 3) BW_ROWS(G, 4) BW_CASE(G, 6, 1) BW_CASE(G, 6, 2) BW_CASE(G, 8, 1)
+#define BW_GROUP(G) BW_ROWS(G, 1) BW_ROWS(G, 2) BW_ROWS(G, 3) BW_ROWS(G, 4) BW_ROWS(G, 6) BW_CASE(G, 8, 1) BW_CASE(G, 8, 2)
     BW_GROUP(128) BW_GROUP(64) BW_GROUP(32)
 #undef BW_GROUP
 #undef BW_ROWS
