@@ -4,6 +4,7 @@
 #include <stddef.h>
 
 bool bw_fast_shape(int64_t M, int64_t N, int64_t K, int64_t ldx, int bits, int group);
+float bw_qgemm_expected_us(int64_t M, int64_t N, int64_t K, int bits);
 
 namespace {
 
@@ -39,42 +40,56 @@ __global__ __launch_bounds__(256) void qbatch_reduce_kernel(const float* __restr
 }
 
 // ---- plan ----
-struct BatchPlan { int ntw, splits; };
+struct BatchPlan { int mt, ntw, splits; };
 
 inline int batch_mt(int64_t M) { const int t = (int)((M + 15) / 16); return t <= 4 ? t : t <= 6 ? 6 : 8; }
 
-// Column tiles per wave and cuts of K for a call, from a model of the launch fitted to timings (17 ... 64 rows: 1500, eleven
-// shapes, 2 / 4 / 8 bits; rms error 7 %, its choice within 0.7 % of the best on average; 65 ... 128 rows, rounds of 256 values: 800,
-// eight shapes, 6 %, 0.8 %): a round costs -0.23 + 0.21 MT + (0.46 + 0.014 MT + 0.19 at 8 bits) NTW us, beyond 64 rows 0.094 MT +
-// (0.258 + 0.004 MT + 0.136 at 8 bits) NTW; every wave of workgroups 0.34 (0.22) MT us more, a launch 2.1 (2.9), a cut of K
-// the reduction: 2.4 (2.7) us and 2.9 (2.5) us per million partial sums.
-BatchPlan batch_plan(int64_t M, int64_t N, int64_t K, int bits, bool may_split) {
-    struct Entry { int64_t m, n, k; int key; BatchPlan plan; };
-    static thread_local Entry cache[32] = {};              // the search takes 2 us of a call's host time
-    const int key = bits * 2 + may_split;
-    Entry& e = cache[(size_t)(M * 7 + N * 3 + K * 5 + key) % 32];
-    if (e.m == M && e.n == N && e.k == K && e.key == key) return e.plan;
-    const int mt = batch_mt(M), nchunks = (int)((K + 127) / 128), cus = bw_device_cus();
-    const bool large = mt > 4;
-    BatchPlan best{1, 1};
-    float best_us = 1e30f;
-    for (int ntw = 1; ntw <= (mt <= 6 ? 3 : 2); ntw++) {
-        const int bn = 32 * ntw;
-        const int64_t tiles = (N + bn - 1) / bn;
-        const float round = large ? 0.094f * mt + (0.258f + 0.004f * mt + (bits == 8 ? 0.136f : 0.f)) * ntw
-                                  : -0.23f + 0.21f * mt + (0.46f + 0.014f * mt + (bits == 8 ? 0.19f : 0.f)) * ntw;
-        for (int s = 1; s <= 16 && (s == 1 || (may_split && 2 * s <= nchunks)); s++) {
-            const int cps = (nchunks + s - 1) / s, used = (nchunks + cps - 1) / cps;
-            if (used != s) continue;
-            const float waves = (float)((tiles * s + cus - 1) / cus), sums = 1e-6f * (float)M * (float)N * s;
-            const float us = large ? 2.9f + waves * ((cps + 1) / 2 * round + 0.22f * mt) + (s > 1 ? 2.7f + 2.5f * sums : 0.f)
-                                   : 2.1f + waves * ((cps + 3) / 4 * round + 0.34f * mt) + (s > 1 ? 2.4f + 2.9f * sums : 0.f);
-            if (us < best_us) { best_us = us; best = {ntw, s}; }
+// Rows of 16 per tile, column tiles per wave and cuts of K for a call, from a model of the launch fitted to 4000 timings (17 ...
+// 1600 rows, 23 shapes, 2 / 4 / 8 bits, both activation types; rms error 6 %, its choice within 1 % of the best on average).
+// A round costs 0.17 MT + (0.33 + 0.024 MT + 0.19 at 8 bits) NTW us, of 256 values (MT > 4) 0.10 MT + (0.22 + (0.004 + 0.013 at 8
+// bits) MT) NTW; every wave of workgroups (0.21 + 0.22 NTW) MT or (0.13 + 0.18 NTW) MT more, a launch 2.4, a cut of K the
+// reduction: 2 us and 1.6 us per million partial sums.  At 8 bits the two shapes whose registers spill cost a quarter more.
+//
+// Lower tiles than the call has rows read the weights (out of L2) once per tile, but fill the chip without a cut of K and its
+// reduction: W4 g128 us, one tile of rows against the plan, 2048 x 2048 at 64 rows 8.5 -> 5.3, at 128 rows 11.4 -> 6.3; 4096 x 4096 at
+// 64 rows 12.4 -> 8.8, at 128 rows 18.1 -> 12.2; 4096 -> 11008 at 128 rows 28.6 -> 23.8.
+struct BatchCost { BatchPlan plan; float us; };
+
+BatchCost batch_search(int64_t M, int64_t N, int64_t K, int bits, bool may_split) {
+    const int nchunks = (int)((K + 127) / 128), cus = bw_device_cus(), whole = batch_mt(M);
+    BatchCost best{{whole, 1, 1}, 1e30f};
+    for (const int mt : {1, 2, 3, 4, 6, 8}) {
+        const int64_t mtiles = (M + 16 * mt - 1) / (16 * mt);
+        if (mt > whole || (mt < 4 && mtiles > 4)) continue;   // (more tiles of few rows: not measured)
+        const bool large = mt > 4;
+        for (int ntw = 1; ntw <= (mt <= 6 ? 3 : 2); ntw++) {
+            const int64_t tiles = mtiles * ((N + 32 * ntw - 1) / (32 * ntw));
+            const float b8 = bits == 8 ? 1.f : 0.f;
+            float round = large ? 0.10f * mt + (0.22f + (0.004f + 0.013f * b8) * mt) * ntw : 0.17f * mt + (0.33f + 0.024f * mt + 0.19f * b8) * ntw;
+            if (bits == 8 && ((mt == 4 && ntw == 3) || (mt == 8 && ntw == 2))) round *= 1.25f;
+            const float wave = large ? (0.13f + 0.18f * ntw) * mt : (0.21f + 0.22f * ntw) * mt;
+            for (int s = 1; s <= 16 && (s == 1 || (may_split && 2 * s <= nchunks)); s++) {
+                const int cps = (nchunks + s - 1) / s, used = (nchunks + cps - 1) / cps, rounds = large ? (cps + 1) / 2 : (cps + 3) / 4;
+                if (used != s || (s > 1 && M * N * s > ((int64_t)32 << 20))) continue;   // (128 MiB of partial sums)
+                const float waves = (float)((tiles * s + cus - 1) / cus);
+                const float us = 2.4f + waves * (rounds * round + wave) + (s > 1 ? 2.f + 0.05f * s + 1.6e-6f * (float)M * (float)N * s : 0.f);
+                if (us < best.us) best = {{mt, ntw, s}, us};
+            }
         }
     }
-    e = {M, N, K, key, best};
     return best;
 }
+
+BatchCost batch_cost(int64_t M, int64_t N, int64_t K, int bits, bool may_split) {
+    struct Entry { int64_t m, n, k; int key; BatchCost cost; };
+    static thread_local Entry cache[32] = {};              // the search takes some us of a call's host time
+    const int key = bits * 2 + may_split;
+    Entry& e = cache[(size_t)(M * 7 + N * 3 + K * 5 + key) % 32];
+    if (e.m != M || e.n != N || e.k != K || e.key != key) e = {M, N, K, key, batch_search(M, N, K, bits, may_split)};
+    return e.cost;
+}
+
+BatchPlan batch_plan(int64_t M, int64_t N, int64_t K, int bits, bool may_split) { return batch_cost(M, N, K, bits, may_split).plan; }
 
 inline size_t batch_ws_bytes(int64_t M, int64_t N, const BatchPlan& p) { return p.splits > 1 ? (size_t)p.splits * M * ((N + 3) & ~(int64_t)3) * 4 : 0; }
 
@@ -99,18 +114,18 @@ inline bool batch_takes_decode_rows(int64_t M, int64_t N, int64_t K, int bits, i
     return bits == 2 && M > 8 && tiles > 3 * cus && (group == 32 || K / group % 2);
 }
 
-// 17 ... 96 rows: this kernel (64 rows of the Llama shapes at 4 bits, us, prefill kernel against this one: 4096 x 4096 17.7
-// -> 11.7, 4096 -> 11008 20.4 -> 17.3, 11008 -> 4096 22.8 -> 19.1; 2048 x 2048 13.0 -> 8.1; 96 rows 1.1 ... 1.4 x faster).
-// Up to 128 rows while one wave of its 64-column tiles covers N and the layer has no more than 64 M weights (128 rows, us,
-// prefill kernel with its cast of bfloat16 against this one: 4096 -> 14336 W4 31.3 -> 27.4, bfloat16 34.0 -> 30.5, W8 g32 36.4 -> 31.3,
-// W2 31.5 -> 26.4; 4096 x 4096 20.9 -> 17.0; but 4096 -> 22016 W4 40.8 against 53.3) - 48 M where K has to be cut and
-// weights are few bytes (14336 -> 4096 W4 28.7 against 29.9, 11008 -> 4096 27.2 -> 26.5).
+// 17 ... 64 rows: this kernel (W4 g128 at 64 rows, us, prefill kernel against this one: 4096 x 4096 17.8 -> 8.8, 4096 -> 11008 20.9
+// -> 17.2, 11008 -> 4096 24.8 -> 18.9; 2048 x 2048 13.3 -> 5.3).  Beyond, whichever is expected to be done first: the prefill
+// kernel's 128 x 256 tiles leave the chip idle on most layers of a few hundred rows, or have to be cut along K (W4 g128, us, prefill
+// against this: 2048 x 2048 at 333 rows 20.4 -> 10.8, at 768 rows 26.7 -> 14.5; 4096 x 4096 at 256 rows 28.6 -> 17.6, at 512
+// rows 32.4 -> 30.0, but at 768 rows 39.8 against 47.9; 4096 -> 14336 at 128 rows 31.3 -> 27.4, at 160 rows 41.5 against 42.9;
+// 512 -> 13056 at 200 rows 11.3 against 15.2).  Both models together lose 0.3 % on average, 15 % at most, against the better of the
+// two on 350 shapes.  (The cast of bfloat16 that only the prefill kernel needs is left out: both types take one route.)
 Route route(int64_t M, int64_t N, int64_t K, int bits, int group) {
     if (M <= 16) return batch_takes_decode_rows(M, N, K, bits, group) ? kBatch : kDecode;
-    if (M <= 96) return kBatch;
-    if (M > 128 || (N + 63) / 64 > bw_device_cus()) return kPrefill;
-    const int64_t most = bits == 8 || batch_plan(M, N, K, bits, true).splits == 1 ? 64 : 48;
-    return N * K <= (most << 20) ? kBatch : kPrefill;
+    if (M <= 64) return kBatch;
+    if (M > 2048) return kPrefill;
+    return batch_cost(M, N, K, bits, true).us < 0.95f * bw_qgemm_expected_us(M, N, K, bits) ? kBatch : kPrefill;
 }
 
 // What the batch kernel asks of a call beyond bw_fast_shape: 4-byte words of scales, offsets of x in 31 bits.
@@ -134,9 +149,9 @@ int launch_batch(const void* x, int act_dtype, int64_t M, int64_t K, int64_t ldx
     a.splits = plan.splits;
     a.chunks_per_split = (a.nchunks + plan.splits - 1) / plan.splits;
     a.x_bf16 = act_dtype == BW_BF16;
-    const int mt = batch_mt(M);
-    const int r = bits == 4 ? bw_launch_qbatch_w4(group, mt, plan.ntw, a, st) : bits == 8 ? bw_launch_qbatch_w8(group, mt, plan.ntw, a, st)
-                                                                                      : bw_launch_qbatch_w2(group, mt, plan.ntw, a, st);
+    const int r = bits == 4   ? bw_launch_qbatch_w4(group, plan.mt, plan.ntw, a, st)
+                  : bits == 8 ? bw_launch_qbatch_w8(group, plan.mt, plan.ntw, a, st)
+                              : bw_launch_qbatch_w2(group, plan.mt, plan.ntw, a, st);
     if (r != BW_OK || a.splits == 1) return r;
     const int64_t items = M * (a.npad / 4);
     hipLaunchKernelGGL(qbatch_reduce_kernel, dim3((unsigned)((items + 255) / 256)), dim3(256), 0, st, a.ws, a.bias, a.y, a.M, a.N, a.npad, a.ldy, a.splits);

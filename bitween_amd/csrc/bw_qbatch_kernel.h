@@ -3,8 +3,8 @@
 //
 // Between the decode kernels (16 rows a launch) and the prefill kernel (tiles of 64 x 256 outputs and more) a call is
 // bound by how many bytes a compute unit has to take in: every workgroup needs its slice of x, so x crosses from L2 to
-// the CUs N / BN times, next to the weights once from HBM.  A workgroup of 8 waves owns all M rows x BN = 32 NTW output
-// columns and a slice of K:
+// the CUs N / BN times, next to the weights once from HBM.  A workgroup of 8 waves owns all M rows (128 of them beyond that) x
+// BN = 32 NTW output columns and a slice of K:
 //   * K is walked in rounds of 512 values (256 beyond 64 rows); of a round's four chunks each wave takes one (kw) and NTW of the
 //     2 NTW column tiles (wn), so that the grid has enough workgroups for narrow layers and a fragment of x read from LDS
 //     feeds NTW MFMAs;
@@ -30,7 +30,7 @@ struct BatchArgs {
     uint32_t x_bytes, w_bytes, meta_bytes;
     int M, N, K, ldx, ldy, npad;
     int groups, row_bytes, nchunks;   // chunks of 128 values of K
-    int splits, chunks_per_split;
+    int splits, chunks_per_split, mtiles, ntiles;
     int x_bf16;
 };
 
@@ -78,12 +78,14 @@ __global__ __launch_bounds__(512, 2) void qbatch_kernel(const BatchArgs a) {
     const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
     const int nl = lane & 15, kq = lane >> 4, kw = wave % WK, wn = wave / WK;
     const int tile = (int)blockIdx.x / a.splits, slice = (int)blockIdx.x - tile * a.splits;
-    const int n_base = tile * BN;
+    const int mtile = tile / a.ntiles, n_base = (tile - mtile * a.ntiles) * BN, m_base = mtile * 16 * MT;
+    const int M = min(a.M - m_base, 16 * MT);                         // rows of this tile
     // chunks of CK values (the slices are counted in 128s)
     const int c_begin = slice * a.chunks_per_split * (128 / CK), c_end = min(a.nchunks, (slice + 1) * a.chunks_per_split) * (128 / CK);
     const int rounds = (c_end - c_begin + WK - 1) / WK;
     const int k_end = min(a.K, c_end * CK);
-    const __amdgpu_buffer_rsrc_t rw = batch_rsrc(a.qweight, a.w_bytes), rx = batch_rsrc(a.x, a.x_bytes);
+    const __amdgpu_buffer_rsrc_t rw = batch_rsrc(a.qweight, a.w_bytes), 
+                                 rx = batch_rsrc((const char*)a.x + (int64_t)m_base * a.ldx * 2, a.x_bytes - (uint32_t)m_base * a.ldx * 2);
 
     uint32_t w_off[NTW];
 #pragma unroll
@@ -122,7 +124,7 @@ __global__ __launch_bounds__(512, 2) void qbatch_kernel(const BatchArgs a) {
 #pragma unroll
     for (int p = 0; p < PASSES; p++) {
         const int row = x_row(p);                             // (row + 1 = M of an odd M lies past the buffer's end)
-        row_off[p] = __builtin_amdgcn_readfirstlane(row < a.M ? (uint32_t)row * a.ldx * 2 : kOobRow);
+        row_off[p] = __builtin_amdgcn_readfirstlane(row < M ? (uint32_t)row * a.ldx * 2 : kOobRow);
     }
     auto x_offset = [&](int r) {
         const int k = (c_begin + WK * r) * CK + col;
@@ -297,7 +299,7 @@ __global__ __launch_bounds__(512, 2) void qbatch_kernel(const BatchArgs a) {
         for (int j = 0; j < NTW; j++) red[(kw * 16 * MT + 16 * i + nl) * (QUADS + 1) + 4 * (wn * NTW + j) + kq] = acc[i][j];
     __syncthreads();
     const bool wide = a.ldy % 4 == 0 && ((uintptr_t)a.y & 7) == 0;
-    const int items = min(a.M, 16 * MT) * QUADS;
+    const int items = M * QUADS;
     for (int t = tid; t < items; t += 512) {
         const int m = t / QUADS, q = t - m * QUADS, n = n_base + 4 * q;
         if (n >= a.N) continue;
@@ -305,13 +307,13 @@ __global__ __launch_bounds__(512, 2) void qbatch_kernel(const BatchArgs a) {
 #pragma unroll
         for (int w = 1; w < WK; w++) v += red[(w * 16 * MT + m) * (QUADS + 1) + q];
         if (a.splits > 1) {
-            *reinterpret_cast<f4*>(a.ws + ((int64_t)slice * a.M + m) * a.npad + n) = v;
+            *reinterpret_cast<f4*>(a.ws + ((int64_t)slice * a.M + m_base + m) * a.npad + n) = v;
             continue;
         }
         _Float16 h[4];
 #pragma unroll
         for (int e = 0; e < 4; e++) h[e] = (_Float16)(v[e] + (a.bias && n + e < a.N ? (float)a.bias[n + e] : 0.f));
-        _Float16* dst = a.y + (int64_t)m * a.ldy + n;
+        _Float16* dst = a.y + (int64_t)(m_base + m) * a.ldy + n;
         if (wide && n + 3 < a.N) {
             *reinterpret_cast<u2*>(dst) = u2{as_u32(h2{h[0], h[1]}), as_u32(h2{h[2], h[3]})};
         } else {
@@ -323,15 +325,15 @@ __global__ __launch_bounds__(512, 2) void qbatch_kernel(const BatchArgs a) {
 }
 
 template <int BITS, int GROUP, int MT, int NTW, bool BF16>
-int launch_qbatch(const BatchArgs& a, hipStream_t stream) {
+int launch_qbatch(BatchArgs a, hipStream_t stream) {
     constexpr int LDS = BatchCfg<MT, NTW>::template lds<GROUP>();
     static_assert(LDS <= 160 * 1024, "the staged x, scales and zero points have to fit LDS twice");
     auto kern = qbatch_kernel<BITS, GROUP, MT, NTW, BF16>;
     static uint64_t big_lds_devices = 0;                   // per instantiation
     if (LDS > 64 * 1024 && !bw_allow_big_lds(reinterpret_cast<const void*>(kern), big_lds_devices)) return BW_ELAUNCH;
-    constexpr int BN = BatchCfg<MT, NTW>::BN;
-    const int tiles = (a.N + BN - 1) / BN;
-    hipLaunchKernelGGL(kern, dim3((unsigned)(tiles * a.splits)), dim3(512), LDS, stream, a);
+    a.mtiles = (a.M + 16 * MT - 1) / (16 * MT);
+    a.ntiles = (a.N + BatchCfg<MT, NTW>::BN - 1) / BatchCfg<MT, NTW>::BN;
+    hipLaunchKernelGGL(kern, dim3((unsigned)(a.mtiles * a.ntiles * a.splits)), dim3(512), LDS, stream, a);
     return hipGetLastError() == hipSuccess ? BW_OK : BW_ELAUNCH;
 }
 

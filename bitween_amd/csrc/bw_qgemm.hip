@@ -136,6 +136,18 @@ __global__ __launch_bounds__(256) void cast_bf16_f16_kernel(const uint16_t* __re
 
 }  // namespace
 
+// What a call of 65 ... 2048 rows takes with 128-row tiles, fitted to 300 timings of 23 shapes at 2, 4 and 8 bits (rms error 9 %): for
+// each round of tiles 1.34 us (1.69 at 8 bits) per 128 values of K, 0.59 more on a full chip; 4.6 us and 1.6 us per million
+// partial sums where a short round is cut along K.
+float bw_qgemm_expected_us(int64_t M, int64_t N, int64_t K, int bits) {
+    const int steps = (int)((K + 127) / 128), cus = bw_device_cus();
+    const GemmPlan p = gemm_plan(M, N, steps, true);
+    const int rest = p.tiles - p.full_tiles, whole = steps * ((p.full_tiles + cus - 1) / cus);
+    const float fill = p.tiles < cus ? (float)p.tiles / cus : 1.f;
+    return 4.5f + (whole + (rest ? p.chunks_per_split : 0)) * (bits == 8 ? 1.69f : 1.34f) + 0.59f * fill * whole +
+           (rest ? 4.6f + 1.63e-6f * rest * p.splits * (128 * BN) : 0.f);
+}
+
 extern "C" int bw_cast_bf16_f16(const void* x, int64_t rows, int64_t cols, int64_t ldx, void* y, int64_t ldy, void* stream) {
     if (!x || !y || rows < 1 || cols < 1 || ldx < cols || ldy < cols) return BW_EINVAL;
     if (cols % 8 || ldx % 8 || ldy % 8 || cols / 8 >= ((int64_t)1 << 31)) return BW_EUNSUPPORTED;

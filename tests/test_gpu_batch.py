@@ -119,3 +119,31 @@ def test_layouts_the_batch_kernel_does_not_take(m):
     check_matmul(yb, xb.to(torch.float16).cpu().numpy(), qw, s16, z16, b16, bits, g)
     assert lib.bw_qlinear_ws(None, 0, m, k, k, d[0].data_ptr(), d[1].data_ptr(), d[2].data_ptr(), None, n, bits, g, y.data_ptr(), n, None, 0, None) == -1
     assert lib.bw_qlinear_ws(x.data_ptr(), 2, m, k, k, d[0].data_ptr(), d[1].data_ptr(), d[2].data_ptr(), None, n, bits, g, y.data_ptr(), n, None, 0, None) == -2
+
+
+@pytest.mark.parametrize("bits,g", FORMATS)
+@pytest.mark.parametrize("m,k,n", [(129, 640, 1003), (333, 1152, 97), (500, 256, 515), (1025, 384, 130), (50, 512, 2050), (200, 4096, 66)])
+def test_several_tiles_of_rows(bits, g, m, k, n):
+    """More rows than a tile (or lower tiles than the call has rows): a last tile of one row, odd row counts, K cut across workgroups or
+    not; rows of x and y padded, one-hot rows at the tiles' edges, every row against the oracle."""
+    from bitween_amd.kernels import hip_loader
+    lib = hip_loader.load()
+    _, qw, s16, z16, b16 = quantized_layer(n, k, bits, g, seed=m + n + bits + g, outliers=True)
+    w16 = orc.dequantize_f16(qw, s16, z16, g, bits)
+    d = [to_gpu(a) for a in (qw, s16, z16, b16)]
+    for dtype in (torch.float16, torch.bfloat16):
+        xbuf = torch.full((m, k + 8), float("nan"), dtype=dtype, device="cuda")
+        xbuf[:, :k] = torch.randn(m, k, device="cuda", generator=torch.Generator(device="cuda").manual_seed(m)).to(dtype)
+        hot = {r: (37 * r) % k for r in (0, 15, 16, 31, 32, 47, 48, 63, 64, 95, 96, 127, 128, m - 1) if r < m}
+        for r, c in hot.items():
+            xbuf[r, :k] = 0
+            xbuf[r, c] = 1.0
+        x = xbuf[:, :k]
+        for ws in (True, False):
+            st, y, _ = _call(lib, x, d, n, bits, g, n + 1, ws=ws)
+            if not ws and st == -5 and dtype is torch.bfloat16:      # the prefill kernel wants room for its cast
+                continue
+            assert st == 0 and (y[:, n:] == 7.0).all()
+            check_matmul(y[:, :n].contiguous(), x.to(torch.float16).cpu().numpy(), qw, s16, z16, None, bits, g)
+            for r, c in hot.items():
+                assert np.array_equal(y[r, :n].cpu().numpy().view(np.uint16), w16[:, c].view(np.uint16))
