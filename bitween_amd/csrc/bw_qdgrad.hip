@@ -244,11 +244,19 @@ __global__ __launch_bounds__(DTHREADS, MT == 4 ? 3 : 2) void qdgrad_kernel(const
     // acc[i][j][r] = grad_x[m0 + wm + 16 j + l16][k0 + wk + 16 i + 4 q + r]
     if (a.splits > 1) {
         float* dst = a.ws + (size_t)blockIdx.x * (DM * DK);
+        if (m0 + DM <= a.M) {
 #pragma unroll
-        for (int i = 0; i < 4; i++)
+            for (int i = 0; i < 4; i++)
 #pragma unroll
-            for (int j = 0; j < MT; j++)
-                *reinterpret_cast<f4*>(dst + (wm + 16 * j + l16) * DK + wk + 16 * i + 4 * q) = acc[i][j];
+                for (int j = 0; j < MT; j++) *reinterpret_cast<f4*>(dst + (wm + 16 * j + l16) * DK + wk + 16 * i + 4 * q) = acc[i][j];
+            return;
+        }
+#pragma unroll
+        for (int j = 0; j < MT; j++) {
+            if (m0 + wm + 16 * j + l16 >= a.M) continue;              // rows past M: 16 rows of a 128-row tile are an eighth of the traffic
+#pragma unroll
+            for (int i = 0; i < 4; i++) *reinterpret_cast<f4*>(dst + (wm + 16 * j + l16) * DK + wk + 16 * i + 4 * q) = acc[i][j];
+        }
     } else {
 #pragma unroll
         for (int j = 0; j < MT; j++) {
@@ -275,11 +283,15 @@ __global__ __launch_bounds__(256) void qdgrad_reduce_kernel(const DgradArgs a) {
     if (m >= a.M || k >= a.K) return;
     const float* src = a.ws + (size_t)tile * a.splits * (DM * DKT) + ml * DKT + kl;
     f4 v = {0.f, 0.f, 0.f, 0.f};
-    for (int z = 0; z < a.splits; z++) {
-        const f4 t = *reinterpret_cast<const f4*>(src + (size_t)z * (DM * DKT));
+    int z = 0;
+    for (; z + 4 <= a.splits; z += 4) {                               // four reads in flight: one memory round trip, not four
+        f4 t[4];
 #pragma unroll
-        for (int i = 0; i < 4; i++) v[i] += t[i];
+        for (int e = 0; e < 4; e++) t[e] = *reinterpret_cast<const f4*>(src + (size_t)(z + e) * (DM * DKT));
+#pragma unroll
+        for (int e = 0; e < 4; e++) v += t[e];
     }
+    for (; z < a.splits; z++) v += *reinterpret_cast<const f4*>(src + (size_t)z * (DM * DKT));
     *reinterpret_cast<u2*>(a.gx + (int64_t)m * a.ldx + k) = u2{pack2<DT>(v[0], v[1]), pack2<DT>(v[2], v[3])};
 }
 
