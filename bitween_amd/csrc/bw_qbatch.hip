@@ -55,14 +55,21 @@ inline int batch_mt(int64_t M) { const int t = (int)((M + 15) / 16); return t <=
 // 64 rows 12.4 -> 8.8, at 128 rows 18.1 -> 12.2; 4096 -> 11008 at 128 rows 28.6 -> 23.8.
 struct BatchCost { BatchPlan plan; float us; };
 
-BatchCost batch_search(int64_t M, int64_t N, int64_t K, int bits, bool may_split) {
+// Calls that scale a group's sum in float32: the rows that are, or by bw_qlinear_decode_rows would be, the decode kernels'.
+inline bool batch_sums(int64_t M, int64_t N, int64_t K, int bits, int group) {
+    return bw_qbatch_sums(bits, group, 1, 1) && M <= bw_qlinear_decode_rows(N, K, bits);
+}
+
+BatchCost batch_search(int64_t M, int64_t N, int64_t K, int bits, int group, bool may_split) {
     const int nchunks = (int)((K + 127) / 128), cus = bw_device_cus(), whole = batch_mt(M);
     BatchCost best{{whole, 1, 1}, 1e30f};
+    const bool sums = batch_sums(M, N, K, bits, group);
     for (const int mt : {1, 2, 3, 4, 6, 8}) {
         const int64_t mtiles = (M + 16 * mt - 1) / (16 * mt);
         if (mt > whole || (mt < 4 && mtiles > 4)) continue;   // (more tiles of few rows: not measured)
         const bool large = mt > 4;
         for (int ntw = 1; ntw <= (mt <= 6 ? 3 : 2); ntw++) {
+            if (sums && !bw_qbatch_sums(bits, group, mt, ntw)) continue;
             const int64_t tiles = mtiles * ((N + 32 * ntw - 1) / (32 * ntw));
             const float b8 = bits == 8 ? 1.f : 0.f;
             float round = large ? 0.10f * mt + (0.22f + (0.004f + 0.013f * b8) * mt) * ntw : 0.17f * mt + (0.33f + 0.024f * mt + 0.19f * b8) * ntw;
@@ -80,16 +87,16 @@ BatchCost batch_search(int64_t M, int64_t N, int64_t K, int bits, bool may_split
     return best;
 }
 
-BatchCost batch_cost(int64_t M, int64_t N, int64_t K, int bits, bool may_split) {
+BatchCost batch_cost(int64_t M, int64_t N, int64_t K, int bits, int group, bool may_split) {
     struct Entry { int64_t m, n, k; int key; BatchCost cost; };
     static thread_local Entry cache[32] = {};              // the search takes some us of a call's host time
-    const int key = bits * 2 + may_split;
+    const int key = (bits * 2 + may_split) * 256 + (group & 255);
     Entry& e = cache[(size_t)(M * 7 + N * 3 + K * 5 + key) % 32];
-    if (e.m != M || e.n != N || e.k != K || e.key != key) e = {M, N, K, key, batch_search(M, N, K, bits, may_split)};
+    if (e.m != M || e.n != N || e.k != K || e.key != key) e = {M, N, K, key, batch_search(M, N, K, bits, group, may_split)};
     return e.cost;
 }
 
-BatchPlan batch_plan(int64_t M, int64_t N, int64_t K, int bits, bool may_split) { return batch_cost(M, N, K, bits, may_split).plan; }
+BatchPlan batch_plan(int64_t M, int64_t N, int64_t K, int bits, int group, bool may_split) { return batch_cost(M, N, K, bits, group, may_split).plan; }
 
 inline size_t batch_ws_bytes(int64_t M, int64_t N, const BatchPlan& p) { return p.splits > 1 ? (size_t)p.splits * M * ((N + 3) & ~(int64_t)3) * 4 : 0; }
 
@@ -125,7 +132,7 @@ Route route(int64_t M, int64_t N, int64_t K, int bits, int group) {
     if (M <= 16) return batch_takes_decode_rows(M, N, K, bits, group) ? kBatch : kDecode;
     if (M <= 64) return kBatch;
     if (M > 2048) return kPrefill;
-    return batch_cost(M, N, K, bits, true).us < 0.95f * bw_qgemm_expected_us(M, N, K, bits) ? kBatch : kPrefill;
+    return batch_cost(M, N, K, bits, group, true).us < 0.95f * bw_qgemm_expected_us(M, N, K, bits) ? kBatch : kPrefill;
 }
 
 // What the batch kernel asks of a call beyond bw_fast_shape: 4-byte words of scales, offsets of x in 31 bits.
@@ -149,6 +156,7 @@ int launch_batch(const void* x, int act_dtype, int64_t M, int64_t K, int64_t ldx
     a.splits = plan.splits;
     a.chunks_per_split = (a.nchunks + plan.splits - 1) / plan.splits;
     a.x_bf16 = act_dtype == BW_BF16;
+    a.sums = batch_sums(M, N, K, bits, group);
     const int r = bits == 4   ? bw_launch_qbatch_w4(group, plan.mt, plan.ntw, a, st)
                   : bits == 8 ? bw_launch_qbatch_w8(group, plan.mt, plan.ntw, a, st)
                               : bw_launch_qbatch_w2(group, plan.mt, plan.ntw, a, st);
@@ -177,7 +185,7 @@ extern "C" size_t bw_qlinear_workspace_bytes(int64_t M, int64_t N, int64_t K, in
     // (a call that this kernel turns out not to take - unaligned scales - falls back to the prefill kernel)
     const size_t prefill = M <= 16 ? 0 : bw_qgemm_workspace_bytes(M, N, K, bits, group);
     size_t split = r == kPrefill ? prefill : 0;
-    if (r == kBatch) split = batch_ws_bytes(M, N, batch_plan(M, N, K, bits, true));
+    if (r == kBatch) split = batch_ws_bytes(M, N, batch_plan(M, N, K, bits, group, true));
     const bool cast = act_dtype == BW_BF16 && (r == kPrefill || !fast);
     return split + (cast ? cast_bytes(M, K) : 0);
 }
@@ -193,8 +201,8 @@ extern "C" int bw_qlinear_ws(const void* x, int act_dtype, int64_t M, int64_t K,
     const bool fast = bw_fast_shape(M, N, K, ldx, bits, group);
     Route r = fast ? route(M, N, K, bits, group) : M <= 16 ? kDecode : kPrefill;
     if (r == kBatch && batch_takes(x, M, N, K, ldx, qweight, scale16, zp16, bits, group)) {
-        BatchPlan plan = batch_plan(M, N, K, bits, true);
-        if (batch_ws_bytes(M, N, plan) > workspace_bytes) plan = batch_plan(M, N, K, bits, false);
+        BatchPlan plan = batch_plan(M, N, K, bits, group, true);
+        if (batch_ws_bytes(M, N, plan) > workspace_bytes) plan = batch_plan(M, N, K, bits, group, false);
         return launch_batch(x, act_dtype, M, K, ldx, qweight, scale16, zp16, bias, N, bits, group, y, ldy, workspace, plan, (hipStream_t)stream);
     }
     if (M <= 16) {
@@ -223,9 +231,9 @@ extern "C" int bw_qlinear(const void* x, int act_dtype, int64_t M, int64_t K, in
         // the batch kernel where it is what bw_qlinear_ws runs too and K needs no cut for want of workgroups
         if (x && qweight && scale16 && zp16 && y && bw_shape_ok(N, K, bits, group) && ldx >= K && ldy >= N &&
             batch_takes(x, M, N, K, ldx, qweight, scale16, zp16, bits, group) && route(M, N, K, bits, group) == kBatch &&
-            batch_plan(M, N, K, bits, true).splits == 1)
+            batch_plan(M, N, K, bits, group, true).splits == 1)
             return launch_batch(x, act_dtype, M, K, ldx, qweight, scale16, zp16, bias, N, bits, group, y, ldy, nullptr,
-                                batch_plan(M, N, K, bits, true), (hipStream_t)stream);
+                                batch_plan(M, N, K, bits, group, true), (hipStream_t)stream);
         for (int64_t m0 = 0; m0 < M; m0 += 16) {
             const int st = bw_qgemv((const _Float16*)x + m0 * ldx, act_dtype, M - m0 < 16 ? M - m0 : 16, K, ldx, qweight, scale16,
                                     zp16, bias, N, bits, group, (_Float16*)y + m0 * ldy, ldy, stream);

@@ -31,13 +31,18 @@ struct BatchArgs {
     int M, N, K, ldx, ldy, npad;
     int groups, row_bytes, nchunks;   // chunks of 128 values of K
     int splits, chunks_per_split, mtiles, ntiles;
-    int x_bf16;
+    int x_bf16, sums;
 };
 
 // rows of 16 (mt) and column tiles per wave (ntw) of the launch; BW_EUNSUPPORTED for a combination that is not built
 int bw_launch_qbatch_w2(int group, int mt, int ntw, const BatchArgs& a, hipStream_t stream);
 int bw_launch_qbatch_w4(int group, int mt, int ntw, const BatchArgs& a, hipStream_t stream);
 int bw_launch_qbatch_w8(int group, int mt, int ntw, const BatchArgs& a, hipStream_t stream);
+
+// Tiles of which there is a kernel that multiplies sums of a group by its scale, and not every weight.
+constexpr bool bw_qbatch_sums(int bits, int group, int mt, int ntw) {
+    return group == 128 && bits != 2 && mt <= 3 && mt * ntw <= (bits == 4 ? 6 : 4);
+}
 
 namespace {
 
@@ -63,7 +68,7 @@ struct BatchCfg {
     }
 };
 
-template <int BITS, int GROUP, int MT, int NTW, bool BF16>
+template <int BITS, int GROUP, int MT, int NTW, bool BF16, bool SUMS>
 __global__ __launch_bounds__(512, 2) void qbatch_kernel(const BatchArgs a) {
     constexpr uint32_t kOob = 0x80000000u, kOobRow = kBatchMaxBytes;   // beyond every buffer, also added to one another
     using C = BatchCfg<MT, NTW>;
@@ -73,6 +78,11 @@ __global__ __launch_bounds__(512, 2) void qbatch_kernel(const BatchArgs a) {
     constexpr int CHUNK_BYTES = CK * BITS / 8, GR = KR / GROUP;       // groups per round
     constexpr int ML = (BN * GR / 2 + 255) / 256;                     // words of scales (zero points) a thread brings in
     constexpr int BUF = X_BYTES + 2 * BN * GR * 2;
+    // SUMS: a wave's chunk is one group; its partial dot product of the exact q - z is multiplied by the scale in float32, as the decode
+    // kernels do it, so that calls of a few rows keep their rounding: 2.07e-4 against scale * (q - z) in 64 bits, 2.76e-4 with
+    // every weight rounded to float16 - the reference's W16, against which the errors are the other way round.  Only tiles
+    // whose registers hold both sums (3 x 3 at 4 bits, 3 x 2 at 8 spill: 20 -> 50 us); as fast as W16.
+    static_assert(!SUMS || GROUP == CK);
     constexpr int XF = MT * NTW >= 12 ? 1 : 2;                        // sets of x fragments: the next step's are read early where registers allow
     extern __shared__ __attribute__((aligned(16))) char smem[];
     const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
@@ -84,7 +94,7 @@ __global__ __launch_bounds__(512, 2) void qbatch_kernel(const BatchArgs a) {
     const int c_begin = slice * a.chunks_per_split * (128 / CK), c_end = min(a.nchunks, (slice + 1) * a.chunks_per_split) * (128 / CK);
     const int rounds = (c_end - c_begin + WK - 1) / WK;
     const int k_end = min(a.K, c_end * CK);
-    const __amdgpu_buffer_rsrc_t rw = batch_rsrc(a.qweight, a.w_bytes), 
+    const __amdgpu_buffer_rsrc_t rw = batch_rsrc(a.qweight, a.w_bytes),
                                  rx = batch_rsrc((const char*)a.x + (int64_t)m_base * a.ldx * 2, a.x_bytes - (uint32_t)m_base * a.ldx * 2);
 
     uint32_t w_off[NTW];
@@ -195,6 +205,14 @@ __global__ __launch_bounds__(512, 2) void qbatch_kernel(const BatchArgs a) {
             const bool past = !MORE && (c_begin + WK * r + kw) * CK + kq * VPL >= a.K;
             gc[j].set(past ? (_Float16)0.f : m[0], past ? (_Float16)0.f : m[BN * GR]);
         }
+        f4 sc[SUMS ? NTW : 1];                                // of the columns a lane accumulates
+        if constexpr (SUMS) {
+#pragma unroll
+            for (int j = 0; j < NTW; j++)
+#pragma unroll
+                for (int e = 0; e < 4; e++) sc[j][e] = (float)reinterpret_cast<const _Float16*>(cur + X_BYTES)[((wn * NTW + j) * 16 + 4 * kq + e) * GR + g];
+        }
+        f4 part[SUMS ? MT : 1][SUMS ? NTW : 1];
         const char* xp = cur + nl * PITCH + (kw * CK + kq * VPL) * 2;
         h8 xf[XF][MT];
         auto read_x = [&](int t) {
@@ -210,15 +228,18 @@ __global__ __launch_bounds__(512, 2) void qbatch_kernel(const BatchArgs a) {
                 if constexpr (j == 0 && XF == 1) read_x(t);
                 if constexpr (j == 0 && XF == 2 && t + 1 < STEPS) read_x(t + 1);
                 h2 o[4];
-                if constexpr (BITS == 4) dequant_word4<true>(s.w[j][0][t], gc[j], o);
+                if constexpr (BITS == 4) dequant_word4<!SUMS>(s.w[j][0][t], gc[j], o);
                 else if constexpr (BITS == 2) dequant_halfword2_nat(s.w[j][0][t / 2], t % 2, gc[j], o);
                 else {
-                    dequant_word8_nat(s.w[j][t / 2][2 * (t % 2)], gc[j], o);
-                    dequant_word8_nat(s.w[j][t / 2][2 * (t % 2) + 1], gc[j], o + 2);
+                    dequant_word8_nat<!SUMS>(s.w[j][t / 2][2 * (t % 2)], gc[j], o);
+                    dequant_word8_nat<!SUMS>(s.w[j][t / 2][2 * (t % 2) + 1], gc[j], o + 2);
                 }
                 const h8 wf = pack_h8(o);
 #pragma unroll
-                for (int i = 0; i < MT; i++) acc[i][j] = __builtin_amdgcn_mfma_f32_16x16x32_f16(wf, xf[t % XF][i], acc[i][j], 0, 0, 0);
+                for (int i = 0; i < MT; i++) {
+                    if constexpr (!SUMS) acc[i][j] = __builtin_amdgcn_mfma_f32_16x16x32_f16(wf, xf[t % XF][i], acc[i][j], 0, 0, 0);
+                    else part[i][j] = __builtin_amdgcn_mfma_f32_16x16x32_f16(wf, xf[t % XF][i], t == 0 ? f4{0.f, 0.f, 0.f, 0.f} : part[i][j], 0, 0, 0);
+                }
                 if constexpr (MORE) {
                     static_for<0, TASKS>([&](auto kc) {
                         constexpr int k = decltype(kc)::value;
@@ -240,6 +261,14 @@ __global__ __launch_bounds__(512, 2) void qbatch_kernel(const BatchArgs a) {
             });
         });
         __builtin_amdgcn_sched_barrier(0);
+        if constexpr (SUMS) {
+#pragma unroll
+            for (int j = 0; j < NTW; j++)
+#pragma unroll
+                for (int i = 0; i < MT; i++)
+#pragma unroll
+                    for (int e = 0; e < 4; e++) acc[i][j][e] = __builtin_fmaf(part[i][j][e], sc[j][e], acc[i][j][e]);
+        }
         if constexpr (MORE) __syncthreads();
     };
     auto request = [&](XSet& xs, WSet& ws, int r) {
@@ -324,11 +353,11 @@ __global__ __launch_bounds__(512, 2) void qbatch_kernel(const BatchArgs a) {
     }
 }
 
-template <int BITS, int GROUP, int MT, int NTW, bool BF16>
+template <int BITS, int GROUP, int MT, int NTW, bool BF16, bool SUMS>
 int launch_qbatch(BatchArgs a, hipStream_t stream) {
     constexpr int LDS = BatchCfg<MT, NTW>::template lds<GROUP>();
     static_assert(LDS <= 160 * 1024, "the staged x, scales and zero points have to fit LDS twice");
-    auto kern = qbatch_kernel<BITS, GROUP, MT, NTW, BF16>;
+    auto kern = qbatch_kernel<BITS, GROUP, MT, NTW, BF16, SUMS>;
     static uint64_t big_lds_devices = 0;                   // per instantiation
     if (LDS > 64 * 1024 && !bw_allow_big_lds(reinterpret_cast<const void*>(kern), big_lds_devices)) return BW_ELAUNCH;
     a.mtiles = (a.M + 16 * MT - 1) / (16 * MT);
@@ -340,7 +369,11 @@ int launch_qbatch(BatchArgs a, hipStream_t stream) {
 template <int BITS>
 int launch_qbatch_bits(int group, int mt, int ntw, const BatchArgs& a, hipStream_t stream) {
 #define BW_CASE(G, T, W) \
-    if (group == G && mt == T && ntw == W) return a.x_bf16 ? launch_qbatch<BITS, G, T, W, true>(a, stream) : launch_qbatch<BITS, G, T, W, false>(a, stream);
+    if (group == G && mt == T && ntw == W) {                                                                                          \
+        if constexpr (bw_qbatch_sums(BITS, G, T, W))                                                                                  \
+            if (a.sums) return a.x_bf16 ? launch_qbatch<BITS, G, T, W, true, true>(a, stream) : launch_qbatch<BITS, G, T, W, false, true>(a, stream); \
+        return a.x_bf16 ? launch_qbatch<BITS, G, T, W, true, false>(a, stream) : launch_qbatch<BITS, G, T, W, false, false>(a, stream);  \
+    }
 #define BW_ROWS(G, T) BW_CASE(G, T, 1) BW_CASE(G, T, 2) BW_CASE(G, T, 3)
 #define BW_GROUP(G) BW_ROWS(G, 1) BW_ROWS(G, 2) BW_ROWS(G, 3) BW_ROWS(G, 4) BW_ROWS(G, 6) BW_CASE(G, 8, 1) BW_CASE(G, 8, 2)
     BW_GROUP(128) BW_GROUP(64) BW_GROUP(32)
