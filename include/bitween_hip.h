@@ -111,7 +111,7 @@ int bw_dequantize(const int32_t* qweight, const void* scale, int scale_dtype, co
  *   bias   [N] float16 or NULL
  * bw_qgemv: decode path, 1 <= M <= 16, HBM-bound, no workspace.
  * bw_qgemm: prefill path, any M >= 1, MFMA-bound.
- * bw_qlinear: picks between them and a third, the batch kernel (5 ... 128 rows, no entry point of its own), by shape; without
+ * bw_qlinear: picks between them and a third, the batch kernel (5 ... 2048 rows, no entry point of its own), by shape; without
  *             a workspace: up to M = bw_qlinear_decode_rows(N, K, bits) (48; 32 for layers of 10 MiB of packed
  *             weights and more; 16 from 40 MiB on) the batch kernel where it needs none, else the decode kernel, 16
  *             rows per launch; the prefill kernel beyond.  BW_BF16 x up to those rows. */
