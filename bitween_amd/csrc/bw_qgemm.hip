@@ -136,16 +136,27 @@ __global__ __launch_bounds__(256) void cast_bf16_f16_kernel(const uint16_t* __re
 
 }  // namespace
 
-// What a call of 65 ... 2048 rows takes with 128-row tiles, fitted to 300 timings of 23 shapes at 2, 4 and 8 bits (rms error 9 %): for
-// each round of tiles 1.34 us (1.69 at 8 bits) per 128 values of K, 0.59 more on a full chip; 4.6 us and 1.6 us per million
-// partial sums where a short round is cut along K.
-float bw_qgemm_expected_us(int64_t M, int64_t N, int64_t K, int bits) {
-    const int steps = (int)((K + 127) / 128), cus = bw_device_cus();
-    const GemmPlan p = gemm_plan(M, N, steps, true);
-    const int rest = p.tiles - p.full_tiles, whole = steps * ((p.full_tiles + cus - 1) / cus);
-    const float fill = p.tiles < cus ? (float)p.tiles / cus : 1.f;
-    return 4.5f + (whole + (rest ? p.chunks_per_split : 0)) * (bits == 8 ? 1.69f : 1.34f) + 0.59f * fill * whole +
-           (rest ? 4.6f + 1.63e-6f * rest * p.splits * (128 * BN) : 0.f);
+// What a call of 65 ... 2048 rows takes, us, with the tiles it would run (gemm_tile_rows, a workspace on offer), float16 x.  Fitted to 1773
+// timings of 65 ... 2048 rows where this kernel and the batch kernel are within a factor of two (all formats, K and N 512 ...
+// 22016; rms error 6 %; 14 % with 128-row tiles assumed throughout and no look at format and N): a base; per 128 values of K of every
+// round of tiles `step` on an empty chip and `fill` more on a full one; the same for the slices of a short round that is cut along K,
+// 7.3 and 0.38 us per million partial sums for the cut; more per step at 8 bits, groups of 32 and K % 128 != 0; rows of y that start
+// off an 8-byte boundary cost a round of uncut tiles `odd`, their stores going out as 2-byte pieces.
+float bw_qgemm_expected_us(int64_t M, int64_t N, int64_t K, int bits, int group) {
+    struct Cost { float base, step, fill, cut_step, cut_fill, b8, odd; };
+    static constexpr Cost k64 = {5.8f, 0.61f, 0.68f, 0.66f, 0.38f, 0.39f, 0.f}, k128 = {7.4f, 0.96f, 0.68f, 0.77f, 0.87f, 0.27f, 7.4f},
+                          k256 = {12.1f, 1.34f, 1.41f, 0.77f, 0.87f, 0.34f, 16.6f};
+    const bool nat = gemm_nat(M, K, K);
+    const int rows = gemm_tile_rows(M, N, K, K, bits, true, ~(size_t)0), nchunks = gemm_chunks(K, bits, nat), cus = bw_device_cus();
+    const Cost& c = rows == 64 ? k64 : rows == 128 ? k128 : k256;
+    const GemmPlan p = gemm_plan(M, N, nchunks, true, rows);
+    const float steps = bits == 2 && !nat ? 2.f : 1.f;       // of 128 values in a chunk
+    const int rest = p.tiles - p.full_tiles, rounds = (p.full_tiles + cus - 1) / cus;
+    const float extra = (bits == 8 ? c.b8 : bits == 2 ? -0.04f : 0.f) + (nat ? 0.f : 0.37f) + (group == 32 ? bits == 8 ? 0.18f : 0.12f : 0.f);
+    float us = c.base + steps * nchunks * ((c.step + extra) * rounds + c.fill * p.full_tiles / cus) + (N % 4 ? c.odd * rounds : 0.f);
+    if (rest)
+        us += 7.3f + 0.38e-6f * rest * p.splits * (rows * BN) + steps * p.chunks_per_split * (c.cut_step + extra + c.cut_fill * rest * p.splits / cus);
+    return us;
 }
 
 extern "C" int bw_cast_bf16_f16(const void* x, int64_t rows, int64_t cols, int64_t ldx, void* y, int64_t ldy, void* stream) {

@@ -1,6 +1,9 @@
-"""Host side of bw_qlinear_ws, without a GPU: the memory of searched plans."""
+"""Host side of bw_qlinear_ws, without a GPU: the memory of searched plans, the choice between the batch and the prefill kernel."""
 import os
 import subprocess
+
+import pytest
+import torch
 
 CSRC = os.path.join(os.path.dirname(os.path.dirname(os.path.abspath(__file__))), "bitween_amd", "csrc")
 
@@ -47,3 +50,28 @@ def test_layers_of_a_model_keep_their_plans(tmp_path):
     out = subprocess.run([str(binary)], capture_output=True, text=True)
     assert out.returncode == 0, out.returncode
     assert int(out.stdout) == 5
+
+
+# (K, N, rows, bits, group, us of the batch kernel, us of the prefill kernel) on an MI355X, float16 x unless marked: calls on which the two
+# differ by 8 % and more.  Beside each the prefill kernel's tile height, or what sets its time.
+MEASURED = [
+    (4096, 14336, 80, 4, 128, 24.0, 27.4), (2048, 2048, 333, 4, 128, 10.8, 20.4), (4096, 4096, 316, 4, 128, 21.1, 25.9),
+    (13824, 5120, 140, 4, 32, 40.3, 47.0), (8192, 8192, 334, 4, 128, 76.2, 61.2), (6912, 8048, 218, 4, 128, 46.9, 42.0),
+    (11008, 4096, 434, 4, 64, 67.0, 55.8), (13824, 5120, 1539, 2, 128, 290.8, 230.9), (5120, 13824, 656, 4, 128, 132.7, 103.5),   # (the last two: 256)
+    (4096, 11008, 310, 4, 128, 53.4, 46.1), (4096, 14336, 269, 4, 128, 53.2, 46.6), (4608, 10864, 321, 4, 128, 58.6, 51.9),      # one round, just over half full
+    (4096, 4096, 1042, 2, 128, 55.0, 49.2), (5888, 8512, 396, 4, 128, 79.5, 69.1), (2304, 4432, 813, 4, 128, 37.0, 32.1),
+    (14336, 4096, 107, 8, 32, 33.6, 37.5), (14336, 4096, 99, 8, 64, 34.8, 39.9),                                                # 64 (the second: bfloat16)
+    (512, 6149, 299, 4, 128, 12.5, 18.6), (896, 6299, 399, 2, 128, 18.6, 24.1), (640, 4945, 389, 2, 128, 17.1, 24.7),            # rows of y off 8 bytes
+    (11968, 3760, 359, 2, 64, 49.0, 57.8), (8768, 3520, 242, 2, 32, 33.3, 40.5),                                                # K % 128 != 0
+    (3840, 5224, 770, 8, 32, 70.0, 61.2), (7040, 2944, 449, 8, 128, 40.2, 45.7),
+]
+
+
+@pytest.mark.skipif(torch.cuda.is_available(), reason="the choice for 256 compute units, what the library assumes without a GPU")
+@pytest.mark.parametrize("k,n,m,bits,g,batch,prefill", MEASURED)
+def test_route_takes_the_faster_kernel(k, n, m, bits, g, batch, prefill):
+    """bw_qlinear_workspace_bytes asks for room to cast a bfloat16 x only where the prefill kernel runs: that tells the route."""
+    from bitween_amd.kernels import hip_loader
+    need = hip_loader.load().bw_qlinear_workspace_bytes
+    takes_prefill = need(m, n, k, bits, g, hip_loader.BW_BF16) > need(m, n, k, bits, g, hip_loader.BW_F16)
+    assert takes_prefill == (prefill < batch)
