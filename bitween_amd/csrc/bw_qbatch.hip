@@ -140,10 +140,10 @@ Route route(int64_t M, int64_t N, int64_t K, int bits, int group) {
     return 1.035f * batch_cost(M, N, K, bits, group, true).us < 0.97f * prefill ? kBatch : kPrefill;
 }
 
-// What the batch kernel asks of a call beyond bw_fast_shape: 4-byte words of scales, offsets of x in 31 bits.
+// What the batch kernel asks of a call beyond bw_fast_shape: whole float16 values of scales, offsets of x in 31 bits.
 inline bool batch_takes(const void* x, int64_t M, int64_t N, int64_t K, int64_t ldx, const void* qweight, const void* scale16, const void* zp16, int bits, int group) {
-    return bw_fast_shape(M, N, K, ldx, bits, group) && bw_aligned(x, 16) && (ldx * 2) % 16 == 0 && bw_aligned(qweight, 16) && bw_aligned(scale16, 4) &&
-           bw_aligned(zp16, 4) && M * ldx * 2 < (int64_t)kBatchMaxBytes;
+    return bw_fast_shape(M, N, K, ldx, bits, group) && bw_aligned(x, 16) && (ldx * 2) % 16 == 0 && bw_aligned(qweight, 16) && bw_aligned(scale16, 2) &&
+           bw_aligned(zp16, 2) && M * ldx * 2 < (int64_t)kBatchMaxBytes;
 }
 
 int launch_batch(const void* x, int act_dtype, int64_t M, int64_t K, int64_t ldx, const int32_t* qweight, const void* scale16, const void* zp16,
@@ -187,9 +187,7 @@ extern "C" size_t bw_qlinear_workspace_bytes(int64_t M, int64_t N, int64_t K, in
     if (!bw_shape_ok(N, K, bits, group) || M < 1 || M >= ((int64_t)1 << 31)) return 0;
     const bool fast = bw_fast_shape(M, N, K, K, bits, group);
     const Route r = fast ? route(M, N, K, bits, group) : M <= 16 ? kDecode : kPrefill;
-    // (a call that this kernel turns out not to take - unaligned scales - falls back to the prefill kernel)
-    const size_t prefill = M <= 16 ? 0 : bw_qgemm_workspace_bytes(M, N, K, bits, group);
-    size_t split = r == kPrefill ? prefill : 0;
+    size_t split = r == kPrefill && M > 16 ? bw_qgemm_workspace_bytes(M, N, K, bits, group) : 0;
     if (r == kBatch) split = batch_ws_bytes(M, N, batch_plan(M, N, K, bits, group, true));
     const bool cast = act_dtype == BW_BF16 && (r == kPrefill || !fast);
     return split + (cast ? cast_bytes(M, K) : 0);

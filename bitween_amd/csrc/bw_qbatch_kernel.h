@@ -142,16 +142,21 @@ __global__ __launch_bounds__(512, 2) void qbatch_kernel(const BatchArgs a) {
     };
     auto issue_x = [&](XSet& xs, int p, uint32_t ko) { xs.x[p] = __builtin_amdgcn_raw_buffer_load_b128(rx, ko + row_off[p], 0, 0); };
     // scales (waves 0 - 3) and zero points (waves 4 - 7) of a round: GR / 2 words for each of the BN columns, neighbouring
-    // threads on neighbouring words; 8 bytes from the 4-byte boundary below, of which the row's parity picks two halves
+    // threads on neighbouring words; 8 bytes from the 4-byte boundary below, of which the row's parity (and the array's, where it starts
+    // off a 4-byte boundary, as a row slice of an odd number of groups may) picks two halves
     uint32_t meta_off[ML], meta_shift[ML];
+    // (of the pointer itself: two more kernel arguments cost every launch 0.2 ... 0.35 us; the two bytes ahead of such an array belong to
+    // the word it starts in)
+    const char* const marr = (const char*)(wave < 4 ? a.scale : a.zp);
+    const uint32_t skew = (uint32_t)(uintptr_t)marr & 2u;
 #pragma unroll
     for (int i = 0; i < ML; i++) {
         const int item = (tid & 255) + 256 * i, n = item / (GR / 2), w = item - n * (GR / 2);
-        const uint32_t off = (uint32_t)(min(n_base + n, a.N - 1) * a.groups + c_begin * CK / GROUP) * 2 + 4 * w;
+        const uint32_t off = (uint32_t)(min(n_base + n, a.N - 1) * a.groups + c_begin * CK / GROUP) * 2 + 4 * w + skew;
         meta_off[i] = n < BN ? off & ~3u : kOob;
         meta_shift[i] = (off & 2) * 8;
     }
-    const __amdgpu_buffer_rsrc_t rm = batch_rsrc(wave < 4 ? a.scale : a.zp, (a.meta_bytes + 3) & ~3u);
+    const __amdgpu_buffer_rsrc_t rm = batch_rsrc(marr - skew, (a.meta_bytes + skew + 3) & ~3u);
     auto issue_meta = [&](XSet& xs, int i, int r) { xs.m[i] = __builtin_amdgcn_raw_buffer_load_b64(rm, meta_off[i] + (uint32_t)r * (GR * 2), 0, 0); };
     auto stage_x = [&](const XSet& xs, int p, char* buf) {
         u4 in = xs.x[p], o;

@@ -1,4 +1,4 @@
-"""The batch kernel (bw_qlinear_ws from 5, 17 or so rows up to 128) against the oracle: every format, row counts at the edges of
+"""The batch kernel (bw_qlinear_ws from 5, 17 or so rows up to 2048) against the oracle: every format, row counts at the edges of
 its row tiles, columns and K that end inside tiles and rounds, K cut across workgroups or not, float16 and bfloat16 x."""
 import ctypes
 
@@ -100,7 +100,7 @@ def test_decode_rows_on_large_layers(bits, g, k, n, m):
 
 @pytest.mark.parametrize("m", [7, 17, 70])
 def test_layouts_the_batch_kernel_does_not_take(m):
-    """Scales off a 4-byte boundary go to the other kernels, with bfloat16 x too; a workspace that is too small is not used."""
+    """Scales off a 4-byte boundary, with bfloat16 x too; no x and an unknown type of x are refused."""
     from bitween_amd.kernels import hip_loader
     lib = hip_loader.load()
     bits, g, k, n = 4, 128, 1280, 260
@@ -147,3 +147,30 @@ def test_several_tiles_of_rows(bits, g, m, k, n):
             check_matmul(y[:, :n].contiguous(), x.to(torch.float16).cpu().numpy(), qw, s16, z16, None, bits, g)
             for r, c in hot.items():
                 assert np.array_equal(y[r, :n].cpu().numpy().view(np.uint16), w16[:, c].view(np.uint16))
+
+
+@pytest.mark.parametrize("bits,g", FORMATS)
+@pytest.mark.parametrize("m", [17, 40, 130])
+def test_scales_off_a_four_byte_boundary(bits, g, m):
+    """Row slices of scales and zero points with an odd number of groups may start inside a 4-byte word: the same kernel, so the same bits,
+    as with arrays of their own (either array off the boundary, or both), for the first and the last group of every column."""
+    from bitween_amd.kernels import hip_loader
+    lib = hip_loader.load()
+    n, k = 205, 9 * 128 + (g if g < 128 else 0)
+    _, qw, s16, z16, b16 = quantized_layer(n, k, bits, g, seed=m + bits + g, outliers=True)
+    qw, s, z, b = [to_gpu(a) for a in (qw, s16, z16, b16)]
+    x = torch.randn(m, k, device="cuda", dtype=torch.float16)
+    x[0], x[1] = 0, 0
+    x[0, 0], x[1, k - 1] = 1, 1
+
+    def shifted(t):
+        buf = torch.full((t.numel() + 2,), float("nan"), dtype=t.dtype, device="cuda")
+        buf[1:-1] = t.reshape(-1)
+        return buf[1:-1].view(t.shape)
+
+    st, want, _ = _call(lib, x, (qw, s, z), n, bits, g, n, bias=b)
+    assert st == 0
+    check_matmul(want, x.cpu().numpy(), qw.cpu().numpy(), s16, z16, b16, bits, g)
+    for sv, zv in ((shifted(s), z), (s, shifted(z)), (shifted(s), shifted(z))):
+        st, y, _ = _call(lib, x, (qw, sv, zv), n, bits, g, n, bias=b)
+        assert st == 0 and torch.equal(y, want)
