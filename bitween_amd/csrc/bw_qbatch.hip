@@ -54,7 +54,7 @@ inline int batch_mt(int64_t M) { const int t = (int)((M + 15) / 16); return t <=
 // Lower tiles than the call has rows read the weights (out of L2) once per tile, but fill the chip without a cut of K and its
 // reduction: W4 g128 us, one tile of rows against the plan, 2048 x 2048 at 64 rows 8.5 -> 5.3, at 128 rows 11.4 -> 6.3; 4096 x 4096 at
 // 64 rows 12.4 -> 8.8, at 128 rows 18.1 -> 12.2; 4096 -> 11008 at 128 rows 28.6 -> 23.8.
-struct BatchCost { BatchPlan plan; float us; };
+struct BatchCost { BatchPlan plan; float us; bool ahead; };   // ahead: this kernel takes a call of 17 rows and more
 
 // Calls that scale a group's sum in float32: the rows that are, or by bw_qlinear_decode_rows would be, the decode kernels'.
 inline bool batch_sums(int64_t M, int64_t N, int64_t K, int bits, int group) {
@@ -63,7 +63,7 @@ inline bool batch_sums(int64_t M, int64_t N, int64_t K, int bits, int group) {
 
 BatchCost batch_search(int64_t M, int64_t N, int64_t K, int bits, int group, bool may_split) {
     const int nchunks = (int)((K + 127) / 128), cus = bw_device_cus(), whole = batch_mt(M);
-    BatchCost best{{whole, 1, 1}, 1e30f};
+    BatchCost best{{whole, 1, 1}, 1e30f, true};
     const bool sums = batch_sums(M, N, K, bits, group);
     for (const int mt : {1, 2, 3, 4, 6, 8}) {
         const int64_t mtiles = (M + 16 * mt - 1) / (16 * mt);
@@ -81,7 +81,7 @@ BatchCost batch_search(int64_t M, int64_t N, int64_t K, int bits, int group, boo
                 if (used != s || (s > 1 && M * N * s > ((int64_t)32 << 20))) continue;   // (128 MiB of partial sums)
                 const float waves = (float)((tiles * s + cus - 1) / cus);
                 const float us = 2.4f + waves * (rounds * round + wave) + (s > 1 ? 2.f + 0.05f * s + 1.6e-6f * (float)M * (float)N * s : 0.f);
-                if (us < best.us) best = {{mt, ntw, s}, us};
+                if (us < best.us) best = {{mt, ntw, s}, us, true};
             }
         }
     }
@@ -91,9 +91,32 @@ BatchCost batch_search(int64_t M, int64_t N, int64_t K, int bits, int group, boo
     return best;
 }
 
+// 17 ... 64 rows: this kernel; on 1337 layers, formats and row counts there it takes 0.35 ... 0.94 of the time of the prefill kernel and of
+// the decode kernels in launches of 16 rows (W4 g128 at 64 rows, us, prefill kernel against this one: 4096 x 4096 17.8 -> 8.8, 4096 ->
+// 11008 20.9 -> 17.2, 11008 -> 4096 24.8 -> 18.9; 2048 x 2048 13.3 -> 5.3).  Beyond, whichever is expected to be done first: the prefill
+// kernel's 128 x 256 tiles leave the chip idle on most layers of a few hundred rows, or have to be cut along K (W4 g128, us, prefill
+// against this: 2048 x 2048 at 333 rows 20.4 -> 10.8, at 768 rows 26.7 -> 14.5; 4096 x 4096 at 256 rows 28.6 -> 17.6, at 512
+// rows 32.4 -> 30.0, but at 768 rows 39.8 against 47.9; 4096 -> 14336 at 128 rows 31.3 -> 27.4, at 160 rows 41.5 against 42.9, at 269
+// 46.5 against 53.2; 4096 -> 11008 at 310 rows 46.1 against 53.4; 512 -> 13056 at 200 rows 11.3 against 15.2).  The models
+// are of float16 x; bfloat16 costs this kernel 7 % and the prefill kernel a cast (3.2 us and 0.5 us per million values).  Both types take
+// one route, so that a bfloat16 x and its float16 rounding give the same bits: half of both is added.  A doubtful call of up
+// to 128 rows stays here (1.06: 14336 -> 4096 W4 g128 at 128 rows replayed from a graph 32.6 against 30.3 us, with bfloat16 34.0 against
+// 33.1, but in eager code, where the cast is one launch more, an MLP with it takes 92 us against 95 ... 98), of more rows
+// with the prefill kernel (0.97).  On 5452 calls of 65 ... 2048 rows the choice loses 0.3 % against the better of the two (27 % at most),
+// and 42 of them are 3 % or more behind the prefill kernel; 0.5 % (51 %) and 78 with a model of 128-row tiles of the prefill kernel alone.
+bool batch_ahead(int64_t M, int64_t N, int64_t K, int bits, int group, float us) {
+    if (M <= 64) return true;
+    const float half_cast = 1.6f + 0.25e-6f * (float)M * (float)K, prefill = bw_qgemm_expected_us(M, N, K, bits, group) + half_cast;
+    return 1.035f * us < (M <= 128 ? 1.06f : 0.97f) * prefill;
+}
+
 BatchCost batch_cost(int64_t M, int64_t N, int64_t K, int bits, int group, bool may_split) {
-    static thread_local BwPlanCache<BatchCost> cache = {};   // the search takes 1 ... 3 us of a call's host time, a look here 10 ns
-    return cache.get(M, N, K, (bits * 2 + may_split) * 256 + group, [&] { return batch_search(M, N, K, bits, group, may_split); });
+    static thread_local BwPlanCache<BatchCost> cache = {};   // the search takes 1 ... 3 us of a call's host time, the prefill kernel's model as much again; a look here 10 ns
+    return cache.get(M, N, K, (bits * 2 + may_split) * 256 + group, [&] {
+        BatchCost found = batch_search(M, N, K, bits, group, may_split);
+        found.ahead = batch_ahead(M, N, K, bits, group, found.us);
+        return found;
+    });
 }
 
 BatchPlan batch_plan(int64_t M, int64_t N, int64_t K, int bits, int group, bool may_split) { return batch_cost(M, N, K, bits, group, may_split).plan; }
@@ -121,23 +144,9 @@ inline bool batch_takes_decode_rows(int64_t M, int64_t N, int64_t K, int bits, i
     return bits == 2 && M > 8 && tiles > 3 * cus && (group == 32 || K / group % 2);
 }
 
-// 17 ... 64 rows: this kernel; on 1337 layers, formats and row counts there it takes 0.35 ... 0.94 of the time of the prefill kernel and of
-// the decode kernels in launches of 16 rows (W4 g128 at 64 rows, us, prefill kernel against this one: 4096 x 4096 17.8 -> 8.8, 4096 ->
-// 11008 20.9 -> 17.2, 11008 -> 4096 24.8 -> 18.9; 2048 x 2048 13.3 -> 5.3).  Beyond, whichever is expected to be done first: the prefill
-// kernel's 128 x 256 tiles leave the chip idle on most layers of a few hundred rows, or have to be cut along K (W4 g128, us, prefill
-// against this: 2048 x 2048 at 333 rows 20.4 -> 10.8, at 768 rows 26.7 -> 14.5; 4096 x 4096 at 256 rows 28.6 -> 17.6, at 512
-// rows 32.4 -> 30.0, but at 768 rows 39.8 against 47.9; 4096 -> 14336 at 128 rows 31.3 -> 27.4, at 160 rows 41.5 against 42.9, at 269
-// 46.5 against 53.2; 4096 -> 11008 at 310 rows 46.1 against 53.4; 512 -> 13056 at 200 rows 11.3 against 15.2).  The models
-// are of float16 x; bfloat16 costs this kernel 7 % and the prefill kernel a cast (3.2 us and 0.5 us per million values).  Both types take
-// one route, so that a bfloat16 x and its float16 rounding give the same bits: half of both is added.  A doubtful call stays with the
-// prefill kernel (0.97).  On 5284 calls of 65 ... 2048 rows the choice loses 0.3 % against the better of the two (27 % at most), and 30
-// of them are 3 % or more behind the prefill kernel; 0.5 % (51 %) and 74 with a model of 128-row tiles of the prefill kernel alone.
 Route route(int64_t M, int64_t N, int64_t K, int bits, int group) {
     if (M <= 16) return batch_takes_decode_rows(M, N, K, bits, group) ? kBatch : kDecode;
-    if (M <= 64) return kBatch;
-    if (M > 2048) return kPrefill;
-    const float half_cast = 1.6f + 0.25e-6f * (float)M * (float)K, prefill = bw_qgemm_expected_us(M, N, K, bits, group) + half_cast;
-    return 1.035f * batch_cost(M, N, K, bits, group, true).us < 0.97f * prefill ? kBatch : kPrefill;
+    return M <= 2048 && batch_cost(M, N, K, bits, group, true).ahead ? kBatch : kPrefill;
 }
 
 // What the batch kernel asks of a call beyond bw_fast_shape: whole float16 values of scales, offsets of x in 31 bits.
