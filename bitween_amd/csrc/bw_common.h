@@ -1,6 +1,7 @@
 // Shared device helpers for the gfx950 kernels of libbitween_hip.so.
 #pragma once
 #include <hip/hip_runtime.h>
+#include <initializer_list>
 #include <type_traits>
 #include <stdint.h>
 
@@ -254,6 +255,12 @@ BW_DEV void wait_loads() {
     static_assert(N >= 0 && N < 64, "vmcnt is a 6-bit counter");
     __builtin_amdgcn_s_waitcnt((N & 15) | ((N >> 4) << 14) | 0x0F70);   // expcnt and lgkmcnt left alone
 }
+
+// Name of the decode or batch kernel this thread launched last (bw_qgemv_last_kernel): lets a benchmark label its numbers
+// with the kernel that actually ran.  The string is built once per kernel instantiation; a launch only stores a pointer.
+const char* bw_kernel_name(const char* base, std::initializer_list<int> params);
+void bw_note_kernel(const char* name);
+#define BW_NOTE_KERNEL(base, ...) do { static const char* const nm = bw_kernel_name(base, {__VA_ARGS__}); bw_note_kernel(nm); } while (0)
 
 // Host-side argument checks shared by the entry points.
 static inline bool bw_bits_ok(int bits) { return bits == 2 || bits == 4 || bits == 8; }

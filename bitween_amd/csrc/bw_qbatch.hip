@@ -210,6 +210,7 @@ extern "C" int bw_qlinear_ws(const void* x, int act_dtype, int64_t M, int64_t K,
     if (act_dtype != BW_F16 && act_dtype != BW_BF16) return BW_EUNSUPPORTED;
     if (workspace && !bw_aligned(workspace, 16)) return BW_EALIGN;
     if (!workspace) workspace_bytes = 0;
+    bw_note_kernel("");
     const bool fast = bw_fast_shape(M, N, K, ldx, bits, group);
     Route r = fast ? route(M, N, K, bits, group) : M <= 16 ? kDecode : kPrefill;
     if (r == kBatch && batch_takes(x, M, N, K, ldx, qweight, scale16, zp16, bits, group)) {
@@ -239,6 +240,7 @@ extern "C" int bw_qlinear_ws(const void* x, int act_dtype, int64_t M, int64_t K,
 extern "C" int bw_qlinear(const void* x, int act_dtype, int64_t M, int64_t K, int64_t ldx, const int32_t* qweight,
                           const void* scale16, const void* zp16, const void* bias, int64_t N, int bits, int group,
                           void* y, int64_t ldy, void* stream) {
+    bw_note_kernel("");
     if (M >= 1 && M <= bw_qlinear_decode_rows(N, K, bits) && (act_dtype == BW_F16 || act_dtype == BW_BF16)) {
         // the batch kernel where it is what bw_qlinear_ws runs too and K needs no cut for want of workgroups
         if (x && qweight && scale16 && zp16 && y && bw_shape_ok(N, K, bits, group) && ldx >= K && ldy >= N &&

@@ -367,6 +367,7 @@ int launch_qbatch(BatchArgs a, hipStream_t stream) {
     if (LDS > 64 * 1024 && !bw_allow_big_lds(reinterpret_cast<const void*>(kern), big_lds_devices)) return BW_ELAUNCH;
     a.mtiles = (a.M + 16 * MT - 1) / (16 * MT);
     a.ntiles = (a.N + BatchCfg<MT, NTW>::BN - 1) / BatchCfg<MT, NTW>::BN;
+    BW_NOTE_KERNEL("qbatch_kernel", BITS, GROUP, MT, NTW, (int)BF16, (int)SUMS);
     hipLaunchKernelGGL(kern, dim3((unsigned)(a.mtiles * a.ntiles * a.splits)), dim3(512), LDS, stream, a);
     return hipGetLastError() == hipSuccess ? BW_OK : BW_ELAUNCH;
 }

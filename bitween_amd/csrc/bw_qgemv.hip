@@ -32,17 +32,6 @@
 
 namespace {
 
-// Name of the decode kernel this thread launched last (bw_qgemv_last_kernel): lets a benchmark label its numbers
-// with the kernel that actually ran.  The string is built once per kernel instantiation; a launch only stores a pointer.
-thread_local const char* g_last_kernel = "";
-inline const char* kernel_name(const char* base, std::initializer_list<int> params) {
-    std::string s = std::string(base) + "<";
-    bool first = true;
-    for (int v : params) { s += (first ? "" : ", ") + std::to_string(v); first = false; }
-    return (new std::string(s + ">"))->c_str();           // lives as long as the library
-}
-#define BW_NOTE_KERNEL(base, ...) do { static const char* const nm = kernel_name(base, {__VA_ARGS__}); g_last_kernel = nm; } while (0)
-
 template <int BITS, int GROUP, int MT>
 struct GemvCfg {
     static constexpr int VPI = 32 / BITS;            // values per int32 word
@@ -1654,6 +1643,17 @@ int launch_gemv(const GemvArgs& a, hipStream_t stream) {
 
 }  // namespace
 
+// ---- the name of the kernel a thread launched last ----
+static thread_local const char* g_last_kernel = "";
+void bw_note_kernel(const char* name) { g_last_kernel = name; }
+const char* bw_kernel_name(const char* base, std::initializer_list<int> params) {
+    std::string s = std::string(base) + "<";
+    bool first = true;
+    for (int v : params) { s += (first ? "" : ", ") + std::to_string(v); first = false; }
+    return (new std::string(s + ">"))->c_str();           // lives as long as the library
+}
+extern "C" const char* bw_qgemv_last_kernel(void) { return g_last_kernel; }
+
 // Shapes the MFMA kernels take: 16-byte lane loads need K*bits/8 % 16 == 0, group in {32, 64, 128}, and
 // every extent must fit the 32-bit offsets of buffer addressing.
 bool bw_fast_shape(int64_t M, int64_t N, int64_t K, int64_t ldx, int bits, int group) {
@@ -1666,15 +1666,13 @@ int bw_qgemm_generic(const void* x, int act_dtype, int64_t M, int64_t K, int64_t
                      const void* scale16, const void* zp16, const void* bias, int64_t N, int bits, int group, void* y,
                      int64_t ldy, void* stream);
 
-extern "C" const char* bw_qgemv_last_kernel(void) { return g_last_kernel; }
-
 extern "C" int bw_qgemv(const void* x, int act_dtype, int64_t M, int64_t K, int64_t ldx, const int32_t* qweight,
                         const void* scale16, const void* zp16, const void* bias, int64_t N, int bits, int group,
                         void* y, int64_t ldy, void* stream) {
     if (!x || !qweight || !scale16 || !zp16 || !y) return BW_EINVAL;
     if (!bw_shape_ok(N, K, bits, group) || M < 1 || M > 16 || ldx < K || ldy < N) return BW_EINVAL;
     if (act_dtype != BW_F16 && act_dtype != BW_BF16) return BW_EUNSUPPORTED;
-    g_last_kernel = "";
+    bw_note_kernel("");
     if (!bw_fast_shape(M, N, K, ldx, bits, group) || !bw_aligned(x, 16) || (ldx * 2) % 16 || !bw_aligned(qweight, 16))
         return bw_qgemm_generic(x, act_dtype, M, K, ldx, qweight, scale16, zp16, bias, N, bits, group, y, ldy, stream);
     GemvArgs a;

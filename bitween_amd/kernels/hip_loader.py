@@ -297,7 +297,7 @@ def quantized_input_grad(grad_y, qweight, scale, zero_point, bits, group_size):
 
 
 def last_decode_kernel():
-    """Name of the decode kernel this thread's last bw_qgemv / bw_qlinear launch ran (a diagnostic for benchmarks)."""
+    """Name of the decode or batch kernel that this thread's last matmul launched; "" if it was another one (a diagnostic for benchmarks)."""
     return load().bw_qgemv_last_kernel().decode()
 
 

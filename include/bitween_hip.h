@@ -168,9 +168,10 @@ int bw_qlinear_ws(const void* x, int act_dtype, int64_t M, int64_t K, int64_t ld
                   int64_t N, int bits, int group, void* y, int64_t ldy,
                   void* workspace, size_t workspace_bytes, void* stream);
 
-/* Diagnostic, no counterpart in the reference: the name (with template arguments) of the decode kernel that the
- * calling thread's last bw_qgemv / bw_qlinear launch ran ("" before the first one, or when the generic kernel ran).
- * For benchmarks that label a timing with the kernel it belongs to; the string lives as long as the library. */
+/* Diagnostic, no counterpart in the reference: the name (with template arguments) of the decode or batch kernel that the
+ * calling thread's last bw_qgemv / bw_qlinear / bw_qlinear_ws call launched ("" before the first one, and when that call ran another
+ * kernel - prefill, generic).  For benchmarks that label a timing with the kernel it belongs to; the string lives as long as the
+ * library. */
 const char* bw_qgemv_last_kernel(void);
 
 int bw_qlinear(const void* x, int act_dtype, int64_t M, int64_t K, int64_t ldx,

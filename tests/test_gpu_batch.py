@@ -174,3 +174,33 @@ def test_scales_off_a_four_byte_boundary(bits, g, m):
     for sv, zv in ((shifted(s), z), (s, shifted(z)), (shifted(s), shifted(z))):
         st, y, _ = _call(lib, x, (qw, sv, zv), n, bits, g, n, bias=b)
         assert st == 0 and torch.equal(y, want)
+
+
+def test_last_kernel_names_the_batch_kernel_and_nothing_else():
+    """bw_qgemv_last_kernel after each call of bw_qlinear_ws (with and without a workspace) and bw_qlinear: the decode or batch kernel of this
+    very call, "" after the prefill and the generic kernel."""
+    from bitween_amd.kernels import hip_loader as hip
+    lib = hip.load()
+    _, qw, s16, z16, _ = quantized_layer(272, 1024, 4, 128, seed=1)
+    d = [to_gpu(a) for a in (qw, s16, z16)]
+
+    def name(m, ws=True, dtype=torch.float16):
+        st, _, _ = _call(lib, torch.randn(m, 1024, device="cuda").to(dtype), d, 272, 4, 128, 272, ws=ws)
+        assert st == 0
+        return hip.last_decode_kernel()
+
+    decode = name(1)
+    assert decode.startswith("qgemv_") and name(40).startswith("qbatch_kernel<4, 128, ") and name(1) == decode
+    assert name(40, ws=False).startswith("qbatch_kernel<4, 128, ") and name(2100) == "" and name(1) == decode
+    x = torch.randn(40, 1024, device="cuda", dtype=torch.float16)
+    y = torch.empty(40, 272, device="cuda", dtype=torch.float16)
+    stream = ctypes.c_void_p(torch.cuda.current_stream().cuda_stream)
+
+    def qlinear(m, bits=4, g=128, k=1024, q=d):
+        assert lib.bw_qlinear(x.data_ptr(), 0, m, k, 1024, q[0].data_ptr(), q[1].data_ptr(), q[2].data_ptr(), None, 272, bits, g, y.data_ptr(), 272, stream) == 0
+        return hip.last_decode_kernel()
+
+    assert qlinear(1) == decode and qlinear(40).startswith("q")
+    _, qw, s16, z16, _ = quantized_layer(272, 960, 4, 48, seed=2)      # groups of 48: the generic kernel
+    assert qlinear(3, g=48, k=960, q=[to_gpu(a) for a in (qw, s16, z16)]) == ""
+    torch.cuda.synchronize()
