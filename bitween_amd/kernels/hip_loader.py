@@ -49,6 +49,9 @@ def load():
     if lib.bw_abi_version() != ABI_VERSION:
         raise BitweenHipError(f"{_LIB_PATH} has ABI version {lib.bw_abi_version()}, this package expects {ABI_VERSION}: "
                               "rebuild it with `python -m bitween_amd.csrc.build`")
+    missing = [name for name in ENTRY_POINTS if not hasattr(lib, name)]    # built before functions were added to this version
+    if missing:
+        raise BitweenHipError(f"{_LIB_PATH} lacks {', '.join(missing)}: rebuild it with `python -m bitween_amd.csrc.build`")
     lib.bw_strerror.restype = ctypes.c_char_p
     lib.bw_strerror.argtypes = [i32]
     lib.bw_quantize_pack.argtypes = [vp, i32, i32, i64, i64, i64, i32, i32, vp, vp, i32, vp, i32, vp]

@@ -205,3 +205,21 @@ def test_scale_division_default_follows_the_tensor_device():
             bitween_amd.set_scale_division("fast")
     finally:
         bitween_amd.set_scale_division(previous)
+
+
+def test_a_library_built_before_an_entry_point_was_added_is_refused_by_name(tmp_path):
+    """Functions are added without a new ABI version (no signature changes): a library that is too old for this package says what it lacks
+    and what to do, in place of an AttributeError from ctypes."""
+    import subprocess
+    import sys
+    stub, lib = tmp_path / "stub.c", tmp_path / "old.so"
+    from bitween_amd.kernels import hip_loader
+    old = [n for n in hip_loader.ENTRY_POINTS if n not in ("bw_abi_version", "bw_qlinear_ws", "bw_qlinear_workspace_bytes")]
+    stub.write_text("int bw_abi_version(void) { return %d; }\n" % hip_loader.ABI_VERSION + "".join("int %s(void) { return 0; }\n" % n for n in old))
+    subprocess.run(["gcc", "-shared", "-fPIC", "-o", str(lib), str(stub)], check=True)
+    program = ("from bitween_amd.kernels import hip_loader as h\n"
+               "try:\n    h.load()\nexcept h.BitweenHipError as e:\n    print(e)\n")
+    out = subprocess.run([sys.executable, "-c", program], capture_output=True, text=True, env=dict(os.environ, BITWEEN_HIP_LIB=str(lib)),
+                         cwd=os.path.dirname(os.path.dirname(os.path.abspath(__file__))))
+    assert out.returncode == 0, out.stderr
+    assert "bw_qlinear_ws, bw_qlinear_workspace_bytes" in out.stdout and "rebuild" in out.stdout
