@@ -81,6 +81,15 @@ struct OnDevice {
     }
 };
 
+// The interpreter lock given up while a call allocates, plans and launches: a full queue or an allocator that goes to the driver would
+// hold every other Python thread up.  Nothing between here and the end of its scope touches a Python object.
+struct Unlocked {
+    PyThreadState* state = PyEval_SaveThread();
+    Unlocked() = default;
+    Unlocked(const Unlocked&) = delete;
+    ~Unlocked() { PyEval_RestoreThread(state); }
+};
+
 struct Layer {
     const void *qweight, *scale, *zero, *bias;
     int64_t n, k;
@@ -269,7 +278,7 @@ bool module_of(PyObject* dict, Module& m) {
 PyObject* py_forward(PyObject*, PyObject* const* args, Py_ssize_t nargs) {
     return guarded([&]() -> PyObject* {
         if (nargs != 2 || !PyDict_Check(args[0]) || !plain(args[1])) return none();
-        const Tensor& x = unpack(args[1]);
+        const Tensor x = unpack(args[1]);
         if (!x.is_cuda() || !x.has_storage()) return none();    // (no storage: a wrapper of vmap or torch.func)
         Module l;
         if (!module_of(args[0], l)) {
@@ -280,14 +289,15 @@ PyObject* py_forward(PyObject*, PyObject* const* args, Py_ssize_t nargs) {
             return nullptr;                                    // the mark says that the native path takes this layer
         int status = 0;
         const char* what = "";
-        if (!(c10::GradMode::is_enabled() && x.requires_grad())) return checked(linear(l.layer, x, status, what), status, what);
-        if (x._fw_grad(0).defined()) return none();            // the Python function refuses forward-mode derivatives
+        const bool recorded = c10::GradMode::is_enabled() && x.requires_grad();
+        if (recorded && x._fw_grad(0).defined()) return none();   // the Python function refuses forward-mode derivatives
         Tensor y;
         {
+            Unlocked unlocked;
             c10::AutoGradMode off(false);
             y = linear(l.layer, x, status, what);
         }
-        if (status == 0 && y.defined()) {
+        if (recorded && status == 0 && y.defined()) {
             std::shared_ptr<QuantizedLinearBackward> node(new QuantizedLinearBackward(), torch::autograd::deleteNode);
             node->set_next_edges(torch::autograd::collect_next_edges(x));
             node->qweight = torch::autograd::SavedVariable(l.qweight, false);
@@ -307,16 +317,19 @@ PyObject* py_matmul(PyObject*, PyObject* const* args, Py_ssize_t nargs) {
         if (nargs != 7 || !PyLong_Check(args[5]) || !PyLong_Check(args[6])) return none();
         for (int i = 0; i < 5; i++)
             if (!plain(args[i]) && !(i == 4 && args[i] == Py_None)) return none();
-        const Tensor& x = unpack(args[0]);
+        const Tensor x = unpack(args[0]);
         if (!x.has_storage() || (x.scalar_type() != at::kHalf && x.scalar_type() != at::kBFloat16)) return none();
+        const Tensor qweight = unpack(args[1]), scale = unpack(args[2]), zero = unpack(args[3]), bias = args[4] == Py_None ? Tensor() : unpack(args[4]);
         Layer l;
-        if (!layer_of(unpack(args[1]), unpack(args[2]), unpack(args[3]), args[4] == Py_None ? nullptr : &unpack(args[4]),
-                      PyLong_AsLong(args[5]), PyLong_AsLong(args[6]), l))
-            return none();
+        if (!layer_of(qweight, scale, zero, bias.defined() ? &bias : nullptr, PyLong_AsLong(args[5]), PyLong_AsLong(args[6]), l)) return none();
         int status = 0;
         const char* what = "";
-        c10::AutoGradMode off(false);
-        Tensor y = linear(l, x, status, what);
+        Tensor y;
+        {
+            Unlocked unlocked;
+            c10::AutoGradMode off(false);
+            y = linear(l, x, status, what);
+        }
         return checked(std::move(y), status, what);
     });
 }
@@ -327,13 +340,17 @@ PyObject* py_input_grad(PyObject*, PyObject* const* args, Py_ssize_t nargs) {
         if (nargs != 6 || !PyLong_Check(args[4]) || !PyLong_Check(args[5])) return none();
         for (int i = 0; i < 4; i++)
             if (!plain(args[i])) return none();
-        const Tensor& go = unpack(args[0]);
+        const Tensor go = unpack(args[0]), qweight = unpack(args[1]), scale = unpack(args[2]), zero = unpack(args[3]);
         Layer l;
-        if (!go.is_cuda() || !go.has_storage() ||
-            !layer_of(unpack(args[1]), unpack(args[2]), unpack(args[3]), nullptr, PyLong_AsLong(args[4]), PyLong_AsLong(args[5]), l))
+        if (!go.is_cuda() || !go.has_storage() || !layer_of(qweight, scale, zero, nullptr, PyLong_AsLong(args[4]), PyLong_AsLong(args[5]), l))
             return none();
         if (go.dim() < 1 || go.size(-1) != l.n || !go.is_floating_point() || go.device().index() != l.device) return none();
-        return THPVariable_Wrap(input_grad(go, unpack(args[1]), unpack(args[2]), unpack(args[3]), l.bits, l.group));
+        Tensor gx;
+        {
+            Unlocked unlocked;
+            gx = input_grad(go, qweight, scale, zero, l.bits, l.group);
+        }
+        return THPVariable_Wrap(std::move(gx));
     });
 }
 
@@ -341,26 +358,29 @@ PyObject* py_input_grad(PyObject*, PyObject* const* args, Py_ssize_t nargs) {
 PyObject* py_quantize(PyObject*, PyObject* const* args, Py_ssize_t nargs) {
     return guarded([&]() -> PyObject* {
         if (nargs != 7 || !plain(args[0]) || !(args[1] == Py_None || plain(args[1]))) return none();
-        c10::AutoGradMode off(false);
-        Tensor w = unpack(args[0]), delta;
+        Tensor w = unpack(args[0]), delta = args[1] == Py_None ? Tensor() : unpack(args[1]);
         const int64_t bits = PyLong_AsLong(args[2]), group = PyLong_AsLong(args[3]);
         const int math = (int)PyLong_AsLong(args[4]), sc = (int)PyLong_AsLong(args[5]), zc = (int)PyLong_AsLong(args[6]);
         if (PyErr_Occurred()) return nullptr;
         const int code = dtype_code(w.scalar_type());
         if (!lib.quantize || !w.is_cuda() || w.dim() != 2 || code < 0 || (bits != 2 && bits != 4 && bits != 8) || group < 1) return none();
-        if (w.stride(1) != 1) w = w.contiguous();
-        if (args[1] != Py_None) {
-            delta = unpack(args[1]);
-            if (delta.device() != w.device() || delta.sizes() != w.sizes() || delta.scalar_type() != w.scalar_type()) return none();
-            if (delta.stride(1) != 1) delta = delta.contiguous();
+        if (delta.defined() && (delta.device() != w.device() || delta.sizes() != w.sizes() || delta.scalar_type() != w.scalar_type())) return none();
+        Tensor q, s, z;
+        int st;
+        {
+            Unlocked unlocked;
+            c10::AutoGradMode off(false);
+            if (w.stride(1) != 1) w = w.contiguous();
+            if (delta.defined() && delta.stride(1) != 1) delta = delta.contiguous();
+            const int64_t n = w.size(0), k = w.size(1);
+            OnDevice on(w.device());
+            q = empty({n, k / (32 / bits)}, at::kInt, w.device());
+            s = empty({n, k / group}, dtype_of(sc), w.device());
+            z = empty({n, k / group}, dtype_of(zc), w.device());
+            st = lib.quantize(w.const_data_ptr(), delta.defined() ? delta.const_data_ptr() : nullptr, code, math, n, k, w.stride(0),
+                              delta.defined() ? delta.stride(0) : 0, (int)bits, (int)group, (int32_t*)q.mutable_data_ptr(),
+                              s.mutable_data_ptr(), sc, z.mutable_data_ptr(), zc, stream_of(w.device().index()));
         }
-        const int64_t n = w.size(0), k = w.size(1);
-        OnDevice on(w.device());
-        Tensor q = empty({n, k / (32 / bits)}, at::kInt, w.device());
-        Tensor s = empty({n, k / group}, dtype_of(sc), w.device()), z = empty({n, k / group}, dtype_of(zc), w.device());
-        const int st = lib.quantize(w.const_data_ptr(), delta.defined() ? delta.const_data_ptr() : nullptr, code, math, n, k, w.stride(0),
-                                    delta.defined() ? delta.stride(0) : 0, (int)bits, (int)group, (int32_t*)q.mutable_data_ptr(),
-                                    s.mutable_data_ptr(), sc, z.mutable_data_ptr(), zc, stream_of(w.device().index()));
         if (st) return checked({}, st, "bw_quantize_pack");
         PyObject* r = PyTuple_New(3);
         if (!r) return nullptr;
@@ -375,21 +395,28 @@ PyObject* py_quantize(PyObject*, PyObject* const* args, Py_ssize_t nargs) {
 PyObject* py_dequantize(PyObject*, PyObject* const* args, Py_ssize_t nargs) {
     return guarded([&]() -> PyObject* {
         if (nargs != 6 || !plain(args[0]) || !plain(args[1]) || !plain(args[2])) return none();
-        c10::AutoGradMode off(false);
         const int64_t group = PyLong_AsLong(args[3]), bits = PyLong_AsLong(args[4]);
         const int oc = (int)PyLong_AsLong(args[5]);
         if (PyErr_Occurred()) return nullptr;
-        const Tensor q = unpack(args[0]).contiguous(), s = unpack(args[1]).contiguous(), z = unpack(args[2]).contiguous();
+        Tensor q = unpack(args[0]), s = unpack(args[1]), z = unpack(args[2]), w;
         const int sc = dtype_code(s.scalar_type()), zc = dtype_code(z.scalar_type());
         if (!lib.dequantize || !q.is_cuda() || s.device() != q.device() || z.device() != q.device() || q.scalar_type() != at::kInt || q.dim() != 2 ||
             sc < 0 || zc < 0 || (bits != 2 && bits != 4 && bits != 8) || group < 1)
             return none();
         const int64_t n = q.size(0), k = q.size(1) * (32 / bits);
         if (s.numel() < n * (k / group) || z.numel() < n * (k / group)) return none();
-        OnDevice on(q.device());
-        Tensor w = empty({n, k}, dtype_of(oc), q.device());
-        const int st = lib.dequantize((const int32_t*)q.const_data_ptr(), s.const_data_ptr(), sc, z.const_data_ptr(), zc, n, k, (int)bits, (int)group,
-                                      w.mutable_data_ptr(), oc, k, stream_of(q.device().index()));
+        int st;
+        {
+            Unlocked unlocked;
+            c10::AutoGradMode off(false);
+            q = q.contiguous();
+            s = s.contiguous();
+            z = z.contiguous();
+            OnDevice on(q.device());
+            w = empty({n, k}, dtype_of(oc), q.device());
+            st = lib.dequantize((const int32_t*)q.const_data_ptr(), s.const_data_ptr(), sc, z.const_data_ptr(), zc, n, k, (int)bits, (int)group,
+                                w.mutable_data_ptr(), oc, k, stream_of(q.device().index()));
+        }
         return checked(std::move(w), st, "bw_dequantize");
     });
 }

@@ -138,3 +138,69 @@ def test_transforms_that_the_python_function_refuses_stay_refused():
     import torch.autograd.forward_ad as fwd
     with fwd.dual_level(), pytest.raises(RuntimeError):         # no jvp
         q(fwd.make_dual(x.clone().requires_grad_(True), torch.ones_like(x)))
+
+
+SLOW_LIBRARY = r"""
+#include <stddef.h>
+#include <stdint.h>
+#include <unistd.h>
+#define SLOW(name) int name() { usleep(300000); return 0; }
+SLOW(bw_qlinear_ws) SLOW(bw_qdgrad) SLOW(bw_quantize_pack_add) SLOW(bw_dequantize) SLOW(bw_cast_bf16_f16)
+size_t bw_qlinear_workspace_bytes() { return 0; }
+size_t bw_qdgrad_workspace_bytes() { return 0; }
+int bw_qdgrad_tile_rows() { return 128; }
+"""
+
+
+def test_other_threads_run_while_a_call_is_under_way(tmp_path):
+    """A launch that blocks (a full queue) must not hold the interpreter lock: a second copy of the native module, bound to a library whose
+    entry points sleep for 0.3 s, leaves another Python thread running in every function."""
+    import ctypes
+    import importlib.util
+    import shutil
+    import subprocess
+    import threading
+    import time
+    from bitween_amd.kernels import hip_loader as hip
+    q = _layer(128, 64, 4, 64)
+    x = torch.randn(3, 128, device="cuda", dtype=torch.float16)
+    go = torch.randn(3, 64, device="cuda", dtype=torch.float16)
+    (tmp_path / "slow.c").write_text(SLOW_LIBRARY)
+    subprocess.run(["gcc", "-shared", "-fPIC", "-o", str(tmp_path / "slow.so"), str(tmp_path / "slow.c")], check=True)
+    slow = ctypes.CDLL(str(tmp_path / "slow.so"))
+    shutil.copy(hip._HOST_PATH, tmp_path / "_bw_host.so")
+    spec = importlib.util.spec_from_file_location("slow_copy._bw_host", tmp_path / "_bw_host.so")
+    host = importlib.util.module_from_spec(spec)
+    spec.loader.exec_module(host)
+    names = [n for n in hip.ENTRY_POINTS if hasattr(slow, n)]
+    _bind(host, {n: ctypes.cast(getattr(slow, n), ctypes.c_void_p).value for n in names})
+    ticks, stop = [0], threading.Event()
+
+    def count():
+        while not stop.is_set():
+            time.sleep(0.001)
+            ticks[0] += 1
+
+    thread = threading.Thread(target=count)
+    thread.start()
+    try:
+        buffers = (q.qweight, q.scale, q.zero_point)
+        calls = {"forward": lambda: host.forward(q.__dict__, x), "matmul": lambda: host.matmul(x, *buffers, q.bias, 4, 64),
+                 "recorded forward": lambda: host.forward(q.__dict__, x.clone().requires_grad_(True)),
+                 "input_grad": lambda: host.input_grad(go, *buffers, 4, 64),
+                 "quantize": lambda: host.quantize(x, None, 4, 64, hip.BW_F32, hip.BW_F16, hip.BW_F16),
+                 "dequantize": lambda: host.dequantize(*buffers, 64, 4, hip.BW_F16)}
+        for name, call in calls.items():
+            call()                                              # (allocator warm: the second call only sleeps)
+            before, start = ticks[0], time.perf_counter()
+            assert call() is not None, name
+            seconds = time.perf_counter() - start
+            assert seconds > 0.25 and ticks[0] - before > 20, (name, seconds, ticks[0] - before)
+    finally:
+        stop.set()
+        thread.join()
+
+
+def _bind(host, table):
+    from bitween_amd.kernels import hip_loader as hip
+    host.bind(table, hip._check, hip.FUSED_DGRAD_MAX_ROWS, hip.FUSED_DGRAD_LARGE_MAX_ROWS)
