@@ -42,7 +42,7 @@ struct Library {
 PyObject* g_check = nullptr;          // Python: check(status, entry point's name) raises for a status other than 0
 int64_t g_fused_rows = 0, g_fused_large_rows = 0;
 
-PyObject *s_buffers, *s_qweight, *s_scale, *s_zero, *s_bias, *s_bits, *s_group, *s_plan;
+PyObject *s_buffers, *s_qweight, *s_scale, *s_zero, *s_bias, *s_bits, *s_group;
 
 int dtype_code(at::ScalarType t) {
     switch (t) {
@@ -285,8 +285,6 @@ PyObject* py_forward(PyObject*, PyObject* const* args, Py_ssize_t nargs) {
             if (PyErr_Occurred()) return nullptr;
             return none();
         }
-        if (!PyDict_GetItemWithError(args[0], s_plan) && (PyErr_Occurred() || PyDict_SetItem(args[0], s_plan, Py_True)))
-            return nullptr;                                    // the mark says that the native path takes this layer
         int status = 0;
         const char* what = "";
         const bool recorded = c10::GradMode::is_enabled() && x.requires_grad();
@@ -476,6 +474,5 @@ PyMODINIT_FUNC PyInit__bw_host() {
     s_bias = PyUnicode_InternFromString("bias");
     s_bits = PyUnicode_InternFromString("bits");
     s_group = PyUnicode_InternFromString("group_size");
-    s_plan = PyUnicode_InternFromString("_decode_plan");
     return PyModule_Create(&module_def);
 }

@@ -102,11 +102,6 @@ class QuantizedLinear(nn.Module):
         y = _hip.quantized_matmul_hip(x2, self.qweight, self.scale, self.zero_point, self.bias, self.bits, self.group_size)
         return y.view(*shape[:-1], self.out_features)
 
-    def __getstate__(self):                                # the native path's mark belongs to this object's buffers
-        state = self.__dict__.copy()
-        state.pop("_decode_plan", None)
-        return state
-
     @classmethod
     def from_float(cls, float_layer: nn.Linear, bits=8, group_size=32):
         """RTN-quantise an nn.Linear.  The reference upcasts the layer to float32, quantises, and stores
