@@ -8,6 +8,7 @@ import weakref
 
 import torch
 import torch.nn as nn
+from torch.nn.modules import module as _nn_module
 
 from . import functional as _functional
 from .kernels import hip_loader as _hip
@@ -123,32 +124,41 @@ class QuantizedLinear(nn.Module):
         qweight, scale, zero_point = _hip.quantize_pack(weight, bits, group_size, math_dtype=torch.float32,
                                                         scale_dtype=torch.float16, zp_dtype=torch.float16,
                                                         scale_reciprocal=_functional.scale_reciprocal_for(float_layer.weight))
-        if qweight.shape[0] != float_layer.out_features or weight.shape[1] != float_layer.in_features:
-            raise BitweenShapeError(f"the layer declares {float_layer.out_features} x {float_layer.in_features}, its weight is {tuple(weight.shape)}")
+        n, k = float_layer.out_features, float_layer.in_features
+        if qweight.shape[0] != n or weight.shape[1] != k:
+            raise BitweenShapeError(f"the layer declares {n} x {k}, its weight is {tuple(weight.shape)}")
         buffers = {"qweight": qweight, "scale": scale, "zero_point": zero_point}
-        if float_layer.bias is not None:
-            buffers["bias"] = float_layer.bias.data.to(device="cuda", dtype=torch.float16, copy=True)
-        if device.type != "cuda":
-            buffers = {name: value.to(device) for name, value in buffers.items()}
-        if cls.__init__ is not QuantizedLinear.__init__:   # a subclass with a constructor of its own
-            with torch.device("meta"):                     # its zero buffers without memory; the kernel's outputs take their place
-                q_layer = cls(float_layer.in_features, float_layer.out_features, bits, group_size,
-                              bias=float_layer.bias is not None, dtype=torch.float16)
-        else:
+        bias = float_layer.bias
+        if bias is not None:
+            buffers["bias"] = bias.data.to(device="cuda", dtype=torch.float16, copy=True)
+            if bias.shape != (n,):
+                raise BitweenShapeError(f"the layer declares {n} outputs, its bias is {tuple(bias.shape)}")
+        if cls is QuantizedLinear and cls.__init__ is _constructor and not getattr(_nn_module, "_global_buffer_registration_hooks", True):
             # what the constructor does, without zero buffers to throw away and without nn.Module's attribute hooks
             # (30 us of a call whose kernel runs for 10 ... 25)
             q_layer = cls.__new__(cls)
             nn.Module.__init__(q_layer)
-            q_layer.__dict__.update(in_features=float_layer.in_features, out_features=float_layer.out_features, bits=bits,
-                                    group_size=group_size, requires_grad=False, dtype=torch.float16)
-            if float_layer.bias is None:
+            q_layer.__dict__.update(in_features=k, out_features=n, bits=bits, group_size=group_size, requires_grad=False, dtype=torch.float16)
+            if bias is None:
                 q_layer.__dict__["bias"] = None
+        else:                                              # a subclass, another constructor, or hooks that want to see the buffers come
+            with torch.device("meta"):                     # its zero buffers without memory; the kernel's outputs take their place
+                q_layer = cls(k, n, bits, group_size, bias=bias is not None, dtype=torch.float16)
+            for name, value in buffers.items():
+                if value.shape != q_layer._buffers[name].shape or value.dtype != q_layer._buffers[name].dtype:
+                    raise BitweenShapeError(f"{name}: kernel produced {tuple(value.shape)} {value.dtype}, the module declares "
+                                            f"{tuple(q_layer._buffers[name].shape)} {q_layer._buffers[name].dtype}")
+        if device.type != "cuda":
+            buffers = {name: value.to(device) for name, value in buffers.items()}
         q_layer._buffers.update(buffers)
         return q_layer
 
     def __repr__(self):
         return (f"QuantizedLinear(in_features={self.in_features}, out_features={self.out_features}, "
                 f"bias={self.bias is not None}, bits={self.bits}, group_size={self.group_size})")
+
+
+_constructor = QuantizedLinear.__init__
 
 
 class _SiblingGroup:

@@ -204,3 +204,41 @@ def test_other_threads_run_while_a_call_is_under_way(tmp_path):
 def _bind(host, table):
     from bitween_amd.kernels import hip_loader as hip
     host.bind(table, hip._check, hip.FUSED_DGRAD_MAX_ROWS, hip.FUSED_DGRAD_LARGE_MAX_ROWS)
+
+
+def test_from_float_runs_the_constructor_where_someone_looks_on(monkeypatch):
+    """Global buffer registration hooks are called for every buffer, a subclass's and a replaced constructor run; the layers are those of the
+    short way, and a bias that does not fit its layer is refused."""
+    from torch.nn.modules.module import register_module_buffer_registration_hook
+    import bitween_amd
+    from bitween_amd.modules import BitweenShapeError
+    lin = torch.nn.Linear(128, 64, device="cuda", dtype=torch.float16)
+    plain = bitween_amd.QuantizedLinear.from_float(lin, 4, 64)
+    seen = []
+    handle = register_module_buffer_registration_hook(lambda module, name, buffer: seen.append((type(module).__name__, name)))
+    try:
+        hooked = bitween_amd.QuantizedLinear.from_float(lin, 4, 64)
+    finally:
+        handle.remove()
+    assert seen == [("QuantizedLinear", n) for n in ("qweight", "scale", "zero_point", "bias")]
+
+    class Sub(bitween_amd.QuantizedLinear):
+        def __setattr__(self, name, value):
+            seen.append(name)
+            super().__setattr__(name, value)
+
+    sub = Sub.from_float(lin, 4, 64)
+    assert "in_features" in seen and "group_size" in seen
+    calls, init = [], bitween_amd.QuantizedLinear.__init__
+    monkeypatch.setattr(bitween_amd.QuantizedLinear, "__init__", lambda self, *a, **k: (calls.append(a), init(self, *a, **k))[1])
+    replaced = bitween_amd.QuantizedLinear.from_float(lin, 4, 64)
+    monkeypatch.undo()
+    assert len(calls) == 1
+    for layer in (hooked, sub, replaced):
+        assert set(layer.__dict__) == set(plain.__dict__) and repr(layer) == repr(plain)
+        for name, value in plain._buffers.items():
+            assert torch.equal(layer._buffers[name], value) and layer._buffers[name].device == value.device
+    bad = torch.nn.Linear(128, 64, device="cuda", dtype=torch.float16)
+    bad.bias = torch.nn.Parameter(torch.zeros(63, device="cuda", dtype=torch.float16))
+    with pytest.raises(BitweenShapeError):
+        bitween_amd.QuantizedLinear.from_float(bad, 4, 64)
