@@ -18,6 +18,7 @@
 #include <c10/hip/HIPStream.h>
 #include <torch/csrc/autograd/function.h>
 #include <torch/csrc/autograd/functions/utils.h>
+#include <torch/csrc/autograd/python_cpp_function.h>
 #include <torch/csrc/autograd/python_variable.h>
 #include <torch/csrc/autograd/saved_variable.h>
 #include <torch/csrc/autograd/variable.h>
@@ -210,23 +211,66 @@ Tensor input_grad(const Tensor& go, const Tensor& qweight, const Tensor& scale, 
     return at::matmul(go, wt == t ? w : w.to(t));
 }
 
+// The node of a recorded forward, in the likeness of QuantizedLinearFunction's: its name, what it saves (x too, so that a change of x in
+// place is noticed, and saved-tensor hooks see it) and the edges it has.
 struct QuantizedLinearBackward : public torch::autograd::Node {
-    torch::autograd::SavedVariable qweight, scale, zero;
+    enum { X, QWEIGHT, SCALE, ZERO, BIAS };
+    torch::autograd::SavedVariable saved[5];
+    bool has_bias = false;
     int bits = 0, group = 0;
-    std::string name() const override { return "QuantizedLinearBackward"; }
+    std::string name() const override { return "QuantizedLinearFunctionBackward"; }
     void release_variables() override {
         std::lock_guard<std::mutex> lock(mutex_);
-        qweight.reset_data();
-        scale.reset_data();
-        zero.reset_data();
+        for (auto& v : saved) v.reset_data();
+    }
+    std::array<Tensor, 5> unpack() const {
+        std::array<Tensor, 5> t;
+        for (int i = 0; i < (has_bias ? 5 : 4); i++) t[i] = saved[i].unpack();
+        return t;
     }
     torch::autograd::variable_list apply(torch::autograd::variable_list&& grads) override {
         std::lock_guard<std::mutex> lock(mutex_);
-        if (!grads[0].defined() || !task_should_compute_output(0)) return {Tensor()};
-        const Tensor q = qweight.unpack(), s = scale.unpack(), z = zero.unpack();
-        return {input_grad(grads[0], q.contiguous(), s.contiguous(), z.contiguous(), bits, group)};
+        const auto t = unpack();
+        torch::autograd::variable_list out(has_bias ? 5 : 4);
+        if (!task_should_compute_output(0)) return out;
+        const Tensor go = grads[0].defined() ? grads[0] : input_metadata(0).zeros_like();
+        out[0] = input_grad(go, t[QWEIGHT].contiguous(), t[SCALE].contiguous(), t[ZERO].contiguous(), bits, group);
+        return out;
     }
 };
+
+QuantizedLinearBackward* node_of(PyObject* self) {
+    return static_cast<QuantizedLinearBackward*>(reinterpret_cast<torch::autograd::THPCppFunction*>(self)->cdata.get());
+}
+
+PyObject* node_saved_tensors(PyObject* self, void*) {
+    HANDLE_TH_ERRORS
+    QuantizedLinearBackward* node = node_of(self);
+    const auto t = node->unpack();
+    PyObject* r = PyTuple_New(5);
+    if (!r) return nullptr;
+    for (int i = 0; i < 5; i++) PyTuple_SET_ITEM(r, i, THPVariable_Wrap(t[i]));   // (an undefined tensor is None)
+    return r;
+    END_HANDLE_TH_ERRORS
+}
+
+PyObject* node_needs_input_grad(PyObject* self, void*) {
+    QuantizedLinearBackward* node = node_of(self);
+    PyObject* r = PyTuple_New(7);
+    if (!r) return nullptr;
+    for (uint32_t i = 0; i < 7; i++)
+        PyTuple_SET_ITEM(r, i, PyBool_FromLong(i < node->num_outputs() && node->task_should_compute_output(i)));
+    return r;
+}
+
+using namespace torch::autograd;                              // (the names of the next macro)
+PyGetSetDef node_properties[] = {THP_FUNCTION_DEFAULT_PROPERTIES,
+                                 {"saved_tensors", node_saved_tensors, nullptr, nullptr, nullptr},
+                                 {"needs_input_grad", node_needs_input_grad, nullptr, nullptr, nullptr},
+                                 {"bits", [](PyObject* self, void*) { return PyLong_FromLong(node_of(self)->bits); }, nullptr, nullptr, nullptr},
+                                 {"group_size", [](PyObject* self, void*) { return PyLong_FromLong(node_of(self)->group); }, nullptr, nullptr, nullptr},
+                                 {nullptr, nullptr, nullptr, nullptr, nullptr}};
+PyTypeObject node_type = {PyVarObject_HEAD_INIT(nullptr, 0)};
 
 // ---- Python side ----
 
@@ -297,10 +341,11 @@ PyObject* py_forward(PyObject*, PyObject* const* args, Py_ssize_t nargs) {
         }
         if (recorded && status == 0 && y.defined()) {
             std::shared_ptr<QuantizedLinearBackward> node(new QuantizedLinearBackward(), torch::autograd::deleteNode);
-            node->set_next_edges(torch::autograd::collect_next_edges(x));
-            node->qweight = torch::autograd::SavedVariable(l.qweight, false);
-            node->scale = torch::autograd::SavedVariable(l.scale, false);
-            node->zero = torch::autograd::SavedVariable(l.zero, false);
+            const Tensor* inputs[5] = {&x, &l.qweight, &l.scale, &l.zero, &l.bias};
+            node->has_bias = l.bias.defined();
+            node->set_next_edges(node->has_bias ? torch::autograd::collect_next_edges(x, l.qweight, l.scale, l.zero, l.bias)
+                                                : torch::autograd::collect_next_edges(x, l.qweight, l.scale, l.zero));
+            for (int i = 0; i < (node->has_bias ? 5 : 4); i++) node->saved[i] = torch::autograd::SavedVariable(*inputs[i], false);
             node->bits = l.layer.bits;
             node->group = l.layer.group;
             torch::autograd::set_history(y, node);
@@ -474,5 +519,9 @@ PyMODINIT_FUNC PyInit__bw_host() {
     s_bias = PyUnicode_InternFromString("bias");
     s_bits = PyUnicode_InternFromString("bits");
     s_group = PyUnicode_InternFromString("group_size");
+    HANDLE_TH_ERRORS
+    torch::autograd::_initFunctionPyTypeObject(node_type, "QuantizedLinearFunctionBackward", node_properties, nullptr);
+    torch::autograd::registerCppFunction(typeid(QuantizedLinearBackward), &node_type);
     return PyModule_Create(&module_def);
+    END_HANDLE_TH_ERRORS
 }

@@ -242,3 +242,57 @@ def test_from_float_runs_the_constructor_where_someone_looks_on(monkeypatch):
     bad.bias = torch.nn.Parameter(torch.zeros(63, device="cuda", dtype=torch.float16))
     with pytest.raises(BitweenShapeError):
         bitween_amd.QuantizedLinear.from_float(bad, 4, 64)
+
+
+@pytest.mark.parametrize("bias", [True, False])
+def test_node_looks_like_that_of_the_autograd_function(bias):
+    """The node of q(x) against that of QuantizedLinearFunction.apply: name, saved tensors, edges, hooks; x changed in place is noticed, and
+    saved-tensor hooks see the same tensors."""
+    from bitween_amd import QuantizedLinearFunction
+    q = _layer(128, 64, 4, 64, bias=bias)
+    leaf = torch.randn(3, 128, device="cuda", dtype=torch.float16, requires_grad=True)
+
+    def make(module, x):
+        return q(x) if module else QuantizedLinearFunction.apply(x, q.qweight, q.scale, q.zero_point, q.bias, q.bits, q.group_size)
+
+    looks = []
+    for module in (True, False):
+        packed, x = [], leaf * 1
+        with torch.autograd.graph.saved_tensors_hooks(lambda t: (packed.append(tuple(t.shape)), t)[1], lambda t: t):
+            y = make(module, x)
+        node, fired = y.grad_fn, []
+        node.register_hook(lambda grad_in, grad_out: fired.append((len(grad_in), grad_in[0].shape, len(grad_out))))
+        saved = node.saved_tensors
+        assert saved[0].data_ptr() == x.data_ptr() and (saved[4] is None) == (not bias)
+        look = [node.name(), type(node).__name__, len(node.next_functions), node.next_functions[0][0].name(), node.bits, node.group_size,
+                packed, [None if t is None else (t.dtype, tuple(t.shape), t.requires_grad) for t in saved], node.needs_input_grad[0]]
+        y.sum().backward()
+        looks.append(look + [fired])
+        with pytest.raises(RuntimeError, match="second time"):
+            node.saved_tensors
+        x = leaf * 1
+        y = make(module, x)
+        x.mul_(2)
+        with pytest.raises(RuntimeError, match="modified by an inplace"):
+            y.sum().backward()
+    assert looks[0] == looks[1]
+
+
+def test_gradient_that_does_not_arrive_counts_as_zero():
+    from bitween_amd import QuantizedLinearFunction
+
+    class Nothing(torch.autograd.Function):
+        @staticmethod
+        def forward(ctx, y):
+            return y.clone()
+
+        @staticmethod
+        def backward(ctx, grad):
+            return None
+
+    q = _layer(128, 64, 4, 64)
+    for module in (True, False):
+        x = torch.randn(3, 128, device="cuda", dtype=torch.float16, requires_grad=True)
+        y = q(x) if module else QuantizedLinearFunction.apply(x, q.qweight, q.scale, q.zero_point, q.bias, q.bits, q.group_size)
+        Nothing.apply(y).sum().backward()
+        assert x.grad is not None and not x.grad.any()
