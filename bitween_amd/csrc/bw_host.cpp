@@ -41,8 +41,9 @@ struct Library {
 } lib;
 
 PyObject* g_check = nullptr;          // Python: check(status, entry point's name) raises for a status other than 0
-int64_t g_fused_rows = 0, g_fused_large_rows = 0;
+PyObject* g_limits = nullptr;         // Python: the dict with the row limits of the fused input gradient
 
+PyObject *s_fused_rows, *s_fused_large_rows;
 PyObject *s_buffers, *s_qweight, *s_scale, *s_zero, *s_bias, *s_bits, *s_group;
 
 int dtype_code(at::ScalarType t) {
@@ -89,6 +90,23 @@ struct Unlocked {
     Unlocked() = default;
     Unlocked(const Unlocked&) = delete;
     ~Unlocked() { PyEval_RestoreThread(state); }
+};
+
+// The row limits as they are now (0 = not a number: no row runs fused); takes the interpreter lock where the thread does not hold it.
+struct FusedRows {
+    int64_t always = 0, large = 0;
+    FusedRows() {
+        const PyGILState_STATE state = PyGILState_Ensure();
+        always = read(s_fused_rows);
+        large = read(s_fused_large_rows);
+        PyGILState_Release(state);
+    }
+    static int64_t read(PyObject* name) {
+        PyObject* v = g_limits ? PyDict_GetItemWithError(g_limits, name) : nullptr;
+        const long long rows = v && PyLong_Check(v) ? PyLong_AsLongLong(v) : 0;
+        if (PyErr_Occurred()) PyErr_Clear();
+        return rows < 0 ? 0 : rows;
+    }
 };
 
 struct Layer {
@@ -168,10 +186,10 @@ Tensor linear(const Layer& l, Tensor x, int& status, const char*& what) {
 }
 
 // grad_x = grad_y @ W, W the dequantised weight in grad_y's dtype (bitween/modules.py:108-141).  float16 / bfloat16
-// gradients run the fused kernel - up to g_fused_rows rows always, up to g_fused_large_rows where the library plans its
+// gradients run the fused kernel - up to `fused.always` rows always, up to `fused.large` where the library plans its
 // 256 x 256 kernel - and dequantise + library GEMM beyond, which is faster there; so does a backward that is itself
 // recorded (create_graph).
-Tensor input_grad(const Tensor& go, const Tensor& qweight, const Tensor& scale, const Tensor& zero, int bits, int group) {
+Tensor input_grad(const Tensor& go, const Tensor& qweight, const Tensor& scale, const Tensor& zero, int bits, int group, const FusedRows& fused) {
     const int64_t n = qweight.size(0), k = qweight.size(1) * (32 / bits);
     OnDevice on(go.device());
     void* stream = stream_of(go.device().index());
@@ -179,7 +197,7 @@ Tensor input_grad(const Tensor& go, const Tensor& qweight, const Tensor& scale, 
     const int64_t m = go.numel() / n;
     const bool recorded = c10::GradMode::is_enabled() && go.requires_grad();
     if ((t == at::kHalf || t == at::kBFloat16) && !recorded && m > 0 &&
-        (m <= g_fused_rows || (m <= g_fused_large_rows && lib.qdgrad_tile_rows(m, n, k, bits, group) == 257))) {
+        (m <= fused.always || (m <= fused.large && lib.qdgrad_tile_rows(m, n, k, bits, group) == 257))) {
         Tensor g = go;
         int64_t ldg = n;
         if (!g.is_contiguous()) {
@@ -229,12 +247,13 @@ struct QuantizedLinearBackward : public torch::autograd::Node {
         return t;
     }
     torch::autograd::variable_list apply(torch::autograd::variable_list&& grads) override {
+        const FusedRows fused;
         std::lock_guard<std::mutex> lock(mutex_);
         const auto t = unpack();
         torch::autograd::variable_list out(has_bias ? 5 : 4);
         if (!task_should_compute_output(0)) return out;
         const Tensor go = grads[0].defined() ? grads[0] : input_metadata(0).zeros_like();
-        out[0] = input_grad(go, t[QWEIGHT].contiguous(), t[SCALE].contiguous(), t[ZERO].contiguous(), bits, group);
+        out[0] = input_grad(go, t[QWEIGHT].contiguous(), t[SCALE].contiguous(), t[ZERO].contiguous(), bits, group, fused);
         return out;
     }
 };
@@ -388,10 +407,11 @@ PyObject* py_input_grad(PyObject*, PyObject* const* args, Py_ssize_t nargs) {
         if (!go.is_cuda() || !go.has_storage() || !layer_of(qweight, scale, zero, nullptr, PyLong_AsLong(args[4]), PyLong_AsLong(args[5]), l))
             return none();
         if (go.dim() < 1 || go.size(-1) != l.n || !go.is_floating_point() || go.device().index() != l.device) return none();
+        const FusedRows fused;
         Tensor gx;
         {
             Unlocked unlocked;
-            gx = input_grad(go, qweight, scale, zero, l.bits, l.group);
+            gx = input_grad(go, qweight, scale, zero, l.bits, l.group, fused);
         }
         return THPVariable_Wrap(std::move(gx));
     });
@@ -464,11 +484,10 @@ PyObject* py_dequantize(PyObject*, PyObject* const* args, Py_ssize_t nargs) {
     });
 }
 
-// bind({entry point name: address}, check, fused rows, fused rows of the large kernel): once, after the kernel library is loaded
+// bind({entry point name: address}, check, dict with the fused gradient's row limits): once, after the kernel library is loaded
 PyObject* py_bind(PyObject*, PyObject* args) {
-    PyObject *table, *check;
-    long long rows, large;
-    if (!PyArg_ParseTuple(args, "O!OLL", &PyDict_Type, &table, &check, &rows, &large)) return nullptr;
+    PyObject *table, *check, *limits;
+    if (!PyArg_ParseTuple(args, "O!OO!", &PyDict_Type, &table, &check, &PyDict_Type, &limits)) return nullptr;
     bool ok = true;
     auto get = [&](auto& fn, const char* name) {
         PyObject* v = PyDict_GetItemString(table, name);
@@ -493,8 +512,8 @@ PyObject* py_bind(PyObject*, PyObject* args) {
     lib = l;
     Py_INCREF(check);
     Py_XSETREF(g_check, check);
-    g_fused_rows = rows;
-    g_fused_large_rows = large;
+    Py_INCREF(limits);
+    Py_XSETREF(g_limits, limits);
     Py_RETURN_NONE;
 }
 
@@ -512,6 +531,8 @@ PyModuleDef module_def = {PyModuleDef_HEAD_INIT, "_bw_host", "Native host path o
 }  // namespace
 
 PyMODINIT_FUNC PyInit__bw_host() {
+    s_fused_rows = PyUnicode_InternFromString("FUSED_DGRAD_MAX_ROWS");
+    s_fused_large_rows = PyUnicode_InternFromString("FUSED_DGRAD_LARGE_MAX_ROWS");
     s_buffers = PyUnicode_InternFromString("_buffers");
     s_qweight = PyUnicode_InternFromString("qweight");
     s_scale = PyUnicode_InternFromString("scale");

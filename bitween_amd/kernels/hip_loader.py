@@ -90,10 +90,6 @@ def load():
 _HOST_PATH = os.path.join(os.path.dirname(os.path.dirname(os.path.abspath(__file__))), "csrc", "_bw_host.so")
 _host = None
 
-FUSED_DGRAD_MAX_ROWS = 512       # measured on MI355X, Llama-shaped layers: the 128-row fused kernel wins up to here (3x at 128 rows)
-FUSED_DGRAD_LARGE_MAX_ROWS = 2048  # ... and the 256 x 256 kernel, where the library plans it (large layers), up to here
-
-
 def host():
     """The native host path (csrc/bw_host.cpp) bound to the kernel library; both are loaded once."""
     global _host
@@ -105,7 +101,8 @@ def host():
         module = importlib.util.module_from_spec(spec)
         spec.loader.exec_module(module)
         table = {name: ctypes.cast(getattr(lib, name), ctypes.c_void_p).value for name in ENTRY_POINTS}
-        module.bind(table, _check, FUSED_DGRAD_MAX_ROWS, FUSED_DGRAD_LARGE_MAX_ROWS)
+        from .. import modules
+        module.bind(table, _check, vars(modules))          # (the row limits of the fused input gradient live there)
         _host = module
     return _host
 
@@ -265,7 +262,7 @@ def _matmul(entry, x, qweight, scale, zero_point, bias, bits, group_size):
 
 def input_grad(grad_output, qweight, scale, zero_point, bits, group_size):
     """grad_output [..., N] @ W -> [..., K] in grad_output's dtype: the fused kernel (bw_qdgrad) for float16 / bfloat16 gradients of
-    up to FUSED_DGRAD_MAX_ROWS rows, and of up to FUSED_DGRAD_LARGE_MAX_ROWS where the library plans its 256 x 256 kernel;
+    up to modules.FUSED_DGRAD_MAX_ROWS rows, and of up to modules.FUSED_DGRAD_LARGE_MAX_ROWS where the library plans its 256 x 256 kernel;
     dequantise + library GEMM otherwise.  None for buffers that are not the contiguous ones a QuantizedLinear keeps."""
     return host().input_grad(grad_output, qweight, scale, zero_point, bits, group_size)
 

@@ -14,6 +14,11 @@ from . import functional as _functional
 from .kernels import hip_loader as _hip
 
 
+# Rows of a gradient up to which backward runs the fused kernel, looked at by every backward.
+FUSED_DGRAD_MAX_ROWS = 512       # measured on MI355X, Llama-shaped layers: the 128-row fused kernel wins up to here (3x at 128 rows)
+FUSED_DGRAD_LARGE_MAX_ROWS = 2048  # ... and the 256 x 256 kernel, where the library plans it (large layers), up to here
+
+
 def _host_forward(fields, x):
     """First call: loads the native host path and puts its forward(module.__dict__, x) in this function's place."""
     global _host_forward

@@ -202,8 +202,9 @@ def test_other_threads_run_while_a_call_is_under_way(tmp_path):
 
 
 def _bind(host, table):
+    from bitween_amd import modules
     from bitween_amd.kernels import hip_loader as hip
-    host.bind(table, hip._check, hip.FUSED_DGRAD_MAX_ROWS, hip.FUSED_DGRAD_LARGE_MAX_ROWS)
+    host.bind(table, hip._check, vars(modules))
 
 
 def test_from_float_runs_the_constructor_where_someone_looks_on(monkeypatch):
@@ -296,3 +297,26 @@ def test_gradient_that_does_not_arrive_counts_as_zero():
         y = q(x) if module else QuantizedLinearFunction.apply(x, q.qweight, q.scale, q.zero_point, q.bias, q.bits, q.group_size)
         Nothing.apply(y).sum().backward()
         assert x.grad is not None and not x.grad.any()
+
+
+def test_row_limits_of_the_fused_gradient_are_looked_at_by_every_backward(monkeypatch):
+    """modules.FUSED_DGRAD_MAX_ROWS and _LARGE_MAX_ROWS, changed between forward and backward, decide which way the gradient takes: the
+    dequantised weight has to be in memory on one way only."""
+    from bitween_amd import QuantizedLinearFunction, modules
+    q = _layer(4096, 4096, 4, 64)
+    go = torch.randn(8, 4096, device="cuda", dtype=torch.float16)
+
+    def memory(module):
+        x = torch.randn(8, 4096, device="cuda", dtype=torch.float16, requires_grad=True)
+        y = q(x) if module else QuantizedLinearFunction.apply(x, q.qweight, q.scale, q.zero_point, q.bias, q.bits, q.group_size)
+        monkeypatch.setattr(modules, "FUSED_DGRAD_MAX_ROWS", rows)
+        monkeypatch.setattr(modules, "FUSED_DGRAD_LARGE_MAX_ROWS", rows)
+        torch.cuda.synchronize()
+        torch.cuda.reset_peak_memory_stats()
+        before = torch.cuda.memory_allocated()
+        y.backward(go)
+        return torch.cuda.max_memory_allocated() - before
+
+    for module in (True, False):
+        for rows, unfused in ((512, False), (7, True), (8, False), (0, True), (512, False)):
+            assert (memory(module) >= 2 * 4096 * 4096) == unfused, (module, rows)
