@@ -184,14 +184,16 @@ __global__ __launch_bounds__(DTHREADS, MT == 4 ? 3 : 2) void qdgrad_kernel(const
         *reinterpret_cast<u4*>(Bs + b_dst) = u4{wd[0], wd[1], wd[2], wd[3]};
         *reinterpret_cast<u4*>(Bs + b_dst + 16) = u4{wd[4], wd[5], wd[6], wd[7]};
         // ... and their columns of grad_y of zero as well: an infinity there times a weight of zero would turn its sum into NaN
-        const int dup = step < s_end ? step * DN - min(step * DN, a.N - DN) : DN;
-        if (dup > 0) {                                                // (uniform)
+        if constexpr (MT == 4) {
+            const int dup = step < s_end ? step * DN - min(step * DN, a.N - DN) : DN;
+            if (dup > 0) {                                            // (uniform)
 #pragma unroll
-            for (int e = 0; e < 4; e++) {
-                const int n = gpart * 8 + 2 * e;
-                const uint32_t keep = (n < dup ? 0u : 0xFFFFu) | (n + 1 < dup ? 0u : 0xFFFF0000u);
+                for (int e = 0; e < 4; e++) {
+                    const int n = gpart * 8 + 2 * e;
+                    const uint32_t keep = (n < dup ? 0u : 0xFFFFu) | (n + 1 < dup ? 0u : 0xFFFF0000u);
 #pragma unroll
-                for (int r = 0; r < GR; r++) greg[slot][r][e] &= keep;
+                    for (int r = 0; r < GR; r++) greg[slot][r][e] &= keep;
+                }
             }
         }
 #pragma unroll
@@ -216,6 +218,19 @@ __global__ __launch_bounds__(DTHREADS, MT == 4 ? 3 : 2) void qdgrad_kernel(const
             const int step = base + d;
             const char* As = smem + (d & 1) * STAGE;                  // PD is even: stages alternate across passes too
             const char* Bs = As + A_BYTES;
+            // The same for the 256-row tile, whose registers do not hold the masks (20 ... 48 bytes a lane were spilled; 756 rows of N = 1216,
+            // K = 1024 at 8 bits 20.2 us, 19.3 without): here, where few are in use, over what lies in LDS, a row to a thread.
+            if constexpr (MT == 8) {
+                const int dup = step < s_end ? step * DN - min(step * DN, a.N - DN) : DN;
+                if (dup > 0) {                                            // (uniform)
+                    char* row = smem + (d & 1) * STAGE + tid * DPITCH;
+                    if (tid < DM) {
+                        for (int n = 0; n < dup / 2; n++) *reinterpret_cast<uint32_t*>(row + 4 * n) = 0;
+                        if (dup & 1) *reinterpret_cast<short*>(row + 2 * (dup - 1)) = 0;
+                    }
+                    __syncthreads();
+                }
+            }
             h8 af[4], bf[MT];
 #pragma unroll
             for (int i = 0; i < 4; i++) {
@@ -243,20 +258,18 @@ __global__ __launch_bounds__(DTHREADS, MT == 4 ? 3 : 2) void qdgrad_kernel(const
 
     // acc[i][j][r] = grad_x[m0 + wm + 16 j + l16][k0 + wk + 16 i + 4 q + r]
     if (a.splits > 1) {
-        float* dst = a.ws + (size_t)blockIdx.x * (DM * DK);
-        if (m0 + DM <= a.M) {
+        // Rows past M lie beyond the descriptor and are dropped by its range check (16 rows of a 128-row tile: an eighth of the traffic).
+        // Masked by hand the stores were there twice, for every launch to fetch: 97 rows of N = 1024, K = 10624 at 4 bits 22.6 us, 21.0 this way,
+        // 756 of N = 1216, K = 1024 at 8 bits 19.3 and 18.5.  The i loop outside: neighbouring stores to the two halves of a line take 1 us
+        // longer.
+        const __amdgpu_buffer_rsrc_t rd = __builtin_amdgcn_make_buffer_rsrc(a.ws + (size_t)blockIdx.x * (DM * DK), (short)0, min(a.M - m0, DM) * (DK * 4), 0x00020000);
+        const uint32_t off = ((wm + l16) * DK + wk + 4 * q) * 4;
+        const int rows = __builtin_amdgcn_readfirstlane(a.M - m0 - wm);   // of this wave; pieces of 16 without any are not asked for
 #pragma unroll
-            for (int i = 0; i < 4; i++)
+        for (int i = 0; i < 4; i++)
 #pragma unroll
-                for (int j = 0; j < MT; j++) *reinterpret_cast<f4*>(dst + (wm + 16 * j + l16) * DK + wk + 16 * i + 4 * q) = acc[i][j];
-            return;
-        }
-#pragma unroll
-        for (int j = 0; j < MT; j++) {
-            if (m0 + wm + 16 * j + l16 >= a.M) continue;              // rows past M: 16 rows of a 128-row tile are an eighth of the traffic
-#pragma unroll
-            for (int i = 0; i < 4; i++) *reinterpret_cast<f4*>(dst + (wm + 16 * j + l16) * DK + wk + 16 * i + 4 * q) = acc[i][j];
-        }
+            for (int j = 0; j < MT; j++)
+                if (16 * j < rows) __builtin_amdgcn_raw_buffer_store_b128(__builtin_bit_cast(u4, acc[i][j]), rd, off + j * (16 * DK * 4) + i * 64, 0, 0);
     } else {
 #pragma unroll
         for (int j = 0; j < MT; j++) {
