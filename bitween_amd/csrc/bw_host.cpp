@@ -382,8 +382,10 @@ PyObject* py_matmul(PyObject*, PyObject* const* args, Py_ssize_t nargs) {
         const Tensor x = unpack(args[0]);
         if (!x.has_storage() || (x.scalar_type() != at::kHalf && x.scalar_type() != at::kBFloat16)) return none();
         const Tensor qweight = unpack(args[1]), scale = unpack(args[2]), zero = unpack(args[3]), bias = args[4] == Py_None ? Tensor() : unpack(args[4]);
+        const int64_t bits = PyLong_AsLong(args[5]), group = PyLong_AsLong(args[6]);
+        if (PyErr_Occurred()) return nullptr;
         Layer l;
-        if (!layer_of(qweight, scale, zero, bias.defined() ? &bias : nullptr, PyLong_AsLong(args[5]), PyLong_AsLong(args[6]), l)) return none();
+        if (!layer_of(qweight, scale, zero, bias.defined() ? &bias : nullptr, bits, group, l)) return none();
         int status = 0;
         const char* what = "";
         Tensor y;
@@ -403,9 +405,10 @@ PyObject* py_input_grad(PyObject*, PyObject* const* args, Py_ssize_t nargs) {
         for (int i = 0; i < 4; i++)
             if (!plain(args[i])) return none();
         const Tensor go = unpack(args[0]), qweight = unpack(args[1]), scale = unpack(args[2]), zero = unpack(args[3]);
+        const int64_t bits = PyLong_AsLong(args[4]), group = PyLong_AsLong(args[5]);
+        if (PyErr_Occurred()) return nullptr;
         Layer l;
-        if (!go.is_cuda() || !go.has_storage() || !layer_of(qweight, scale, zero, nullptr, PyLong_AsLong(args[4]), PyLong_AsLong(args[5]), l))
-            return none();
+        if (!go.is_cuda() || !go.has_storage() || !layer_of(qweight, scale, zero, nullptr, bits, group, l)) return none();
         if (go.dim() < 1 || go.size(-1) != l.n || !go.is_floating_point() || go.device().index() != l.device) return none();
         const FusedRows fused;
         Tensor gx;

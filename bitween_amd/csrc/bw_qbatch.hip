@@ -91,7 +91,7 @@ BatchCost batch_search(int64_t M, int64_t N, int64_t K, int bits, int group, boo
     return best;
 }
 
-// 17 ... 64 rows: this kernel; on 1337 layers, formats and row counts there it takes 0.35 ... 0.94 of the time of the prefill kernel and of
+// 17 ... 64 rows: this kernel; on 1493 layers, formats and row counts there it takes 0.15 ... 0.94 of the time of the prefill kernel and of
 // the decode kernels in launches of 16 rows (W4 g128 at 64 rows, us, prefill kernel against this one: 4096 x 4096 17.8 -> 8.8, 4096 ->
 // 11008 20.9 -> 17.2, 11008 -> 4096 24.8 -> 18.9; 2048 x 2048 13.3 -> 5.3).  Beyond, whichever is expected to be done first: the prefill
 // kernel's 128 x 256 tiles leave the chip idle on most layers of a few hundred rows, or have to be cut along K (W4 g128, us, prefill

@@ -223,3 +223,16 @@ def test_a_library_built_before_an_entry_point_was_added_is_refused_by_name(tmp_
                          cwd=os.path.dirname(os.path.dirname(os.path.abspath(__file__))))
     assert out.returncode == 0, out.stderr
     assert "bw_qlinear_ws, bw_qlinear_workspace_bytes" in out.stdout and "rebuild" in out.stdout
+
+
+def test_sizes_beyond_64_bits_are_an_overflow_error():
+    from bitween_amd.kernels import hip_loader
+    host = hip_loader.host()
+    x, q, s = torch.zeros(2, 64, dtype=torch.float16), torch.zeros(8, 8, dtype=torch.int32), torch.zeros(8, 1, dtype=torch.float16)
+    for bits, group in ((2 ** 70, 64), (4, 2 ** 70)):
+        with pytest.raises(OverflowError):
+            host.matmul(x, q, s, s, None, bits, group)
+        with pytest.raises(OverflowError):
+            host.input_grad(x, q, s, s, bits, group)
+        with pytest.raises(OverflowError):
+            host.dequantize(q, s, s, group, bits, hip_loader.BW_F16)
