@@ -132,7 +132,8 @@ int bw_qgemm(const void* x, int act_dtype, int64_t M, int64_t K, int64_t ldx,
 size_t bw_qgemm_workspace_bytes(int64_t M, int64_t N, int64_t K, int bits, int group);
 
 /* Rows of the output tile the prefill kernel runs this shape with (x rows K apart, any workspace it asks for granted):
- * 128, or 256 once a grid of 256-row tiles fills most of the device; 0 = the shape-generic kernel.
+ * 64 (up to 64 rows, and up to 128 where N is at most 16 tiles of 256 wide), 128, or 256 once a grid of 256-row tiles fills most of the
+ * device; 0 = the shape-generic kernel.
  * A diagnostic for benchmarks and tests; no counterpart in the reference. */
 int bw_qgemm_tile_rows(int64_t M, int64_t N, int64_t K, int bits, int group);
 
@@ -158,8 +159,8 @@ int bw_qgemm_static(const void* x, int act_dtype, int64_t M, int64_t K, int64_t 
 int bw_qlinear_decode_rows(int64_t N, int64_t K, int bits);
 
 /* bw_qlinear with a workspace: what the Python forward calls for any number of rows.  Adds to it the batch kernel with K cut
- * across workgroups, the split-K plans of the prefill kernel, and BW_BF16 x for every M (cast into the workspace where the
- * prefill kernel runs).  `workspace` (16-byte aligned) holds at least bw_qlinear_workspace_bytes(...) bytes (0 = none needed);
+ * across workgroups (also beyond bw_qlinear_decode_rows: up to 2048 rows while it is expected to be done before the prefill kernel), the
+ * split-K plans of the prefill kernel, and BW_BF16 x for every M (cast into the workspace where the prefill kernel runs).  `workspace` (16-byte aligned) holds at least bw_qlinear_workspace_bytes(...) bytes (0 = none needed);
  * with less, plans that need it are not used, and BW_BF16 x that has to be cast returns BW_EWORKSPACE. */
 size_t bw_qlinear_workspace_bytes(int64_t M, int64_t N, int64_t K, int bits, int group, int act_dtype);
 

@@ -92,8 +92,9 @@ def test_split_k_workspace_size_is_a_pure_host_function():
 
 
 def test_decode_rows_switch_is_a_pure_host_function():
-    """bw_qlinear keeps up to 48 rows on the decode kernel for layers under 10 MiB of packed weights, 32 under 40 MiB
-    (a third 16-row launch loses to one launch of the prefill kernel's 64-row tiles) and 16 from 40 MiB on."""
+    """Without a workspace bw_qlinear stays off the prefill kernel (batch kernel or decode launches of 16 rows) up to 48 rows for layers
+    under 10 MiB of packed weights, 32 under 40 MiB (a third 16-row launch loses to one launch of the prefill kernel's 64-row tiles)
+    and 16 from 40 MiB on."""
     from bitween_amd.kernels import hip_loader
     rows = hip_loader.load().bw_qlinear_decode_rows
     assert rows(4096, 4096, 4) == 48 and rows(4096, 4096, 8) == 32 and rows(4096, 11008, 2) == 32

@@ -100,7 +100,8 @@ def test_decode_rows_on_large_layers(bits, g, k, n, m):
 
 @pytest.mark.parametrize("m", [7, 17, 70])
 def test_layouts_the_batch_kernel_does_not_take(m):
-    """Scales off a 4-byte boundary, with bfloat16 x too; no x and an unknown type of x are refused."""
+    """Rows of x off a 16-byte boundary go to the generic kernel; scales off a 4-byte boundary do not, with bfloat16 x too; no x and an
+    unknown type of x are refused."""
     from bitween_amd.kernels import hip_loader
     lib = hip_loader.load()
     bits, g, k, n = 4, 128, 1280, 260
@@ -114,6 +115,11 @@ def test_layouts_the_batch_kernel_does_not_take(m):
     assert st == 0
     check_matmul(y, x.cpu().numpy(), qw, s16, z16, None, bits, g)
     from bitween_amd.kernels import hip_loader as hip
+    shifted = torch.empty(m, k + 8, device="cuda", dtype=torch.float16)[:, 1:k + 1]
+    shifted.copy_(x)
+    st, y, _ = _call(lib, shifted, d, n, bits, g, n)
+    assert st == 0 and hip.last_decode_kernel() == ""
+    check_matmul(y, x.cpu().numpy(), qw, s16, z16, None, bits, g)
     xb = x.to(torch.bfloat16)
     yb = hip.quantized_matmul_hip(xb, d[0], s_odd, d[2], to_gpu(b16), bits, g)
     check_matmul(yb, xb.to(torch.float16).cpu().numpy(), qw, s16, z16, b16, bits, g)

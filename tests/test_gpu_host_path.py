@@ -26,7 +26,7 @@ def _close(y, x16, q):
 
 
 @pytest.mark.parametrize("dtype", [torch.float16, torch.bfloat16, torch.float32])
-@pytest.mark.parametrize("rows", [1, 16, 17, 49, 130])         # one decode launch, two, and the prefill kernel
+@pytest.mark.parametrize("rows", [1, 16, 17, 49, 130])         # the decode kernels, the batch kernel
 def test_layouts_of_x(dtype, rows):
     q = _layer(256, 97, 4, 64)
     base = torch.randn(rows, 3, 2 * 256 + 8, device="cuda").to(dtype)

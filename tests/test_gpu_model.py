@@ -66,7 +66,7 @@ def test_llama_quantize_forward_generate_save(fuse):
 
     twin = _oracle_twin(qmodel)
     gen = torch.Generator(device="cuda").manual_seed(5)
-    for shape in ((1, 1), (1, 7), (2, 33), (1, 130)):          # decode kernel, its 16-row slices, prefill kernel
+    for shape in ((1, 1), (1, 7), (2, 33), (1, 130)):          # decode kernels (1, 7), the others beyond 16 rows
         ids = torch.randint(0, 512, shape, device="cuda", generator=gen)
         with torch.no_grad():
             got = qmodel(input_ids=ids).logits.float()

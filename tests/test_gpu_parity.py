@@ -604,8 +604,8 @@ def test_full_size_properties(bits, g, k, n):
 @pytest.mark.parametrize("bits,g", COMBOS)
 def test_bfloat16_activations_are_rounded_to_float16_in_the_kernel(bits, g):
     """x.to(float16) of the reference's forward (bitween/modules.py:74) fused into the decode kernels: a bfloat16 x
-    gives bit for bit what its float16 rounding gives, for every decode kernel variant, through bw_qlinear's 16-row
-    slices and (cast on the host side) through the prefill kernel; tiny and huge values included."""
+    gives bit for bit what its float16 rounding gives, for every decode kernel variant and for the batch kernel; tiny
+    and huge values included."""
     hip = _hip()
     k, n = 1024, 272
     _, qw, s16, z16, b16 = quantized_layer(n, k, bits, g, seed=bits * 31 + g, outliers=True)
@@ -780,9 +780,9 @@ def test_forward_under_graph_capture_replays_like_eager(m, dtype):
 @pytest.mark.parametrize("dtype", [torch.float16, torch.bfloat16])
 @pytest.mark.parametrize("bits,switch,ms", [(4, 32, (32, 33, 40, 48)), (8, 16, (16, 17, 32, 33))])
 def test_rows_33_to_48_on_a_large_layer_take_the_prefill_kernel(dtype, bits, switch, ms):
-    """For a layer of 10 MiB of packed weights and more bw_qlinear hands 33-48 rows to the prefill kernel, from 40 MiB on
-    (4096 -> 11008 at 8 bits) 17-32 rows too; the module forward (validated-buffer path, bfloat16 cast included) must
-    follow it and agree with the C entry point."""
+    """For a layer of 10 MiB of packed weights and more bw_qlinear, which has no workspace, hands 33-48 rows to the prefill kernel, from
+    40 MiB on (4096 -> 11008 at 8 bits) 17-32 rows too; the module forward, which has one, runs the batch kernel there.  Both against the
+    dequantised weights in 64 bits, and bit for bit the same where they run the same kernel."""
     import ctypes
     from bitween_amd import QuantizedLinear
     from bitween_amd.kernels import hip_loader as hip
@@ -806,7 +806,7 @@ def test_rows_33_to_48_on_a_large_layer_take_the_prefill_kernel(dtype, bits, swi
         assert st == 0
         torch.cuda.synchronize()
         if m <= switch:
-            assert torch.equal(y, yc)                            # same decode launches either way
+            assert torch.equal(y, yc)                            # the same launch either way
         else:
             assert ((y.double() - yc.double()).abs() <= 2.0 ** -9 * ref.abs() + 2.0 ** -12 * mag).all()   # split-K or not
 
