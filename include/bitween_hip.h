@@ -159,9 +159,10 @@ int bw_qgemm_static(const void* x, int act_dtype, int64_t M, int64_t K, int64_t 
 int bw_qlinear_decode_rows(int64_t N, int64_t K, int bits);
 
 /* bw_qlinear with a workspace: what the Python forward calls for any number of rows.  Adds to it the batch kernel with K cut
- * across workgroups (also beyond bw_qlinear_decode_rows: up to 2048 rows while it is expected to be done before the prefill kernel), the
- * split-K plans of the prefill kernel, and BW_BF16 x for every M (cast into the workspace where the prefill kernel runs).  `workspace` (16-byte aligned) holds at least bw_qlinear_workspace_bytes(...) bytes (0 = none needed);
- * with less, plans that need it are not used, and BW_BF16 x that has to be cast returns BW_EWORKSPACE. */
+ * across workgroups and beyond bw_qlinear_decode_rows (up to 2048 rows while it is expected to be done before the prefill kernel),
+ * the split-K plans of the prefill kernel, and BW_BF16 x for every M (cast into the workspace where the prefill kernel runs).
+ * `workspace` (16-byte aligned) holds at least bw_qlinear_workspace_bytes(...) bytes (0 = none needed); with less, plans that
+ * need it are not used, and BW_BF16 x that has to be cast returns BW_EWORKSPACE. */
 size_t bw_qlinear_workspace_bytes(int64_t M, int64_t N, int64_t K, int bits, int group, int act_dtype);
 
 int bw_qlinear_ws(const void* x, int act_dtype, int64_t M, int64_t K, int64_t ldx,
