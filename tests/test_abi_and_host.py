@@ -237,3 +237,33 @@ def test_sizes_beyond_64_bits_are_an_overflow_error():
             host.input_grad(x, q, s, s, bits, group)
         with pytest.raises(OverflowError):
             host.dequantize(q, s, s, group, bits, hip_loader.BW_F16)
+
+
+def _kernel_metadata(path):
+    """The AMDGPU metadata notes of every gfx950 code object in the library: one dict per kernel."""
+    import struct
+    msgpack = pytest.importorskip("msgpack")
+    data = open(path, "rb").read()
+    at = data.find(b"\x7fELF", 4)
+    while at >= 0:
+        if struct.unpack_from("<H", data, at + 18)[0] == 224:                        # EM_AMDGPU
+            headers, = struct.unpack_from("<Q", data, at + 32)
+            size, count = struct.unpack_from("<HH", data, at + 54)
+            for i in range(count):
+                kind, _, offset, _, _, length = struct.unpack_from("<IIQQQQ", data, at + headers + i * size)
+                p = at + offset
+                while kind == 4 and p < at + offset + length:                        # PT_NOTE
+                    name, desc, note = struct.unpack_from("<III", data, p)
+                    body = p + 12 + (name + 3) // 4 * 4
+                    if note == 32 and data[p + 12:p + 18] == b"AMDGPU":              # NT_AMDGPU_METADATA
+                        yield from msgpack.unpackb(data[body:body + desc])["amdhsa.kernels"]
+                    p = body + (desc + 3) // 4 * 4
+        at = data.find(b"\x7fELF", at + 4)
+
+
+def test_stepping_input_gradient_kernel_spills_no_registers():
+    """A few spilled bytes cost a launch of the input gradient 1 ... 2 us: its 256-row tile uses nearly all registers."""
+    from bitween_amd.kernels import hip_loader
+    kernels = [k for k in _kernel_metadata(hip_loader.library_path()) if "qdgrad_kernel" in k[".name"]]
+    assert len(kernels) == 36                                                        # formats x tile heights x gradient types
+    assert not [k[".name"] for k in kernels if k[".vgpr_spill_count"] or k[".private_segment_fixed_size"]]
