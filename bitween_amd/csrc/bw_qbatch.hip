@@ -45,15 +45,16 @@ struct BatchPlan { int mt, ntw, splits; };
 
 inline int batch_mt(int64_t M) { const int t = (int)((M + 15) / 16); return t <= 4 ? t : t <= 6 ? 6 : 8; }
 
-// Rows of 16 per tile, column tiles per wave and cuts of K for a call, from a model of the launch fitted to 4000 timings (17 ...
-// 1600 rows, 23 shapes, 2 / 4 / 8 bits, both activation types; rms error 6 %, its choice within 1 % of the best on average).
-// A round costs 0.17 MT + (0.33 + 0.024 MT + 0.19 at 8 bits) NTW us, of 256 values (MT > 4) 0.10 MT + (0.22 + (0.004 + 0.013 at 8
-// bits) MT) NTW; every wave of workgroups (0.21 + 0.22 NTW) MT or (0.13 + 0.18 NTW) MT more, a launch 2.4, a cut of K the
-// reduction: 2 us and 1.6 us per million partial sums.  At 8 bits the two shapes whose registers spill cost a quarter more.
+// Rows of 16 per tile, column tiles per wave and cuts of K for a call, from a model of the launch fitted to 270000 timings of 45000 calls
+// (17 ... 640 rows, K 512 ... 14336, N 512 ... 22016, 2 / 4 / 8 bits, both activation types; rms error 6 %, its choice within 0.7 % of the
+// best on average).  A round costs 0.20 MT + (0.39 + 0.16 at 8 bits) NTW us, of 256 values (MT > 4) 0.13 MT + (0.29 - 0.01 MT + 0.05 at 8 bits)
+// NTW; every wave of workgroups (0.01 + 0.25 NTW) MT or (0.04 + 0.19 NTW) MT more, a launch 2.5 ... 3, a cut of K the reduction: 2 us and
+// 1.5 us per million partial sums.  Four column tiles a wave halve the LDS traffic of 8 x 2 tiles for the same outputs: W4 g128 us, 128 rows of 4096
+// -> 14336 float16 27.7 -> 25.6, bfloat16 30.2 -> 26.0; 14336 -> 4096 32.0 -> 28.5 - not at 8 bits, where their weights spill (59 ... 126 registers).
 //
 // Lower tiles than the call has rows read the weights (out of L2) once per tile, but fill the chip without a cut of K and its
 // reduction: W4 g128 us, one tile of rows against the plan, 2048 x 2048 at 64 rows 8.5 -> 5.3, at 128 rows 11.4 -> 6.3; 4096 x 4096 at
-// 64 rows 12.4 -> 8.8, at 128 rows 18.1 -> 12.2; 4096 -> 11008 at 128 rows 28.6 -> 23.8.
+// 64 rows 12.4 -> 8.8, at 128 rows 18.1 -> 12.2; 4096 -> 11008 at 128 rows 28.6 -> 23.8 (with two sets of x in flight).
 struct BatchCost { BatchPlan plan; float us; bool ahead; };   // ahead: this kernel takes a call of 17 rows and more
 
 // Calls that scale a group's sum in float32: the rows that are, or by bw_qlinear_decode_rows would be, the decode kernels'.
@@ -69,25 +70,28 @@ BatchCost batch_search(int64_t M, int64_t N, int64_t K, int bits, int group, boo
         const int64_t mtiles = (M + 16 * mt - 1) / (16 * mt);
         if (mt > whole || (mt < 4 && mtiles > 4)) continue;   // (more tiles of few rows: not measured)
         const bool large = mt > 4;
-        for (int ntw = 1; ntw <= (mt <= 6 ? 3 : 2); ntw++) {
+        for (int ntw = 1; ntw <= (mt <= 4 ? bits == 8 ? 3 : 4 : mt == 6 ? 3 : 2); ntw++) {
             if (sums && !bw_qbatch_sums(bits, group, mt, ntw)) continue;
             const int64_t tiles = mtiles * ((N + 32 * ntw - 1) / (32 * ntw));
             const float b8 = bits == 8 ? 1.f : 0.f;
-            float round = large ? 0.10f * mt + (0.22f + (0.004f + 0.013f * b8) * mt) * ntw : 0.17f * mt + (0.33f + 0.024f * mt + 0.19f * b8) * ntw;
-            if (bits == 8 && ((mt == 4 && ntw == 3) || (mt == 8 && ntw == 2))) round *= 1.25f;
-            const float wave = large ? (0.13f + 0.18f * ntw) * mt : (0.21f + 0.22f * ntw) * mt;
+            float round = large ? 0.128f * mt + (0.291f - 0.009f * mt + (0.086f - 0.006f * mt) * b8) * ntw - 0.185f
+                                : 0.196f * mt + (0.386f + 0.004f * mt + (0.155f - 0.005f * mt) * b8) * ntw - 0.081f;
+            if (bits == 4 && group == 32 && ntw == 4) round *= 1.04f;   // (12 registers spill)
+            const float wave = large ? (0.04f + 0.19f * ntw) * mt + 0.78f : (0.01f + 0.254f * ntw) * mt + 0.18f;
             for (int s = 1; s <= 16 && (s == 1 || (may_split && 2 * s <= nchunks)); s++) {
                 const int cps = (nchunks + s - 1) / s, used = (nchunks + cps - 1) / cps, rounds = large ? (cps + 1) / 2 : (cps + 3) / 4;
                 if (used != s || (s > 1 && M * N * s > ((int64_t)32 << 20))) continue;   // (128 MiB of partial sums)
                 const float waves = (float)((tiles * s + cus - 1) / cus);
-                const float us = 2.4f + waves * (rounds * round + wave) + (s > 1 ? 2.f + 0.05f * s + 1.6e-6f * (float)M * (float)N * s : 0.f);
+                const float us = (large ? 2.5f : 2.95f) + waves * (rounds * round + wave) + (s > 1 ? (large ? 1.7f : 2.3f) + 0.08f * s + 1.5e-6f * (float)M * (float)N * s : 0.f);
                 if (us < best.us) best = {{mt, ntw, s}, us, true};
             }
         }
     }
-    // what the model reads low or high by, per format (2600 timings of the plans it picks, float16 x; 5 % rms around that): the plan stays
-    best.us *= bits == 4 ? group == 32 ? 1.09f : 1.055f : bits == 2 ? 1.f : group == 32 && best.plan.mt == 6 && best.plan.ntw == 3 ? 1.14f : 0.97f;
-    if (N % 4) best.us *= 1.03f;                              // rows of y off an 8-byte boundary
+    // what a format costs more or less than that; the plan stays
+    best.us *= bits == 2 ? 0.965f : bits == 8 ? group == 32 ? 1.015f : 0.98f : group == 32 ? 1.03f : group == 64 ? 1.01f : 1.f;
+    if (N % 4) best.us *= 1.02f;                              // rows of y off an 8-byte boundary
+    // the chosen plan on a chip that others of the fit left idle: 2 % more, 9 % at 1 PFLOP/s (the clock comes down)
+    best.us *= 1.02f + 0.14e-9f * (float)M * (float)N * (float)K / best.us;
     return best;
 }
 
@@ -98,16 +102,15 @@ BatchCost batch_search(int64_t M, int64_t N, int64_t K, int bits, int group, boo
 // against this: 2048 x 2048 at 333 rows 20.4 -> 10.8, at 768 rows 26.7 -> 14.5; 4096 x 4096 at 256 rows 28.6 -> 17.6, at 512
 // rows 32.4 -> 30.0, but at 768 rows 39.8 against 47.9; 4096 -> 14336 at 128 rows 31.3 -> 27.4, at 160 rows 41.5 against 42.9, at 269
 // 46.5 against 53.2; 4096 -> 11008 at 310 rows 46.1 against 53.4; 512 -> 13056 at 200 rows 11.3 against 15.2).  The models
-// are of float16 x; bfloat16 costs this kernel 7 % and the prefill kernel a cast (3.2 us and 0.5 us per million values).  Both types take
+// are of float16 x; bfloat16 costs this kernel 4 % and the prefill kernel a cast (3.2 us and 0.5 us per million values).  Both types take
 // one route, so that a bfloat16 x and its float16 rounding give the same bits: half of both is added.  A doubtful call of up
-// to 128 rows stays here (1.06: 14336 -> 4096 W4 g128 at 128 rows replayed from a graph 32.6 against 30.3 us, with bfloat16 34.0 against
-// 33.1, but in eager code, where the cast is one launch more, an MLP with it takes 92 us against 95 ... 98), of more rows
-// with the prefill kernel (0.97).  On 5452 calls of 65 ... 2048 rows the choice loses 0.3 % against the better of the two (27 % at most),
-// and 42 of them are 3 % or more behind the prefill kernel; 0.5 % (51 %) and 78 with a model of 128-row tiles of the prefill kernel alone.
+// to 128 rows stays here (1.06: in eager code the prefill kernel's cast is one launch more, and an MLP that takes 92 us here takes 95 ...
+// 98 there), one beyond 512 with the prefill kernel (0.95).  On 15500 calls of 17 ... 1500 rows the choice loses 0.3 % against the better of the two;
+// they take 0.958 of the time they took with two sets of x, three column tiles and no order by XCD, and 38 of them 5 % or more longer.
 bool batch_ahead(int64_t M, int64_t N, int64_t K, int bits, int group, float us) {
     if (M <= 64) return true;
     const float half_cast = 1.6f + 0.25e-6f * (float)M * (float)K, prefill = bw_qgemm_expected_us(M, N, K, bits, group) + half_cast;
-    return 1.035f * us < (M <= 128 ? 1.06f : 0.97f) * prefill;
+    return 1.035f * us < (M <= 128 ? 1.06f : M <= 512 ? 1.f : 0.95f) * prefill;
 }
 
 BatchCost batch_cost(int64_t M, int64_t N, int64_t K, int bits, int group, bool may_split) {

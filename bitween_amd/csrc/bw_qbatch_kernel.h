@@ -8,12 +8,18 @@
 //   * K is walked in rounds of 512 values (256 beyond 64 rows); of a round's four chunks each wave takes one (kw) and NTW of the
 //     2 NTW column tiles (wn), so that the grid has enough workgroups for narrow layers and a fragment of x read from LDS
 //     feeds NTW MFMAs;
-//   * x goes global -> registers -> LDS (double buffered, one round ahead), converted from bfloat16 and permuted to the
-//     order the unpack emits on the way; scales and zero points of a round come in with it, whole rows at a time;
+//   * x goes global -> registers -> LDS (double buffered, one round ahead), converted from bfloat16 straight into the order the unpack
+//     emits, or permuted to it, on the way; scales and zero points of a round come in with it, whole rows at a time.  One set of
+//     registers, asked for a round before it is staged: x comes out of L2, a round is long enough for that, and the first multiplication
+//     waits for one request fewer (two sets: 40 rows of 4096 -> 12288, W4 g64, bfloat16 16.3 us, one 15.4; 128 rows of 4096 -> 14336, g128, 26.6 and
+//     25.9; permuting after the conversion instead of converting into the order 16.7 and 27.2);
 //   * weights go global -> registers two rounds ahead, four lanes to the 64 bytes of a row, are permuted between the lanes
 //     to operand layout (ds_bpermute) and unpacked to the reference's W16 in registers.  Asking for them in operand layout
 //     right away (neighbouring lanes on neighbouring rows) costs the address unit 60 cycles an instruction instead of 16:
 //     37 bytes/ns per CU out of L2 instead of 109;
+//   * what bounds it (128 rows of 4096 -> 14336, MT = NTW = 4, float16, 25.6 us): without a loop 10.8 (launch 2.4, the first requests 6,
+//     the sums of the four waves 2.2), without unpack and MFMAs 19.2, without memory 21.2 - LDS (x in once, out twice: 1.5 MB a
+//     workgroup), the vector unit and the matrix pipe each need 8 ... 10 us and two waves a SIMD in step overlap them in part;
 //   * the four waves that share columns add up through LDS at the end.  Where N / BN leaves CUs idle K is also cut
 //     across workgroups: float32 partial sums in the caller's workspace, added by qbatch_reduce_kernel.
 #pragma once
@@ -87,8 +93,33 @@ __global__ __launch_bounds__(512, 2) void qbatch_kernel(const BatchArgs a) {
     extern __shared__ __attribute__((aligned(16))) char smem[];
     const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
     const int nl = lane & 15, kq = lane >> 4, kw = wave % WK, wn = wave / WK;
-    const int tile = (int)blockIdx.x / a.splits, slice = (int)blockIdx.x - tile * a.splits;
-    const int mtile = tile / a.ntiles, n_base = (tile - mtile * a.ntiles) * BN, m_base = mtile * 16 * MT;
+    // Which tile.  Workgroups go to the 8 XCDs round-robin.  Where x is more than an XCD's L2 takes beside the weights (2 MB) each XCD works
+    // through one contiguous eighth of the tiles, slice by slice of K, in panels of four tiles of rows, columns last, instead of
+    // reading all of x: W4 g128 us, 999 x 8192 -> 544 29.8 -> 23.1, 300 x 4096 -> 4096 20.7 -> 19.4; W2 1146 x 10240 -> 529 38.4 -> 28.2.
+    // Elsewhere the slices of a tile, then its columns, lie side by side: 128 x 14336 -> 4096 in four slices 28.0, the other way 28.7.
+    // (Divisions only where there is something to divide: the five of the first order cost 0.15 us a launch.)
+    int slice = 0, ntile, mtile = 0;
+    if (a.mtiles >= 4 && a.x_bytes > (2u << 20)) {
+        const int xcd = (int)blockIdx.x & 7, share = (int)gridDim.x >> 3, extra = (int)gridDim.x & 7, tiles = a.mtiles * a.ntiles;
+        int tile = xcd * share + min(xcd, extra) + ((int)blockIdx.x >> 3);
+        slice = tile / tiles;
+        tile -= slice * tiles;
+        const int panel = tile / (4 * a.ntiles), rows = min(4, a.mtiles - 4 * panel);
+        tile -= panel * 4 * a.ntiles;
+        ntile = tile / rows;
+        mtile = 4 * panel + tile - ntile * rows;
+    } else {
+        ntile = (int)blockIdx.x;
+        if (a.splits > 1) {
+            ntile /= a.splits;
+            slice = (int)blockIdx.x - ntile * a.splits;
+        }
+        if (a.mtiles > 1) {
+            mtile = ntile / a.ntiles;
+            ntile -= mtile * a.ntiles;
+        }
+    }
+    const int n_base = ntile * BN, m_base = mtile * 16 * MT;
     const int M = min(a.M - m_base, 16 * MT);                         // rows of this tile
     // chunks of CK values (the slices are counted in 128s)
     const int c_begin = slice * a.chunks_per_split * (128 / CK), c_end = min(a.nchunks, (slice + 1) * a.chunks_per_split) * (128 / CK);
@@ -127,7 +158,7 @@ __global__ __launch_bounds__(512, 2) void qbatch_kernel(const BatchArgs a) {
     // the same time, which L2 serves better than requests that start at different rows (16.4 against 17.0 us at 40 rows of
     // 4096 -> 14336).
     struct XSet { u4 x[PASSES]; u2 m[ML]; };                  // a thread's share of a round: x, and scales or zero points
-    XSet xset[2];
+    XSet xset;
     auto x_row = [&](int p) { return (p * 8 + wave) * C::RPW; };
     const int sub = C::RPW == 1 ? 0 : lane / (KR / 8), col = (C::RPW == 1 ? lane : lane % (KR / 8)) * 8;   // of the lane in its wave's pass
     uint32_t row_off[PASSES];                                 // scalars
@@ -159,21 +190,30 @@ __global__ __launch_bounds__(512, 2) void qbatch_kernel(const BatchArgs a) {
     const __amdgpu_buffer_rsrc_t rm = batch_rsrc(marr - skew, (a.meta_bytes + skew + 3) & ~3u);
     auto issue_meta = [&](XSet& xs, int i, int r) { xs.m[i] = __builtin_amdgcn_raw_buffer_load_b64(rm, meta_off[i] + (uint32_t)r * (GR * 2), 0, 0); };
     auto stage_x = [&](const XSet& xs, int p, char* buf) {
-        u4 in = xs.x[p], o;
+        const u4 in = xs.x[p];
+        u4 o;                                                 // pairs (k, k + 4) at 4 bits: the order dequant_word4 emits
         if constexpr (BF16) {
+            float lo[4], hi[4];
 #pragma unroll
             for (int j = 0; j < 4; j++) {
-                const float lo = __builtin_bit_cast(float, in[j] << 16), hi = __builtin_bit_cast(float, in[j] & 0xFFFF0000u);
-                in[j] = as_u32(h2{(_Float16)lo, (_Float16)hi});
+                lo[j] = __builtin_bit_cast(float, in[j] << 16);
+                hi[j] = __builtin_bit_cast(float, in[j] & 0xFFFF0000u);
             }
-        }
-        o = in;
-        if constexpr (BITS == 4) {                            // pairs (k, k + 4): the order dequant_word4 emits
+            if constexpr (BITS == 4) {
+                o[0] = as_u32(h2{(_Float16)lo[0], (_Float16)lo[2]});
+                o[1] = as_u32(h2{(_Float16)hi[0], (_Float16)hi[2]});
+                o[2] = as_u32(h2{(_Float16)lo[1], (_Float16)lo[3]});
+                o[3] = as_u32(h2{(_Float16)hi[1], (_Float16)hi[3]});
+            } else {
+#pragma unroll
+                for (int j = 0; j < 4; j++) o[j] = as_u32(h2{(_Float16)lo[j], (_Float16)hi[j]});
+            }
+        } else if constexpr (BITS == 4) {
             o[0] = __builtin_amdgcn_perm(in[2], in[0], 0x05040100u);
             o[1] = __builtin_amdgcn_perm(in[2], in[0], 0x07060302u);
             o[2] = __builtin_amdgcn_perm(in[3], in[1], 0x05040100u);
             o[3] = __builtin_amdgcn_perm(in[3], in[1], 0x07060302u);
-        }
+        } else o = in;
         *reinterpret_cast<u4*>(buf + (x_row(p) + sub) * PITCH + col * 2) = o;
     };
     auto stage_meta = [&](const XSet& xs, int i, char* buf) {
@@ -195,13 +235,14 @@ __global__ __launch_bounds__(512, 2) void qbatch_kernel(const BatchArgs a) {
     };
     // One round: multiply what lies in `cur` and `s`; and, dealt out over the column tiles' MFMA groups so that neither the
     // address unit nor LDS sees a burst while the matrix pipe idles (12288 x 4096 at 40 rows 18.2 -> 15.9 us),
-    // put round r + 1 into `nxt` and `sn` from the registers it was requested into, and request round r + 3 there.
+    // put round r + 1 into `nxt` and `sn` from the registers it was requested into, and request x of round r + 2 and weights
+    // of round r + 3 there.
     constexpr int TASKS = PASSES + ML + NTW * WL, SLOTS = STEPS * NTW;
     auto round = [&](auto more, const char* cur, char* nxt, XSet& xs, WSet& wq, const WSet& s, WSet& sn, int r) {
         constexpr bool MORE = decltype(more)::value;
         // the lane's group of the round, kept inside the row
         const int g = min((kw * CK + kq * VPL) / GROUP, a.groups - 1 - (c_begin + WK * r) * CK / GROUP);
-        const uint32_t ko = x_offset(r + 3), so = w_scalar(r + 3);
+        const uint32_t ko = x_offset(r + 2), so = w_scalar(r + 3);
         GC gc[NTW];
 #pragma unroll
         for (int j = 0; j < NTW; j++) {
@@ -254,7 +295,7 @@ __global__ __launch_bounds__(512, 2) void qbatch_kernel(const BatchArgs a) {
                                 issue_x(xs, k, ko);
                             } else if constexpr (k < PASSES + ML) {
                                 stage_meta(xs, k - PASSES, nxt);
-                                issue_meta(xs, k - PASSES, r + 3);
+                                issue_meta(xs, k - PASSES, r + 2);
                             } else {
                                 constexpr int jl = k - PASSES - ML;
                                 permute_w(sn, wq, jl / WL, jl % WL);
@@ -276,46 +317,53 @@ __global__ __launch_bounds__(512, 2) void qbatch_kernel(const BatchArgs a) {
         }
         if constexpr (MORE) __syncthreads();
     };
-    auto request = [&](XSet& xs, WSet& ws, int r) {
-        const uint32_t ko = x_offset(r), so = w_scalar(r);
+    auto request_x = [&](int r) {
+        const uint32_t ko = x_offset(r);
 #pragma unroll
-        for (int p = 0; p < PASSES; p++) issue_x(xs, p, ko);
+        for (int p = 0; p < PASSES; p++) issue_x(xset, p, ko);
 #pragma unroll
-        for (int i = 0; i < ML; i++) issue_meta(xs, i, r);
+        for (int i = 0; i < ML; i++) issue_meta(xset, i, r);
+    };
+    auto request_w = [&](WSet& ws, int r) {
+        const uint32_t so = w_scalar(r);
 #pragma unroll
         for (int j = 0; j < NTW; j++)
 #pragma unroll
             for (int l = 0; l < WL; l++) issue_w(ws, j, l, so);
     };
     WSet s0, s1;                                              // weights in operand layout: this round's, the next one's
-    request(xset[0], wset[0], 0);
+    request_x(0);
+    request_w(wset[0], 0);
     __builtin_amdgcn_sched_barrier(0);                        // the loop's wait counts assume this order of the requests
-    request(xset[1], wset[1], 1);
+    request_w(wset[1], 1);
     __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
-    for (int p = 0; p < PASSES; p++) stage_x(xset[0], p, smem);
+    for (int p = 0; p < PASSES; p++) stage_x(xset, p, smem);
 #pragma unroll
-    for (int i = 0; i < ML; i++) stage_meta(xset[0], i, smem);
+    for (int i = 0; i < ML; i++) stage_meta(xset, i, smem);
+    __builtin_amdgcn_sched_barrier(0);
+    request_x(1);
+    __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
     for (int j = 0; j < NTW; j++)
 #pragma unroll
         for (int l = 0; l < WL; l++) permute_w(s0, wset[0], j, l);
     __builtin_amdgcn_sched_barrier(0);
-    request(xset[0], wset[0], 2);
+    request_w(wset[0], 2);
     __builtin_amdgcn_sched_barrier(0);
     __syncthreads();
     auto last = [&](const char* buf, const WSet& s, int r) {  // only the last round of a slice can have chunks past its end
-        if (c_begin + WK * r + kw < c_end) round(std::false_type{}, buf, nullptr, xset[0], wset[0], s, s1, r);
+        if (c_begin + WK * r + kw < c_end) round(std::false_type{}, buf, nullptr, xset, wset[0], s, s1, r);
     };
     // (whole pairs of rounds in a loop without a way out in the middle: another path to the loop's head, with fewer requests
     // behind it, would make every wait of the first half as strict as that path needs)
     int r = 0;
     for (; r + 2 < rounds; r += 2) {
-        round(std::true_type{}, smem, smem + BUF, xset[1], wset[1], s0, s1, r);
-        round(std::true_type{}, smem + BUF, smem, xset[0], wset[0], s1, s0, r + 1);
+        round(std::true_type{}, smem, smem + BUF, xset, wset[1], s0, s1, r);
+        round(std::true_type{}, smem + BUF, smem, xset, wset[0], s1, s0, r + 1);
     }
     if (r + 1 < rounds) {
-        round(std::true_type{}, smem, smem + BUF, xset[1], wset[1], s0, s1, r);
+        round(std::true_type{}, smem, smem + BUF, xset, wset[1], s0, s1, r);
         last(smem + BUF, s1, r + 1);
     } else {
         last(smem, s0, r);
@@ -381,8 +429,13 @@ int launch_qbatch_bits(int group, int mt, int ntw, const BatchArgs& a, hipStream
         return a.x_bf16 ? launch_qbatch<BITS, G, T, W, true, false>(a, stream) : launch_qbatch<BITS, G, T, W, false, false>(a, stream);  \
     }
 #define BW_ROWS(G, T) BW_CASE(G, T, 1) BW_CASE(G, T, 2) BW_CASE(G, T, 3)
-#define BW_GROUP(G) BW_ROWS(G, 1) BW_ROWS(G, 2) BW_ROWS(G, 3) BW_ROWS(G, 4) BW_ROWS(G, 6) BW_CASE(G, 8, 1) BW_CASE(G, 8, 2)
+#define BW_WIDE(G) BW_CASE(G, 1, 4) BW_CASE(G, 2, 4) BW_CASE(G, 3, 4) BW_CASE(G, 4, 4)
+#define BW_GROUP(G) BW_ROWS(G, 1) BW_ROWS(G, 2) BW_ROWS(G, 3) BW_ROWS(G, 4) BW_CASE(G, 6, 1) BW_CASE(G, 6, 2) BW_CASE(G, 6, 3) BW_CASE(G, 8, 1) BW_CASE(G, 8, 2)
     BW_GROUP(128) BW_GROUP(64) BW_GROUP(32)
+    if constexpr (BITS != 8) {                                // (at 8 bits four column tiles' weights spill)
+        BW_WIDE(128) BW_WIDE(64) BW_WIDE(32)
+    }
+#undef BW_WIDE
 #undef BW_GROUP
 #undef BW_ROWS
 #undef BW_CASE

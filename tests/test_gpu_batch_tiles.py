@@ -1,0 +1,60 @@
+"""The batch kernel's widest tiles and the order of its tiles on calls with many rows, against the oracle."""
+import numpy as np
+import pytest
+import torch
+
+from gpu_util import check_matmul
+from test_gpu_batch import _call
+
+pytestmark = pytest.mark.gpu
+
+
+def _layer(n, k, bits, g):
+    import bitween_amd
+    torch.manual_seed(n + k)
+    lin = torch.nn.Linear(k, n, bias=True, device="cuda", dtype=torch.float16)
+    q = bitween_amd.QuantizedLinear.from_float(lin, bits, g)
+    return (q.qweight, q.scale, q.zero_point), q.bias
+
+
+def _check(x, d, bias, bits, g, columns, y):
+    part = [a[torch.from_numpy(columns).cuda()].cpu().numpy() for a in (*d, bias)]
+    check_matmul(y[:, torch.from_numpy(columns).cuda()], x.to(torch.float16).cpu().numpy(), *part, bits, g)
+
+
+def _columns(n, step=97):
+    """A sample, with both ends and the edges of the 32-column tiles around them."""
+    return np.unique(np.clip(np.concatenate([np.arange(0, n, step), [1, 15, 16, 31, 32, 63, 64, 127, 128], n - np.array([1, 2, 16, 17, 33])]), 0, n - 1))
+
+
+@pytest.mark.parametrize("bits,g", [(4, 128), (4, 64), (4, 32), (2, 128), (2, 32)])
+@pytest.mark.parametrize("m,n,k", [(33, 8501, 256), (17, 24751, 3200), (45, 24751, 1152), (260, 5501, 1024), (128, 14336, 640)])
+def test_four_column_tiles(bits, g, m, n, k):
+    """Layers wide enough for four column tiles a wave: rows and columns that end inside a tile, one to three rounds of K; bfloat16 x has
+    the bits of its float16 cast."""
+    from bitween_amd.kernels import hip_loader as hip
+    d, bias = _layer(n, k, bits, g)
+    gen = torch.Generator(device="cuda").manual_seed(m)
+    x = torch.randn(m, k, device="cuda", generator=gen).to(torch.bfloat16)
+    st, y, _ = _call(hip.load(), x.to(torch.float16), d, n, bits, g, n + 1, bias=bias)
+    name = hip.last_decode_kernel()
+    assert st == 0 and (y[:, n:] == 7.0).all() and name.startswith("qbatch_kernel<%d, %d, " % (bits, g))
+    if g == 128 and n % 2 and m > 32:                         # (fewer rows of it scale sums of a group, on narrower tiles)
+        assert name.split(", ")[3] == "4", name
+    _check(x, d, bias, bits, g, _columns(n), y)
+    st, yb, _ = _call(hip.load(), x, d, n, bits, g, n + 1, bias=bias)
+    assert st == 0 and torch.equal(y, yb)
+
+
+@pytest.mark.parametrize("bits,g,m,n,k", [(4, 128, 1100, 130, 1024), (4, 128, 700, 2050, 1664), (2, 64, 1030, 70, 4096), (8, 32, 620, 66, 2304),
+                                          (4, 64, 530, 515, 2176), (4, 32, 257, 1030, 4192)])
+def test_many_rows_every_tile_once(bits, g, m, n, k):
+    """x beyond 2 MB in four and more tiles of rows, whose workgroups are numbered by XCD: panels of four and a shorter last one, grids that
+    are no multiple of eight, K cut or not; nothing is left out and nothing beyond y is written."""
+    from bitween_amd.kernels import hip_loader as hip
+    d, bias = _layer(n, k, bits, g)
+    x = torch.randn(m, k, device="cuda", generator=torch.Generator(device="cuda").manual_seed(m)).to(torch.float16)
+    assert m * k * 2 > 2 << 20
+    st, y, _ = _call(hip.load(), x, d, n, bits, g, n + 3, bias=bias)
+    assert st == 0 and (y[:, n:] == 7.0).all() and hip.last_decode_kernel().startswith("qbatch_kernel<")
+    _check(x, d, bias, bits, g, np.arange(n) if n < 200 else _columns(n, 23), y)
