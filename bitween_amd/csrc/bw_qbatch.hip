@@ -129,22 +129,32 @@ inline size_t batch_ws_bytes(int64_t M, int64_t N, const BatchPlan& p) { return 
 // ---- which kernel ----
 enum Route { kDecode, kBatch, kPrefill };
 
-// Up to 16 rows the decode kernels keep the call except where they stage x several times over: rows longer than one round
-// of theirs (K > 4096), or more column tiles than their resident workgroups hold.  5 ... 16 rows, timed on 60 shapes x
-// nine formats (us, decode against this kernel): W4 g32 5120 -> 22016 36 ... 48 against 20 ... 22, W2 g64 5120 -> 14336 21 ...
-// 30 against 11 ... 13, W4 g128 4096 -> 22016 15.7 ... 18.3 against 13.5 ... 14.8, W8 g64 4096 -> 14336 16.0 ... 20.5 against
-// 15.4 ... 16.1; on the other side of the lines W4 g128 4096 -> 14336 9.5 ... 10.8 against 10.3 ... 11.4, W4 g128 11008 -> 4096
-// 8.8 ... 12.1 against 11.7 ... 12.9.
+// Up to 16 rows the decode kernels keep the call except where they stage x several times over: rows longer than one round of theirs
+// (K > 4096), or more column tiles than their resident workgroups hold; and except on narrow layers with long rows, where this kernel cuts
+// K and they have a few workgroups that walk all of it.  From 49000 timings (5 ... 16 rows, nine formats, K 512 ... 14336, N 512 ...
+// 22016; this kernel's time over theirs at 9 ... 16 rows, and at 5 ... 8): K > 4096 with tiles > CUs 0.40 ... 0.89 (0.55 ... 0.98);
+// tiles > 3 CUs 0.73 ... 0.97; tiles <= CUs / 2 at K > 11008 0.51 ... 0.83 (0.72 ... 1.04), at K <= 4096 1.0 ... 1.2; between CUs / 2 and
+// CUs, where every CU has one decode workgroup, 0.85 ... 1.1 at K > 8192 and 1.0 ... 1.5 below; at 8 bits CUs ... 2 CUs tiles 0.67 ... 0.97
+// for K > 3072, 5 ... 8 rows 0.9 ... 1.1.  Layers of 8 bits in groups of 64 keep the lines they had: their decode kernels scale a group's
+// sum in float32, this kernel rounds every weight.
 inline bool batch_takes_decode_rows(int64_t M, int64_t N, int64_t K, int bits, int group) {
     const int64_t tiles = (N + 15) / 16, cus = bw_device_cus();
+    const bool many = M > 8, narrow = tiles <= cus / 2;
     if (M < 5) return false;
-    if (bits == 8) return tiles > 3 * cus || (M > 8 && K >= 8192);
-    if (K > 4096) {
-        if (tiles > cus) return !(bits == 4 && group == 128) || M > 8;
-        return M > 8 && (group == 32 || (bits == 4 && group == 64));
+    if (bits == 8) {
+        if (tiles > 3 * cus) return many ? K > 1024 : K > 3072 && (tiles <= 4 * cus || group == 32);
+        if (group == 64) return many && K >= 8192;
+        if (tiles > 2 * cus) return many && K > 6144;
+        if (tiles > cus) return many && K > 3072;
+        if (narrow) return K > (many ? group == 32 ? 6144 : 8191 : group == 32 ? 8192 : 11008);
+        return many && K > (group == 32 ? 8192 : 11008);
     }
-    if (K >= 3072 && tiles > 4 * cus) return true;
-    return bits == 2 && M > 8 && tiles > 3 * cus && (group == 32 || K / group % 2);
+    if (K > 4096 ? tiles > cus : K >= 3072 && tiles > 4 * cus) return true;
+    if (many && tiles > 3 * cus) return true;
+    if (many && group == 32) return K > 4096 || (tiles > cus && tiles <= 2 * cus);
+    if (K <= 4096) return false;
+    if (narrow) return many ? K > 6144 : group != 128 && K > (group == 32 ? 8192 : 11008);
+    return many && (bits == 2 ? K > 8192 : group == 64 && K > 11008);
 }
 
 Route route(int64_t M, int64_t N, int64_t K, int bits, int group) {

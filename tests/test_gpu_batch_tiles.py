@@ -1,4 +1,5 @@
-"""The batch kernel's widest tiles and the order of its tiles on calls with many rows, against the oracle."""
+"""The batch kernel's widest tiles, the order of its tiles on calls with many rows, and the lines between it and the decode kernels
+up to 16 rows, against the oracle."""
 import numpy as np
 import pytest
 import torch
@@ -58,3 +59,22 @@ def test_many_rows_every_tile_once(bits, g, m, n, k):
     st, y, _ = _call(hip.load(), x, d, n, bits, g, n + 3, bias=bias)
     assert st == 0 and (y[:, n:] == 7.0).all() and hip.last_decode_kernel().startswith("qbatch_kernel<")
     _check(x, d, bias, bits, g, np.arange(n) if n < 200 else _columns(n, 23), y)
+
+
+@pytest.mark.parametrize("bits,g,k,n,m,kernel", [
+    (4, 128, 6272, 2048, 9, "qbatch"), (4, 128, 6144, 2048, 16, "qgemv"), (4, 128, 6272, 2048, 8, "qgemv"), (4, 128, 6272, 2064, 16, "qgemv"),
+    (4, 128, 4224, 4112, 5, "qbatch"), (4, 128, 4096, 4112, 16, "qgemv"), (4, 64, 11072, 2064, 9, "qbatch"), (4, 64, 11008, 2064, 9, "qgemv"),
+    (4, 32, 544, 4112, 9, "qbatch"), (4, 32, 544, 4096, 9, "qgemv"), (4, 32, 8224, 640, 5, "qbatch"), (2, 128, 8320, 2064, 12, "qbatch"),
+    (4, 128, 1024, 12304, 9, "qbatch"), (8, 128, 3200, 4112, 16, "qbatch"), (8, 128, 3072, 4112, 16, "qgemv"), (8, 128, 3200, 4112, 8, "qgemv"),
+    (8, 128, 8192, 2048, 9, "qbatch"), (8, 32, 8224, 640, 5, "qbatch"), (8, 64, 8192, 2064, 9, "qbatch"), (8, 64, 8128, 2064, 9, "qgemv")])
+def test_lines_between_decode_and_batch_rows(bits, g, k, n, m, kernel):
+    """5 ... 16 rows on both sides of each line (256 compute units), K cut across workgroups where the layer is narrow."""
+    from bitween_amd.kernels import hip_loader as hip
+    d, bias = _layer(n, k, bits, g)
+    x = torch.randn(m, k, device="cuda", generator=torch.Generator(device="cuda").manual_seed(m)).to(torch.float16)
+    st, y, _ = _call(hip.load(), x, d, n, bits, g, n, bias=bias)
+    assert st == 0 and hip.last_decode_kernel().startswith(kernel)
+    _check(x, d, bias, bits, g, _columns(n), y)
+    st, y, _ = _call(hip.load(), x, d, n, bits, g, n, ws=False, bias=bias)
+    assert st == 0
+    _check(x, d, bias, bits, g, _columns(n), y)
