@@ -32,15 +32,15 @@
 #include <hip/hip_runtime.h>
 
 #include "bw_common.h"
+#include "bw_plan_cache.h"
 
 namespace {
 
 constexpr int DK = 128, DN = 32, DTHREADS = 256;
 constexpr int DPITCH = 80;                           // bytes per LDS row of the grad_y tile: 32 halves + 16 (rows stay 16-byte aligned)
 constexpr int B_BYTES = DN * DK * 2;                 // n-major weight tile: 32 rows of 128 halves, unpadded
-// MT = 16-row m tiles per wave (the workgroup's 2 x 2 waves cover 32 MT rows of m).  MT = 4 (161 registers, three
-// workgroups per CU) up to 512 rows of grad_y; MT = 8 (251 registers, two per CU, a quarter fewer LDS reads per MFMA)
-// beyond: 15-20 % faster there, slower below.
+// MT = 16-row m tiles per wave (the workgroup's 2 x 2 waves cover 32 MT rows of m): 4 (161 registers, three workgroups
+// per CU) or 8 (251 registers, two per CU, a quarter fewer LDS reads per MFMA), whichever the plan predicts the faster.
 template <int MT> struct DgradTile {
     static constexpr int DM = 32 * MT;
     static constexpr int A_BYTES = DM * DPITCH;      // grad_y tile
@@ -610,9 +610,6 @@ inline int dgrad_cus() {
     return cus;
 }
 
-// Three workgroups fit a CU and hide each other's barriers.  With fewer tiles than two per CU N is cut into slices:
-// to two workgroups per CU (three measured slower: more partial-tile traffic) when a slice keeps at least 24 steps,
-// else to one per CU with at least 8 (short slices pay their prologue and the partial tiles' traffic).
 // The 256 x 256 kernel takes a problem when it is large enough, counted in tile-steps (tiles x steps of 64 rows of n),
 // K in whole tiles, N in whole steps, extents that fit the 32-bit offsets of buffer addressing - and, below one
 // workgroup per CU, a workspace: N is then cut into slices of at least 8 steps so that every CU has one.  Measured
@@ -656,32 +653,62 @@ inline DgradPlan dgrad256_plan(int64_t M, int64_t N, int64_t K, bool have_worksp
     return p;
 }
 
-inline DgradPlan dgrad_plan(int64_t M, int64_t N, int64_t K, bool have_workspace) {
-    DgradPlan p;
-    p.mt = M > 512 ? 8 : 4;
-    const int DM = 32 * p.mt;
-    p.tiles_k = (int)((K + DK - 1) / DK);
-    p.tiles = p.tiles_k * (int)((M + DM - 1) / DM);
-    const int nsteps = (int)((N + DN - 1) / DN);
-    p.splits = 1;
-    p.steps_per_split = nsteps;
-    p.ws_bytes = 0;
-    if (!have_workspace) return p;
-    const int cus = dgrad_cus();
-    int s = (2 * cus + p.tiles - 1) / p.tiles;
-    if (s < 2 || nsteps / s < 24) {
-        s = (cus + p.tiles - 1) / p.tiles;
-        if (s > nsteps / 8) s = nsteps / 8;
+// The stepping kernel's tile height and slices of N, by predicted time.  A step is bound by its own chain (weight words ->
+// LDS -> transposed reads -> MFMAs -> barrier), not by memory: 0.41 us alone on a CU, 0.65 / 0.88 with two / three
+// workgroups (128-row tiles; 0.67 / 1.03 with one / two of 256 rows), so co-resident workgroups pay - 2.1 times the
+// throughput at three - and a launch lasts as long as the CU with the most of them.  Counted that way two slices too many
+// cost more than a few idle CUs: 20 CUs with a second workgroup make the rest wait for a second set of steps.  Beside the
+// steps: a workgroup's prologue and epilogue, and for slices the second launch and the partial tiles (0.29 us per MB
+// written and read, 0.11 us per slice read one behind the other).  128-row tiles dequantise a weight twice as often per
+// MFMA, which long launches pay in clock rate (up to 12 %).
+// Fitted on 113184 timings of 16303 calls (1 ... 2048 rows, layers of 512 ... 14336 on either side, all formats, ragged
+// sizes; the order of plans hardly depends on type and bits).  Against two workgroups per CU where a slice keeps 24 steps,
+// else one with 8, and 256-row tiles beyond 512 rows, calls take 0.888 of the time on average (the best plan of each:
+// 0.876), 0.82-0.84 beyond 512 rows and 0.88 up to 16; 1.3 % of them take over 5 % longer.  W4 g64, float16: 333 rows of
+// 3001 -> 2880 27.9 -> 22.4 us (276 workgroups of 4 slices: now 207 of 3), 333 of 1000 -> 8192 26.9 -> 18.1 (unsliced),
+// 700 of 1100 -> 1088 17.9 -> 15.2 (128-row tiles), 128 of 8000 -> 1024 17.9 -> 15.8 (24 slices instead of 16).
+struct DgradSearch {
+    static constexpr int MAX_SPLITS = 32;
+    static float us(int mt, int tiles, int splits, int steps, int64_t M, int cus) {
+        const int DM = 32 * mt, slots = mt == 4 ? 3 : 2;
+        const int per_cu = (int)(((int64_t)tiles * splits + cus - 1) / cus);      // workgroups of the busiest CU
+        auto step = [&](int resident) { return mt == 4 ? 0.177f + 0.235f * resident : 0.313f + 0.359f * resident; };
+        float t = steps * ((per_cu / slots) * step(slots) + (per_cu % slots ? step(per_cu % slots) : 0.f));
+        if (mt == 4) t *= 1.f + 0.12f * (t < 300.f ? t / 300.f : 1.f);
+        t += (mt == 4 ? 0.66f : 1.f) * per_cu;
+        if (splits > 1) t += 2.2f + 0.11f * splits + 0.285e-6f * ((float)tiles * splits * (M < DM ? M : DM) * DK * 4);
+        return t;
     }
-    if (s > 32) s = 32;
-    if (s < 2) return p;
-    const int sps = (nsteps + s - 1) / s;
-    s = (nsteps + sps - 1) / sps;
-    if (s < 2) return p;
-    p.splits = s;
-    p.steps_per_split = sps;
-    p.ws_bytes = (size_t)p.tiles * s * DM * DK * sizeof(float);
-    return p;
+    static DgradPlan run(int64_t M, int64_t N, int64_t K, bool have_workspace) {
+        const int cus = dgrad_cus(), nsteps = (int)((N + DN - 1) / DN);
+        DgradPlan best{};
+        float best_us = 0.f;
+        for (int mt = 4; mt <= (M > 256 ? 8 : 4); mt += 4) {                     // up to 256 rows the taller tile has no second row of tiles to save
+            const int DM = 32 * mt;
+            DgradPlan p;
+            p.mt = mt;
+            p.tiles_k = (int)((K + DK - 1) / DK);
+            p.tiles = p.tiles_k * (int)((M + DM - 1) / DM);
+            for (int s = 1; s <= (have_workspace ? MAX_SPLITS : 1) && s <= nsteps; s++) {
+                // four 128-row workgroups per CU bound the workspace to 64 MiB (more of them gains 0.03 % on average)
+                if (s > 1 && (int64_t)p.tiles * s * mt > (int64_t)16 * cus) break;
+                p.steps_per_split = (nsteps + s - 1) / s;
+                p.splits = (nsteps + p.steps_per_split - 1) / p.steps_per_split;
+                if (p.splits != s) continue;                                     // the same slices as a smaller s
+                const float t = us(mt, p.tiles, s, p.steps_per_split, M, cus);
+                if (best_us > 0.f && t >= best_us) continue;
+                p.ws_bytes = s > 1 ? (size_t)p.tiles * s * DM * DK * sizeof(float) : 0;
+                best = p;
+                best_us = t;
+            }
+        }
+        return best;
+    }
+};
+
+inline DgradPlan dgrad_plan(int64_t M, int64_t N, int64_t K, bool have_workspace) {
+    thread_local BwPlanCache<DgradPlan> cache{};                                 // a search takes about a microsecond; the launch and both queries ask
+    return cache.get(M, N, K, have_workspace, [&] { return DgradSearch::run(M, N, K, have_workspace); });
 }
 
 inline bool dgrad_fast_shape(int64_t M, int64_t N, int64_t K, int64_t ldg, int64_t ldx, int bits, int group) {
@@ -778,7 +805,7 @@ extern "C" size_t bw_qdgrad_workspace_bytes(int64_t M, int64_t N, int64_t K, int
 extern "C" int bw_qdgrad_tile_rows(int64_t M, int64_t N, int64_t K, int bits, int group) {
     if (!bw_shape_ok(N, K, bits, group) || !dgrad_fast_shape(M, N, K, N, K, bits, group)) return 0;
     if (const int rows = dgrad_use256(M, N, K, N, bits, group, true)) return rows + 1;
-    return M > 512 ? 256 : 128;
+    return 32 * dgrad_plan(M, N, K, true).mt;
 }
 
 extern "C" int bw_qdgrad(const void* grad_y, int act_dtype, int64_t M, int64_t N, int64_t ldg, const int32_t* qweight,

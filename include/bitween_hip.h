@@ -198,7 +198,7 @@ int bw_cast_bf16_f16(const void* x, int64_t rows, int64_t cols, int64_t ldx, voi
  * When M * K is small the reduction over N is cut into slices whose float32 partial sums go through a
  * caller-provided workspace of bw_qdgrad_workspace_bytes(...) bytes (16-byte aligned; 0 = none needed);
  * workspace == NULL runs unsliced.
- * Two kernels: one that owns 128 (256 beyond 512 rows) x 128 tiles of grad_x and walks N in steps of 32 rows, and - for
+ * Two kernels: one that owns 128 or 256 x 128 tiles of grad_x and walks N in steps of 32 rows, and - for
  * large problems with K % 256 == 0 and N % 64 == 0 - one with 256 x 256 tiles and steps of 64 rows;
  * bw_qdgrad_tile_rows tells which a shape gets (128, 256; 129, 257 = the 256 x 256 kernel with 128 (up to 512 rows of
  * grad_y) or 256 rows of m per tile; 0 = no fused path): a diagnostic,

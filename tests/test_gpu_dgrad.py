@@ -348,3 +348,35 @@ def test_dgrad_infinite_gradients_of_a_ragged_n(n, m):
     gx = hip.quantized_input_grad(go.cuda(), *(to_gpu(a) for a in (qw, s16, z16)), bits, g).double().cpu()
     assert torch.equal(torch.isnan(gx), torch.isnan(want)) and torch.equal(torch.isinf(gx), torch.isinf(want))
     assert torch.equal(gx[torch.isinf(want)], want[torch.isinf(want)])
+
+
+@pytest.mark.parametrize("m,n,k,rows,slices", [
+    (333, 1000, 8192, 128, 1),      # 192 tiles: a second slice would give half the CUs a second workgroup
+    (333, 3001, 2880, 128, 3),      # 69 tiles, the last column half empty; the last slice ends within a step of 32 rows
+    (128, 8000, 1024, 128, 21),     # 8 tiles of 250 steps
+    (700, 1100, 1088, 128, 4),      # the shorter tiles beyond 512 rows
+    (411, 5728, 4160, 256, 7),      # the taller tiles below, the last column half empty
+])
+def test_dgrad_plan_of_tiles_and_slices(m, n, k, rows, slices):
+    """The stepping kernel's tile height and slices of N come from a predicted time: each plan against the oracle, with its
+    workspace (exactly what the query names; four bytes less are refused) and without one (unsliced)."""
+    from bitween_amd.kernels import hip_loader
+    lib = hip_loader.load()
+    bits, g = 4, 64
+    if torch.cuda.get_device_properties(0).multi_processor_count == 256:     # the prediction counts workgroups per CU
+        assert lib.bw_qdgrad_tile_rows(m, n, k, bits, g) == rows
+        tiles = -(-m // rows) * -(-k // 128)
+        assert lib.bw_qdgrad_workspace_bytes(m, n, k, bits, g) == (tiles * slices * rows * 128 * 4 if slices > 1 else 0)
+    _, qw, s16, z16, _ = quantized_layer(n, k, bits, g, seed=n + k, outliers=True, bias=False)
+    d = [to_gpu(a) for a in (qw, s16, z16)]
+    go16 = np.random.default_rng(m).standard_normal((m, n)).astype(np.float16)
+    go = to_gpu(go16)
+    for use_ws in (True, False):
+        st, gx, need = _call(lib, go, d, m, n, k, bits, g, use_ws)
+        assert st == 0
+        _check(gx, go16, qw, s16, z16, bits, g)
+    if slices > 1:
+        ws = torch.empty(lib.bw_qdgrad_workspace_bytes(m, n, k, bits, g), dtype=torch.uint8, device="cuda")
+        gx = torch.empty((m, k), dtype=torch.float16, device="cuda")
+        assert lib.bw_qdgrad(go.data_ptr(), 0, m, n, n, d[0].data_ptr(), d[1].data_ptr(), d[2].data_ptr(), k, bits, g, gx.data_ptr(),
+                             k, ws.data_ptr(), ws.numel() - 4, ctypes.c_void_p(torch.cuda.current_stream().cuda_stream)) == -5
