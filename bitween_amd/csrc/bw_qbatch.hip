@@ -133,7 +133,7 @@ enum Route { kDecode, kBatch, kPrefill };
 // (K > 4096), or more column tiles than their resident workgroups hold; and except on narrow layers with long rows, where this kernel cuts
 // K and they have a few workgroups that walk all of it.  From 49000 timings (5 ... 16 rows, nine formats, K 512 ... 14336, N 512 ...
 // 22016; this kernel's time over theirs at 9 ... 16 rows, and at 5 ... 8): K > 4096 with tiles > CUs 0.40 ... 0.89 (0.55 ... 0.98);
-// tiles > 3 CUs 0.73 ... 0.97; tiles <= CUs / 2 at K > 11008 0.51 ... 0.83 (0.72 ... 1.04), at K <= 4096 1.0 ... 1.2; between CUs / 2 and
+// tiles > 3 CUs at 8 bits, groups of 32 or an odd number of them 0.73 ... 0.97, else 0.94 ... 1.03 at K <= 2048 (g64: 3072), 1.0 ... 1.06 up to K = 4096; tiles <= CUs / 2 at K > 11008 0.51 ... 0.83 (0.72 ... 1.04), at K <= 4096 1.0 ... 1.2; between CUs / 2 and
 // CUs, where every CU has one decode workgroup, 0.85 ... 1.1 at K > 8192 and 1.0 ... 1.5 below; at 8 bits CUs ... 2 CUs tiles 0.67 ... 0.97
 // for K > 3072, 5 ... 8 rows 0.9 ... 1.1.  Layers of 8 bits in groups of 64 keep the lines they had: their decode kernels scale a group's
 // sum in float32, this kernel rounds every weight.
@@ -150,7 +150,7 @@ inline bool batch_takes_decode_rows(int64_t M, int64_t N, int64_t K, int bits, i
         return many && K > (group == 32 ? 8192 : 11008);
     }
     if (K > 4096 ? tiles > cus : K >= 3072 && tiles > 4 * cus) return true;
-    if (many && tiles > 3 * cus) return true;
+    if (many && tiles > 3 * cus && (group == 32 || K / group % 2 || K <= (group == 64 ? 3072 : 2048))) return true;
     if (many && group == 32) return K > 4096 || (tiles > cus && tiles <= 2 * cus);
     if (K <= 4096) return false;
     if (narrow) return many ? K > 6144 : group != 128 && K > (group == 32 ? 8192 : 11008);
@@ -226,9 +226,12 @@ extern "C" int bw_qlinear_ws(const void* x, int act_dtype, int64_t M, int64_t K,
     bw_note_kernel("");
     const bool fast = bw_fast_shape(M, N, K, ldx, bits, group);
     Route r = fast ? route(M, N, K, bits, group) : M <= 16 ? kDecode : kPrefill;
+    const bool cut = r != kBatch || batch_ws_bytes(M, N, batch_plan(M, N, K, bits, group, true)) <= workspace_bytes;   // room for the plan's cut of K
+    // Up to 16 rows a narrow layer comes here for that cut: without room for it the decode kernels are ahead (9 rows, us: W4 g128
+    // 14336 -> 512 uncut 15.1, theirs 10.6; W8 g32 14336 -> 4096 23.6 and 19.9; 83 calls with tiles <= CUs 0.6 ... 1.01).
+    if (!cut && M <= 16 && (N + 15) / 16 <= bw_device_cus()) r = kDecode;
     if (r == kBatch && batch_takes(x, M, N, K, ldx, qweight, scale16, zp16, bits, group)) {
-        BatchPlan plan = batch_plan(M, N, K, bits, group, true);
-        if (batch_ws_bytes(M, N, plan) > workspace_bytes) plan = batch_plan(M, N, K, bits, group, false);
+        const BatchPlan plan = batch_plan(M, N, K, bits, group, cut);
         return launch_batch(x, act_dtype, M, K, ldx, qweight, scale16, zp16, bias, N, bits, group, y, ldy, workspace, plan, (hipStream_t)stream);
     }
     if (M <= 16) {
