@@ -133,10 +133,12 @@ enum Route { kDecode, kBatch, kPrefill };
 // (K > 4096), or more column tiles than their resident workgroups hold; and except on narrow layers with long rows, where this kernel cuts
 // K and they have a few workgroups that walk all of it.  From 49000 timings (5 ... 16 rows, nine formats, K 512 ... 14336, N 512 ...
 // 22016; this kernel's time over theirs at 9 ... 16 rows, and at 5 ... 8): K > 4096 with tiles > CUs 0.40 ... 0.89 (0.55 ... 0.98);
-// tiles > 3 CUs at 8 bits, groups of 32 or an odd number of them 0.73 ... 0.97, else 0.94 ... 1.03 at K <= 2048 (g64: 3072), 1.0 ... 1.06 up to K = 4096; tiles <= CUs / 2 at K > 11008 0.51 ... 0.83 (0.72 ... 1.04), at K <= 4096 1.0 ... 1.2; between CUs / 2 and
-// CUs, where every CU has one decode workgroup, 0.85 ... 1.1 at K > 8192 and 1.0 ... 1.5 below; at 8 bits CUs ... 2 CUs tiles 0.67 ... 0.97
-// for K > 3072, 5 ... 8 rows 0.9 ... 1.1.  Layers of 8 bits in groups of 64 keep the lines they had: their decode kernels scale a group's
-// sum in float32, this kernel rounds every weight.
+// tiles > 3 CUs at 8 bits, groups of 32 or an odd number of them 0.73 ... 0.97, else 0.94 ... 1.03 at K <= 2048 (g64: 3072) and 1.0 ... 1.06 up
+// to K = 4096; tiles <= CUs / 2 at K > 11008 0.51 ... 0.83 (0.72 ... 1.04), at K <= 4096 1.0 ... 1.2; between CUs / 2 and CUs, where
+// every CU has one decode workgroup, 0.85 ... 1.1 at K > 8192 and 1.0 ... 1.5 below, of that up to 3/4 CUs at 2 bits 0.72 ... 1.06 (W4 g64 at K
+// > 11008 0.84 ... 1.05), beyond 0.95 ... 1.07 (1.02 ... 1.15) until the rows are long: W2 g64 12800 0.94 ... 1.0, 14336 0.80 ... 0.87, W4 g64
+// 14336 0.83 ... 1.01; at 8 bits CUs ... 2 CUs tiles 0.67 ... 0.97 for K > 3072, 5 ... 8 rows 0.9 ... 1.1.  Layers of 8 bits in groups of
+// 64 keep the lines they had: their decode kernels scale a group's sum in float32, this kernel rounds every weight.
 inline bool batch_takes_decode_rows(int64_t M, int64_t N, int64_t K, int bits, int group) {
     const int64_t tiles = (N + 15) / 16, cus = bw_device_cus();
     const bool many = M > 8, narrow = tiles <= cus / 2;
@@ -154,7 +156,8 @@ inline bool batch_takes_decode_rows(int64_t M, int64_t N, int64_t K, int bits, i
     if (many && group == 32) return K > 4096 || (tiles > cus && tiles <= 2 * cus);
     if (K <= 4096) return false;
     if (narrow) return many ? K > 6144 : group != 128 && K > (group == 32 ? 8192 : 11008);
-    return many && (bits == 2 ? K > 8192 : group == 64 && K > 11008);
+    const bool full = 4 * tiles > 3 * cus && K / group % 2 == 0;
+    return many && (bits == 2 ? K > (!full ? 8192 : group == 64 ? 12288 : 13312) : group == 64 && K > (full ? 13312 : 11008));
 }
 
 Route route(int64_t M, int64_t N, int64_t K, int bits, int group) {

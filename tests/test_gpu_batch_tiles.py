@@ -66,6 +66,8 @@ def test_many_rows_every_tile_once(bits, g, m, n, k):
     (4, 128, 4224, 4112, 5, "qbatch"), (4, 128, 4096, 4112, 16, "qgemv"), (4, 64, 11072, 2064, 9, "qbatch"), (4, 64, 11008, 2064, 9, "qgemv"),
     (4, 32, 544, 4112, 9, "qbatch"), (4, 32, 544, 4096, 9, "qgemv"), (4, 32, 8224, 640, 5, "qbatch"), (2, 128, 8320, 2064, 12, "qbatch"),
     (4, 128, 1024, 12304, 9, "qbatch"), (4, 128, 4096, 12304, 9, "qgemv"), (4, 128, 3968, 12304, 9, "qbatch"),
+    (2, 128, 8448, 4096, 9, "qgemv"), (2, 128, 8320, 4096, 9, "qbatch"),
+    (2, 64, 12288, 4096, 9, "qgemv"), (2, 64, 12416, 4096, 9, "qbatch"), (4, 64, 13312, 4096, 9, "qgemv"), (4, 64, 13440, 4096, 9, "qbatch"),
     (2, 64, 3072, 12304, 16, "qbatch"), (2, 64, 3200, 12304, 16, "qgemv"), (8, 128, 3200, 4112, 16, "qbatch"), (8, 128, 3072, 4112, 16, "qgemv"), (8, 128, 3200, 4112, 8, "qgemv"),
     (8, 128, 8192, 2048, 9, "qbatch"), (8, 32, 8224, 640, 5, "qbatch"), (8, 64, 8192, 2064, 9, "qbatch"), (8, 64, 8128, 2064, 9, "qgemv")])
 def test_lines_between_decode_and_batch_rows(bits, g, k, n, m, kernel):
