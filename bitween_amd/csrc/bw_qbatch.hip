@@ -229,6 +229,9 @@ extern "C" int bw_qlinear_ws(const void* x, int act_dtype, int64_t M, int64_t K,
     bw_note_kernel("");
     const bool fast = bw_fast_shape(M, N, K, ldx, bits, group);
     Route r = fast ? route(M, N, K, bits, group) : M <= 16 ? kDecode : kPrefill;
+    // Without room for the prefill kernel's cast of a bfloat16 x this kernel takes the call, which reads x as it is (and cuts K only if
+    // there is room for that).
+    if (fast && r == kPrefill && M <= 2048 && act_dtype == BW_BF16 && workspace_bytes < cast_bytes(M, K)) r = kBatch;
     const bool cut = r != kBatch || batch_ws_bytes(M, N, batch_plan(M, N, K, bits, group, true)) <= workspace_bytes;   // room for the plan's cut of K
     // Up to 16 rows a narrow layer comes here for that cut: without room for it the decode kernels are ahead (9 rows, us: W4 g128
     // 14336 -> 512 uncut 15.1, theirs 10.6; W8 g32 14336 -> 4096 23.6 and 19.9; 83 calls with tiles <= CUs 0.6 ... 1.01).

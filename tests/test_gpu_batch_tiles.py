@@ -1,5 +1,7 @@
 """The batch kernel's widest tiles, the order of its tiles on calls with many rows, and the lines between it and the decode kernels
 up to 16 rows, against the oracle."""
+import ctypes
+
 import numpy as np
 import pytest
 import torch
@@ -82,3 +84,31 @@ def test_lines_between_decode_and_batch_rows(bits, g, k, n, m, kernel):
     st, y, _ = _call(hip.load(), x, d, n, bits, g, n, ws=False, bias=bias)
     assert st == 0 and hip.last_decode_kernel().startswith("qgemv" if need and n <= 4096 else kernel)
     _check(x, d, bias, bits, g, _columns(n), y)
+
+
+@pytest.mark.parametrize("bits,g,m,n,k", [(4, 128, 813, 4432, 2304), (4, 64, 200, 9000, 6912), (2, 64, 1167, 3340, 1024), (8, 32, 1171, 3842, 1024)])
+def test_bfloat16_without_room_for_its_cast(bits, g, m, n, k):
+    """Calls that the prefill kernel is expected to finish first, with bfloat16 x: with no workspace, and with 16 bytes less than the cast takes,
+    the batch kernel runs them (and writes nothing beyond the workspace); beyond 2048 rows there is none that could."""
+    from bitween_amd.kernels import hip_loader as hip
+    lib = hip.load()
+    d, bias = _layer(n, k, bits, g)
+    x = torch.randn(m, k, device="cuda", generator=torch.Generator(device="cuda").manual_seed(m)).to(torch.bfloat16)
+    st, y, need = _call(lib, x, d, n, bits, g, n, bias=bias)
+    if torch.cuda.get_device_properties(0).multi_processor_count == 256:
+        assert hip.last_decode_kernel() == "" and need >= 2 * m * k
+    _check(x, d, bias, bits, g, _columns(n), y)
+    short = 2 * m * k - 16
+    ws = torch.full((short + 64,), 85, dtype=torch.uint8, device="cuda")
+    y = torch.full((m, n), 7.0, dtype=torch.float16, device="cuda")
+    stream = ctypes.c_void_p(torch.cuda.current_stream().cuda_stream)
+    for buffer, size in ((None, 0), (ws.data_ptr(), short)):
+        y.fill_(7.0)
+        st = lib.bw_qlinear_ws(x.data_ptr(), 1, m, k, k, d[0].data_ptr(), d[1].data_ptr(), d[2].data_ptr(), bias.data_ptr(), n, bits, g, y.data_ptr(), n,
+                               buffer, size, stream)
+        torch.cuda.synchronize()
+        assert st == 0 and hip.last_decode_kernel().startswith("qbatch_kernel<%d, %d, " % (bits, g)) and (ws[short:] == 85).all()
+        _check(x, d, bias, bits, g, _columns(n), y)
+    x = torch.zeros(2050, k, dtype=torch.bfloat16, device="cuda")
+    y = torch.zeros(2050, n, dtype=torch.float16, device="cuda")
+    assert lib.bw_qlinear_ws(x.data_ptr(), 1, 2050, k, k, d[0].data_ptr(), d[1].data_ptr(), d[2].data_ptr(), None, n, bits, g, y.data_ptr(), n, None, 0, stream) == -5
