@@ -105,12 +105,14 @@ BatchCost batch_search(int64_t M, int64_t N, int64_t K, int bits, int group, boo
 // are of float16 x; bfloat16 costs this kernel 4 % and the prefill kernel a cast (3.2 us and 0.5 us per million values).  Both types take
 // one route, so that a bfloat16 x and its float16 rounding give the same bits: half of both is added.  A doubtful call of up
 // to 128 rows stays here (1.06: in eager code the prefill kernel's cast is one launch more, and an MLP that takes 92 us here takes 95 ...
-// 98 there), one beyond 512 with the prefill kernel (0.95).  On 15500 calls of 17 ... 1500 rows the choice loses 0.3 % against the better of the two;
-// they take 0.958 of the time they took with two sets of x, three column tiles and no order by XCD, and 38 of them 5 % or more longer.
+// 98 there).  No allowance beyond: near the line both models are 2 ... 10 % high, this one more, and 760 calls of 513 ... 2048 rows that a
+// factor of 0.95 sends to the prefill kernel take 0.955 (float16) and 0.887 (bfloat16) of its time here (weights out of HBM); with 1.04 as
+// many calls would lose as gain with float16 x.  Against the lines of two sets of x and three column tiles: 7978 calls within 15 % of the
+// line, 74 with float16 and 78 with bfloat16 x 5 % and more longer (0.95 beyond 512 rows: 132 and 270).
 bool batch_ahead(int64_t M, int64_t N, int64_t K, int bits, int group, float us) {
     if (M <= 64) return true;
     const float half_cast = 1.6f + 0.25e-6f * (float)M * (float)K, prefill = bw_qgemm_expected_us(M, N, K, bits, group) + half_cast;
-    return 1.035f * us < (M <= 128 ? 1.06f : M <= 512 ? 1.f : 0.95f) * prefill;
+    return 1.035f * us < (M <= 128 ? 1.06f : 1.f) * prefill;
 }
 
 BatchCost batch_cost(int64_t M, int64_t N, int64_t K, int bits, int group, bool may_split) {
