@@ -655,25 +655,27 @@ inline DgradPlan dgrad256_plan(int64_t M, int64_t N, int64_t K, bool have_worksp
 
 // The stepping kernel's tile height and slices of N, by predicted time.  A step is bound by its own chain (weight words ->
 // LDS -> transposed reads -> MFMAs -> barrier), not by memory: 0.41 us alone on a CU, 0.65 / 0.88 with two / three
-// workgroups (128-row tiles; 0.67 / 1.03 with one / two of 256 rows), so co-resident workgroups pay - 2.1 times the
+// workgroups (128-row tiles; 0.67 / 1.03 with one / two of 256 rows), so co-resident workgroups pay - 1.4 times the
 // throughput at three - and a launch lasts as long as the CU with the most of them.  Counted that way two slices too many
-// cost more than a few idle CUs: 20 CUs with a second workgroup make the rest wait for a second set of steps.  Beside the
-// steps: a workgroup's prologue and epilogue, and for slices the second launch and the partial tiles (0.29 us per MB
-// written and read, 0.11 us per slice read one behind the other).  128-row tiles dequantise a weight twice as often per
-// MFMA, which long launches pay in clock rate (up to 12 %).
+// cost more than a few idle CUs: 20 CUs with a second workgroup make the rest wait for a second set of steps.  Steps count in
+// twos, as the loop takes them (a slice of 7 takes as long as one of 8: counted singly, 21 rows of 1024 <- 5120 ran 23 slices of 7,
+// 11.7 us, where 20 of 8 take 10.5).  Beside the steps: a workgroup's prologue and epilogue, and for slices the second launch and
+// the partial tiles (0.29 us per MB written and read, 0.11 us per slice read one behind the other).  128-row tiles dequantise a
+// weight twice as often per MFMA, which long launches pay in clock rate (up to 12 %).
 // Fitted on 113184 timings of 16303 calls (1 ... 2048 rows, layers of 512 ... 14336 on either side, all formats, ragged
-// sizes; the order of plans hardly depends on type and bits).  Against two workgroups per CU where a slice keeps 24 steps,
-// else one with 8, and 256-row tiles beyond 512 rows, calls take 0.888 of the time on average (the best plan of each:
-// 0.876), 0.82-0.84 beyond 512 rows and 0.88 up to 16; 1.3 % of them take over 5 % longer.  W4 g64, float16: 333 rows of
-// 3001 -> 2880 27.9 -> 22.4 us (276 workgroups of 4 slices: now 207 of 3), 333 of 1000 -> 8192 26.9 -> 18.1 (unsliced),
-// 700 of 1100 -> 1088 17.9 -> 15.2 (128-row tiles), 128 of 8000 -> 1024 17.9 -> 15.8 (24 slices instead of 16).
+// sizes; the order of plans hardly depends on type and bits).  On 11051 other calls of 1 ... 512 rows its choice loses 1.0 % against the
+// best of up to 14 plans (2.3 % with steps counted singly).  Against two workgroups per CU where a slice keeps 24 steps, else one with
+// 8 (the calls whose plans both were timed): 0.83 of the time up to 4 rows, 0.87 up to 16, 0.91 from 33 on; 62 of 8411 take over 5 %
+// longer, 110 with steps counted singly.  W4 g64, float16, us (graphs): 333 rows of 3001 -> 2880 28.5 -> 22.7 (276
+// workgroups of 4 slices: now 207 of 3), 333 of 1000 -> 8192 27.5 -> 19.0 (unsliced), 700 of 1100 -> 1088 19.6 -> 16.2 (128-row tiles),
+// 128 of 8000 -> 1024 18.1 -> 15.5 (21 slices instead of 28).
 struct DgradSearch {
     static constexpr int MAX_SPLITS = 32;
     static float us(int mt, int tiles, int splits, int steps, int64_t M, int cus) {
         const int DM = 32 * mt, slots = mt == 4 ? 3 : 2;
         const int per_cu = (int)(((int64_t)tiles * splits + cus - 1) / cus);      // workgroups of the busiest CU
         auto step = [&](int resident) { return mt == 4 ? 0.177f + 0.235f * resident : 0.313f + 0.359f * resident; };
-        float t = steps * ((per_cu / slots) * step(slots) + (per_cu % slots ? step(per_cu % slots) : 0.f));
+        float t = (steps + steps % 2) * ((per_cu / slots) * step(slots) + (per_cu % slots ? step(per_cu % slots) : 0.f));
         if (mt == 4) t *= 1.f + 0.12f * (t < 300.f ? t / 300.f : 1.f);
         t += (mt == 4 ? 0.66f : 1.f) * per_cu;
         if (splits > 1) t += 2.2f + 0.11f * splits + 0.285e-6f * ((float)tiles * splits * (M < DM ? M : DM) * DK * 4);

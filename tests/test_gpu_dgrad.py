@@ -354,7 +354,7 @@ def test_dgrad_infinite_gradients_of_a_ragged_n(n, m):
     (333, 1000, 8192, 128, 1),      # 192 tiles: a second slice would give half the CUs a second workgroup
     (333, 3001, 2880, 128, 3),      # 69 tiles, the last column half empty; the last slice ends within a step of 32 rows
     (128, 8000, 1024, 128, 21),     # 8 tiles of 250 steps
-    (700, 1100, 1088, 128, 4),      # the shorter tiles beyond 512 rows
+    (700, 1100, 1088, 128, 3),      # the shorter tiles beyond 512 rows
     (411, 5728, 4160, 256, 7),      # the taller tiles below, the last column half empty
 ])
 def test_dgrad_plan_of_tiles_and_slices(m, n, k, rows, slices):

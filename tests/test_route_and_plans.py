@@ -1,4 +1,5 @@
-"""Host side of bw_qlinear_ws, without a GPU: the memory of searched plans, the choice between the batch and the prefill kernel."""
+"""Host side of bw_qlinear_ws and bw_qdgrad, without a GPU: the memory of searched plans, the choice between the batch and the prefill kernel,
+slices of the input gradient."""
 import os
 import subprocess
 
@@ -78,3 +79,17 @@ def test_route_takes_the_faster_kernel(k, n, m, bits, g, batch, prefill):
     need = hip_loader.load().bw_qlinear_workspace_bytes
     takes_prefill = need(m, n, k, bits, g, hip_loader.BW_BF16) > need(m, n, k, bits, g, hip_loader.BW_F16)
     assert takes_prefill == (prefill < batch)
+
+
+@pytest.mark.skipif(torch.cuda.is_available(), reason="the plan for 256 compute units, what the library assumes without a GPU")
+@pytest.mark.parametrize("m,n,k,slices", [
+    (21, 5120, 1024, 20), (10, 4096, 1536, 16), (19, 2304, 2816, 9), (30, 1024, 4288, 6), (48, 1216, 5376, 5), (39, 2048, 2048, 11)])
+def test_input_gradient_slices_are_whole_passes(m, n, k, slices):
+    """The stepping kernel takes its steps of 32 rows of N in twos, so slices of an odd number of steps are not worth their number: 23 of 7
+    instead of 20 of 8 steps cost 11 %."""
+    from bitween_amd.kernels import hip_loader
+    lib = hip_loader.load()
+    assert lib.bw_qdgrad_tile_rows(m, n, k, 4, 64) == 128
+    need = lib.bw_qdgrad_workspace_bytes(m, n, k, 4, 64)
+    assert need == -(-k // 128) * slices * 128 * 128 * 4
+    assert -(-(-(-n // 32)) // slices) % 2 == 0
