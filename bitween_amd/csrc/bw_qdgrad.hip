@@ -262,7 +262,7 @@ __global__ __launch_bounds__(DTHREADS, MT == 4 ? 3 : 2) void qdgrad_kernel(const
         // Masked by hand the stores were there twice, for every launch to fetch: 97 rows of N = 1024, K = 10624 at 4 bits 22.6 us, 21.0 this way,
         // 756 of N = 1216, K = 1024 at 8 bits 19.3 and 18.5.  The i loop outside: neighbouring stores to the two halves of a line take 1 us
         // longer.
-        const __amdgpu_buffer_rsrc_t rd = __builtin_amdgcn_make_buffer_rsrc(a.ws + (size_t)blockIdx.x * (DM * DK), (short)0, min(a.M - m0, DM) * (DK * 4), 0x00020000);
+        const __amdgpu_buffer_rsrc_t rd = __builtin_amdgcn_make_buffer_rsrc(a.ws + (size_t)blockIdx.x * (min(a.M, DM) * DK), (short)0, min(a.M - m0, DM) * (DK * 4), 0x00020000);
         const uint32_t off = ((wm + l16) * DK + wk + 4 * q) * 4;
         const int rows = __builtin_amdgcn_readfirstlane(a.M - m0 - wm);   // of this wave; pieces of 16 without any are not asked for
 #pragma unroll
@@ -294,17 +294,18 @@ __global__ __launch_bounds__(256) void qdgrad_reduce_kernel(const DgradArgs a) {
     const int ml = quad / (DKT / 4), kl = (quad % (DKT / 4)) * 4;
     const int m = (tile / a.tiles_k) * DM + ml, k = (tile % a.tiles_k) * DKT + kl;
     if (m >= a.M || k >= a.K) return;
-    const float* src = a.ws + (size_t)tile * a.splits * (DM * DKT) + ml * DKT + kl;
+    const int part = min(a.M, DM) * DKT;                              // values of a partial tile: a call of fewer rows than a tile has no room for the rest
+    const float* src = a.ws + (size_t)tile * a.splits * part + ml * DKT + kl;
     f4 v = {0.f, 0.f, 0.f, 0.f};
     int z = 0;
     for (; z + 4 <= a.splits; z += 4) {                               // four reads in flight: one memory round trip, not four
         f4 t[4];
 #pragma unroll
-        for (int e = 0; e < 4; e++) t[e] = *reinterpret_cast<const f4*>(src + (size_t)(z + e) * (DM * DKT));
+        for (int e = 0; e < 4; e++) t[e] = *reinterpret_cast<const f4*>(src + (size_t)(z + e) * part);
 #pragma unroll
         for (int e = 0; e < 4; e++) v += t[e];
     }
-    for (; z < a.splits; z++) v += *reinterpret_cast<const f4*>(src + (size_t)z * (DM * DKT));
+    for (; z < a.splits; z++) v += *reinterpret_cast<const f4*>(src + (size_t)z * part);
     *reinterpret_cast<u2*>(a.gx + (int64_t)m * a.ldx + k) = u2{pack2<DT>(v[0], v[1]), pack2<DT>(v[2], v[3])};
 }
 
@@ -555,7 +556,7 @@ __global__ __launch_bounds__(256) void qdgrad256_kernel(const DgradArgs a) {
     }
     // acc[i][j][r] = grad_x[m0 + 16 i + nl][k0 + 64 wave + 16 j + 4 kq + r]
     if (a.splits > 1) {
-        float* dst = a.ws + (size_t)blockIdx.x * (QMv * QK) + 64 * wave + 4 * kq;
+        float* dst = a.ws + (size_t)blockIdx.x * (min(a.M, QMv) * QK) + 64 * wave + 4 * kq;
 #pragma unroll
         for (int i = 0; i < MT; i++) {
             if (m0 + 16 * i + nl >= a.M) continue;
@@ -649,7 +650,7 @@ inline DgradPlan dgrad256_plan(int64_t M, int64_t N, int64_t K, bool have_worksp
     if (s < 2) return p;
     p.splits = s;
     p.steps_per_split = sps;
-    p.ws_bytes = (size_t)p.tiles * s * qm * QK * sizeof(float);
+    p.ws_bytes = (size_t)p.tiles * s * (M < qm ? M : qm) * QK * sizeof(float);
     return p;
 }
 
@@ -699,7 +700,7 @@ struct DgradSearch {
                 if (p.splits != s) continue;                                     // the same slices as a smaller s
                 const float t = us(mt, p.tiles, s, p.steps_per_split, M, cus);
                 if (best_us > 0.f && t >= best_us) continue;
-                p.ws_bytes = s > 1 ? (size_t)p.tiles * s * DM * DK * sizeof(float) : 0;
+                p.ws_bytes = s > 1 ? (size_t)p.tiles * s * (M < DM ? M : DM) * DK * sizeof(float) : 0;   // rows past M have no place
                 best = p;
                 best_us = t;
             }

@@ -380,3 +380,25 @@ def test_dgrad_plan_of_tiles_and_slices(m, n, k, rows, slices):
         gx = torch.empty((m, k), dtype=torch.float16, device="cuda")
         assert lib.bw_qdgrad(go.data_ptr(), 0, m, n, n, d[0].data_ptr(), d[1].data_ptr(), d[2].data_ptr(), k, bits, g, gx.data_ptr(),
                              k, ws.data_ptr(), ws.numel() - 4, ctypes.c_void_p(torch.cuda.current_stream().cuda_stream)) == -5
+
+
+@pytest.mark.parametrize("bits,g,m,n,k", [(4, 64, 1, 4096, 512), (8, 32, 8, 8752, 4864), (4, 128, 17, 3001, 1152), (2, 64, 127, 5000, 640),
+                                          (4, 128, 101, 14336, 4096)])
+def test_partial_tiles_of_few_rows(bits, g, m, n, k):
+    """Calls of fewer rows than a tile: a slice's partial tile is the call's rows and no more (the last: of the 256 x 256 kernel), so the next
+    slice's begins where they end; nothing is written beyond the workspace that the query names."""
+    from bitween_amd.kernels import hip_loader
+    lib = hip_loader.load()
+    need = lib.bw_qdgrad_workspace_bytes(m, n, k, bits, g)
+    assert need > 0 and need % (m * 128 * 4) == 0
+    _, qw, s16, z16, _ = quantized_layer(n, k, bits, g, seed=n + k, outliers=True, bias=False)
+    d = [to_gpu(a) for a in (qw, s16, z16)]
+    go16 = np.random.default_rng(m).standard_normal((m, n)).astype(np.float16)
+    go = to_gpu(go16)
+    ws = torch.full((need + 4096,), 85, dtype=torch.uint8, device="cuda")
+    gx = torch.full((m, k), 7.0, dtype=torch.float16, device="cuda")
+    st = lib.bw_qdgrad(go.data_ptr(), 0, m, n, n, d[0].data_ptr(), d[1].data_ptr(), d[2].data_ptr(), k, bits, g, gx.data_ptr(), k,
+                       ws.data_ptr(), need, ctypes.c_void_p(torch.cuda.current_stream().cuda_stream))
+    torch.cuda.synchronize()
+    assert st == 0 and (ws[need:] == 85).all()
+    _check(gx, go16, qw, s16, z16, bits, g)

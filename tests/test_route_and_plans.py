@@ -91,5 +91,5 @@ def test_input_gradient_slices_are_whole_passes(m, n, k, slices):
     lib = hip_loader.load()
     assert lib.bw_qdgrad_tile_rows(m, n, k, 4, 64) == 128
     need = lib.bw_qdgrad_workspace_bytes(m, n, k, 4, 64)
-    assert need == -(-k // 128) * slices * 128 * 128 * 4
+    assert need == -(-k // 128) * slices * m * 128 * 4                        # a partial tile is the call's m rows
     assert -(-(-(-n // 32)) // slices) % 2 == 0
