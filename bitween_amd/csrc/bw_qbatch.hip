@@ -140,7 +140,14 @@ enum Route { kDecode, kBatch, kPrefill };
 // every CU has one decode workgroup, 0.85 ... 1.1 at K > 8192 and 1.0 ... 1.5 below, of that up to 3/4 CUs at 2 bits 0.72 ... 1.06 (W4 g64 at K
 // > 11008 0.84 ... 1.05), beyond 0.95 ... 1.07 (1.02 ... 1.15) until the rows are long: W2 g64 12800 0.94 ... 1.0, 14336 0.80 ... 0.87, W4 g64
 // 14336 0.83 ... 1.01; at 8 bits CUs ... 2 CUs tiles 0.67 ... 0.97 for K > 3072, 5 ... 8 rows 0.9 ... 1.1.  Layers of 8 bits in groups of
-// 64 keep the lines they had: their decode kernels scale a group's sum in float32, this kernel rounds every weight.
+// 64 with up to 3 CUs tiles keep the line they had, as their decode kernels scale a group's sum in float32 and this kernel rounds every
+// weight; beyond 3 CUs, where all of their calls of 5 rows and more were this kernel's, the wide line gave some back.
+// The timings above are graphs.  In eager code the cut costs the host an allocation and a second launch, 8.1 us a call against 6 ... 7, so a
+// narrow layer's line lies where the decode kernels take that long (this kernel's time over theirs in a loop of eager calls, and in a
+// graph, tiles <= CUs / 2): W2 9 ... 16 rows K = 8192 1.16 ... 1.28 (0.85 ... 0.99), 9216 0.90 ... 0.98 (0.69 ... 0.82); W4 g128 9216 1.05 ...
+// 1.17 (0.83 ... 0.98), 11264 0.85 ... 1.04 (0.77 ... 0.90); W8 g32 6400 0.86 ... 1.12 (0.82 ... 0.94), 7168 0.81 ... 1.06 (0.79 ... 0.90); 5 ... 8
+// rows W2 g64 12288 1.12 ... 1.20 (0.84 ... 1.04), 12800 0.95 ... 1.02 (0.76 ... 0.95); W4 g64 11264 0.99 ... 1.17 (0.88 ... 1.0), 12288 0.88 ... 1.05
+// (0.75 ... 0.89); W4 g32 9216 0.97 ... 1.10 (0.78 ... 0.93), 10240 0.90 ... 1.06 (0.79 ... 0.89).
 inline bool batch_takes_decode_rows(int64_t M, int64_t N, int64_t K, int bits, int group) {
     const int64_t tiles = (N + 15) / 16, cus = bw_device_cus();
     const bool many = M > 8, narrow = tiles <= cus / 2;
@@ -150,14 +157,15 @@ inline bool batch_takes_decode_rows(int64_t M, int64_t N, int64_t K, int bits, i
         if (group == 64) return many && K >= 8192;
         if (tiles > 2 * cus) return many && K > 6144;
         if (tiles > cus) return many && K > 3072;
-        if (narrow) return K > (many ? group == 32 ? 6144 : 8191 : group == 32 ? 8192 : 11008);
+        if (narrow) return K > (many ? group == 32 ? 6400 : 8191 : group == 32 ? 8192 : 11008);
         return many && K > (group == 32 ? 8192 : 11008);
     }
     if (K > 4096 ? tiles > cus : K >= 3072 && tiles > 4 * cus) return true;
     if (many && tiles > 3 * cus && (group == 32 || K / group % 2 || K <= (group == 64 ? 3072 : 2048))) return true;
     if (many && group == 32) return K > 4096 || (tiles > cus && tiles <= 2 * cus);
     if (K <= 4096) return false;
-    if (narrow) return many ? K > 6144 : group != 128 && K > (group == 32 ? 8192 : 11008);
+    if (narrow && many) return K > (bits == 2 ? 8192 : group == 128 ? 10240 : 6144);
+    if (narrow) return group != 128 && K > (bits == 2 ? 12288 : group == 32 ? 9216 : 11264);
     const bool full = 4 * tiles > 3 * cus && K / group % 2 == 0;
     return many && (bits == 2 ? K > (!full ? 8192 : group == 64 ? 12288 : 13312) : group == 64 && K > (full ? 13312 : 11008));
 }

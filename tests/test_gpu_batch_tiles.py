@@ -111,9 +111,11 @@ def test_padded_rows_in_the_order_by_xcd(bits, g, m, n, k, ldx):
 
 
 @pytest.mark.parametrize("bits,g,k,n,m,kernel", [
-    (4, 128, 6272, 2048, 9, "qbatch"), (4, 128, 6144, 2048, 16, "qgemv"), (4, 128, 6272, 2048, 8, "qgemv"), (4, 128, 6272, 2064, 16, "qgemv"),
+    (4, 128, 10368, 2048, 9, "qbatch"), (4, 128, 10240, 2048, 16, "qgemv"), (4, 128, 10368, 2048, 8, "qgemv"), (4, 128, 10368, 2064, 16, "qgemv"),
     (4, 128, 4224, 4112, 5, "qbatch"), (4, 128, 4096, 4112, 16, "qgemv"), (4, 64, 11072, 2064, 9, "qbatch"), (4, 64, 11008, 2064, 9, "qgemv"),
-    (4, 32, 544, 4112, 9, "qbatch"), (4, 32, 544, 4096, 9, "qgemv"), (4, 32, 8224, 640, 5, "qbatch"), (2, 128, 8320, 2064, 12, "qbatch"),
+    (4, 32, 544, 4112, 9, "qbatch"), (4, 32, 544, 4096, 9, "qgemv"), (4, 32, 9248, 640, 5, "qbatch"), (4, 32, 9216, 640, 5, "qgemv"), (4, 64, 11328, 512, 5, "qbatch"), (4, 64, 11264, 512, 8, "qgemv"),
+    (2, 64, 12352, 512, 5, "qbatch"), (2, 64, 12288, 512, 8, "qgemv"), (2, 64, 8256, 1024, 9, "qbatch"), (2, 128, 8192, 1024, 16, "qgemv"),
+    (8, 32, 6432, 1024, 9, "qbatch"), (8, 32, 6400, 1024, 9, "qgemv"), (2, 128, 8320, 2064, 12, "qbatch"),
     (4, 128, 1024, 12304, 9, "qbatch"), (4, 128, 4096, 12304, 9, "qgemv"), (4, 128, 3968, 12304, 9, "qbatch"),
     (2, 128, 8448, 4096, 9, "qgemv"), (2, 128, 8320, 4096, 9, "qbatch"),
     (2, 64, 12288, 4096, 9, "qgemv"), (2, 64, 12416, 4096, 9, "qbatch"), (4, 64, 13312, 4096, 9, "qgemv"), (4, 64, 13440, 4096, 9, "qbatch"),
