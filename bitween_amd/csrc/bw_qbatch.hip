@@ -50,7 +50,9 @@ inline int batch_mt(int64_t M) { const int t = (int)((M + 15) / 16); return t <=
 // best on average).  A round costs 0.20 MT + (0.39 + 0.16 at 8 bits) NTW us, of 256 values (MT > 4) 0.13 MT + (0.29 - 0.01 MT + 0.05 at 8 bits)
 // NTW; every wave of workgroups (0.01 + 0.25 NTW) MT or (0.04 + 0.19 NTW) MT more, a launch 2.5 ... 3, a cut of K the reduction: 2 us and
 // 1.5 us per million partial sums.  Four column tiles a wave halve the LDS traffic of 8 x 2 tiles for the same outputs: W4 g128 us, 128 rows of 4096
-// -> 14336 float16 27.7 -> 25.6, bfloat16 30.2 -> 26.0; 14336 -> 4096 32.0 -> 28.5 - not at 8 bits, where their weights spill (59 ... 126 registers).
+// -> 14336 float16 27.7 -> 25.6, bfloat16 30.2 -> 26.0; 14336 -> 4096 32.0 -> 28.5.  Not built at 8 bits: in
+// 64-row tiles their weights spill 59 ... 135 registers; lower ones spill none (48 rows in groups of 32: 10 ... 13) and have not been timed.  Of the tiles
+// that are, W4 g32 4 x 4 spills 12, W4 g64 4, W8 6 x 3 8 ... 12; the fit has their timings.
 //
 // Lower tiles than the call has rows read the weights (out of L2) once per tile, but fill the chip without a cut of K and its
 // reduction: W4 g128 us, one tile of rows against the plan, 2048 x 2048 at 64 rows 8.5 -> 5.3, at 128 rows 11.4 -> 6.3; 4096 x 4096 at

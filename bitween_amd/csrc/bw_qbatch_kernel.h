@@ -432,7 +432,7 @@ int launch_qbatch_bits(int group, int mt, int ntw, const BatchArgs& a, hipStream
 #define BW_WIDE(G) BW_CASE(G, 1, 4) BW_CASE(G, 2, 4) BW_CASE(G, 3, 4) BW_CASE(G, 4, 4)
 #define BW_GROUP(G) BW_ROWS(G, 1) BW_ROWS(G, 2) BW_ROWS(G, 3) BW_ROWS(G, 4) BW_CASE(G, 6, 1) BW_CASE(G, 6, 2) BW_CASE(G, 6, 3) BW_CASE(G, 8, 1) BW_CASE(G, 8, 2)
     BW_GROUP(128) BW_GROUP(64) BW_GROUP(32)
-    if constexpr (BITS != 8) {                                // (at 8 bits four column tiles' weights spill)
+    if constexpr (BITS != 8) {                                // (at 8 bits 64-row tiles of them spill 59 ... 135 registers)
         BW_WIDE(128) BW_WIDE(64) BW_WIDE(32)
     }
 #undef BW_WIDE
