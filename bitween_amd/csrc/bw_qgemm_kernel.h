@@ -136,6 +136,22 @@ BW_DEV void lds_read_b128(h8& dst, uint32_t addr) {
     asm volatile("ds_read_b128 %0, %1 offset:%2" : "=v"(dst) : "v"(addr), "n"(OFF));
 }
 
+// LDS operations of a wave younger than the read of slot S's activation fragment when slot S begins: a K step starts with the reads of
+// its first RING slots; every slot then ends with the read of slot S + RING, and with PW > 0 the first slot of each of the four regions of an
+// MFMA step (MT slots) hands over PW words before that.  The words a slot's unpack takes were handed over one MFMA step earlier and
+// have to be there too.  At most what the counter can express: a smaller number waits for more.
+template <int RING, int SLOTS, int MT, int PW>
+constexpr int frag_younger(int S) {
+    int n = S < RING ? RING - 1 - S : 0;
+    for (int q = S < RING ? 0 : S - RING + 1; q < S; q++) n += (q + RING < SLOTS ? 1 : 0) + (q % (MT / 4) == 0 ? PW : 0);
+    if (PW && S >= MT) {
+        int m = 0;
+        for (int q = S - MT; q < S; q++) m += (q + RING < SLOTS ? 1 : 0) + (q > S - MT && q % (MT / 4) == 0 ? PW : 0);
+        n = n < m ? n : m;
+    }
+    return n < 15 ? n : 15;
+}
+
 BW_DEV void tile_coords(int tile, const GemmArgs& a, int& tm, int& tn) {
     const int per_panel = a.panel * a.tiles_n;
     const int p = tile / per_panel, within = tile - p * per_panel;
@@ -169,6 +185,14 @@ __global__ __launch_bounds__(WAVES * 64) void qgemm_kernel(const GemmArgs a) {
     // 60.5 -> 55.7).  Not at larger groups (an odd number of them), where several lanes share a scale anyway and it gained
     // nothing, and not with 256-row tiles: their step has twice the MFMAs for the same requests, and no register to spare.
     constexpr bool QMETA = NAT && !META4 && GROUP == 32 && MT <= 8;
+    // QW: weights, too, are asked for four lanes to a row, and the words of an MFMA step are handed to the lanes that multiply them by
+    // ds_bpermute one step ahead.  A K step's 8 requests a wave at 8 bits were 1920 address-unit cycles a CU of the 2048 that the MFMAs of
+    // a 128-row tile take, next to 512 for x and, at groups of 32, 512 for the scales; now 512.  us, out of HBM: W8 g32 4096 -> 11008 at 64 / 333 /
+    // 509 rows 26.2 -> 24.5, 57.8 -> 53.5, 59.5 -> 55.1, 11008 -> 4096 at 509 60.7 -> 58.7; g64 4096 -> 11008 at 509 59.6 -> 56.5; g128 (one
+    // request for the scales of four steps) 51.2 -> 50.9.  Not at 4 and 2 bits, half as many requests: the handing over costs what it
+    // saves (W4 g128 46.1 -> 47.3, g32 51.3 -> 52.1, W2 g128 45.8 -> 47.3); not with 256-row tiles, twice the MFMAs and no registers.
+    constexpr bool QW = NAT && MT <= 8 && BITS == 8;
+    constexpr int PW = BITS == 8 ? 2 : 1;                        // QW: words of a tile an MFMA step multiplies
     constexpr uint32_t kOob = 0x80000000u;
     extern __shared__ __attribute__((aligned(16))) char smem[];
 #ifdef BW_TUNE
@@ -197,7 +221,8 @@ __global__ __launch_bounds__(WAVES * 64) void qgemm_kernel(const GemmArgs a) {
         const int row = n0 + 16 * j + nl;
         // (256-row tiles add a scalar chunk offset that is itself "out of range" past the last chunk: rows past N then
         // read the last row's bytes instead of relying on a sum that could wrap; their outputs are never stored)
-        w_off[j] = row < a.N ? (uint32_t)row * a.row_bytes + kq * C::LB * C::WL : NAT ? (uint32_t)(a.N - 1) * a.row_bytes + kq * C::LB * C::WL : kOob;
+        if constexpr (QW) w_off[j] = (uint32_t)min(n0 + 16 * j + (lane >> 2), a.N - 1) * a.row_bytes + (lane & 3) * C::LB * C::WL;
+        else w_off[j] = row < a.N ? (uint32_t)row * a.row_bytes + kq * C::LB * C::WL : NAT ? (uint32_t)(a.N - 1) * a.row_bytes + kq * C::LB * C::WL : kOob;
         m_off[j] = (uint32_t)min(QMETA ? n0 + 16 * j + (lane >> 2) : row, a.N - 1) * groups * 2;
     }
     // 128-row tiles: byte offsets of the staging units of a thread
@@ -262,6 +287,13 @@ __global__ __launch_bounds__(WAVES * 64) void qgemm_kernel(const GemmArgs a) {
     auto issue_meta4 = [&](int j, int which, int c, u2 (*m)[2]) {
         m[j][which] = __builtin_amdgcn_raw_buffer_load_b64(which == 0 ? rs : rz, m_off[j] + c * (2 * C::GPS), 0, 0);
     };
+    // The lane's packed word e of MFMA step t.
+    auto word_of = [&](const WSet& ws, int j, int t, int e) -> uint32_t {
+        if constexpr (BITS == 8) return ws.w[j][t / C::SPL][2 * (t % C::SPL) + e];
+        else return ws.w[j][0][BITS == 4 ? t : t / 2];
+    };
+    // QW: the words of MFMA step t, in pw[(t + 1) & 1]: handed over during step t - 2, unpacked during step t - 1
+    uint32_t pw[2][NT][PW];
     // Weight fragment of MFMA step t: values [8 t, 8 t + 8) of the lane's VPL, from lane load t / SPL.
     auto unpack = [&](const WSet& ws, int j, int t, const auto* gcj) {
         static_assert(C::WL == 1 || C::NG == 1, "two lane loads share one group");
@@ -298,7 +330,7 @@ __global__ __launch_bounds__(WAVES * 64) void qgemm_kernel(const GemmArgs a) {
     h8 xf[C::XSETS][C::XRING];
     h2 wf[2][NT][4];                                      // weight fragments as 4 register pairs each
     uint32_t pm[NT];                                      // QMETA: (scale | zero point << 16) of the lane's row and values
-    const uint32_t pm_from = (uint32_t)(((nl << 2) | kq) << 2);
+    const uint32_t pm_from = (uint32_t)(((nl << 2) | kq) << 2);   // QMETA, QW: the lane that asked for what this one multiplies
     // group constants of tile j for the step that reads `from` (META4: half `half` of m_cur / m_next)
     auto set_consts = [&](GC* gj, int j, const WSet& from, const u2 (*m)[2], int half) {
 #pragma unroll
@@ -441,8 +473,8 @@ __global__ __launch_bounds__(WAVES * 64) void qgemm_kernel(const GemmArgs a) {
     // reading one slot then spreads over all banks (rows are 256 bytes apart: unswizzled they would share 4 banks).
     // The fragment reads are written as assembly: the compiler orders every LDS read it knows of behind all pending
     // loads with LDS destination, and would so wait for the next chunk before reading this one.  It does not track
-    // assembly results either, so the waits are here too: fragment reads complete in order and nothing else uses LDS
-    // in the loop, so before slot S of a K step (S = 16 t + i) at most 7 - max(0, S - 56) younger reads are in flight.
+    // assembly results either, so the waits are here too: LDS operations complete in order, and before a slot begins at most
+    // frag_younger(slot) operations younger than its fragment's read may be in flight (QMETA's are not counted, which waits for more).
     // Request addresses are one VGPR per thread plus a scalar: the chunk part of an offset is uniform, and past the
     // slice it is replaced by an offset beyond every buffer, so that the hardware's range check returns zeros.
     // Requires K % CHUNK_K == 0 (the launcher's condition for this variant): no request straddles the end of a row.
@@ -500,9 +532,9 @@ __global__ __launch_bounds__(WAVES * 64) void qgemm_kernel(const GemmArgs a) {
                 // RG gaps (SLOTS slots) per region: 16 (4) with 256-row tiles, 8 (2) with 128-row tiles
                 constexpr int RG = 4 * MT / NT, SLOTS = RG / 4;
                 constexpr int g = decltype(gcnt)::value, i = g / NT, j = g % NT, r = g / RG, k = g % RG;
-                constexpr int S = MT * t + i, SLAST = MT * C::MF - 1 - C::XRING;          // SLAST: the last slot that issues a fragment read
+                constexpr int S = MT * t + i;
                 __builtin_amdgcn_sched_barrier(0);
-                if constexpr (j == 0) __builtin_amdgcn_s_waitcnt(0xC07F | ((C::XRING - 1 - (S > SLAST + 1 ? S - SLAST - 1 : 0)) << 8));
+                if constexpr (j == 0) __builtin_amdgcn_s_waitcnt(0xC07F | (frag_younger<C::XRING, MT * C::MF, MT, QW ? PW : 0>(S) << 8));
                 mfma_acc(acc[i][j], pack_h8(wf[cu][j]), xf[0][(MT * t + i) % C::XRING]);
                 __builtin_amdgcn_sched_barrier(0);
                 // ---- unpack of n-tile r: instruction v of its sequence ----
@@ -510,7 +542,7 @@ __global__ __launch_bounds__(WAVES * 64) void qgemm_kernel(const GemmArgs a) {
                 auto unpack_op = [&](auto vc) {
                     constexpr int v = decltype(vc)::value;
                     if constexpr (BITS == 4) {
-                        const uint32_t word = src.w[r][0][tt];
+                        const uint32_t word = QW ? pw[cu][r][0] : word_of(src, r, tt, 0);
                         if constexpr (v == 0) pq[r][0] = __builtin_amdgcn_perm(word, word, 0x01000100u);
                         if constexpr (v == 1) pq[r][1] = __builtin_amdgcn_perm(word, word, 0x03020302u);
                         if constexpr (v == 2) up[r][0] = as_h2(and_or(pq[r][0], 0x00F0000Fu, kMagic));
@@ -523,7 +555,7 @@ __global__ __launch_bounds__(WAVES * 64) void qgemm_kernel(const GemmArgs a) {
                         if constexpr (v >= 12) wf[nx][r][v - 12] = up[r][v - 12] * gr.s;
                     } else if constexpr (BITS == 2) {
                         // half-word tt of the lane's 8 bytes
-                        const uint32_t word = src.w[r][0][tt / 2];
+                        const uint32_t word = QW ? pw[cu][r][0] : word_of(src, r, tt, 0);
                         if constexpr (v == 0) pq[r][0] = tt % 2 ? __builtin_amdgcn_perm(word, word, 0x03020302u) : __builtin_amdgcn_perm(word, word, 0x01000100u);
                         if constexpr (v == 1) uw[r] = pq[r][0] >> 8;
                         if constexpr (v == 2) up[r][0] = as_h2(and_or(pq[r][0], 0x000C0003u, kMagic));
@@ -534,7 +566,7 @@ __global__ __launch_bounds__(WAVES * 64) void qgemm_kernel(const GemmArgs a) {
                         if constexpr (v >= 10 && v < 14) wf[nx][r][v - 10] = up[r][v - 10] * gr.s;
                     } else {
                         // 8 bits: the two words of MFMA step tt are words 2 (tt % 2), + 1 of lane load tt / 2
-                        const uint32_t w0 = src.w[r][tt / C::SPL][2 * (tt % C::SPL)], w1 = src.w[r][tt / C::SPL][2 * (tt % C::SPL) + 1];
+                        const uint32_t w0 = QW ? pw[cu][r][0] : word_of(src, r, tt, 0), w1 = QW ? pw[cu][r][PW - 1] : word_of(src, r, tt, 1);
                         if constexpr (v == 0) up[r][0] = as_h2(__builtin_amdgcn_perm(0x64646464u, w0, 0x04010400u));
                         if constexpr (v == 1) up[r][1] = as_h2(__builtin_amdgcn_perm(0x64646464u, w0, 0x04030402u));
                         if constexpr (v == 2) up[r][2] = as_h2(__builtin_amdgcn_perm(0x64646464u, w1, 0x04010400u));
@@ -568,6 +600,12 @@ __global__ __launch_bounds__(WAVES * 64) void qgemm_kernel(const GemmArgs a) {
                     const uint32_t pair = wsn.s[r][0] | (wsn.z[r][0] << 16);
                     asm volatile("ds_bpermute_b32 %0, %1, %2" : "=v"(pm[r]) : "v"(pm_from), "v"(pair));
                 }
+                // ---- QW: tile r's words of the MFMA step after next, in the first slot of its region (frag_younger counts them)
+                if constexpr (QW && k >= 1 && k <= PW) {
+                    constexpr int t2 = (t + 2) % C::MF;
+                    const uint32_t word = word_of(t + 2 < C::MF ? ws : wsn, r, t2, k - 1);
+                    asm volatile("ds_bpermute_b32 %0, %1, %2" : "=v"(pw[nx][r][k - 1]) : "v"(pm_from), "v"(word));
+                }
                 // ---- fragment ring ----
                 if constexpr (j == NT - 1) {
                     constexpr int i2 = (i + C::XRING) % MT, t2 = t + (i + C::XRING) / MT;
@@ -588,10 +626,11 @@ __global__ __launch_bounds__(WAVES * 64) void qgemm_kernel(const GemmArgs a) {
                     if constexpr (META4) set_consts(gn[r], r, wsn, ph < C::SPR - 1 ? m_cur : m_next, ph < C::SPR - 1 ? ph + 1 : 0);
                     else set_consts(gn[r], r, wsn, m_cur, 0);
                 }
+                constexpr int T_WREQ = QW ? C::MF - 2 : C::MF - 1;         // the words are handed over (or unpacked) by then
                 if constexpr (SLOTS == 4) {
                     if constexpr (t == C::MF - 1 && j == 1 && sl >= 4 - C::WL) w_req16(r, sl - (4 - C::WL), c + 2, ws);
                 } else {                                                   // two slots: gaps 1 (and 2 at 8 bits) of the second
-                    if constexpr (t == C::MF - 1 && sl == SLOTS - 1 && j >= 1 && j <= C::WL) w_req16(r, j - 1, c + 2, ws);
+                    if constexpr (t == T_WREQ && sl == SLOTS - 1 && j >= 1 && j <= C::WL) w_req16(r, j - 1, c + 2, ws);
                 }
                 asm volatile("" ::: "memory");
             });
@@ -605,6 +644,13 @@ __global__ __launch_bounds__(WAVES * 64) void qgemm_kernel(const GemmArgs a) {
         else if ((META4 && ph != 0)) wait_loads<NT * C::WL>();
         else wait_loads<NT * C::WL + 2 * NT>();
         lds_barrier();
+        // What was handed over keeps its registers until it is there, also in a last step that has no use for it.
+#pragma unroll
+        for (int j = 0; j < NT; j++) {
+            if constexpr (QMETA) asm volatile("" ::"v"(pm[j]));
+#pragma unroll
+            for (int e = 0; e < (QW ? PW : 0); e++) asm volatile("" ::"v"(pw[0][j][e]), "v"(pw[1][j][e]));
+        }
     };
     auto step = [&](int c, _Float16* cur, _Float16* nxt, WSet& ws, const WSet& wsn, GC (&gc)[NT][C::NG], GC (&gn)[NT][C::NG],
                     const int ph, const bool tail = false) {
@@ -711,7 +757,16 @@ __global__ __launch_bounds__(WAVES * 64) void qgemm_kernel(const GemmArgs a) {
     for (int j = 0; j < NT; j++) {
         if constexpr (QMETA) pm[j] = __builtin_amdgcn_ds_bpermute((int)pm_from, (int)(set0.s[j][0] | (set0.z[j][0] << 16)));
         set_consts(gc0[j], j, set0, m_cur, 0);
-        const h8 f = unpack(set0, j, 0, gc0[j]);
+        h8 f;
+        if constexpr (QW) {
+            WSet first;                                           // words of MFMA step 0, and into pw those of step 1
+#pragma unroll
+            for (int e = 0; e < PW; e++) {
+                first.w[j][0][e] = __builtin_amdgcn_ds_bpermute((int)pm_from, (int)word_of(set0, j, 0, e));
+                pw[0][j][e] = __builtin_amdgcn_ds_bpermute((int)pm_from, (int)word_of(set0, j, 1, e));
+            }
+            f = unpack(first, j, 0, gc0[j]);
+        } else f = unpack(set0, j, 0, gc0[j]);
 #pragma unroll
         for (int e = 0; e < 4; e++) wf[0][j][e] = h2{f[2 * e], f[2 * e + 1]};
     }

@@ -222,3 +222,26 @@ def test_prefill_one_to_three_k_steps(bits, g, k):
         w16 = to_gpu(orc.dequantize_f16(qw, s16, z16, g, bits))
         ref = (x @ w16.T).float() + to_gpu(b16).float()
         assert ((y.float() - ref).abs().max() <= 2.0 ** -8 * ref.abs().max()).item()
+
+
+@pytest.mark.parametrize("g", [32, 64, 128])
+@pytest.mark.parametrize("k,n,m", [(128, 301, 20), (640, 300, 64), (256, 17, 65), (384, 513, 130), (768, 301, 200), (1152, 255, 300)])
+def test_prefill_8_bit_words_handed_over_between_lanes(g, k, n, m):
+    """64- and 128-row tiles at 8 bits ask for weights four lanes to a row and hand the words over an MFMA step ahead: one to nine K
+    steps (odd counts run one on zeros), columns past N repeating the last row, a value of every lane and word in its own place."""
+    from bitween_amd.kernels import hip_loader
+    lib = hip_loader.load()
+    _, qw, s16, z16, b16 = quantized_layer(n, k, 8, g, seed=k + n + g, outliers=True)
+    x = np.random.default_rng(m).standard_normal((m, k)).astype(np.float16)
+    d, b = [to_gpu(a) for a in (qw, s16, z16)], to_gpu(b16)
+    st = ctypes.c_void_p(torch.cuda.current_stream().cuda_stream)
+    y = torch.empty((m, n), dtype=torch.float16, device="cuda")
+    assert lib.bw_qgemm(to_gpu(x).data_ptr(), 0, m, k, k, *[t.data_ptr() for t in d], b.data_ptr(), n, 8, g, y.data_ptr(), n, st) == 0
+    check_matmul(y, x, qw, s16, z16, b16, 8, g)
+    # one-hot rows return columns of W16 bit for bit
+    cols = np.linspace(0, k - 1, m).astype(int)
+    hot = np.zeros((m, k), np.float16)
+    hot[np.arange(m), cols] = 1
+    assert lib.bw_qgemm(to_gpu(hot).data_ptr(), 0, m, k, k, *[t.data_ptr() for t in d], None, n, 8, g, y.data_ptr(), n, st) == 0
+    w16 = orc.dequantize_f16(qw, s16, z16, g, 8)
+    assert np.array_equal(y.cpu().numpy(), w16[:, cols].T)
