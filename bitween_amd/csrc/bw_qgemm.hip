@@ -20,11 +20,13 @@
 // Grids that fill the device run the natural-order schedule with 256 x 256
 // tiles (a wave owns 256 x 64: all 256 accumulation registers): every weight
 // is unpacked once for twice the rows.  Which tile height a call gets is
-// gemm_tile_rows(); a short last round of tiles is cut along K (gemm_plan()),
+// gemm_tile(); a short last round of tiles is cut along K (gemm_plan()),
 // and the tiles are numbered so that the workgroups an XCD runs together share
-// operand tiles in its L2 (GemmArgs::panel).
+// operand tiles in its L2 (GemmArgs::panel).  Both heights also come 192 columns
+// wide (a wave owns 48): finer tiles for the grids that 256 columns would fill badly.
 // Also holds the shape-generic fallback used when the fast layouts do not
 // apply (odd K or group size): correct for everything the reference accepts.
+#include "bw_plan_cache.h"
 #include "bw_qgemm_kernel.h"
 
 #include <atomic>
@@ -42,7 +44,9 @@ inline bool gemm_nat(int64_t M, int64_t K, int64_t ldx) {
     return K % 128 == 0 && (M + 256) * ldx * 2 < ((int64_t)1 << 32);
 }
 
-// Rows of a tile for this call.  Calls of at most 64 rows take 64-row tiles: half the MFMAs and half the activation
+struct GemmTile { int rows, cols; };
+
+// Tile of 256 columns for this call.  Calls of at most 64 rows take 64-row tiles: half the MFMAs and half the activation
 // traffic of a 128-row tile that would be at least half padding (17 ... 64 rows on the five Llama MLP / attention shapes at
 // 4 bits: 0.84-0.95 of the 128-row time, same bits).  A 256-row tile unpacks every weight once for twice the rows and keeps the matrix pipe
 // busier: a full round of 256-row tiles takes about 1.65 x the time of a full round of 128-row tiles for twice the
@@ -53,28 +57,79 @@ inline bool gemm_nat(int64_t M, int64_t K, int64_t ldx) {
 // 184 us; 4096 x 4096 at 2048 rows: 1.0 against 1.24, measured 60 against 75 us); the 256-row grid is taken when it is
 // ahead by 5 % or more.  Only with the natural-order schedule, and only while the split-K blocks of its plan fit the
 // workspace on offer.
-inline int gemm_tile_rows(int64_t M, int64_t N, int64_t K, int64_t ldx, int bits, bool have_workspace, size_t workspace_bytes) {
-    if (!gemm_nat(M, K, ldx)) return 128;
+inline GemmTile gemm_tile_wide(int64_t M, int64_t N, int64_t K, int64_t ldx, int bits, bool have_workspace, size_t workspace_bytes) {
+    constexpr int wide = tile_cols(4);
+    if (!gemm_nat(M, K, ldx)) return {128, wide};
     const int nchunks = gemm_chunks(K, bits, true);
 #ifdef BW_TUNE
-    if (const char* e = getenv("BW_GEMM_BM")) return atoi(e) == 256 ? 256 : atoi(e) == 64 ? 64 : 128;
+    if (const char* e = getenv("BW_GEMM_BM")) return {atoi(e) == 256 ? 256 : atoi(e) == 64 ? 64 : 128, wide};
 #endif
     // (up to 128 rows as two 64-row tiles where N is at most 16 tiles wide: 4096 x 4096, 11008 -> 4096 and 14336 -> 4096 at
     // 80 ... 128 rows 0.88-0.95 of the 128-row time - half the partial-tile traffic of the K split -, but 1.06-1.11 at
     // N = 11008 and 14336, where every weight would be unpacked twice for nothing)
-    if (M <= 64) return 64;
-    if (M <= 128 && (N + BN - 1) / BN <= 16 && !(have_workspace && gemm_plan(M, N, nchunks, true, 64).ws_bytes > workspace_bytes)) return 64;
+    if (M <= 64) return {64, wide};
+    auto fits = [&](int rows, int cols) { return !have_workspace || gemm_plan(M, N, nchunks, true, rows, cols).ws_bytes <= workspace_bytes; };
+    if (M <= 128 && (N + wide - 1) / wide <= 16 && fits(64, wide)) return {64, wide};
     const int64_t cus = bw_device_cus();
     auto rounds = [&](int64_t tiles) {
         const int64_t full = tiles / cus, rest = tiles % cus;
         const bool split = have_workspace && nchunks >= 8 && rest <= cus / 2;
         return (double)full + (rest == 0 ? 0.0 : split ? 0.75 : 1.0);
     };
-    const int64_t tiles_n = (N + BN - 1) / BN;
+    const int64_t tiles_n = (N + wide - 1) / wide;
     const double t128 = rounds(tiles_n * ((M + 127) / 128)), t256 = 1.65 * rounds(tiles_n * ((M + 255) / 256));
-    if (t256 > 0.95 * t128) return 128;
-    if (have_workspace && gemm_plan(M, N, nchunks, true, 256).ws_bytes > workspace_bytes) return 128;
-    return 256;
+    return {t256 > 0.95 * t128 || !fits(256, wide) ? 128 : 256, wide};
+}
+
+// What a call takes, us, with 128- or 256-row tiles of the natural-order schedule (float16 x, weights out of HBM): a base; per 128 values of K
+// of every round of tiles `step` on an empty chip and `fill` more on a full one; where the tiles of a short round are cut along K, `cut`, `part`
+// per million partial sums, and the same two for their slices; more per step at 8 bits and in groups of 32; rows of y that start off an 8-byte
+// boundary cost a round of tiles `odd`, their stores going out as 2-byte pieces.  Fitted to 11796 calls of 129 ... 2048 rows, each timed with
+// the four tiles (all formats, K 512 ... 14336, N 512 ... 22016; rms error 6 ... 7 % each).
+inline float gemm_us(int64_t M, int64_t N, int64_t K, int bits, int group, GemmTile tile, bool have_workspace) {
+    struct Cost { float base, step, fill, cut, part, cut_step, cut_fill, b8, g32, odd; };
+    static constexpr Cost k128 = {8.1f, 0.864f, 0.924f, 4.1f, 0.85f, 1.11f, 0.41f, 0.16f, 0.09f, 7.2f},
+                          k256 = {12.1f, 1.468f, 1.507f, 7.0f, 0.42f, 1.37f, 1.32f, 0.31f, 0.07f, 13.6f},
+                          n128 = {7.1f, 0.745f, 0.564f, 2.8f, 1.32f, 0.97f, 0.12f, 0.17f, 0.08f, 5.1f},
+                          n256 = {10.9f, 1.077f, 1.266f, 4.3f, 0.57f, 1.21f, 0.83f, 0.26f, 0.06f, 8.9f};
+    const Cost& c = tile.cols == tile_cols(4) ? tile.rows == 128 ? k128 : k256 : tile.rows == 128 ? n128 : n256;
+    const int nchunks = gemm_chunks(K, bits, true), cus = bw_device_cus();
+    const GemmPlan p = gemm_plan(M, N, nchunks, have_workspace, tile.rows, tile.cols);
+    const int rest = p.tiles - p.full_tiles, rounds = (p.full_tiles + cus - 1) / cus;
+    const float extra = (bits == 8 ? c.b8 : 0.f) + (group == 32 ? c.g32 : 0.f);
+    float us = c.base + nchunks * ((c.step + extra) * rounds + c.fill * p.full_tiles / cus) + (N % 4 ? c.odd * rounds : 0.f);
+    if (rest)
+        us += c.cut + c.part * 1e-6f * rest * p.splits * (tile.rows * tile.cols) + p.chunks_per_split * (c.cut_step + extra + c.cut_fill * rest * p.splits / cus);
+    return us;
+}
+
+// Tile for this call: 192 columns where the model above is ahead of the 256-column tile's by 5 % (10 % of a 256-row tile on less than eight
+// K steps, which it has too slow).  Finer tiles leave fewer CUs idle in a short round (4096 -> 11008 at 509 rows: 172 tiles of 128 x 256 on 256
+// CUs, 232 of 128 x 192; W4 g128 52.2 -> 46.7 us), their base is smaller, and a K step takes 0.86 of the time where CUs are idle and 0.73 on
+// a full chip, for 0.75 of the work.  8489 of the 11796 calls take 192 columns; all together they take 0.917 of the time, 16 of them over 5 %
+// more (K below 1024), and the best of the four tiles each time would save another 1 %.
+inline GemmTile gemm_tile(int64_t M, int64_t N, int64_t K, int64_t ldx, int bits, int group, bool have_workspace, size_t workspace_bytes) {
+    const GemmTile wide = gemm_tile_wide(M, N, K, ldx, bits, have_workspace, workspace_bytes);
+    if (M <= 128 || !gemm_nat(M, K, ldx)) return wide;
+    const int nchunks = gemm_chunks(K, bits, true);
+    if (have_workspace && gemm_plan(M, N, nchunks, true, wide.rows, wide.cols).ws_bytes > workspace_bytes) return wide;   // refused, whatever a narrow plan needs
+#ifdef BW_TUNE
+    if (const char* e = getenv("BW_GEMM_BN")) return {wide.rows, atoi(e) == tile_cols(3) && wide.rows != 64 ? tile_cols(3) : tile_cols(4)};
+    if (getenv("BW_GEMM_BM")) return wide;
+#endif
+    static thread_local BwPlanCache<GemmTile> cache = {};    // the four models take 0.2 us
+    const GemmTile best = cache.get(M, N, K, (bits * 4 + 2 * have_workspace + (wide.rows == 256)) * 256 + group, [&] {
+        GemmTile b = wide;
+        float us = gemm_us(M, N, K, bits, group, wide, have_workspace) * (wide.rows == 256 && nchunks < 8 ? 0.9f : 0.95f);
+        for (const int rows : {128, 256}) {
+            const GemmTile narrow = {rows, tile_cols(3)};
+            const float t = gemm_us(M, N, K, bits, group, narrow, have_workspace);
+            if (t < us) { b = narrow; us = t; }
+        }
+        return b;
+    });
+    if (best.cols != wide.cols && have_workspace && gemm_plan(M, N, nchunks, true, best.rows, best.cols).ws_bytes > workspace_bytes) return wide;
+    return best;
 }
 
 // Shape-generic fallback: one thread per output element, any group size and
@@ -136,18 +191,19 @@ __global__ __launch_bounds__(256) void cast_bf16_f16_kernel(const uint16_t* __re
 
 }  // namespace
 
-// What a call of 65 ... 2048 rows takes, us, with the tiles it would run (gemm_tile_rows, a workspace on offer), float16 x.  Fitted to 1773
+// What a call of 65 ... 2048 rows takes, us, with the 256-column tiles it would run (gemm_tile_wide, a workspace on offer), float16 x.  Fitted to 1773
 // timings of 65 ... 2048 rows where this kernel and the batch kernel are within a factor of two (all formats, K and N 512 ...
 // 22016; rms error 6 %; 14 % with 128-row tiles assumed throughout and no look at format and N): a base; per 128 values of K of every
 // round of tiles `step` on an empty chip and `fill` more on a full one; the same for the slices of a short round that is cut along K,
 // 7.3 and 0.38 us per million partial sums for the cut; more per step at 8 bits, groups of 32 and K % 128 != 0; rows of y that start
-// off an 8-byte boundary cost a round of uncut tiles `odd`, their stores going out as 2-byte pieces.
+// off an 8-byte boundary cost a round of uncut tiles `odd`, their stores going out as 2-byte pieces.  (192-column tiles have not moved the line between the
+// kernels: by gemm_us of the chosen tile 955 of 22338 calls more would come here and take 0.906 of the batch kernel's time, 28 of them over 8 % longer.)
 float bw_qgemm_expected_us(int64_t M, int64_t N, int64_t K, int bits, int group) {
     struct Cost { float base, step, fill, cut_step, cut_fill, b8, odd; };
     static constexpr Cost k64 = {5.8f, 0.61f, 0.68f, 0.66f, 0.38f, 0.39f, 0.f}, k128 = {7.4f, 0.96f, 0.68f, 0.77f, 0.87f, 0.27f, 7.4f},
                           k256 = {12.1f, 1.34f, 1.41f, 0.77f, 0.87f, 0.34f, 16.6f};
     const bool nat = gemm_nat(M, K, K);
-    const int rows = gemm_tile_rows(M, N, K, K, bits, true, ~(size_t)0), nchunks = gemm_chunks(K, bits, nat), cus = bw_device_cus();
+    const int rows = gemm_tile_wide(M, N, K, K, bits, true, ~(size_t)0).rows, nchunks = gemm_chunks(K, bits, nat), cus = bw_device_cus();
     const Cost& c = rows == 64 ? k64 : rows == 128 ? k128 : k256;
     const GemmPlan p = gemm_plan(M, N, nchunks, true, rows);
     const float steps = bits == 2 && !nat ? 2.f : 1.f;       // of 128 values in a chunk
@@ -155,7 +211,7 @@ float bw_qgemm_expected_us(int64_t M, int64_t N, int64_t K, int bits, int group)
     const float extra = (bits == 8 ? c.b8 : bits == 2 ? -0.04f : 0.f) + (nat ? 0.f : 0.37f) + (group == 32 ? bits == 8 ? 0.18f : 0.12f : 0.f);
     float us = c.base + steps * nchunks * ((c.step + extra) * rounds + c.fill * p.full_tiles / cus) + (N % 4 ? c.odd * rounds : 0.f);
     if (rest)
-        us += 7.3f + 0.38e-6f * rest * p.splits * (rows * BN) + steps * p.chunks_per_split * (c.cut_step + extra + c.cut_fill * rest * p.splits / cus);
+        us += 7.3f + 0.38e-6f * rest * p.splits * (rows * tile_cols(4)) + steps * p.chunks_per_split * (c.cut_step + extra + c.cut_fill * rest * p.splits / cus);
     return us;
 }
 
@@ -186,14 +242,13 @@ static unsigned long long* g_tune_clk = nullptr;
 extern "C" void bw_tune_clock_buffer(void* p) { g_tune_clk = (unsigned long long*)p; }   // 4096 bytes of device memory, or null
 #endif
 
-extern "C" size_t bw_qgemm_workspace_bytes(int64_t M, int64_t N, int64_t K, int bits, int group) {
-    if (!bw_shape_ok(N, K, bits, group) || M < 1 || M >= ((int64_t)1 << 31) || !bw_fast_shape(M, N, K, K, bits, group)) return 0;
-    // any of the plans may run (the call's own ldx and workspace decide): enough for each of them
+// Workspace of the plans with 256-column tiles: the call's own ldx and workspace decide which of them runs.
+static size_t gemm_wide_ws_bytes(int64_t M, int64_t N, int64_t K, int bits) {
     size_t need = gemm_plan(M, N, gemm_chunks(K, bits, false), true, 128).ws_bytes;
     if (gemm_nat(M, K, K)) {
         const size_t nat128 = gemm_plan(M, N, gemm_chunks(K, bits, true), true, 128).ws_bytes;
         if (nat128 > need) need = nat128;
-        const int rows = gemm_tile_rows(M, N, K, K, bits, true, ~(size_t)0);
+        const int rows = gemm_tile_wide(M, N, K, K, bits, true, ~(size_t)0).rows;
         if (rows != 128) {
             const size_t other = gemm_plan(M, N, gemm_chunks(K, bits, true), true, rows).ws_bytes;
             if (other > need) need = other;
@@ -202,9 +257,18 @@ extern "C" size_t bw_qgemm_workspace_bytes(int64_t M, int64_t N, int64_t K, int 
     return need;
 }
 
+extern "C" size_t bw_qgemm_workspace_bytes(int64_t M, int64_t N, int64_t K, int bits, int group) {
+    if (!bw_shape_ok(N, K, bits, group) || M < 1 || M >= ((int64_t)1 << 31) || !bw_fast_shape(M, N, K, K, bits, group)) return 0;
+    const size_t need = gemm_wide_ws_bytes(M, N, K, bits);
+    if (!gemm_nat(M, K, K)) return need;
+    const GemmTile tile = gemm_tile(M, N, K, K, bits, group, true, ~(size_t)0);
+    const size_t chosen = gemm_plan(M, N, gemm_chunks(K, bits, true), true, tile.rows, tile.cols).ws_bytes;
+    return chosen > need ? chosen : need;
+}
+
 extern "C" int bw_qgemm_tile_rows(int64_t M, int64_t N, int64_t K, int bits, int group) {
     if (!bw_shape_ok(N, K, bits, group) || M < 1 || M >= ((int64_t)1 << 31) || !bw_fast_shape(M, N, K, K, bits, group)) return 0;
-    return gemm_tile_rows(M, N, K, K, bits, true, ~(size_t)0);
+    return gemm_tile(M, N, K, K, bits, group, true, ~(size_t)0).rows;
 }
 
 extern "C" int bw_qgemm_ws(const void* x, int act_dtype, int64_t M, int64_t K, int64_t ldx, const int32_t* qweight,
@@ -237,8 +301,9 @@ extern "C" int bw_qgemm_ws(const void* x, int act_dtype, int64_t M, int64_t K, i
     a.splits = 1;
     a.chunks_per_split = a.nchunks;
     hipStream_t st = (hipStream_t)stream;
-    const int rows = nat ? gemm_tile_rows(M, N, K, ldx, bits, workspace != nullptr, workspace_bytes) : 128;
-    if (rows != 128) return bw_launch_gemm_rows(bits, group, rows, a, workspace, workspace_bytes, st);
+    const GemmTile tile = gemm_tile(M, N, K, ldx, bits, group, workspace != nullptr, workspace_bytes);
+    if (tile.cols != tile_cols(4)) return bw_launch_gemm_cols192(bits, group, tile.rows, a, workspace, workspace_bytes, st);
+    if (tile.rows != 128) return bw_launch_gemm_rows(bits, group, tile.rows, a, workspace, workspace_bytes, st);
 #define BW_CASE(B, G)                                                                               \
     if (bits == B && group == G)                                                                     \
         return nat ? launch_gemm<B, G, 8, true>(a, workspace, workspace_bytes, st)                   \
@@ -270,7 +335,9 @@ extern "C" int bw_qgemm_static(const void* x, int act_dtype, int64_t M, int64_t 
         if (hipGetSymbolAddress(&ptr, HIP_SYMBOL(scratch)) != hipSuccess || !ptr) return BW_ELAUNCH;
         g_scratch_ptr[dev].store(ptr, std::memory_order_release);
     }
-    if (bw_qgemm_workspace_bytes(M, N, K, bits, group) > kScratchBytes) return BW_EWORKSPACE;
+    // (a plan of 192-column tiles that needs more than the array is passed over for the 256-column tiles)
+    const bool fast = bw_shape_ok(N, K, bits, group) && M >= 1 && M < ((int64_t)1 << 31) && bw_fast_shape(M, N, K, K, bits, group);
+    if (fast && gemm_wide_ws_bytes(M, N, K, bits) > kScratchBytes) return BW_EWORKSPACE;
     return bw_qgemm_ws(x, act_dtype, M, K, ldx, qweight, scale16, zp16, bias, N, bits, group, y, ldy, ptr, kScratchBytes, stream);
 }
 

@@ -20,7 +20,7 @@ struct GemmArgs {
     // partial tiles go to ws (one BM x BN block per id) for qgemm_reduce_kernel to add up.
     float* ws;
     int tiles_n, full_tiles, splits, chunks_per_split;
-    int bm;                                        // rows of a tile: 128 or 256
+    int bm, bn;                                    // rows and columns of a tile
     // Order of the tiles.  Tile t sits in panel t / (panel * tiles_n) of `panel` m-tiles, n-major inside the panel, so
     // consecutive tiles form blocks a few m-tiles high.  Workgroup ids go to the 8 XCDs round-robin; id i < xcd_tiles (a
     // multiple of 8) takes tile (i % 8) * xcd_tiles / 8 + i / 8: an XCD works through one contiguous eighth of the tile
@@ -35,11 +35,14 @@ struct GemmArgs {
 
 // 64- and 256-row tiles of the natural-order schedule (bw_qgemm_rows.hip); BW_EUNSUPPORTED for any other `rows`
 int bw_launch_gemm_rows(int bits, int group, int rows, const GemmArgs& a, void* workspace, size_t workspace_bytes, hipStream_t stream);
+// 128- and 256-row tiles of 192 columns (bw_qgemm_cols.hip)
+int bw_launch_gemm_cols192(int bits, int group, int rows, const GemmArgs& a, void* workspace, size_t workspace_bytes, hipStream_t stream);
 
 namespace {
 
 
-constexpr int WAVES = 4, NT = 4, BN = WAVES * NT * 16;   // a wave owns MT x NT MFMA tiles; MT = 8 or 16 (128 or 256 rows)
+constexpr int WAVES = 4;                                // a wave owns MT x NT MFMA tiles: 64, 128 or 256 rows of 64 or 48 columns
+constexpr int tile_cols(int nt) { return WAVES * nt * 16; }
 
 template <int BITS, int GROUP, int MT = 8, bool NAT = false>
 struct GemmCfg {
@@ -140,13 +143,23 @@ BW_DEV void lds_read_b128(h8& dst, uint32_t addr) {
 // its first RING slots; every slot then ends with the read of slot S + RING, and with PW > 0 the first slot of each of the four regions of an
 // MFMA step (MT slots) hands over PW words before that.  The words a slot's unpack takes were handed over one MFMA step earlier and
 // have to be there too.  At most what the counter can express: a smaller number waits for more.
-template <int RING, int SLOTS, int MT, int PW>
+// gap of its region in which a tile's first word is handed over: with three column tiles regions begin inside slots, and the words have to lie
+// in the slot in which their unpack begins, or before
+constexpr int hand_gap(int nt) { return nt == 4 ? 1 : 0; }
+
+template <int RING, int SLOTS, int MT, int NT, int PW>
 constexpr int frag_younger(int S) {
+    auto handed = [](int q) {                                 // words handed over in slot q
+        int n = 0;
+        for (int r = 0; r < NT; r++)
+            for (int k = 0; k < PW; k++) n += (MT * r + hand_gap(NT) + k) / NT == q % MT ? 1 : 0;
+        return n;
+    };
     int n = S < RING ? RING - 1 - S : 0;
-    for (int q = S < RING ? 0 : S - RING + 1; q < S; q++) n += (q + RING < SLOTS ? 1 : 0) + (q % (MT / 4) == 0 ? PW : 0);
+    for (int q = S < RING ? 0 : S - RING + 1; q < S; q++) n += (q + RING < SLOTS ? 1 : 0) + handed(q);
     if (PW && S >= MT) {
         int m = 0;
-        for (int q = S - MT; q < S; q++) m += (q + RING < SLOTS ? 1 : 0) + (q > S - MT && q % (MT / 4) == 0 ? PW : 0);
+        for (int q = S - MT; q < S; q++) m += (q + RING < SLOTS ? 1 : 0) + (q > S - MT ? handed(q) : 0);
         n = n < m ? n : m;
     }
     return n < 15 ? n : 15;
@@ -170,11 +183,12 @@ BW_DEV __amdgpu_buffer_rsrc_t make_rsrc(const void* p, uint32_t bytes) {
 //   the activations of chunk c+1 were requested one step earlier and are written to buffer (c+1)&1 during
 //   step c, then re-requested for chunk c+2; the weights of chunk c+2 are requested into step c's own set
 //   once its last fragment is unpacked.  Every global load has a full K step (~2000 MFMA cycles) to land.
-template <int BITS, int GROUP, bool WIDE_META, int MT, bool NAT>
+template <int BITS, int GROUP, bool WIDE_META, int MT, bool NAT, int NT>
 __global__ __launch_bounds__(WAVES * 64) void qgemm_kernel(const GemmArgs a) {
     static_assert(MT == 8 || (NAT && (MT == 4 || MT == 16)), "64- and 256-row tiles exist with the natural-order schedule only");
     using C = GemmCfg<BITS, GROUP, MT, NAT>;
-    constexpr int BM = C::BM;
+    constexpr int BM = C::BM, BN = tile_cols(NT);
+    static_assert(NT == 4 || (NT == 3 && NAT && MT >= 8), "192-column tiles exist with 128 and 256 rows of the natural-order schedule");
     // WIDE_META (rows of scales on 4-byte boundaries): META4 = 8-byte requests over runs of K steps; PAIR = a lane whose
     // values span two groups fetches both scales (zero points) with one 4-byte request instead of two 2-byte ones
     constexpr bool META4 = WIDE_META && C::CAN_META4, PAIR = WIDE_META && !C::CAN_META4 && C::NG == 2;
@@ -528,13 +542,13 @@ __global__ __launch_bounds__(WAVES * 64) void qgemm_kernel(const GemmArgs a) {
             constexpr bool early = t == C::MF - 1;
             const WSet& src = early ? wsn : ws;
             constexpr int tt = early ? 0 : t + 1;
-            static_for<0, 4 * MT>([&](auto gcnt) {
+            static_for<0, NT * MT>([&](auto gcnt) {
                 // RG gaps (SLOTS slots) per region: 16 (4) with 256-row tiles, 8 (2) with 128-row tiles
-                constexpr int RG = 4 * MT / NT, SLOTS = RG / 4;
+                constexpr int RG = MT, SLOTS = RG / 4;
                 constexpr int g = decltype(gcnt)::value, i = g / NT, j = g % NT, r = g / RG, k = g % RG;
                 constexpr int S = MT * t + i;
                 __builtin_amdgcn_sched_barrier(0);
-                if constexpr (j == 0) __builtin_amdgcn_s_waitcnt(0xC07F | (frag_younger<C::XRING, MT * C::MF, MT, QW ? PW : 0>(S) << 8));
+                if constexpr (j == 0) __builtin_amdgcn_s_waitcnt(0xC07F | (frag_younger<C::XRING, MT * C::MF, MT, NT, QW ? PW : 0>(S) << 8));
                 mfma_acc(acc[i][j], pack_h8(wf[cu][j]), xf[0][(MT * t + i) % C::XRING]);
                 __builtin_amdgcn_sched_barrier(0);
                 // ---- unpack of n-tile r: instruction v of its sequence ----
@@ -588,8 +602,11 @@ __global__ __launch_bounds__(WAVES * 64) void qgemm_kernel(const GemmArgs a) {
                 // (64-row tiles, one slot per region: 12 -> 4 4 4, 16 -> 6 5 5)
                 constexpr int n0 = PER_SLOT == 3 ? 1 : PER_SLOT == 8 ? 3 : PER_SLOT == 12 ? 4 : PER_SLOT == 16 ? 6 : 2,
                               n1 = PER_SLOT <= 4 ? 1 : PER_SLOT == 8 ? 3 : PER_SLOT == 12 ? 4 : PER_SLOT == 16 ? 5 : 2;
-                constexpr int first = sl * PER_SLOT + (j == 0 ? 0 : j == 1 ? n0 : n0 + n1);
-                constexpr int count = j == 0 ? n0 : j == 1 ? n1 : j == 2 ? PER_SLOT - n0 - n1 : 0;
+                // Three column tiles (192-column tiles of the workgroup): a slot has two such gaps, a region RG gaps that begin inside a slot; its
+                // instructions are dealt out evenly over those that are not a read's.
+                constexpr int free_before = k - ((r * RG + k) / NT - r * RG / NT), free_all = RG - ((r + 1) * RG / NT - r * RG / NT);
+                constexpr int first = NT == 3 ? free_before * OPS / free_all : sl * PER_SLOT + (j == 0 ? 0 : j == 1 ? n0 : n0 + n1);
+                constexpr int count = NT == 3 ? (j == NT - 1 ? 0 : (free_before + 1) * OPS / free_all - first) : j == 0 ? n0 : j == 1 ? n1 : j == 2 ? PER_SLOT - n0 - n1 : 0;
                 static_for<0, count>([&](auto oc) { unpack_op(std::integral_constant<int, first + decltype(oc)::value>{}); });
                 // ---- the next chunk's activations: unit i of the wave in slot i of the first MFMA step ----
                 if constexpr (t == 0 && j == 1) x_dma16(i, c + 1, nxt);
@@ -600,11 +617,11 @@ __global__ __launch_bounds__(WAVES * 64) void qgemm_kernel(const GemmArgs a) {
                     const uint32_t pair = wsn.s[r][0] | (wsn.z[r][0] << 16);
                     asm volatile("ds_bpermute_b32 %0, %1, %2" : "=v"(pm[r]) : "v"(pm_from), "v"(pair));
                 }
-                // ---- QW: tile r's words of the MFMA step after next, in the first slot of its region (frag_younger counts them)
-                if constexpr (QW && k >= 1 && k <= PW) {
+                // ---- QW: tile r's words of the MFMA step after next, in the first slot of its region (frag_younger counts them; hand_gap)
+                if constexpr (QW && k >= hand_gap(NT) && k < hand_gap(NT) + PW) {
                     constexpr int t2 = (t + 2) % C::MF;
-                    const uint32_t word = word_of(t + 2 < C::MF ? ws : wsn, r, t2, k - 1);
-                    asm volatile("ds_bpermute_b32 %0, %1, %2" : "=v"(pw[nx][r][k - 1]) : "v"(pm_from), "v"(word));
+                    const uint32_t word = word_of(t + 2 < C::MF ? ws : wsn, r, t2, k - hand_gap(NT));
+                    asm volatile("ds_bpermute_b32 %0, %1, %2" : "=v"(pw[nx][r][k - hand_gap(NT)]) : "v"(pm_from), "v"(word));
                 }
                 // ---- fragment ring ----
                 if constexpr (j == NT - 1) {
@@ -613,9 +630,9 @@ __global__ __launch_bounds__(WAVES * 64) void qgemm_kernel(const GemmArgs a) {
                 }
                 // ---- requests and constants (second gap of a slot) ----
                 // two requests per region: slots 2 and 3 of four (second gap), or gaps 1 and 2 of the second slot of two
-                constexpr bool meta_here = SLOTS == 4 ? (j == 1 && sl >= 2) : (sl == SLOTS - 1 && (j == 1 || j == 2));
+                constexpr bool meta_here = NT == 3 ? (k == RG - 4 || k == RG - 3) : SLOTS == 4 ? (j == 1 && sl >= 2) : (sl == SLOTS - 1 && (j == 1 || j == 2));
                 if constexpr (t == 1 && meta_here) {
-                    constexpr int which = SLOTS == 4 ? sl - 2 : j - 1;
+                    constexpr int which = NT == 3 ? k - (RG - 4) : SLOTS == 4 ? sl - 2 : j - 1;
                     if constexpr (META4) {
                         if (ph == 0) issue_meta4(r, which, c + C::SPR, m_next);
                     } else {
@@ -627,7 +644,9 @@ __global__ __launch_bounds__(WAVES * 64) void qgemm_kernel(const GemmArgs a) {
                     else set_consts(gn[r], r, wsn, m_cur, 0);
                 }
                 constexpr int T_WREQ = QW ? C::MF - 2 : C::MF - 1;         // the words are handed over (or unpacked) by then
-                if constexpr (SLOTS == 4) {
+                if constexpr (NT == 3) {
+                    if constexpr (t == T_WREQ && k >= RG - C::WL) w_req16(r, k - (RG - C::WL), c + 2, ws);
+                } else if constexpr (SLOTS == 4) {
                     if constexpr (t == C::MF - 1 && j == 1 && sl >= 4 - C::WL) w_req16(r, sl - (4 - C::WL), c + 2, ws);
                 } else {                                                   // two slots: gaps 1 (and 2 at 8 bits) of the second
                     if constexpr (t == T_WREQ && sl == SLOTS - 1 && j >= 1 && j <= C::WL) w_req16(r, j - 1, c + 2, ws);
@@ -853,7 +872,7 @@ __global__ __launch_bounds__(WAVES * 64) void qgemm_kernel(const GemmArgs a) {
         for (int q = 0; q < BM / 8; q++) {
             const int row = 8 * q + (lane >> 3), unit = lane & 7;
             const u4 v = *reinterpret_cast<const u4*>(ob + row * 128 + ((unit ^ (row & 7)) * 16));
-            if (m0 + row < a.M) *reinterpret_cast<u4*>(a.y + (int64_t)(m0 + row) * a.ldy + n0 + unit * 8) = v;
+            if (unit < 2 * NT && m0 + row < a.M) *reinterpret_cast<u4*>(a.y + (int64_t)(m0 + row) * a.ldy + n0 + unit * 8) = v;
         }
         return;
     }
@@ -889,8 +908,8 @@ __global__ __launch_bounds__(WAVES * 64) void qgemm_kernel(const GemmArgs a) {
 // a thread four consecutive n.  y[m][n] = fp16( sum_z partial_z[m][n] + bias[n] ).
 __global__ __launch_bounds__(256) void qgemm_reduce_kernel(const GemmArgs a) {
     const int tile = a.full_tiles + (int)blockIdx.y;
-    const int quad = (int)(blockIdx.x * blockDim.x + threadIdx.x);          // < bm * BN / 4
-    const int ml = quad / (BN / 4), nl4 = (quad % (BN / 4)) * 4;
+    const int quad = (int)(blockIdx.x * blockDim.x + threadIdx.x);          // < bm * bn / 4
+    const int BN = a.bn, ml = quad / (BN / 4), nl4 = (quad % (BN / 4)) * 4;
     int tm, tn;
     tile_coords(tile, a, tm, tn);
     const int m = tm * a.bm + ml, n = tn * BN + nl4;
@@ -930,9 +949,9 @@ inline int gemm_chunks(int64_t K, int bits, bool nat) {   // K steps of a whole 
     return (int)((K * bits / 8 + chunk - 1) / chunk);
 }
 
-inline GemmPlan gemm_plan(int64_t M, int64_t N, int nchunks, bool have_workspace, int bm = 128) {
+inline GemmPlan gemm_plan(int64_t M, int64_t N, int nchunks, bool have_workspace, int bm = 128, int bn = tile_cols(4)) {
     GemmPlan p;
-    p.tiles_n = (int)((N + BN - 1) / BN);
+    p.tiles_n = (int)((N + bn - 1) / bn);
     p.tiles = p.tiles_n * (int)((M + bm - 1) / bm);
     p.full_tiles = p.tiles;
     p.splits = 1;
@@ -953,32 +972,33 @@ inline GemmPlan gemm_plan(int64_t M, int64_t N, int nchunks, bool have_workspace
     p.full_tiles = p.tiles - rest;
     p.splits = s;
     p.chunks_per_split = cps;
-    p.ws_bytes = (size_t)rest * s * bm * BN * sizeof(float);
+    p.ws_bytes = (size_t)rest * s * bm * bn * sizeof(float);
     return p;
 }
 
-template <int BITS, int GROUP, int MT, bool NAT>
+template <int BITS, int GROUP, int MT, bool NAT, int NT = 4>
 int launch_gemm(GemmArgs a, void* workspace, size_t workspace_bytes, hipStream_t stream) {
     using C = GemmCfg<BITS, GROUP, MT, NAT>;
-    constexpr int BM = C::BM;
+    constexpr int BM = C::BM, BN = tile_cols(NT);
     static_assert(C::CHUNK_BYTES == (BITS == 8 ? 128 : (BITS == 2 && NAT) ? 32 : 64), "gemm_chunks() counts K steps of this size");
     const size_t lds = 2 * (size_t)C::STAGE_BYTES;
-    void (*kern)(const GemmArgs) = qgemm_kernel<BITS, GROUP, false, MT, NAT>;
+    void (*kern)(const GemmArgs) = qgemm_kernel<BITS, GROUP, false, MT, NAT, NT>;
     static uint64_t big_lds_devices[2] = {0, 0};           // per kernel
     int which = 0;
     if constexpr (C::CAN_META4 || C::NG == 2) {
         // an even number of K steps (so that the loop never pads with a step that would read past the row's scales)
         // and rows of scales on 4-byte boundaries
         if (a.groups % (C::CAN_META4 ? 2 * C::GPS : 2) == 0 && bw_aligned(a.scale, 4) && bw_aligned(a.zp, 4)) {
-            kern = qgemm_kernel<BITS, GROUP, true, MT, NAT>;
+            kern = qgemm_kernel<BITS, GROUP, true, MT, NAT, NT>;
             which = 1;
         }
     }
     if (lds > 64 * 1024 && !bw_allow_big_lds(reinterpret_cast<const void*>(kern), big_lds_devices[which])) return BW_ELAUNCH;
-    const GemmPlan p = gemm_plan(a.M, a.N, a.nchunks, workspace != nullptr, BM);
+    const GemmPlan p = gemm_plan(a.M, a.N, a.nchunks, workspace != nullptr, BM, BN);
     if (p.ws_bytes > workspace_bytes) return BW_EWORKSPACE;
     a.ws = (float*)workspace;
     a.bm = BM;
+    a.bn = BN;
     a.tiles_n = p.tiles_n;
     a.tiles_m = p.tiles / p.tiles_n;
     a.panel = a.tiles_m < 4 ? a.tiles_m : 4;

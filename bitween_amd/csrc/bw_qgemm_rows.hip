@@ -4,7 +4,7 @@
 //            activation traffic of a 128-row tile that would be at least half padding; two workgroups fit a CU
 //   256 rows (a wave owns 256 x 64, all 256 accumulation registers): grids that fill the device - every weight is
 //            unpacked once for twice the rows
-// Which height a call gets is decided in bw_qgemm.hip (gemm_tile_rows).
+// Which height a call gets is decided in bw_qgemm.hip (gemm_tile).
 #include "bw_qgemm_kernel.h"
 
 int bw_launch_gemm_rows(int bits, int group, int rows, const GemmArgs& a, void* workspace, size_t workspace_bytes, hipStream_t stream) {

@@ -1,0 +1,85 @@
+"""The prefill kernel's 192-column tiles (three column tiles a wave) against the oracle: forced through the measurement build, which takes
+the tile from the environment, and as the library chooses them."""
+import ctypes
+
+import numpy as np
+import pytest
+import torch
+
+from gpu_util import check_matmul, quantized_layer, to_gpu
+from oracle import rtn_oracle as orc
+
+pytestmark = pytest.mark.gpu
+
+FORMATS = [(4, 128), (4, 64), (4, 32), (8, 128), (8, 64), (8, 32), (2, 128), (2, 64), (2, 32)]
+
+
+def _forced(monkeypatch, rows, cols):
+    from bitween_amd.csrc import build
+    from bitween_amd.kernels import hip_loader
+    lib, ref = ctypes.CDLL(build.TUNE_LIB), hip_loader.load()
+    for name in ("bw_qgemm_ws", "bw_qgemm_workspace_bytes"):
+        fn = getattr(lib, name)
+        fn.argtypes, fn.restype = getattr(ref, name).argtypes, getattr(ref, name).restype
+    monkeypatch.setenv("BW_GEMM_BM", str(rows))
+    monkeypatch.setenv("BW_GEMM_BN", str(cols))
+    return lib
+
+
+def _run(lib, x, d, bias, n, bits, g, ldy, with_workspace=False):
+    m, k = x.shape
+    y = torch.full((m, ldy), 7.0, dtype=torch.float16, device="cuda")
+    need = lib.bw_qgemm_workspace_bytes(m, n, k, bits, g) if with_workspace else 0
+    ws = torch.empty(max(need, 16), dtype=torch.uint8, device="cuda")
+    st = lib.bw_qgemm_ws(x.data_ptr(), 0, m, k, k, *[t.data_ptr() for t in d], bias.data_ptr() if bias is not None else None, n, bits, g,
+                         y.data_ptr(), ldy, ws.data_ptr() if need else None, need, ctypes.c_void_p(torch.cuda.current_stream().cuda_stream))
+    assert st == 0
+    torch.cuda.synchronize()
+    assert (y[:, n:] == 7.0).all()
+    return y[:, :n]
+
+
+@pytest.mark.parametrize("rows", [128, 256])
+@pytest.mark.parametrize("bits,g", FORMATS)
+@pytest.mark.parametrize("k,n,m,pad", [(128, 191, 129, 1), (256, 193, 257, 7), (384, 48, 130, 0), (640, 400, 200, 0), (896, 239, 300, 1), (1024, 576, 513, 8)])
+def test_192_column_tiles(monkeypatch, rows, bits, g, k, n, m, pad):
+    """One to eight K steps (odd counts, runs of four and what is left of them), columns that end in every quarter of a tile and inside a
+    wave's 48, rows past a tile, rows of y on and off 16 bytes; one-hot rows return columns of W16 bit for bit."""
+    lib = _forced(monkeypatch, rows, 192)
+    _, qw, s16, z16, b16 = quantized_layer(n, k, bits, g, seed=k + n + g + bits, outliers=True)
+    x = np.random.default_rng(m).standard_normal((m, k)).astype(np.float16)
+    d = [to_gpu(a) for a in (qw, s16, z16)]
+    check_matmul(_run(lib, to_gpu(x), d, to_gpu(b16), n, bits, g, n + pad), x, qw, s16, z16, b16, bits, g)
+    cols = np.linspace(0, k - 1, m).astype(int)
+    hot = np.zeros((m, k), np.float16)
+    hot[np.arange(m), cols] = 1
+    y = _run(lib, to_gpu(hot), d, None, n, bits, g, n + pad)
+    assert np.array_equal(y.cpu().numpy(), orc.dequantize_f16(qw, s16, z16, g, bits)[:, cols].T)
+
+
+@pytest.mark.parametrize("rows", [128, 256])
+@pytest.mark.parametrize("bits,g", [(4, 128), (8, 32), (2, 64)])
+def test_192_column_tiles_cut_along_k(monkeypatch, rows, bits, g):
+    """Partial tiles of 192 columns and their sum: slices of whole pairs of K steps and a shorter last one."""
+    n, k, m = 401, 128 * 22, 300
+    lib = _forced(monkeypatch, rows, 192)
+    assert lib.bw_qgemm_workspace_bytes(m, n, k, bits, g) > 0
+    _, qw, s16, z16, b16 = quantized_layer(n, k, bits, g, seed=rows + g, outliers=True)
+    x = np.random.default_rng(rows).standard_normal((m, k)).astype(np.float16)
+    d = [to_gpu(a) for a in (qw, s16, z16)]
+    check_matmul(_run(lib, to_gpu(x), d, to_gpu(b16), n, bits, g, n + 3, with_workspace=True), x, qw, s16, z16, b16, bits, g)
+
+
+@pytest.mark.parametrize("bits,g,m,n,k", [(8, 32, 509, 11008, 4096), (4, 128, 1000, 11008, 4096), (4, 64, 160, 6000, 2048)])
+def test_tiles_the_library_chooses(bits, g, m, n, k):
+    """Columns at the edges of the 192- and 256-column tiles."""
+    import bitween_amd
+    from bitween_amd.kernels import hip_loader
+    lib = hip_loader.load()
+    torch.manual_seed(n)
+    q = bitween_amd.QuantizedLinear.from_float(torch.nn.Linear(k, n, bias=True, device="cuda", dtype=torch.float16), bits, g)
+    x = torch.randn(m, k, device="cuda", dtype=torch.float16)
+    y = _run(lib, x, (q.qweight, q.scale, q.zero_point), q.bias, n, bits, g, n, with_workspace=True)
+    cols = np.unique(np.clip(np.concatenate([np.arange(0, n, 331)] + [e + np.arange(-1, 2) for e in (48, 64, 192, 256, n - n % 192, n)]), 0, n - 1))
+    part = [t[torch.from_numpy(cols).cuda()].cpu().numpy() for t in (q.qweight, q.scale, q.zero_point, q.bias)]
+    check_matmul(y[:, torch.from_numpy(cols).cuda()], x.cpu().numpy(), *part, bits, g)
