@@ -250,15 +250,19 @@ BW_DEV float half_of(uint32_t word, int hi) {
 // zero point) pairs.
 // The registers that requests land in are not touched until the code that uses them, so every wait sits where
 // the data is needed; nothing is requested under a branch (a request under a branch costs a full wait).
+// LINES (4 bits): weights are asked for as whole 128-byte lines - eight lanes a line, non-temporal - and go through the wave's x tile in LDS
+// to operand layout; the wave's x, the same for all tiles, waits in registers by then.  us at 16 rows, graph replay, weights out
+// of HBM: 4096 -> 11008 g128 9.34 -> 8.78, g32 10.9 -> 10.6; at 6 rows 8.18 -> 7.48, 9.47 -> 8.79.
 // What bounds it: a CU keeps a limited number of cache lines requested at once, and a line of x from L2 holds
 // its place for a few hundred cycles, a line of weights from HBM for over a thousand: the x lines of 16
 // activation rows (128 KB per CU at K = 4096) add about 2 us to what the weights alone need.
-template <int BITS, int GROUP, int MT, int NT>
+template <int BITS, int GROUP, int MT, int NT, bool LINES>
 __global__ __launch_bounds__(1024) void qgemv_tiles_kernel(const GemvArgs a) {
     using C = GemvCfg<BITS, GROUP, MT>;
     constexpr int KBW = BITS == 4 ? 2 : (BITS == 8 ? 4 : 1);     // chunks per wave: 256 values of K
     constexpr int BK = KBW * C::CHUNK_K, PITCH = BK + 8, UPR = BK / C::UNIT, XL = (MT * UPR + 63) / 64;
-    constexpr int X_BYTES = MT * PITCH * 2, UW = C::UNIT / 8;
+    constexpr int X_BYTES = MT * PITCH * 2, UW = C::UNIT / 8, XF = KBW * C::MF;
+    static_assert(!LINES || (BITS == 4 && X_BYTES >= 16 * 128), "a wave's 256 values are one line of a row; a tile of them fits its x tile");
     constexpr int kOutPerTile = 16 * MT;
     constexpr uint32_t kOob = 0x80000000u;
     extern __shared__ __attribute__((aligned(16))) char smem[];
@@ -325,14 +329,14 @@ __global__ __launch_bounds__(1024) void qgemv_tiles_kernel(const GemvArgs a) {
     asm volatile("" ::: "memory");
     u4 wr[NT][KBW];
     auto issue_w = [&](int t) {
-        const uint32_t n = (uint32_t)tile_of(t) * 16 + nl;
 #pragma unroll
         for (int b = 0; b < KBW; b++) {
-            const int c = wave * KBW + b;
-            uint32_t off = n * a.row_bytes + c * 64 + kq * 16;
+            const uint32_t n = (uint32_t)tile_of(t) * 16 + (LINES ? 8 * b + (lane >> 3) : nl);
+            const int c = wave * KBW + (LINES ? (lane & 7) >> 2 : b);
+            uint32_t off = n * a.row_bytes + c * 64 + (LINES ? lane & 3 : kq) * 16;
             asm volatile("" : "+v"(off));
             off = (tile_of(t) < a.ntiles && c < a.nchunks) ? off : kOob;
-            wr[t][b] = __builtin_amdgcn_raw_buffer_load_b128(rw, off, 0, 0);
+            wr[t][b] = __builtin_amdgcn_raw_buffer_load_b128(rw, off, 0, LINES ? 2 : 0);   // 2: non-temporal
         }
         asm volatile("" ::: "memory");
     };
@@ -376,20 +380,39 @@ __global__ __launch_bounds__(1024) void qgemv_tiles_kernel(const GemvArgs a) {
         }
     }
     __builtin_amdgcn_wave_barrier();
+    const int arow = nl < MT ? nl : MT - 1;              // MFMA rows >= MT repeat a valid row; never stored
+    h8 xf[LINES ? XF : 1];
+    if constexpr (LINES) {                               // x is the same for all tiles: its LDS is free for the weights
+#pragma unroll
+        for (int s = 0; s < XF; s++) xf[s] = *reinterpret_cast<const h8*>(xs + arow * PITCH + s / C::MF * C::CHUNK_K + kq * C::VPL + s % C::MF * 8);
+        asm volatile("" ::: "memory");
+    }
     while (__hip_atomic_load(ready, __ATOMIC_ACQUIRE, __HIP_MEMORY_SCOPE_WORKGROUP) < (uint32_t)meta_waves) __builtin_amdgcn_s_sleep(1);
 
     // ---- the tiles, as their weights arrive
     f4 acc[NT][2];
-    const int arow = nl < MT ? nl : MT - 1;              // MFMA rows >= MT repeat a valid row; never stored
 #pragma unroll
     for (int t = 0; t < NT; t++) {
         if (t + 2 < NT) issue_w(t + 2);
+        if constexpr (LINES) {                                // whole lines -> operand layout, the pieces of a row swizzled by its number
+            char* const lines = reinterpret_cast<char*>(xs);
+#pragma unroll
+            for (int b = 0; b < KBW; b++) {
+                u4 wv = wr[t][b];
+                asm volatile("" : "+v"(wv));                  // the wait for them belongs here
+                *reinterpret_cast<u4*>(lines + (8 * b + (lane >> 3)) * 128 + ((lane & 7) ^ (lane >> 3)) * 16) = wv;
+            }
+            asm volatile("" ::: "memory");                    // (a wave's LDS operations complete in order)
+#pragma unroll
+            for (int b = 0; b < KBW; b++) wr[t][b] = *reinterpret_cast<const u4*>(lines + nl * 128 + ((4 * b + kq) ^ (nl & 7)) * 16);
+            asm volatile("" ::: "memory");
+        }
         acc[t][0] = acc[t][1] = f4{0.f, 0.f, 0.f, 0.f};
         const uint32_t* mrow = meta + t * 16 * GP + nl * GP;
 #pragma unroll
         for (int b = 0; b < KBW; b++) {
             u4 wv = wr[t][b];
-            asm volatile("" : "+v"(wv));                      // use the registers here and not before
+            if constexpr (!LINES) asm volatile("" : "+v"(wv));   // use the registers here and not before
             // (a chunk may reach past the end of K: those lanes take the row's last groups, their x is zero)
             const int gb = min(((wave * KBW + b) * C::CHUNK_K + kq * C::VPL) / GROUP, groups - C::NG);
             GroupConst<BITS> gc[C::NG];
@@ -401,18 +424,22 @@ __global__ __launch_bounds__(1024) void qgemv_tiles_kernel(const GemvArgs a) {
             h2 wp[C::VPL / 2];
             dequant_lane16<BITS, C::NG, !C::POST>(wv, gc, wp);
             const _Float16* xp = xs + arow * PITCH + b * C::CHUNK_K + kq * C::VPL;
+            auto x_of = [&](int s) -> h8 {
+                if constexpr (LINES) return xf[b * C::MF + s];
+                else return *reinterpret_cast<const h8*>(xp + 8 * s);
+            };
             if constexpr (C::POST) {
                 f4 part = {0.f, 0.f, 0.f, 0.f};
 #pragma unroll
                 for (int s = 0; s < C::MF; s++)
-                    part = __builtin_amdgcn_mfma_f32_16x16x32_f16(*reinterpret_cast<const h8*>(xp + 8 * s), pack_h8(wp + 4 * s), part, 0, 0, 0);
+                    part = __builtin_amdgcn_mfma_f32_16x16x32_f16(x_of(s), pack_h8(wp + 4 * s), part, 0, 0, 0);
                 const float sf = (float)gc[0].s[0];
 #pragma unroll
                 for (int q = 0; q < 4; q++) acc[t][b & 1][q] = __builtin_fmaf(sf, part[q], acc[t][b & 1][q]);
             } else {
 #pragma unroll
                 for (int s = 0; s < C::MF; s++)
-                    acc[t][s & 1] = __builtin_amdgcn_mfma_f32_16x16x32_f16(*reinterpret_cast<const h8*>(xp + 8 * s), pack_h8(wp + 4 * s), acc[t][s & 1], 0, 0, 0);
+                    acc[t][s & 1] = __builtin_amdgcn_mfma_f32_16x16x32_f16(x_of(s), pack_h8(wp + 4 * s), acc[t][s & 1], 0, 0, 0);
             }
         }
     }
@@ -1440,14 +1467,25 @@ int launch_w2(const GemvArgs& a, hipStream_t stream) {
 
 constexpr int kLdsBudget = 150 * 1024;
 
-template <int BITS, int GROUP, int MT, int NT>
-int launch_tiles_nt(const GemvArgs& a, int grid, int nwaves, size_t lds, hipStream_t stream) {
-    auto kern = qgemv_tiles_kernel<BITS, GROUP, MT, NT>;
+template <int BITS, int GROUP, int MT, int NT, bool LINES>
+int launch_tiles_lines(const GemvArgs& a, int grid, int nwaves, size_t lds, hipStream_t stream) {
+    auto kern = qgemv_tiles_kernel<BITS, GROUP, MT, NT, LINES>;
     BW_NOTE_KERNEL("qgemv_tiles_kernel", BITS, GROUP, MT, NT);
     static uint64_t big_lds_devices = 0;                   // per instantiation
     if (lds > 64 * 1024 && !bw_allow_big_lds(reinterpret_cast<const void*>(kern), big_lds_devices)) return BW_ELAUNCH;
     hipLaunchKernelGGL(kern, dim3((unsigned)grid), dim3(nwaves * 64), lds, stream, a);
     return hipGetLastError() == hipSuccess ? BW_OK : BW_ELAUNCH;
+}
+
+template <int BITS, int GROUP, int MT, int NT>
+int launch_tiles_nt(const GemvArgs& a, int grid, int nwaves, size_t lds, hipStream_t stream) {
+    // Whole lines (LINES): 4 bits, where a wave's 256 values of a row are one line of it, and several tiles a workgroup.  Timed on 420 calls (K 512
+    // ... 4096, N 512 ... 14336, 5 ... 16 rows, three groups), the time over that of operand layout: two tiles 0.91 ... 0.98, three 0.92 ... 0.98, four at
+    // 9 ... 16 rows 0.955 ... 0.97; four at 5 ... 8 rows 1.01 ... 1.08, one tile 1.0 ... 1.06 (the way through LDS before the first MFMA
+    // is not made up for), rows that are no whole number of lines 1.08 ... 1.13 (K = 2880), up to 4 rows 0.98 ... 1.09.
+    if constexpr (BITS == 4 && MT >= 8 && NT >= 2 && !(MT == 8 && NT == 4))
+        if (a.row_bytes % 128 == 0 && bw_aligned(a.qweight, 128)) return launch_tiles_lines<BITS, GROUP, MT, NT, true>(a, grid, nwaves, lds, stream);
+    return launch_tiles_lines<BITS, GROUP, MT, NT, false>(a, grid, nwaves, lds, stream);
 }
 
 template <int BITS, int GROUP, int MT, int DEPTH, bool LOOP>

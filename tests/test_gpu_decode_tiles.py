@@ -110,3 +110,23 @@ def test_layouts_the_tile_kernels_do_not_take_fall_back():
         assert st == 0
         torch.cuda.synchronize()
         check_matmul(y, x, qw, s16, z16, b16, bits, g)
+
+
+@pytest.mark.parametrize("g", [128, 64, 32])
+@pytest.mark.parametrize("k,n", [(2048, 8209), (3840, 6200), (4096, 9000), (4096, 12500), (3968, 6200)])   # 2, 2, 3, 4 tiles a workgroup; rows of 15.5 lines
+def test_whole_lines_and_operand_layout_agree(g, k, n):
+    """Weights asked for as whole lines (4 bits, 5 rows and more, several tiles a workgroup, rows of whole lines) meet the oracle, and give
+    the bits of the same weights 16 bytes off a line, which go to operand layout directly."""
+    if k % g:
+        pytest.skip("no whole number of groups")
+    rows = np.unique(np.concatenate([np.arange(0, n, n // 24), [15, 16, n - 17, n - 1]]))
+    q, qw_o, s16, z16, b16 = _layer_rows(n, k, 4, g, seed=k + n + g, rows=rows)
+    off = torch.empty(q.qweight.numel() + 4, dtype=torch.int32, device="cuda")
+    off[4:] = q.qweight.reshape(-1)
+    moved = off[4:].view(q.qweight.shape)
+    from bitween_amd.kernels import hip_loader as hip
+    for m, dtype in ((5, torch.float16), (8, torch.bfloat16), (9, torch.bfloat16), (16, torch.float16)):
+        x = torch.randn(m, k, device="cuda").to(dtype)
+        y = _gemv(q, x, 4, g)
+        check_matmul(y[:, rows], x.to(torch.float16).cpu().numpy(), qw_o, s16, z16, b16, 4, g)
+        assert torch.equal(y, hip.quantized_gemv_hip(x, moved, q.scale, q.zero_point, q.bias, 4, g))
