@@ -110,7 +110,7 @@ inline float gemm_us(int64_t M, int64_t N, int64_t K, int bits, int group, GemmT
 // more (K below 1024), and the best of the four tiles each time would save another 1 %.
 inline GemmTile gemm_tile(int64_t M, int64_t N, int64_t K, int64_t ldx, int bits, int group, bool have_workspace, size_t workspace_bytes) {
     const GemmTile wide = gemm_tile_wide(M, N, K, ldx, bits, have_workspace, workspace_bytes);
-    if (M <= 128 || !gemm_nat(M, K, ldx)) return wide;
+    if (wide.rows == 64 || !gemm_nat(M, K, ldx)) return wide;
     const int nchunks = gemm_chunks(K, bits, true);
     if (have_workspace && gemm_plan(M, N, nchunks, true, wide.rows, wide.cols).ws_bytes > workspace_bytes) return wide;   // refused, whatever a narrow plan needs
 #ifdef BW_TUNE
