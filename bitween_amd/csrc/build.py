@@ -11,7 +11,7 @@ import subprocess
 import sys
 
 HERE = os.path.dirname(os.path.abspath(__file__))
-SOURCES = ["bw_quantize.hip", "bw_qgemv.hip", "bw_qgemm.hip", "bw_qgemm_rows.hip", "bw_qgemm_cols.hip", "bw_qbatch.hip", "bw_qbatch_w2.hip", "bw_qbatch_w4.hip", "bw_qbatch_w8.hip", "bw_qdgrad.hip"]
+SOURCES = ["bw_quantize.hip", "bw_qgemv.hip", "bw_qgemm.hip", "bw_qgemm_rows.hip", "bw_qgemm_cols.hip", "bw_qbatch.hip", "bw_qbatch_w2.hip", "bw_qbatch_w4.hip", "bw_qbatch_w8.hip", "bw_qdgrad.hip", "bw_qdgrad_rows.hip"]
 TUNE_SOURCES = ["bw_qgemm.hip", "bw_qgemm_rows.hip", "bw_qgemm_cols.hip"]      # compiled a second time with -DBW_TUNE for the measurement build
 LIB = os.path.join(HERE, "libbitween_hip.so")
 HOST_SOURCE, HOST_LIB = os.path.join(HERE, "bw_host.cpp"), os.path.join(HERE, "_bw_host.so")

@@ -33,6 +33,7 @@
 
 #include "bw_common.h"
 #include "bw_plan_cache.h"
+#include "bw_qdgrad_rows.h"
 
 namespace {
 
@@ -767,6 +768,24 @@ inline int dgrad_use256(int64_t M, int64_t N, int64_t K, int64_t ldg, int bits, 
     return (have_workspace || tiles > dgrad_cus() / 2) ? rows : 0;
 }
 
+// Slices of N for the kernel of a few rows (bw_qdgrad_rows.hip) in a workspace of `need` bytes, the one that the plan of the others asks for; 0 =
+// the others run.  One workgroup a CU at most (4096 <- 4096 at 16 rows: 8 or 16 slices of 16 strips of K 11 us, 24 slices 16), and eight steps of 32 n a slice
+// so that every wave has one.  The lines are from 33324 calls of 1 ... 48 rows (all formats, K and N 512 ... 14336), the time over that of the other
+// kernels: up to 16 rows from 4 M weights 0.757 (float16), from 6 M 0.773 (bfloat16), one in a thousand 2 % slower; 17 ... 32 rows from 6 M
+// 0.843 (float16; 1 % of them 2 % slower), from 30 M 0.756 (bfloat16, whose float32 products keep the vector unit busy twice as long; 2 %);
+// 33 ... 48 rows from 30 M 0.80 (float16); below these lines, and from 33 rows with bfloat16, it falls behind (1 ... 1.5).
+inline int dgrad_rows_slices(int64_t M, int64_t N, int64_t K, int dtype, size_t need) {
+    const int64_t weights = N * K, m = 1000000;
+    if (M > (dtype == BW_F16 ? 48 : 32) || weights < (M <= 16 ? dtype == BW_F16 ? 4 * m : 6 * m : M <= 32 && dtype == BW_F16 ? 6 * m : 30 * m)) return 0;
+    const int64_t strips = (K + 255) / 256, steps = (N + 31) / 32, room = (int64_t)(need / ((size_t)M * K * sizeof(float)));
+    int64_t s = dgrad_cus() / strips;
+    if (s > room) s = room;
+    if (s > (steps + 7) / 8) s = (steps + 7) / 8;
+    if (s < 2) return 0;
+    const int64_t per = (steps + s - 1) / s;
+    return (int)((steps + per - 1) / per);
+}
+
 #ifdef BW_TUNE
 static int g_dgrad_force = 0;                              // measurement builds: 1 = stepping kernel, 16 / 8 = the 256 x 256 kernel with 256 / 128 rows
 extern "C" void bw_tune_dgrad_kernel(int kind) { g_dgrad_force = kind; }
@@ -779,9 +798,26 @@ int launch_dgrad(DgradArgs a, void* workspace, size_t workspace_bytes, hipStream
     if (g_dgrad_force == 8) return launch_dgrad256<BITS, GROUP, DT, 8>(a, workspace, workspace_bytes, stream);
     if (g_dgrad_force != 1)
 #endif
-    if (const int rows = bw_aligned(a.go, 16) ? dgrad_use256(a.M, a.N, a.K, a.ldg, BITS, GROUP, workspace != nullptr) : 0)
-        return rows == QM ? launch_dgrad256<BITS, GROUP, DT, 16>(a, workspace, workspace_bytes, stream)
-                          : launch_dgrad256<BITS, GROUP, DT, 8>(a, workspace, workspace_bytes, stream);
+    {
+        const int rows = bw_aligned(a.go, 16) ? dgrad_use256(a.M, a.N, a.K, a.ldg, BITS, GROUP, workspace != nullptr) : 0;
+        const size_t need = rows ? dgrad256_plan(a.M, a.N, a.K, workspace != nullptr, rows).ws_bytes : dgrad_plan(a.M, a.N, a.K, workspace != nullptr).ws_bytes;
+        if (need > workspace_bytes) return BW_EWORKSPACE;
+        const int64_t lim = (int64_t)1 << 31;
+        const bool takes = a.M <= 48 && a.N % 8 == 0 && a.groups % 2 == 0 && a.ldg % 8 == 0 && bw_aligned(a.go, 16) && bw_aligned(a.scale, 4) && bw_aligned(a.zp, 4) &&
+                           (int64_t)a.N * a.row_bytes < lim && (int64_t)a.M * a.ldg * 2 < lim && (int64_t)a.N * a.groups * 2 < lim;
+        if (const int slices = takes ? dgrad_rows_slices(a.M, a.N, a.K, DT, need) : 0) {
+            DgradRowsArgs r;
+            r.go = a.go; r.qweight = a.qweight; r.scale = a.scale; r.zp = a.zp; r.gx = a.gx; r.ws = (float*)workspace;
+            r.M = a.M; r.N = a.N; r.K = a.K; r.ldg = a.ldg; r.ldx = a.ldx; r.groups = a.groups; r.row_bytes = a.row_bytes;
+            r.splits = slices;
+            r.steps_per_split = ((a.N + 31) / 32 + slices - 1) / slices;
+            r.go_bytes = (uint32_t)((((int64_t)a.M - 1) * a.ldg + a.N) * 2);
+            r.w_bytes = (uint32_t)((int64_t)a.N * a.row_bytes);
+            r.meta_bytes = (uint32_t)((int64_t)a.N * a.groups * 2);
+            return bw_launch_dgrad_rows(r, BITS, GROUP, DT, stream);
+        }
+        if (rows) return rows == QM ? launch_dgrad256<BITS, GROUP, DT, 16>(a, workspace, workspace_bytes, stream) : launch_dgrad256<BITS, GROUP, DT, 8>(a, workspace, workspace_bytes, stream);
+    }
     const DgradPlan p = dgrad_plan(a.M, a.N, a.K, workspace != nullptr);
     if (p.ws_bytes > workspace_bytes) return BW_EWORKSPACE;
     a.ws = (float*)workspace;
