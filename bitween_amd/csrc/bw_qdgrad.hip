@@ -29,6 +29,8 @@
 // problems run qdgrad256_kernel further down: 256 columns of k per tile and 256 or 128 rows of m, one wave per SIMD,
 // steps of 64 rows of n with the side work dealt out between the wave's own MFMAs - the forward kernel's natural-order
 // schedule turned around.  dgrad256_rows() holds the measured rule that picks between them.
+// Up to 48 rows both spend their time on the transposition: large enough layers run the kernel of bw_qdgrad_rows.hip, which needs none
+// (dgrad_rows_slices() holds the rule).
 #include <hip/hip_runtime.h>
 
 #include "bw_common.h"

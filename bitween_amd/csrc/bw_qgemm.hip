@@ -46,6 +46,8 @@ inline bool gemm_nat(int64_t M, int64_t K, int64_t ldx) {
 
 struct GemmTile { int rows, cols; };
 
+constexpr size_t kScratchBytes = (size_t)32 << 20;       // bw_qgemm_static's device array: 256 partial tiles of 128 x 256 floats, one full round
+
 // Tile of 256 columns for this call.  Calls of at most 64 rows take 64-row tiles: half the MFMAs and half the activation
 // traffic of a 128-row tile that would be at least half padding (17 ... 64 rows on the five Llama MLP / attention shapes at
 // 4 bits: 0.84-0.95 of the 128-row time, same bits).  A 256-row tile unpacks every weight once for twice the rows and keeps the matrix pipe
@@ -123,6 +125,8 @@ inline GemmTile gemm_tile(int64_t M, int64_t N, int64_t K, int64_t ldx, int bits
         float us = gemm_us(M, N, K, bits, group, wide, have_workspace) * (wide.rows == 256 && nchunks < 8 ? 0.9f : 0.95f);
         for (const int rows : {128, 256}) {
             const GemmTile narrow = {rows, tile_cols(3)};
+            // (no plan that bw_qgemm_static could not run: its results are bw_qgemm_ws's bit for bit)
+            if (have_workspace && gemm_plan(M, N, nchunks, true, rows, narrow.cols).ws_bytes > kScratchBytes) continue;
             const float t = gemm_us(M, N, K, bits, group, narrow, have_workspace);
             if (t < us) { b = narrow; us = t; }
         }
@@ -318,7 +322,6 @@ extern "C" int bw_qgemm_ws(const void* x, int act_dtype, int64_t M, int64_t K, i
 // ---- the same without a caller's workspace: the split-K partial tiles go to a device array of the library ----
 // For callers that cannot allocate (code under graph capture, serving loops, harnesses that forbid it).  The array
 // is one per GPU, shared by every call on that GPU and kept for the life of the process.
-constexpr size_t kScratchBytes = (size_t)32 << 20;       // 256 partial tiles of 128 x 256 floats: one full round
 static __device__ __align__(256) unsigned char scratch[kScratchBytes];
 constexpr int kMaxDevices = 64;
 static std::atomic<void*> g_scratch_ptr[kMaxDevices];    // device address of `scratch` on each GPU, looked up once
@@ -335,7 +338,7 @@ extern "C" int bw_qgemm_static(const void* x, int act_dtype, int64_t M, int64_t 
         if (hipGetSymbolAddress(&ptr, HIP_SYMBOL(scratch)) != hipSuccess || !ptr) return BW_ELAUNCH;
         g_scratch_ptr[dev].store(ptr, std::memory_order_release);
     }
-    // (a plan of 192-column tiles that needs more than the array is passed over for the 256-column tiles)
+    // (plans of 192-column tiles always fit)
     const bool fast = bw_shape_ok(N, K, bits, group) && M >= 1 && M < ((int64_t)1 << 31) && bw_fast_shape(M, N, K, K, bits, group);
     if (fast && gemm_wide_ws_bytes(M, N, K, bits) > kScratchBytes) return BW_EWORKSPACE;
     return bw_qgemm_ws(x, act_dtype, M, K, ldx, qweight, scale16, zp16, bias, N, bits, group, y, ldy, ptr, kScratchBytes, stream);

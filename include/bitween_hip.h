@@ -133,7 +133,7 @@ size_t bw_qgemm_workspace_bytes(int64_t M, int64_t N, int64_t K, int bits, int g
 
 /* Rows of the output tile the prefill kernel runs this shape with (x rows K apart, any workspace it asks for granted):
  * 64 (up to 64 rows, and up to 128 where N is at most 16 tiles of 256 wide), 128, or 256 once a grid of 256-row tiles fills most of the
- * device; 0 = the shape-generic kernel.
+ * device; 0 = the shape-generic kernel.  (128- and 256-row tiles are 256 or 192 columns wide, which this does not tell.)
  * A diagnostic for benchmarks and tests; no counterpart in the reference. */
 int bw_qgemm_tile_rows(int64_t M, int64_t N, int64_t K, int bits, int group);
 
@@ -199,7 +199,9 @@ int bw_cast_bf16_f16(const void* x, int64_t rows, int64_t cols, int64_t ldx, voi
  * When M * K is small the reduction over N is cut into slices whose float32 partial sums go through a
  * caller-provided workspace of bw_qdgrad_workspace_bytes(...) bytes (16-byte aligned; 0 = none needed);
  * workspace == NULL runs unsliced.
- * Two kernels: one that owns 128 or 256 x 128 tiles of grad_x and walks N in steps of 32 rows, and - for
+ * Up to 48 rows of a large enough layer (N a multiple of 8, an even number of groups, 16-byte rows of grad_y, a workspace) a kernel that
+ * unpacks the weights straight to operand layout runs, in the workspace of the others.  Else
+ * two kernels: one that owns 128 or 256 x 128 tiles of grad_x and walks N in steps of 32 rows, and - for
  * large problems with K % 256 == 0 and N % 64 == 0 - one with 256 x 256 tiles and steps of 64 rows;
  * bw_qdgrad_tile_rows tells which a shape gets (128, 256; 129, 257 = the 256 x 256 kernel with 128 (up to 512 rows of
  * grad_y) or 256 rows of m per tile; 0 = no fused path): a diagnostic,

@@ -83,3 +83,20 @@ def test_tiles_the_library_chooses(bits, g, m, n, k):
     cols = np.unique(np.clip(np.concatenate([np.arange(0, n, 331)] + [e + np.arange(-1, 2) for e in (48, 64, 192, 256, n - n % 192, n)]), 0, n - 1))
     part = [t[torch.from_numpy(cols).cuda()].cpu().numpy() for t in (q.qweight, q.scale, q.zero_point, q.bias)]
     check_matmul(y[:, torch.from_numpy(cols).cuda()], x.cpu().numpy(), *part, bits, g)
+
+
+@pytest.mark.parametrize("m,n,k", [(1255, 4656, 12160), (467, 12000, 11904), (300, 4096, 4096)])
+def test_the_librarys_own_array_runs_the_same_plan(m, n, k):
+    """bw_qgemm_static gives the bits of bw_qgemm_ws with all the workspace it asks for: no plan of 192-column tiles needs more than the 32 MiB array
+    (the first two would, with 256 rows, and were accepted before)."""
+    import bitween_amd
+    from bitween_amd.kernels import hip_loader
+    lib = hip_loader.load()
+    q = bitween_amd.QuantizedLinear.from_float(torch.nn.Linear(k, n, bias=True, device="cuda", dtype=torch.float16), 4, 128)
+    x = torch.randn(m, k, device="cuda", dtype=torch.float16)
+    y = _run(lib, x, (q.qweight, q.scale, q.zero_point), q.bias, n, 4, 128, n, with_workspace=True)
+    z = torch.empty_like(y)
+    st = lib.bw_qgemm_static(x.data_ptr(), 0, m, k, k, q.qweight.data_ptr(), q.scale.data_ptr(), q.zero_point.data_ptr(), q.bias.data_ptr(), n, 4, 128,
+                             z.data_ptr(), n, ctypes.c_void_p(torch.cuda.current_stream().cuda_stream))
+    torch.cuda.synchronize()
+    assert st == 0 and torch.equal(y, z)
