@@ -771,9 +771,9 @@ inline int dgrad_use256(int64_t M, int64_t N, int64_t K, int64_t ldg, int bits, 
 }
 
 // Slices of N for the kernel of a few rows (bw_qdgrad_rows.hip) in a workspace of `need` bytes, the one that the plan of the others asks for; 0 =
-// the others run.  One workgroup a CU at most (4096 <- 4096 at 16 rows: 8 or 16 slices of 16 strips of K 11 us, 24 slices 16), and eight steps of 32 n a slice
-// so that every wave has one.  The lines are from 33324 calls of 1 ... 48 rows (all formats, K and N 512 ... 14336), the time over that of the other
-// kernels: up to 16 rows from 4 M weights 0.757 (float16), from 6 M 0.773 (bfloat16), one in a thousand 2 % slower; 17 ... 32 rows from 6 M
+// the others run.  One workgroup a CU at most (4096 <- 4096 at 16 rows: 8 or 16 slices of 16 strips of K 11 us, 24 slices 16), and eight steps of 32 n a slice,
+// two for a wave.  The lines are from 33324 calls of 1 ... 48 rows (all formats, K and N 512 ... 14336), the time over that of the other
+// kernels with eight waves a workgroup (four, as now, take 0.9 ... 0.97 of it on large layers and as long on small ones): up to 16 rows from 4 M weights 0.757 (float16), from 6 M 0.773 (bfloat16), one in a thousand 2 % slower; 17 ... 32 rows from 6 M
 // 0.843 (float16; 1 % of them 2 % slower), from 30 M 0.756 (bfloat16, whose float32 products keep the vector unit busy twice as long; 2 %);
 // 33 ... 48 rows from 30 M 0.80 (float16); below these lines, and from 33 rows with bfloat16, it falls behind (1 ... 1.5).
 inline int dgrad_rows_slices(int64_t M, int64_t N, int64_t K, int dtype, size_t need) {

@@ -10,7 +10,7 @@
 //     requested ahead, 16 lanes to the 128 bytes (4 bits) of a row.  Scales and zero points of a step - two, four or eight groups of 32
 //     rows - come in 32 lanes to an array and are turned to [group][n] in the wave's own LDS.
 //   * What bounds it now: the unpack (28 vector instructions for 16 weights, pairs included) and the sums of the waves, 64 KB a workgroup for 16
-//     rows; 16 rows of 4096 <- 11008 take 12 us here and 3 in the reduction, of which the weights' way out of HBM is 3.5.
+//     rows; 16 rows of 4096 <- 11008 take 11 us here and 3 in the reduction, of which the weights' way out of HBM is 3.5.
 //   * The waves' sums meet in LDS, sixteen rows of m at a time; slices of N go through the caller's workspace and qdgrad_rows_reduce_kernel.
 #include "bw_qdgrad_rows.h"
 
@@ -31,13 +31,13 @@ BW_DEV __amdgpu_buffer_rsrc_t rows_rsrc(const void* p, uint32_t bytes) {
     return __builtin_amdgcn_make_buffer_rsrc(const_cast<void*>(p), (short)0, (int)bytes, 0x00020000);
 }
 
-constexpr int RK = 256, RN = 32;                         // columns of a workgroup, n of a step
-
-constexpr int rows_waves(int mt) { return mt <= 2 ? 8 : 4; }   // 64 accumulation registers a row tile: 256 or 512 registers a wave
+// Columns of a workgroup, n of a step, waves.  Eight waves write twice the sums into LDS and read them back: 16 rows of 4096 <- 4096 11.3 us, with four
+// waves 10.4; 4096 <- 11008 15.5 and 14.2; 32 rows 14.4 and 13.2, 19.3 and 17.8 (W4 g128).
+constexpr int RK = 256, RN = 32, RW = 4;
 
 template <int BITS, int GROUP, int DT, int MT>
-__global__ __launch_bounds__(64 * rows_waves(MT), rows_waves(MT) / 4) void qdgrad_rows_kernel(const DgradRowsArgs a) {
-    constexpr int W = rows_waves(MT), GS = RK / GROUP, LANE_BYTES = 2 * BITS, WORDS = LANE_BYTES / 4;
+__global__ __launch_bounds__(64 * RW, MT <= 2 ? 2 : 1) void qdgrad_rows_kernel(const DgradRowsArgs a) {
+    constexpr int W = RW, GS = RK / GROUP, LANE_BYTES = 2 * BITS, WORDS = LANE_BYTES / 4;
     constexpr uint32_t kOob = 0x80000000u;
     constexpr int META = 2 * GS * RN * 2;                              // a wave's scales and zero points of a step, [array][group][n]
     extern __shared__ __attribute__((aligned(16))) char smem[];
@@ -233,12 +233,12 @@ __global__ __launch_bounds__(256) void qdgrad_rows_reduce_kernel(const float* __
 
 template <int BITS, int GROUP, int DT, int MT>
 int launch_rows(const DgradRowsArgs& a, hipStream_t stream) {
-    constexpr int W = rows_waves(MT), LDS = W * 16 * (RK / 4 + 1) * 16;
+    constexpr int LDS = RW * 16 * (RK / 4 + 1) * 16;
     static_assert(LDS <= 160 * 1024 && 2 * (RK / GROUP) * RN * 2 <= 16 * (RK / 4 + 1) * 16, "a wave's scales lie where its sums go later");
     auto kern = qdgrad_rows_kernel<BITS, GROUP, DT, MT>;
     static uint64_t big_lds_devices = 0;                   // per instantiation
     if (LDS > 64 * 1024 && !bw_allow_big_lds(reinterpret_cast<const void*>(kern), big_lds_devices)) return BW_ELAUNCH;
-    hipLaunchKernelGGL(kern, dim3((unsigned)((a.K + RK - 1) / RK * a.splits)), dim3(64 * W), LDS, stream, a);
+    hipLaunchKernelGGL(kern, dim3((unsigned)((a.K + RK - 1) / RK * a.splits)), dim3(64 * RW), LDS, stream, a);
     if (hipGetLastError() != hipSuccess) return BW_ELAUNCH;
     if (a.splits > 1) {
         hipLaunchKernelGGL(qdgrad_rows_reduce_kernel<DT>, dim3((unsigned)(((int64_t)a.M * (a.K / 4) + 255) / 256)), dim3(256), 0, stream, a.ws, a.gx, a.M, a.K, a.ldx, a.splits);
