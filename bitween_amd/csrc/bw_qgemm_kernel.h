@@ -139,13 +139,16 @@ BW_DEV void lds_read_b128(h8& dst, uint32_t addr) {
     asm volatile("ds_read_b128 %0, %1 offset:%2" : "=v"(dst) : "v"(addr), "n"(OFF));
 }
 
-// LDS operations of a wave younger than the read of slot S's activation fragment when slot S begins: a K step starts with the reads of
-// its first RING slots; every slot then ends with the read of slot S + RING, and with PW > 0 the first slot of each of the four regions of an
-// MFMA step (MT slots) hands over PW words before that.  The words a slot's unpack takes were handed over one MFMA step earlier and
-// have to be there too.  At most what the counter can express: a smaller number waits for more.
-// gap of its region in which a tile's first word is handed over: with three column tiles regions begin inside slots, and the words have to lie
-// in the slot in which their unpack begins, or before
+// Gap of its region in which a tile's first word is handed over: with three column tiles regions begin inside slots, and the words have to lie
+// in the slot in which their unpack begins, or before.
 constexpr int hand_gap(int nt) { return nt == 4 ? 1 : 0; }
+
+// LDS operations of a wave younger than the read of slot S's activation fragment when slot S begins: a K step starts with the reads of
+// its first RING slots; every slot then ends with the read of slot S + RING, and with PW > 0 each of the NT regions of an
+// MFMA step (MT slots of NT gaps, a region MT gaps) hands over PW words from its gap hand_gap on, before the read of the same slot.  The words
+// a slot's unpack takes were handed over one MFMA step earlier and have to be there too.  A smaller number waits for more; kLgkmNone, the most that the
+// counter's four bits hold, waits for nothing, so one less is the largest (8 bits, tiles of 128 x 256: the odd slots 7 ... 23 have 15 younger ones).
+constexpr int kLgkmNone = 15;
 
 template <int RING, int SLOTS, int MT, int NT, int PW>
 constexpr int frag_younger(int S) {
@@ -162,7 +165,7 @@ constexpr int frag_younger(int S) {
         for (int q = S - MT; q < S; q++) m += (q + RING < SLOTS ? 1 : 0) + (q > S - MT ? handed(q) : 0);
         n = n < m ? n : m;
     }
-    return n < 15 ? n : 15;
+    return n < kLgkmNone ? n : kLgkmNone - 1;
 }
 
 BW_DEV void tile_coords(int tile, const GemmArgs& a, int& tm, int& tn) {
@@ -548,7 +551,11 @@ __global__ __launch_bounds__(WAVES * 64) void qgemm_kernel(const GemmArgs a) {
                 constexpr int g = decltype(gcnt)::value, i = g / NT, j = g % NT, r = g / RG, k = g % RG;
                 constexpr int S = MT * t + i;
                 __builtin_amdgcn_sched_barrier(0);
-                if constexpr (j == 0) __builtin_amdgcn_s_waitcnt(0xC07F | (frag_younger<C::XRING, MT * C::MF, MT, NT, QW ? PW : 0>(S) << 8));
+                if constexpr (j == 0) {
+                    constexpr int younger = frag_younger<C::XRING, MT * C::MF, MT, NT, QW ? PW : 0>(S);
+                    static_assert(younger >= 0 && younger < kLgkmNone, "every slot waits for its fragment");
+                    __builtin_amdgcn_s_waitcnt(0xC07F | (younger << 8));
+                }
                 mfma_acc(acc[i][j], pack_h8(wf[cu][j]), xf[0][(MT * t + i) % C::XRING]);
                 __builtin_amdgcn_sched_barrier(0);
                 // ---- unpack of n-tile r: instruction v of its sequence ----
