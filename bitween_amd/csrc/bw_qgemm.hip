@@ -270,6 +270,13 @@ extern "C" size_t bw_qgemm_workspace_bytes(int64_t M, int64_t N, int64_t K, int 
     return chosen > need ? chosen : need;
 }
 
+// Least workspace with which bw_qgemm_ws runs this shape cut along K (0 = not at all, or only with the tile of bw_qgemm_workspace_bytes): below what
+// that asks for, the tiles of 256 columns take over.
+size_t bw_qgemm_least_workspace_bytes(int64_t M, int64_t N, int64_t K, int bits, int group) {
+    if (!bw_shape_ok(N, K, bits, group) || M < 1 || M >= ((int64_t)1 << 31) || !bw_fast_shape(M, N, K, K, bits, group)) return 0;
+    return gemm_wide_ws_bytes(M, N, K, bits);
+}
+
 extern "C" int bw_qgemm_tile_rows(int64_t M, int64_t N, int64_t K, int bits, int group) {
     if (!bw_shape_ok(N, K, bits, group) || M < 1 || M >= ((int64_t)1 << 31) || !bw_fast_shape(M, N, K, K, bits, group)) return 0;
     return gemm_tile(M, N, K, K, bits, group, true, ~(size_t)0).rows;

@@ -100,3 +100,30 @@ def test_the_librarys_own_array_runs_the_same_plan(m, n, k):
                              z.data_ptr(), n, ctypes.c_void_p(torch.cuda.current_stream().cuda_stream))
     torch.cuda.synchronize()
     assert st == 0 and torch.equal(y, z)
+
+
+@pytest.mark.parametrize("m,n,k,bits,g", [(214, 11232, 2944, 4, 128), (198, 11184, 3072, 4, 64), (210, 11184, 3200, 8, 32)])
+@pytest.mark.parametrize("dtype", [torch.float16, torch.bfloat16])
+def test_a_smaller_workspace_still_cuts_k(m, n, k, bits, g, dtype):
+    """bw_qlinear_ws with 16 bytes less than the chosen plan of 192-column tiles asks for: the cut plan of the 256-column tiles runs, bit for bit
+    bw_qgemm_ws's, and not the uncut one (which leaves the workspace alone)."""
+    import bitween_amd
+    from bitween_amd.kernels import hip_loader
+    lib = hip_loader.load()
+    torch.manual_seed(k)
+    q = bitween_amd.QuantizedLinear.from_float(torch.nn.Linear(k, n, bias=True, device="cuda", dtype=torch.float16), bits, g)
+    x = torch.randn(m, k, device="cuda").to(dtype)
+    bf16 = int(dtype == torch.bfloat16)
+    full = lib.bw_qlinear_workspace_bytes(m, n, k, bits, g, bf16)
+    cast = full - lib.bw_qgemm_workspace_bytes(m, n, k, bits, g)
+    assert cast == (-(-m * k * 2 // 256) * 256 if bf16 else 0), "case is meant to run on the prefill kernel"
+    args = [t.data_ptr() for t in (q.qweight, q.scale, q.zero_point, q.bias)]
+    st = ctypes.c_void_p(torch.cuda.current_stream().cuda_stream)
+    y, z = (torch.empty(m, n, dtype=torch.float16, device="cuda") for _ in range(2))
+    ws, other = (torch.full((full,), 85, dtype=torch.uint8, device="cuda") for _ in range(2))
+    assert lib.bw_qlinear_ws(x.data_ptr(), bf16, m, k, k, *args, n, bits, g, y.data_ptr(), n, ws.data_ptr(), full - 16, st) == 0
+    x16 = x.half()
+    assert lib.bw_qgemm_ws(x16.data_ptr(), 0, m, k, k, *args, n, bits, g, z.data_ptr(), n, other.data_ptr(), full - cast - 16, st) == 0
+    torch.cuda.synchronize()
+    assert torch.equal(y, z) and (ws[full - 16:] == 85).all()
+    assert not (ws[cast:cast + 65536] == 85).all(), "the cut needs its partial sums in the workspace"
