@@ -260,8 +260,9 @@ template <int BITS, int GROUP, int MT, int NT, bool LINES>
 __global__ __launch_bounds__(1024) void qgemv_tiles_kernel(const GemvArgs a) {
     using C = GemvCfg<BITS, GROUP, MT>;
     constexpr int KBW = BITS == 4 ? 2 : (BITS == 8 ? 4 : 1);     // chunks per wave: 256 values of K
-    constexpr int BK = KBW * C::CHUNK_K, PITCH = BK + 8, UPR = BK / C::UNIT, XL = (MT * UPR + 63) / 64;
+    constexpr int BK = KBW * C::CHUNK_K, PITCH = BK + 8, UPR = BK / C::UNIT, XL = MT * UPR / 64;
     constexpr int X_BYTES = MT * PITCH * 2, UW = C::UNIT / 8, XF = KBW * C::MF;
+    static_assert(MT * UPR % 64 == 0, "x is staged in whole units of 64 lanes");
     static_assert(!LINES || (BITS == 4 && X_BYTES >= 16 * 128), "a wave's 256 values are one line of a row; a tile of them fits its x tile");
     constexpr int kOutPerTile = 16 * MT;
     constexpr uint32_t kOob = 0x80000000u;
@@ -319,7 +320,7 @@ __global__ __launch_bounds__(1024) void qgemv_tiles_kernel(const GemvArgs a) {
 #pragma unroll
     for (int j = 0; j < XL; j++) {
         const int jr = j + xrot < XL ? j + xrot : j + xrot - XL;
-        const int u = lane + 64 * jr, m = u / UPR, k = wave * BK + (u - m * UPR) * C::UNIT;
+        const int u = lane + 64 * jr, m = (uint32_t)u / UPR, k = wave * BK + (uint32_t)u % UPR * C::UNIT;
         uint32_t off = (uint32_t)(m * a.ldx + k) * 2;
         asm volatile("" : "+v"(off));
         off = (m < a.M && k < a.K) ? off : kOob;
@@ -360,37 +361,36 @@ __global__ __launch_bounds__(1024) void qgemv_tiles_kernel(const GemvArgs a) {
         }
         if (lane == 0) __hip_atomic_fetch_add(ready, 1u, __ATOMIC_RELEASE, __HIP_MEMORY_SCOPE_WORKGROUP);
     }
-    // ---- x -> this wave's LDS tile, permuted to the unpack order
+    // ---- x -> this wave's LDS tile, permuted to the unpack order (a unit's row and place from unsigned numbers, here and above: from signed ones the
+    // compiler may make a branch and a subtraction for each, 40 instructions at 16 rows)
 #pragma unroll
     for (int j = 0; j < XL; j++) {
         const int jr = j + xrot < XL ? j + xrot : j + xrot - XL;
-        const int u = lane + 64 * jr, m = u / UPR, ku = u - m * UPR;
-        if (m < MT) {
-            uint32_t in[4 * UW], o[4 * UW];
+        const int u = lane + 64 * jr, m = (uint32_t)u / UPR, ku = (uint32_t)u % UPR;
+        uint32_t in[4 * UW], o[4 * UW];
 #pragma unroll
-            for (int q = 0; q < UW; q++) { in[4 * q] = xr[j * UW + q][0]; in[4 * q + 1] = xr[j * UW + q][1]; in[4 * q + 2] = xr[j * UW + q][2]; in[4 * q + 3] = xr[j * UW + q][3]; }
-            if (a.x_bf16) {
+        for (int q = 0; q < UW; q++) { in[4 * q] = xr[j * UW + q][0]; in[4 * q + 1] = xr[j * UW + q][1]; in[4 * q + 2] = xr[j * UW + q][2]; in[4 * q + 3] = xr[j * UW + q][3]; }
+        if (a.x_bf16) {
 #pragma unroll
-                for (int q = 0; q < 4 * UW; q++) in[q] = bf16x2_to_f16x2(in[q]);
-            }
-            permute_unit<BITS>(in, o);
-            u4* dst = reinterpret_cast<u4*>(xs + m * PITCH + ku * C::UNIT);
-#pragma unroll
-            for (int q = 0; q < UW; q++) dst[q] = u4{o[4 * q], o[4 * q + 1], o[4 * q + 2], o[4 * q + 3]};
+            for (int q = 0; q < 4 * UW; q++) in[q] = bf16x2_to_f16x2(in[q]);
         }
+        permute_unit<BITS>(in, o);
+        u4* dst = reinterpret_cast<u4*>(xs + m * PITCH + ku * C::UNIT);
+#pragma unroll
+        for (int q = 0; q < UW; q++) dst[q] = u4{o[4 * q], o[4 * q + 1], o[4 * q + 2], o[4 * q + 3]};
     }
     __builtin_amdgcn_wave_barrier();
-    const int arow = nl < MT ? nl : MT - 1;              // MFMA rows >= MT repeat a valid row; never stored
     h8 xf[LINES ? XF : 1];
     if constexpr (LINES) {                               // x is the same for all tiles: its LDS is free for the weights
 #pragma unroll
-        for (int s = 0; s < XF; s++) xf[s] = *reinterpret_cast<const h8*>(xs + arow * PITCH + s / C::MF * C::CHUNK_K + kq * C::VPL + s % C::MF * 8);
+        for (int s = 0; s < XF; s++) xf[s] = *reinterpret_cast<const h8*>(xs + (nl < MT ? nl : MT - 1) * PITCH + s / C::MF * C::CHUNK_K + kq * C::VPL + s % C::MF * 8);
         asm volatile("" ::: "memory");
     }
     while (__hip_atomic_load(ready, __ATOMIC_ACQUIRE, __HIP_MEMORY_SCOPE_WORKGROUP) < (uint32_t)meta_waves) __builtin_amdgcn_s_sleep(1);
 
     // ---- the tiles, as their weights arrive
     f4 acc[NT][2];
+    const int arow = nl < MT ? nl : MT - 1;              // MFMA rows >= MT repeat a valid row; never stored
 #pragma unroll
     for (int t = 0; t < NT; t++) {
         if (t + 2 < NT) issue_w(t + 2);
