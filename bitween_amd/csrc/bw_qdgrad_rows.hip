@@ -35,8 +35,15 @@ BW_DEV __amdgpu_buffer_rsrc_t rows_rsrc(const void* p, uint32_t bytes) {
 // waves 10.4; 4096 <- 11008 15.5 and 14.2; 32 rows 14.4 and 13.2, 19.3 and 17.8 (W4 g128).
 constexpr int RK = 256, RN = 32, RW = 4;
 
+// Waves a SIMD that the registers leave room for (a grid has one workgroup a CU at most: what counts is how the compiler lays them out).  Two, as long as
+// nothing spills: a spilled register comes back through the counter of the loads and waits for all that is requested ahead.  8 bits, bfloat16, two
+// row tiles in groups of 32 and 64 do not fit (4 and 2 spilled, with two waves 1.03 ... 1.04 and 0.93 ... 0.97 of the other kernels' time on 2981 calls, with one
+// 0.79 ... 0.85 and 0.73 ... 0.81); in groups of 128 two are ahead (0.69 ... 0.77 against 0.72 ... 0.80), as at 4 and 2 bits (one takes 1.03 ... 1.07 of their time).
 template <int BITS, int GROUP, int DT, int MT>
-__global__ __launch_bounds__(64 * RW, MT <= 2 ? 2 : 1) void qdgrad_rows_kernel(const DgradRowsArgs a) {
+constexpr int rows_waves = MT > 2 || (MT == 2 && BITS == 8 && GROUP < 128 && DT == BW_BF16) ? 1 : 2;
+
+template <int BITS, int GROUP, int DT, int MT>
+__global__ __launch_bounds__(64 * RW, (rows_waves<BITS, GROUP, DT, MT>)) void qdgrad_rows_kernel(const DgradRowsArgs a) {
     constexpr int W = RW, GS = RK / GROUP, LANE_BYTES = 2 * BITS, WORDS = LANE_BYTES / 4;
     constexpr uint32_t kOob = 0x80000000u;
     constexpr int META = 2 * GS * RN * 2;                              // a wave's scales and zero points of a step, [array][group][n]

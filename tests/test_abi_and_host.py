@@ -267,3 +267,11 @@ def test_stepping_input_gradient_kernel_spills_no_registers():
     kernels = [k for k in _kernel_metadata(hip_loader.library_path()) if "qdgrad_kernel" in k[".name"]]
     assert len(kernels) == 36                                                        # formats x tile heights x gradient types
     assert not [k[".name"] for k in kernels if k[".vgpr_spill_count"] or k[".private_segment_fixed_size"]]
+
+
+def test_input_gradient_kernels_of_a_few_rows_spill_no_registers():
+    """A spilled register comes back through the counter of the loads, so that every step waits for what it has requested ahead."""
+    from bitween_amd.kernels import hip_loader
+    kernels = [k for k in _kernel_metadata(hip_loader.library_path()) if "qdgrad_rows_kernel" in k[".name"]]
+    assert len(kernels) == 45                                                        # formats x (three row tiles of float16, two of bfloat16)
+    assert not [k[".name"] for k in kernels if k[".vgpr_spill_count"] or k[".private_segment_fixed_size"]]
