@@ -770,6 +770,12 @@ inline int dgrad_use256(int64_t M, int64_t N, int64_t K, int64_t ldg, int bits, 
     return (have_workspace || tiles > dgrad_cus() / 2) ? rows : 0;
 }
 
+// calls that the kernel of a few rows can take, as far as their sizes go
+inline bool dgrad_rows_shape(int64_t M, int64_t N, int64_t K, int64_t ldg, int bits, int group) {
+    const int64_t lim = (int64_t)1 << 31, groups = K / group;
+    return M <= 48 && N % 8 == 0 && groups % 2 == 0 && ldg % 8 == 0 && N * (K * bits / 8) < lim && M * ldg * 2 < lim && N * groups * 2 < lim;
+}
+
 // Slices of N for the kernel of a few rows (bw_qdgrad_rows.hip) in a workspace of `need` bytes, the one that the plan of the others asks for; 0 =
 // the others run.  One workgroup a CU at most (4096 <- 4096 at 16 rows: 8 or 16 slices of 16 strips of K 11 us, 24 slices 16), and eight steps of 32 n a slice,
 // two for a wave.  The lines are from 33324 calls of 1 ... 48 rows (all formats, K and N 512 ... 14336), the time over that of the other
@@ -804,9 +810,7 @@ int launch_dgrad(DgradArgs a, void* workspace, size_t workspace_bytes, hipStream
         const int rows = bw_aligned(a.go, 16) ? dgrad_use256(a.M, a.N, a.K, a.ldg, BITS, GROUP, workspace != nullptr) : 0;
         const size_t need = rows ? dgrad256_plan(a.M, a.N, a.K, workspace != nullptr, rows).ws_bytes : dgrad_plan(a.M, a.N, a.K, workspace != nullptr).ws_bytes;
         if (need > workspace_bytes) return BW_EWORKSPACE;
-        const int64_t lim = (int64_t)1 << 31;
-        const bool takes = a.M <= 48 && a.N % 8 == 0 && a.groups % 2 == 0 && a.ldg % 8 == 0 && bw_aligned(a.go, 16) && bw_aligned(a.scale, 4) && bw_aligned(a.zp, 4) &&
-                           (int64_t)a.N * a.row_bytes < lim && (int64_t)a.M * a.ldg * 2 < lim && (int64_t)a.N * a.groups * 2 < lim;
+        const bool takes = dgrad_rows_shape(a.M, a.N, a.K, a.ldg, BITS, GROUP) && bw_aligned(a.go, 16) && bw_aligned(a.scale, 4) && bw_aligned(a.zp, 4);
         if (const int slices = takes ? dgrad_rows_slices(a.M, a.N, a.K, DT, need) : 0) {
             DgradRowsArgs r;
             r.go = a.go; r.qweight = a.qweight; r.scale = a.scale; r.zp = a.zp; r.gx = a.gx; r.ws = (float*)workspace;
@@ -847,6 +851,15 @@ extern "C" int bw_qdgrad_tile_rows(int64_t M, int64_t N, int64_t K, int bits, in
     if (!bw_shape_ok(N, K, bits, group) || !dgrad_fast_shape(M, N, K, N, K, bits, group)) return 0;
     if (const int rows = dgrad_use256(M, N, K, N, bits, group, true)) return rows + 1;
     return 32 * dgrad_plan(M, N, K, true).mt;
+}
+
+// Slices of N with which the kernel of a few rows (bw_qdgrad_rows.hip) runs this shape, with a workspace on offer, rows of grad_y N apart on 16 bytes and scales
+// and zero points on 4; 0 where another does.  A diagnostic.
+extern "C" int bw_qdgrad_rows_slices(int64_t M, int64_t N, int64_t K, int bits, int group, int act_dtype) {
+    if (!bw_shape_ok(N, K, bits, group) || M < 1 || (act_dtype != BW_F16 && act_dtype != BW_BF16)) return 0;
+    if (!dgrad_fast_shape(M, N, K, N, K, bits, group) || !dgrad_rows_shape(M, N, K, N, bits, group)) return 0;
+    const int rows = dgrad_use256(M, N, K, N, bits, group, true);
+    return dgrad_rows_slices(M, N, K, act_dtype, rows ? dgrad256_plan(M, N, K, true, rows).ws_bytes : dgrad_plan(M, N, K, true).ws_bytes);
 }
 
 extern "C" int bw_qdgrad(const void* grad_y, int act_dtype, int64_t M, int64_t N, int64_t ldg, const int32_t* qweight,

@@ -23,7 +23,7 @@ _DTYPE_CODE = {torch.float16: BW_F16, torch.bfloat16: BW_BF16, torch.float32: BW
 
 ABI_VERSION = 10           # what bw_abi_version() of a matching library returns
 ENTRY_POINTS = ("bw_abi_version", "bw_strerror", "bw_quantize_pack", "bw_quantize_pack_add", "bw_dequantize", "bw_qgemv", "bw_qgemm",
-                "bw_qgemm_ws", "bw_qgemm_static", "bw_qgemm_workspace_bytes", "bw_qgemm_tile_rows", "bw_qlinear", "bw_qlinear_ws", "bw_qlinear_workspace_bytes", "bw_qdgrad", "bw_qdgrad_workspace_bytes", "bw_qdgrad_tile_rows", "bw_cast_bf16_f16", "bw_qlinear_decode_rows", "bw_qgemv_last_kernel")
+                "bw_qgemm_ws", "bw_qgemm_static", "bw_qgemm_workspace_bytes", "bw_qgemm_tile_rows", "bw_qlinear", "bw_qlinear_ws", "bw_qlinear_workspace_bytes", "bw_qdgrad", "bw_qdgrad_workspace_bytes", "bw_qdgrad_tile_rows", "bw_qdgrad_rows_slices", "bw_cast_bf16_f16", "bw_qlinear_decode_rows", "bw_qgemv_last_kernel")
 
 
 class BitweenHipError(RuntimeError):
@@ -73,6 +73,8 @@ def load():
     lib.bw_qdgrad_workspace_bytes.restype = ctypes.c_size_t
     lib.bw_qdgrad_tile_rows.argtypes = [i64, i64, i64, i32, i32]
     lib.bw_qdgrad_tile_rows.restype = i32
+    lib.bw_qdgrad_rows_slices.argtypes = [i64, i64, i64, i32, i32, i32]
+    lib.bw_qdgrad_rows_slices.restype = i32
     lib.bw_qdgrad.argtypes = [vp, i32, i64, i64, i64, vp, vp, vp, i64, i32, i32, vp, i64, vp, ctypes.c_size_t, vp]
     lib.bw_qdgrad.restype = i32
     lib.bw_cast_bf16_f16.argtypes = [vp, i64, i64, i64, vp, i64, vp]

@@ -200,7 +200,8 @@ int bw_cast_bf16_f16(const void* x, int64_t rows, int64_t cols, int64_t ldx, voi
  * caller-provided workspace of bw_qdgrad_workspace_bytes(...) bytes (16-byte aligned; 0 = none needed);
  * workspace == NULL runs unsliced.
  * Up to 48 rows of a large enough layer (N a multiple of 8, an even number of groups, 16-byte rows of grad_y, a workspace) a kernel that
- * unpacks the weights straight to operand layout runs, in the workspace of the others.  Else
+ * unpacks the weights straight to operand layout runs, in the workspace of the others: bw_qdgrad_rows_slices tells in how many slices of N (rows of
+ * grad_y N apart, a workspace granted; 0 = not that kernel), whatever bw_qdgrad_tile_rows says of the shape.  Else
  * two kernels: one that owns 128 or 256 x 128 tiles of grad_x and walks N in steps of 32 rows, and - for
  * large problems with K % 256 == 0 and N % 64 == 0 - one with 256 x 256 tiles and steps of 64 rows;
  * bw_qdgrad_tile_rows tells which a shape gets (128, 256; 129, 257 = the 256 x 256 kernel with 128 (up to 512 rows of
@@ -209,6 +210,8 @@ int bw_cast_bf16_f16(const void* x, int64_t rows, int64_t cols, int64_t ldx, voi
 size_t bw_qdgrad_workspace_bytes(int64_t M, int64_t N, int64_t K, int bits, int group);
 
 int bw_qdgrad_tile_rows(int64_t M, int64_t N, int64_t K, int bits, int group);
+
+int bw_qdgrad_rows_slices(int64_t M, int64_t N, int64_t K, int bits, int group, int act_dtype);
 
 int bw_qdgrad(const void* grad_y, int act_dtype, int64_t M, int64_t N, int64_t ldg,
               const int32_t* qweight, const void* scale16, const void* zp16,

@@ -103,3 +103,14 @@ def test_input_gradient_slices_are_whole_passes(m, n, k, slices):
     need = lib.bw_qdgrad_workspace_bytes(m, n, k, 4, 64)
     assert need == -(-k // 128) * slices * m * 128 * 4                        # a partial tile is the call's m rows
     assert -(-(-(-n // 32)) // slices) % 2 == 0
+
+
+@pytest.mark.skipif(torch.cuda.is_available(), reason="the plan for 256 compute units, what the library assumes without a GPU")
+@pytest.mark.parametrize("m,n,k,bits,g,dtype,taken", [
+    (16, 1024, 4096, 4, 128, 0, True), (16, 960, 4096, 4, 128, 0, False), (16, 1472, 4096, 2, 32, 1, True), (16, 1024, 4096, 4, 128, 1, False),
+    (32, 1472, 4096, 8, 64, 0, True), (17, 1024, 4096, 4, 128, 0, False), (17, 7424, 4096, 8, 32, 1, True), (32, 6400, 4096, 4, 128, 1, False),
+    (48, 7424, 4096, 4, 128, 0, True), (33, 6400, 4096, 4, 128, 0, False), (33, 11008, 4096, 4, 128, 1, False), (49, 11008, 4096, 4, 128, 0, False),
+    (9, 6252, 4096, 4, 128, 0, False), (9, 4096, 4224, 4, 128, 0, False)])                 # n off eights, an odd number of groups
+def test_input_gradients_of_few_rows_that_have_their_own_kernel(m, n, k, bits, g, dtype, taken):
+    from bitween_amd.kernels import hip_loader
+    assert (hip_loader.load().bw_qdgrad_rows_slices(m, n, k, bits, g, dtype) > 0) == taken
