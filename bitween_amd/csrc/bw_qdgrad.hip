@@ -778,13 +778,16 @@ inline bool dgrad_rows_shape(int64_t M, int64_t N, int64_t K, int64_t ldg, int b
 
 // Slices of N for the kernel of a few rows (bw_qdgrad_rows.hip) in a workspace of `need` bytes, the one that the plan of the others asks for; 0 =
 // the others run.  One workgroup a CU at most (4096 <- 4096 at 16 rows: 8 or 16 slices of 16 strips of K 11 us, 24 slices 16), and eight steps of 32 n a slice,
-// two for a wave.  The lines are from 33324 calls of 1 ... 48 rows (all formats, K and N 512 ... 14336), the time over that of the other
-// kernels with eight waves a workgroup (four, as now, take 0.9 ... 0.97 of it on large layers and as long on small ones): up to 16 rows from 4 M weights 0.757 (float16), from 6 M 0.773 (bfloat16), one in a thousand 2 % slower; 17 ... 32 rows from 6 M
-// 0.843 (float16; 1 % of them 2 % slower), from 30 M 0.756 (bfloat16, whose float32 products keep the vector unit busy twice as long; 2 %);
-// 33 ... 48 rows from 30 M 0.80 (float16); below these lines, and from 33 rows with bfloat16, it falls behind (1 ... 1.5).
-inline int dgrad_rows_slices(int64_t M, int64_t N, int64_t K, int dtype, size_t need) {
-    const int64_t weights = N * K, m = 1000000;
-    if (M > (dtype == BW_F16 ? 48 : 32) || weights < (M <= 16 ? dtype == BW_F16 ? 4 * m : 6 * m : M <= 32 && dtype == BW_F16 ? 6 * m : 30 * m)) return 0;
+// two for a wave.
+// The lines are from 33324 calls of 1 ... 48 rows (all formats, K and N 512 ... 14336) with eight waves a workgroup; with four, as now, 20198 calls above them, half
+// of them within a factor of two of a line, take of the time of the other kernels, weights out of HBM or the Infinity Cache: up to 16 rows from 4 M weights
+// 0.762 (float16), from 6 M 0.774 (bfloat16); 17 ... 32 rows from 6 M 0.829 (float16), from 30 M 0.714 (bfloat16, whose float32 products keep the
+// vector unit busy twice as long); 33 ... 48 rows from 30 M, at 8 bits from 40 M, 0.808 (float16; 8 bits between 30 and 40 M: 0.94, but 109 of 769 calls
+// over 2 % longer, up to 1.12).  12 calls over 2 % longer, none over 8 %.  Below the lines, and from 33 rows with bfloat16, it fell behind (1 ... 1.5).
+inline int dgrad_rows_slices(int64_t M, int64_t N, int64_t K, int bits, int dtype, size_t need) {
+    const bool f16 = dtype == BW_F16;
+    const int millions = M <= 16 ? (f16 ? 4 : 6) : M <= 32 ? (f16 ? 6 : 30) : bits == 8 ? 40 : 30;
+    if (M > (f16 ? 48 : 32) || N * K < millions * (int64_t)1000000) return 0;
     const int64_t strips = (K + 255) / 256, steps = (N + 31) / 32, room = (int64_t)(need / ((size_t)M * K * sizeof(float)));
     int64_t s = dgrad_cus() / strips;
     if (s > room) s = room;
@@ -811,7 +814,7 @@ int launch_dgrad(DgradArgs a, void* workspace, size_t workspace_bytes, hipStream
         const size_t need = rows ? dgrad256_plan(a.M, a.N, a.K, workspace != nullptr, rows).ws_bytes : dgrad_plan(a.M, a.N, a.K, workspace != nullptr).ws_bytes;
         if (need > workspace_bytes) return BW_EWORKSPACE;
         const bool takes = dgrad_rows_shape(a.M, a.N, a.K, a.ldg, BITS, GROUP) && bw_aligned(a.go, 16) && bw_aligned(a.scale, 4) && bw_aligned(a.zp, 4);
-        if (const int slices = takes ? dgrad_rows_slices(a.M, a.N, a.K, DT, need) : 0) {
+        if (const int slices = takes ? dgrad_rows_slices(a.M, a.N, a.K, BITS, DT, need) : 0) {
             DgradRowsArgs r;
             r.go = a.go; r.qweight = a.qweight; r.scale = a.scale; r.zp = a.zp; r.gx = a.gx; r.ws = (float*)workspace;
             r.M = a.M; r.N = a.N; r.K = a.K; r.ldg = a.ldg; r.ldx = a.ldx; r.groups = a.groups; r.row_bytes = a.row_bytes;
@@ -859,7 +862,7 @@ extern "C" int bw_qdgrad_rows_slices(int64_t M, int64_t N, int64_t K, int bits, 
     if (!bw_shape_ok(N, K, bits, group) || M < 1 || (act_dtype != BW_F16 && act_dtype != BW_BF16)) return 0;
     if (!dgrad_fast_shape(M, N, K, N, K, bits, group) || !dgrad_rows_shape(M, N, K, N, bits, group)) return 0;
     const int rows = dgrad_use256(M, N, K, N, bits, group, true);
-    return dgrad_rows_slices(M, N, K, act_dtype, rows ? dgrad256_plan(M, N, K, true, rows).ws_bytes : dgrad_plan(M, N, K, true).ws_bytes);
+    return dgrad_rows_slices(M, N, K, bits, act_dtype, rows ? dgrad256_plan(M, N, K, true, rows).ws_bytes : dgrad_plan(M, N, K, true).ws_bytes);
 }
 
 extern "C" int bw_qdgrad(const void* grad_y, int act_dtype, int64_t M, int64_t N, int64_t ldg, const int32_t* qweight,

@@ -110,6 +110,7 @@ def test_input_gradient_slices_are_whole_passes(m, n, k, slices):
     (16, 1024, 4096, 4, 128, 0, True), (16, 960, 4096, 4, 128, 0, False), (16, 1472, 4096, 2, 32, 1, True), (16, 1024, 4096, 4, 128, 1, False),
     (32, 1472, 4096, 8, 64, 0, True), (17, 1024, 4096, 4, 128, 0, False), (17, 7424, 4096, 8, 32, 1, True), (32, 6400, 4096, 4, 128, 1, False),
     (48, 7424, 4096, 4, 128, 0, True), (33, 6400, 4096, 4, 128, 0, False), (33, 11008, 4096, 4, 128, 1, False), (49, 11008, 4096, 4, 128, 0, False),
+    (40, 8192, 4096, 8, 32, 0, False), (48, 9792, 4096, 8, 32, 0, True), (40, 8192, 4096, 2, 32, 0, True),
     (9, 6252, 4096, 4, 128, 0, False), (9, 4096, 4224, 4, 128, 0, False)])                 # n off eights, an odd number of groups
 def test_input_gradients_of_few_rows_that_have_their_own_kernel(m, n, k, bits, g, dtype, taken):
     from bitween_amd.kernels import hip_loader
