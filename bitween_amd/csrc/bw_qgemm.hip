@@ -282,6 +282,11 @@ extern "C" int bw_qgemm_tile_rows(int64_t M, int64_t N, int64_t K, int bits, int
     return gemm_tile(M, N, K, K, bits, group, true, ~(size_t)0).rows;
 }
 
+extern "C" int bw_qgemm_tile_cols(int64_t M, int64_t N, int64_t K, int bits, int group) {
+    if (!bw_shape_ok(N, K, bits, group) || M < 1 || M >= ((int64_t)1 << 31) || !bw_fast_shape(M, N, K, K, bits, group)) return 0;
+    return gemm_tile(M, N, K, K, bits, group, true, ~(size_t)0).cols;
+}
+
 extern "C" int bw_qgemm_ws(const void* x, int act_dtype, int64_t M, int64_t K, int64_t ldx, const int32_t* qweight,
                            const void* scale16, const void* zp16, const void* bias, int64_t N, int bits, int group,
                            void* y, int64_t ldy, void* workspace, size_t workspace_bytes, void* stream) {

@@ -23,7 +23,7 @@ _DTYPE_CODE = {torch.float16: BW_F16, torch.bfloat16: BW_BF16, torch.float32: BW
 
 ABI_VERSION = 10           # what bw_abi_version() of a matching library returns
 ENTRY_POINTS = ("bw_abi_version", "bw_strerror", "bw_quantize_pack", "bw_quantize_pack_add", "bw_dequantize", "bw_qgemv", "bw_qgemm",
-                "bw_qgemm_ws", "bw_qgemm_static", "bw_qgemm_workspace_bytes", "bw_qgemm_tile_rows", "bw_qlinear", "bw_qlinear_ws", "bw_qlinear_workspace_bytes", "bw_qdgrad", "bw_qdgrad_workspace_bytes", "bw_qdgrad_tile_rows", "bw_qdgrad_rows_slices", "bw_cast_bf16_f16", "bw_qlinear_decode_rows", "bw_qgemv_last_kernel")
+                "bw_qgemm_ws", "bw_qgemm_static", "bw_qgemm_workspace_bytes", "bw_qgemm_tile_rows", "bw_qgemm_tile_cols", "bw_qlinear", "bw_qlinear_ws", "bw_qlinear_workspace_bytes", "bw_qdgrad", "bw_qdgrad_workspace_bytes", "bw_qdgrad_tile_rows", "bw_qdgrad_rows_slices", "bw_cast_bf16_f16", "bw_qlinear_decode_rows", "bw_qgemv_last_kernel")
 
 
 class BitweenHipError(RuntimeError):
@@ -69,6 +69,8 @@ def load():
     lib.bw_qlinear_workspace_bytes.restype = ctypes.c_size_t
     lib.bw_qgemm_tile_rows.argtypes = [i64, i64, i64, i32, i32]
     lib.bw_qgemm_tile_rows.restype = i32
+    lib.bw_qgemm_tile_cols.argtypes = [i64, i64, i64, i32, i32]
+    lib.bw_qgemm_tile_cols.restype = i32
     lib.bw_qdgrad_workspace_bytes.argtypes = [i64, i64, i64, i32, i32]
     lib.bw_qdgrad_workspace_bytes.restype = ctypes.c_size_t
     lib.bw_qdgrad_tile_rows.argtypes = [i64, i64, i64, i32, i32]

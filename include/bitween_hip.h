@@ -131,11 +131,13 @@ int bw_qgemm(const void* x, int act_dtype, int64_t M, int64_t K, int64_t ldx,
  * GEMM, bitween/modules.py:97). */
 size_t bw_qgemm_workspace_bytes(int64_t M, int64_t N, int64_t K, int bits, int group);
 
-/* Rows of the output tile the prefill kernel runs this shape with (x rows K apart, any workspace it asks for granted):
- * 64 (up to 64 rows, and up to 128 where N is at most 16 tiles of 256 wide), 128, or 256 once a grid of 256-row tiles fills most of the
- * device; 0 = the shape-generic kernel.  (128- and 256-row tiles are 256 or 192 columns wide, which this does not tell.)
- * A diagnostic for benchmarks and tests; no counterpart in the reference. */
+/* Rows and columns of the output tile the prefill kernel runs this shape with (x rows K apart, any workspace it asks for granted):
+ * 64 rows (up to 64 rows, and up to 128 where N is at most 16 tiles of 256 wide), else 128 or 256, and of those 256 or 192 columns,
+ * whichever of the four is expected to be done first; 0 = the shape-generic kernel.
+ * Diagnostics for benchmarks and tests; no counterpart in the reference. */
 int bw_qgemm_tile_rows(int64_t M, int64_t N, int64_t K, int bits, int group);
+
+int bw_qgemm_tile_cols(int64_t M, int64_t N, int64_t K, int bits, int group);
 
 int bw_qgemm_ws(const void* x, int act_dtype, int64_t M, int64_t K, int64_t ldx,
                 const int32_t* qweight, const void* scale16, const void* zp16, const void* bias,

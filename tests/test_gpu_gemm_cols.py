@@ -1,5 +1,6 @@
-"""The prefill kernel's 192-column tiles (three column tiles a wave) against the oracle: forced through the measurement build, which takes
-the tile from the environment, and as the library chooses them."""
+"""The prefill kernel's tiles - 192 columns (three column tiles a wave) and 256 - against the oracle: forced through the measurement build, which takes
+the tile from the environment, and, every format on every tile, as the library itself chooses them (the kernel's waits are counted by hand around
+assembly: what has been compiled is what has to be run)."""
 import ctypes
 
 import numpy as np
@@ -68,6 +69,69 @@ def test_192_column_tiles_cut_along_k(monkeypatch, rows, bits, g):
     x = np.random.default_rng(rows).standard_normal((m, k)).astype(np.float16)
     d = [to_gpu(a) for a in (qw, s16, z16)]
     check_matmul(_run(lib, to_gpu(x), d, to_gpu(b16), n, bits, g, n + 3, with_workspace=True), x, qw, s16, z16, b16, bits, g)
+
+
+@pytest.mark.parametrize("rows", [64, 128, 256])
+@pytest.mark.parametrize("bits,g", FORMATS)
+@pytest.mark.parametrize("k,n,m,pad", [(128, 255, 65, 1), (256, 257, 257, 7), (384, 64, 130, 0), (640, 400, 200, 0), (896, 301, 300, 1), (1024, 576, 513, 8)])
+def test_256_column_tiles(monkeypatch, rows, bits, g, k, n, m, pad):
+    """The same for 256 columns, which small calls have given up to the narrower tiles: 8 bits hands weights over between lanes here too (64 and
+    128 rows; in groups of 32 the scales as well)."""
+    lib = _forced(monkeypatch, rows, 256)
+    _, qw, s16, z16, b16 = quantized_layer(n, k, bits, g, seed=k + n + g + bits, outliers=True)
+    x = np.random.default_rng(m).standard_normal((m, k)).astype(np.float16)
+    d = [to_gpu(a) for a in (qw, s16, z16)]
+    check_matmul(_run(lib, to_gpu(x), d, to_gpu(b16), n, bits, g, n + pad), x, qw, s16, z16, b16, bits, g)
+    cols = np.linspace(0, k - 1, m).astype(int)
+    hot = np.zeros((m, k), np.float16)
+    hot[np.arange(m), cols] = 1
+    y = _run(lib, to_gpu(hot), d, None, n, bits, g, n + pad)
+    assert np.array_equal(y.cpu().numpy(), orc.dequantize_f16(qw, s16, z16, g, bits)[:, cols].T)
+
+
+@pytest.mark.parametrize("rows", [64, 128])
+@pytest.mark.parametrize("g", [32, 64, 128])
+def test_256_column_tiles_of_8_bits_cut_along_k(monkeypatch, rows, g):
+    bits, n, k, m = 8, 401, 128 * 22, 300
+    lib = _forced(monkeypatch, rows, 256)
+    assert lib.bw_qgemm_workspace_bytes(m, n, k, bits, g) > 0
+    _, qw, s16, z16, b16 = quantized_layer(n, k, bits, g, seed=rows + g, outliers=True)
+    x = np.random.default_rng(rows).standard_normal((m, k)).astype(np.float16)
+    d = [to_gpu(a) for a in (qw, s16, z16)]
+    check_matmul(_run(lib, to_gpu(x), d, to_gpu(b16), n, bits, g, n + 3, with_workspace=True), x, qw, s16, z16, b16, bits, g)
+
+
+# rows, columns of the tile: calls that get it for some K of the list below (256 compute units), and whether K is cut
+TILES = [(64, 256, [(65, 301), (113, 517)]), (128, 192, [(139, 301), (80, 4505)]), (128, 256, [(1400, 197), (816, 194), (1200, 203), (69, 9721), (66, 5840)]),
+         (256, 192, [(1900, 9601), (2213, 8223), (2743, 6607)]), (256, 256, [(1180, 9860), (1060, 11078), (2563, 4654), (2907, 4511), (1159, 9877)])]
+
+
+@pytest.mark.parametrize("bits,g", FORMATS)
+@pytest.mark.parametrize("rows,cols,calls", TILES, ids=["%dx%d" % t[:2] for t in TILES])
+def test_every_tile_of_the_library_itself(rows, cols, calls, bits, g):
+    """The first call of the list that gets the tile with more than two K steps, else with two: one-hot rows return columns of W16 bit for bit,
+    random rows agree with the library product of W16 everywhere and with the oracle on samples."""
+    from bitween_amd.kernels import hip_loader
+    lib = hip_loader.load()
+    if torch.cuda.get_device_properties(0).multi_processor_count != 256:
+        pytest.skip("which tile a call gets depends on the number of compute units")
+    picked = [(m, n, k) for k in (1152, 640, 384, 2560, 3072, 4096, 256) for m, n in calls
+              if (lib.bw_qgemm_tile_rows(m, n, k, bits, g), lib.bw_qgemm_tile_cols(m, n, k, bits, g)) == (rows, cols)]
+    assert picked, "no call of the list has this tile any more"
+    m, n, k = picked[0]
+    _, qw, s16, z16, b16 = quantized_layer(n, k, bits, g, seed=m + n + g, outliers=True)
+    d = [to_gpu(a) for a in (qw, s16, z16)]
+    w16 = to_gpu(orc.dequantize_f16(qw, s16, z16, g, bits))
+    at = torch.linspace(0, k - 1, m).long().cuda()
+    hot = torch.zeros(m, k, dtype=torch.float16, device="cuda")
+    hot[torch.arange(m, device="cuda"), at] = 1
+    assert torch.equal(_run(lib, hot, d, None, n, bits, g, n + 1, with_workspace=True), w16[:, at].T)
+    x = torch.randn(m, k, device="cuda").half()
+    y = _run(lib, x, d, to_gpu(b16), n, bits, g, n, with_workspace=True)
+    ref = (x @ w16.T).float() + to_gpu(b16).float()
+    assert ((y.float() - ref).abs().max() <= 2.0 ** -8 * ref.abs().max()).item()
+    sample = torch.unique(torch.cat([torch.arange(0, m, max(1, m // 24)), torch.arange(m - 3, m)]))
+    check_matmul(y[sample.cuda()], x[sample.cuda()].cpu().numpy(), qw, s16, z16, b16, bits, g)
 
 
 @pytest.mark.parametrize("bits,g,m,n,k", [(8, 32, 509, 11008, 4096), (4, 128, 1000, 11008, 4096), (4, 64, 160, 6000, 2048)])

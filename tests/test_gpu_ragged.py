@@ -228,7 +228,8 @@ def test_prefill_one_to_three_k_steps(bits, g, k):
 @pytest.mark.parametrize("k,n,m", [(128, 301, 20), (640, 300, 64), (256, 17, 65), (384, 513, 130), (768, 301, 200), (1152, 255, 300)])
 def test_prefill_8_bit_words_handed_over_between_lanes(g, k, n, m):
     """64- and 128-row tiles at 8 bits ask for weights four lanes to a row and hand the words over an MFMA step ahead: one to nine K
-    steps (odd counts run one on zeros), columns past N repeating the last row, a value of every lane and word in its own place."""
+    steps (odd counts run one on zeros), columns past N repeating the last row, a value of every lane and word in its own place.  (These calls
+    get tiles of 64 x 256 and 128 x 192; 128 x 256 is forced in test_gpu_gemm_cols.py.)"""
     from bitween_amd.kernels import hip_loader
     lib = hip_loader.load()
     _, qw, s16, z16, b16 = quantized_layer(n, k, 8, g, seed=k + n + g, outliers=True)
