@@ -8,9 +8,9 @@ struct DgradRowsArgs {
     const void* scale;
     const void* zp;
     _Float16* gx;
-    float* ws;                                   // splits > 1: [splits][M][K] partial sums
+    float* ws;                                   // [splits][M][K] partial sums
     int M, N, K, ldg, ldx, groups, row_bytes;
-    int splits, steps_per_split;                 // slices of N, in steps of 32
+    int splits, steps_per_split;                 // slices of N (two and more), in steps of 32
     uint32_t go_bytes, w_bytes, meta_bytes;
 };
 

@@ -211,8 +211,7 @@ __global__ __launch_bounds__(64 * RW, (rows_waves<BITS, GROUP, DT, MT>)) void qd
             f4 v = red[at];
 #pragma unroll
             for (int w = 1; w < W; w++) v += red[w * 16 * PIECES + at];
-            if (a.splits > 1) *reinterpret_cast<f4*>(a.ws + ((int64_t)slice * a.M + m) * a.K + k) = v;
-            else *reinterpret_cast<u2*>(a.gx + (int64_t)m * a.ldx + k) = u2{round2<DT>(v[0], v[1]), round2<DT>(v[2], v[3])};
+            *reinterpret_cast<f4*>(a.ws + ((int64_t)slice * a.M + m) * a.K + k) = v;
         }
     }
 }
@@ -247,11 +246,8 @@ int launch_rows(const DgradRowsArgs& a, hipStream_t stream) {
     if (LDS > 64 * 1024 && !bw_allow_big_lds(reinterpret_cast<const void*>(kern), big_lds_devices)) return BW_ELAUNCH;
     hipLaunchKernelGGL(kern, dim3((unsigned)((a.K + RK - 1) / RK * a.splits)), dim3(64 * RW), LDS, stream, a);
     if (hipGetLastError() != hipSuccess) return BW_ELAUNCH;
-    if (a.splits > 1) {
-        hipLaunchKernelGGL(qdgrad_rows_reduce_kernel<DT>, dim3((unsigned)(((int64_t)a.M * (a.K / 4) + 255) / 256)), dim3(256), 0, stream, a.ws, a.gx, a.M, a.K, a.ldx, a.splits);
-        if (hipGetLastError() != hipSuccess) return BW_ELAUNCH;
-    }
-    return BW_OK;
+    hipLaunchKernelGGL(qdgrad_rows_reduce_kernel<DT>, dim3((unsigned)(((int64_t)a.M * (a.K / 4) + 255) / 256)), dim3(256), 0, stream, a.ws, a.gx, a.M, a.K, a.ldx, a.splits);
+    return hipGetLastError() == hipSuccess ? BW_OK : BW_ELAUNCH;
 }
 
 template <int BITS, int GROUP>

@@ -209,7 +209,7 @@ __global__ __launch_bounds__(WAVES * 64) void qgemm_kernel(const GemmArgs a) {
     // request for the scales of four steps) 51.2 -> 50.9.  Not at 4 and 2 bits, half as many requests: the handing over costs what it
     // saves (W4 g128 46.1 -> 47.3, g32 51.3 -> 52.1, W2 g128 45.8 -> 47.3); not with 256-row tiles, twice the MFMAs and no registers.
     constexpr bool QW = NAT && MT <= 8 && BITS == 8;
-    constexpr int PW = BITS == 8 ? 2 : 1;                        // QW: words of a tile an MFMA step multiplies
+    constexpr int PW = 2;                                        // QW: words of a tile an MFMA step multiplies
     constexpr uint32_t kOob = 0x80000000u;
     extern __shared__ __attribute__((aligned(16))) char smem[];
 #ifdef BW_TUNE
@@ -563,7 +563,7 @@ __global__ __launch_bounds__(WAVES * 64) void qgemm_kernel(const GemmArgs a) {
                 auto unpack_op = [&](auto vc) {
                     constexpr int v = decltype(vc)::value;
                     if constexpr (BITS == 4) {
-                        const uint32_t word = QW ? pw[cu][r][0] : word_of(src, r, tt, 0);
+                        const uint32_t word = word_of(src, r, tt, 0);
                         if constexpr (v == 0) pq[r][0] = __builtin_amdgcn_perm(word, word, 0x01000100u);
                         if constexpr (v == 1) pq[r][1] = __builtin_amdgcn_perm(word, word, 0x03020302u);
                         if constexpr (v == 2) up[r][0] = as_h2(and_or(pq[r][0], 0x00F0000Fu, kMagic));
@@ -576,7 +576,7 @@ __global__ __launch_bounds__(WAVES * 64) void qgemm_kernel(const GemmArgs a) {
                         if constexpr (v >= 12) wf[nx][r][v - 12] = up[r][v - 12] * gr.s;
                     } else if constexpr (BITS == 2) {
                         // half-word tt of the lane's 8 bytes
-                        const uint32_t word = QW ? pw[cu][r][0] : word_of(src, r, tt, 0);
+                        const uint32_t word = word_of(src, r, tt, 0);
                         if constexpr (v == 0) pq[r][0] = tt % 2 ? __builtin_amdgcn_perm(word, word, 0x03020302u) : __builtin_amdgcn_perm(word, word, 0x01000100u);
                         if constexpr (v == 1) uw[r] = pq[r][0] >> 8;
                         if constexpr (v == 2) up[r][0] = as_h2(and_or(pq[r][0], 0x000C0003u, kMagic));
@@ -587,7 +587,7 @@ __global__ __launch_bounds__(WAVES * 64) void qgemm_kernel(const GemmArgs a) {
                         if constexpr (v >= 10 && v < 14) wf[nx][r][v - 10] = up[r][v - 10] * gr.s;
                     } else {
                         // 8 bits: the two words of MFMA step tt are words 2 (tt % 2), + 1 of lane load tt / 2
-                        const uint32_t w0 = QW ? pw[cu][r][0] : word_of(src, r, tt, 0), w1 = QW ? pw[cu][r][PW - 1] : word_of(src, r, tt, 1);
+                        const uint32_t w0 = QW ? pw[cu][r][0] : word_of(src, r, tt, 0), w1 = QW ? pw[cu][r][1] : word_of(src, r, tt, 1);
                         if constexpr (v == 0) up[r][0] = as_h2(__builtin_amdgcn_perm(0x64646464u, w0, 0x04010400u));
                         if constexpr (v == 1) up[r][1] = as_h2(__builtin_amdgcn_perm(0x64646464u, w0, 0x04030402u));
                         if constexpr (v == 2) up[r][2] = as_h2(__builtin_amdgcn_perm(0x64646464u, w1, 0x04010400u));
