@@ -54,7 +54,7 @@ def build(verbose=False, tune=False):
     """Compile every source to an object file (in parallel, one hipcc per file), then link the shared library.
 
     tune=True also makes libbitween_hip_tune.so, the measurement build: the same library with the prefill kernel
-    compiled with -DBW_TUNE, which adds (1) kernel choices from the environment (BW_GEMM_NAT, BW_GEMM_BM,
+    compiled with -DBW_TUNE, which adds (1) kernel choices from the environment (BW_GEMM_NAT, BW_GEMM_BM, BW_GEMM_BN,
     BW_GEMM_PANEL) for same-process A/B runs and (2) bw_tune_clock_buffer(): workgroups 0..255 of a prefill launch leave
     the core-clock and real-time ticks of their K loop there, from which the shader clock under that kernel follows
     (bench.py --only prefill_clock).  The package never loads it."""

@@ -10,7 +10,7 @@
 //     requested ahead, 16 lanes to the 128 bytes (4 bits) of a row.  Scales and zero points of a step - two, four or eight groups of 32
 //     rows - come in 32 lanes to an array and are turned to [group][n] in the wave's own LDS.
 //   * What bounds it now: the unpack (28 vector instructions for 16 weights, pairs included) and the sums of the waves, 64 KB a workgroup for 16
-//     rows; 16 rows of 4096 <- 11008 take 11 us here and 3 in the reduction, of which the weights' way out of HBM is 3.5.
+//     rows; 16 rows of 4096 <- 11008 take 12.0 us here and 3.8 in the reduction (kernel trace; 14.2 as a graph), of which the weights' way out of HBM is 3.5.
 //   * The waves' sums meet in LDS, sixteen rows of m at a time; slices of N go through the caller's workspace and qdgrad_rows_reduce_kernel.
 #include "bw_qdgrad_rows.h"
 

@@ -109,7 +109,9 @@ inline float gemm_us(int64_t M, int64_t N, int64_t K, int bits, int group, GemmT
 // K steps, which it has too slow).  Finer tiles leave fewer CUs idle in a short round (4096 -> 11008 at 509 rows: 172 tiles of 128 x 256 on 256
 // CUs, 232 of 128 x 192; W4 g128 52.2 -> 46.7 us), their base is smaller, and a K step takes 0.86 of the time where CUs are idle and 0.73 on
 // a full chip, for 0.75 of the work.  8489 of the 11796 calls take 192 columns; all together they take 0.917 of the time, 16 of them over 5 %
-// more (K below 1024), and the best of the four tiles each time would save another 1 %.
+// more (K below 1024), and the best of the four tiles each time would save another 1 %.  Beyond the rows that the model is fitted to, half of the calls of
+// 2049 ... 8192 rows and a third of those up to 32768 take 192 columns: 13553 of them timed against the 256-column rule, 0.866 on average (0.872 up to 4096 rows,
+// 0.863 to 8192, 0.864 beyond), 24 over 5 % more, at most 1.17 (26142 rows of 11520 -> 672).
 inline GemmTile gemm_tile(int64_t M, int64_t N, int64_t K, int64_t ldx, int bits, int group, bool have_workspace, size_t workspace_bytes) {
     const GemmTile wide = gemm_tile_wide(M, N, K, ldx, bits, have_workspace, workspace_bytes);
     if (wide.rows == 64 || !gemm_nat(M, K, ldx)) return wide;

@@ -942,7 +942,8 @@ __global__ __launch_bounds__(256) void qgemm_reduce_kernel(const GemmArgs a) {
     }
 }
 
-// One workgroup fits per CU, so a grid runs in rounds of `cus` workgroups.  Two cases cut K:
+// A grid is counted in rounds of `cus` workgroups.  (One fits a CU with 256 rows and with 128 x 256; two do with 64 rows and, but for 8 bits in groups of 128
+// with wide requests for the scales, with 128 x 192.  What the second one gains is in the times that gemm_us is fitted to, not in this count.)  Two cases cut K:
 //   * a grid of at most half a round (small M * N, long K): every tile is split so that one round is filled;
 //   * a last round that is at most half full: its tiles are split so that it takes a fraction of a tile's time.
 // Never below 4 chunks per slice.  Without a workspace nothing is split.

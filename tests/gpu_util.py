@@ -30,7 +30,7 @@ def to_gpu(a):
 def check_matmul(y_gpu, x16, qw, s16, z16, b16, bits, g, tol_rel=1e-2):
     """Compare a float16 kernel result with the oracle.
 
-    Bars (written out as the north star asks):
+    Bars:
       * max |y - ref| / max |ref| <= 1e-2            (max relative error, fp32 accumulate)
       * mean |y - ref| / mean |ref| < 1e-2           (main.py:471-477)
       * elementwise: |y - y64| <= 2^-10 |y64| + 6 * 2^-11 * sqrt(x^2 @ (W16^2)^T) + 2e-6 * (|x| @ |W16|^T) + 1e-7:
