@@ -105,6 +105,12 @@ inline float gemm_us(int64_t M, int64_t N, int64_t K, int bits, int group, GemmT
     return us;
 }
 
+// rounds of a grid of tiles t, `per_cu` workgroups at once on every CU
+inline int64_t tile_rounds(int64_t M, int64_t N, GemmTile t, int per_cu) {
+    const int64_t tiles = ((M + t.rows - 1) / t.rows) * ((N + t.cols - 1) / t.cols), places = (int64_t)per_cu * bw_device_cus();
+    return (tiles + places - 1) / places;
+}
+
 // Tile for this call: 192 columns where the model above is ahead of the 256-column tile's by 5 % (10 % of a 256-row tile on less than eight
 // K steps, which it has too slow).  Finer tiles leave fewer CUs idle in a short round (4096 -> 11008 at 509 rows: 172 tiles of 128 x 256 on 256
 // CUs, 232 of 128 x 192; W4 g128 52.2 -> 46.7 us), their base is smaller, and a K step takes 0.86 of the time where CUs are idle and 0.73 on
@@ -129,6 +135,11 @@ inline GemmTile gemm_tile(int64_t M, int64_t N, int64_t K, int64_t ldx, int bits
             const GemmTile narrow = {rows, tile_cols(3)};
             // (no plan that bw_qgemm_static could not run: its results are bw_qgemm_ws's bit for bit)
             if (have_workspace && gemm_plan(M, N, nchunks, true, rows, narrow.cols).ws_bytes > kScratchBytes) continue;
+            // Three and four K steps: the model has one round of 256 x 256 tiles too slow beside 128 x 192 tiles that need a second one of two workgroups a CU (10257
+            // calls of 129 ... 2048 rows with K = 128 ... 640, each with the four tiles: at K = 384 42 of 46 such calls took longer, 1.06 on average, up to 1.14; rows of y
+            // off 16 bytes make 256 columns the slower ones all the same).  One and two steps are left: 46 of 4355 calls over 2 % longer than with 256 columns, up
+            // to 1.17, 0.871 of the time on average; this line would help 17 of them and cost 24 others as much.
+            if ((nchunks == 3 || nchunks == 4) && rows == 128 && wide.rows == 256 && N % 8 == 0 && tile_rounds(M, N, wide, 1) == 1 && tile_rounds(M, N, narrow, 2) > 1) continue;
             const float t = gemm_us(M, N, K, bits, group, narrow, have_workspace);
             if (t < us) { b = narrow; us = t; }
         }

@@ -207,7 +207,9 @@ __global__ __launch_bounds__(WAVES * 64) void qgemm_kernel(const GemmArgs a) {
     // a 128-row tile take, next to 512 for x and, at groups of 32, 512 for the scales; now 512.  us, out of HBM: W8 g32 4096 -> 11008 at 64 / 333 /
     // 509 rows 26.2 -> 24.5, 57.8 -> 53.5, 59.5 -> 55.1, 11008 -> 4096 at 509 60.7 -> 58.7; g64 4096 -> 11008 at 509 59.6 -> 56.5; g128 (one
     // request for the scales of four steps) 51.2 -> 50.9.  Not at 4 and 2 bits, half as many requests: the handing over costs what it
-    // saves (W4 g128 46.1 -> 47.3, g32 51.3 -> 52.1, W2 g128 45.8 -> 47.3); not with 256-row tiles, twice the MFMAs and no registers.
+    // saves (W4 g128 46.1 -> 47.3, g32 51.3 -> 52.1, W2 g128 45.8 -> 47.3); not with 256-row tiles, twice the MFMAs and no registers. A layer of up
+    // to 192 columns leaves waves of its one tile without weights and has nothing to save: 65 ... 128 rows of 64 ... 128 columns, K uncut, take 1.08 of the time (at most 1.15), 193
+    // ... 256 columns 0.94, wider ones 0.80 ... 0.91.
     constexpr bool QW = NAT && MT <= 8 && BITS == 8;
     constexpr int PW = 2;                                        // QW: words of a tile an MFMA step multiplies
     constexpr uint32_t kOob = 0x80000000u;
