@@ -283,11 +283,16 @@ extern "C" size_t bw_qgemm_workspace_bytes(int64_t M, int64_t N, int64_t K, int 
     return chosen > need ? chosen : need;
 }
 
-// Least workspace with which bw_qgemm_ws runs this shape cut along K (0 = not at all, or only with the tile of bw_qgemm_workspace_bytes): below what
-// that asks for, the tiles of 256 columns take over.
-size_t bw_qgemm_least_workspace_bytes(int64_t M, int64_t N, int64_t K, int bits, int group) {
-    if (!bw_shape_ok(N, K, bits, group) || M < 1 || M >= ((int64_t)1 << 31) || !bw_fast_shape(M, N, K, K, bits, group)) return 0;
-    return gemm_wide_ws_bytes(M, N, K, bits);
+// Whether a workspace smaller than bw_qgemm_workspace_bytes asks for is worth passing on: it has room for the plan of the 256-column tiles, which
+// bw_qgemm_ws then runs, and that is expected to be done before the best of the uncut plans is.
+bool bw_qgemm_small_workspace_serves(int64_t M, int64_t N, int64_t K, int bits, int group, size_t workspace_bytes) {
+    if (!bw_shape_ok(N, K, bits, group) || M < 1 || M >= ((int64_t)1 << 31) || !bw_fast_shape(M, N, K, K, bits, group)) return false;
+    const size_t least = gemm_wide_ws_bytes(M, N, K, bits);
+    if (!least || workspace_bytes < least) return false;
+    if (!gemm_nat(M, K, K)) return true;
+    const GemmTile cut = gemm_tile_wide(M, N, K, K, bits, true, workspace_bytes), uncut = gemm_tile(M, N, K, K, bits, group, false, 0);
+    if (cut.rows == 64 || uncut.rows == 64) return true;
+    return gemm_us(M, N, K, bits, group, cut, true) <= gemm_us(M, N, K, bits, group, uncut, false);
 }
 
 extern "C" int bw_qgemm_tile_rows(int64_t M, int64_t N, int64_t K, int bits, int group) {

@@ -166,14 +166,17 @@ def test_the_librarys_own_array_runs_the_same_plan(m, n, k):
     assert st == 0 and torch.equal(y, z)
 
 
-@pytest.mark.parametrize("m,n,k,bits,g", [(214, 11232, 2944, 4, 128), (198, 11184, 3072, 4, 64), (210, 11184, 3200, 8, 32)])
+@pytest.mark.parametrize("m,n,k,bits,g,cuts", [(1287, 2000, 6016, 4, 128, True), (98, 9472, 6272, 8, 32, True), (339, 7376, 2688, 4, 64, False),
+                                                  (227, 11728, 2688, 4, 64, False)])
 @pytest.mark.parametrize("dtype", [torch.float16, torch.bfloat16])
-def test_a_smaller_workspace_still_cuts_k(m, n, k, bits, g, dtype):
-    """bw_qlinear_ws with 16 bytes less than the chosen plan of 192-column tiles asks for: the cut plan of the 256-column tiles runs, bit for bit
-    bw_qgemm_ws's, and not the uncut one (which leaves the workspace alone)."""
+def test_a_workspace_smaller_than_asked_for(m, n, k, bits, g, cuts, dtype):
+    """bw_qlinear_ws with 16 bytes less than the chosen plan of 192-column tiles asks for: the cut plan of the 256-column tiles runs where it is expected to
+    be done before the uncut ones (then bit for bit bw_qgemm_ws's), else the uncut one, which leaves the workspace alone."""
     import bitween_amd
     from bitween_amd.kernels import hip_loader
     lib = hip_loader.load()
+    if torch.cuda.get_device_properties(0).multi_processor_count != 256:
+        pytest.skip("the plans depend on the number of compute units")
     torch.manual_seed(k)
     q = bitween_amd.QuantizedLinear.from_float(torch.nn.Linear(k, n, bias=True, device="cuda", dtype=torch.float16), bits, g)
     x = torch.randn(m, k, device="cuda").to(dtype)
@@ -187,7 +190,10 @@ def test_a_smaller_workspace_still_cuts_k(m, n, k, bits, g, dtype):
     ws, other = (torch.full((full,), 85, dtype=torch.uint8, device="cuda") for _ in range(2))
     assert lib.bw_qlinear_ws(x.data_ptr(), bf16, m, k, k, *args, n, bits, g, y.data_ptr(), n, ws.data_ptr(), full - 16, st) == 0
     x16 = x.half()
-    assert lib.bw_qgemm_ws(x16.data_ptr(), 0, m, k, k, *args, n, bits, g, z.data_ptr(), n, other.data_ptr(), full - cast - 16, st) == 0
+    assert lib.bw_qgemm_ws(x16.data_ptr(), 0, m, k, k, *args, n, bits, g, z.data_ptr(), n, other.data_ptr() if cuts else None, full - cast - 16 if cuts else 0, st) == 0
     torch.cuda.synchronize()
     assert torch.equal(y, z) and (ws[full - 16:] == 85).all()
-    assert not (ws[cast:cast + 65536] == 85).all(), "the cut needs its partial sums in the workspace"
+    assert (ws[cast:] == 85).all().item() != cuts
+    cols = np.unique(np.linspace(0, n - 1, 60).astype(int))
+    part = [t[torch.from_numpy(cols).cuda()].cpu().numpy() for t in (q.qweight, q.scale, q.zero_point, q.bias)]
+    check_matmul(y[:, torch.from_numpy(cols).cuda()], x16.cpu().numpy(), *part, bits, g)
