@@ -164,7 +164,7 @@ int bw_qlinear_decode_rows(int64_t N, int64_t K, int bits);
  * across workgroups and beyond bw_qlinear_decode_rows (up to 2048 rows while it is expected to be done before the prefill kernel),
  * the split-K plans of the prefill kernel, and BW_BF16 x for every M (cast into the workspace where the prefill kernel runs).
  * `workspace` (16-byte aligned) holds at least bw_qlinear_workspace_bytes(...) bytes (0 = none needed); with less, plans that
- * need it are not used: BW_BF16 x without room for its cast runs on the batch kernel, and returns BW_EWORKSPACE where that does
+ * need it are not used (the prefill kernel takes what there is for a smaller plan where that is expected to pay): BW_BF16 x without room for its cast runs on the batch kernel, and returns BW_EWORKSPACE where that does
  * not take the call either (beyond 2048 rows, other shapes and layouts than its). */
 size_t bw_qlinear_workspace_bytes(int64_t M, int64_t N, int64_t K, int bits, int group, int act_dtype);
 
