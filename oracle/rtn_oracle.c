@@ -1,6 +1,6 @@
 /* Scalar C restatement of Bitween's quantized-linear hot path.
  *
- * TEST INFRASTRUCTURE ONLY: the checker the HIP kernels are compared with and
+ * TEST INFRASTRUCTURE ONLY: the oracle the HIP kernels are compared with and
  * the CPU baseline that bench.py times.  Nothing in the shipped library links
  * or loads this file.
  *

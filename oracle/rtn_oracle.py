@@ -1,6 +1,6 @@
 """CPU restatement (numpy) of Bitween's quantized-linear hot path.
 
-TEST INFRASTRUCTURE ONLY.  This module is the checker that the HIP kernels are
+TEST INFRASTRUCTURE ONLY.  This module is the oracle that the HIP kernels are
 compared against; nothing in the shipped package imports it.  Only tests/,
 __graft_entry__.smoke() and bench.py's cpu_baseline leg may use it.
 
@@ -84,7 +84,7 @@ def quantize_rtn(weight, bits=8, group_size=32, math="f32", scale_div="ieee"):
     carried out.  "ieee" = a correctly rounded division, what eager torch does
     on the CPU.  "reciprocal" = what eager torch does on a GPU for a scalar
     divisor: a multiplication by float32(1) / float32(Qmax), the product
-    rounded to float32 and then to the tensor's type (pinned on the GPU box
+    rounded to float32 and then to the tensor's type (pinned on a GPU
     against torch itself, tests/test_gpu_eager_torch.py, and by exact-rational
     vectors).
 

@@ -1,9 +1,9 @@
-"""The reference's CPU path, restated in eager torch ops (TEST INFRASTRUCTURE: checker and timed CPU baseline).
+"""The reference's CPU path, restated in eager torch ops (TEST INFRASTRUCTURE: oracle and timed CPU baseline).
 
 Only tests/, __graft_entry__.smoke() and bench.py's cpu_baseline leg may use this module; nothing in the
-shipped package imports it.  It exists because the reference's own files do not travel to the GPU box: this
+shipped package imports it.  It exists because the reference's own files are not there where the benchmark runs: this
 is the same sequence of eager torch operations, written out from the reference lines cited per function
-(paths relative to the reference checkout), so that timing it on the box's host cores times what the
+(paths relative to the reference checkout), so that timing it on that machine's host cores times what the
 reference would execute there:
 
     quantize_rtn     bitween/functional.py:3-45
